@@ -22,6 +22,7 @@ namespace {
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
 
 thread_local std::string g_err;
 
@@ -165,154 +166,399 @@ __global__ __launch_bounds__(256) void conv_fwd(const uint16_t* __restrict__ x, 
     }
 }
 
-// Forward convolution with the input staged in LDS (Cin a multiple of 32).
-// A workgroup owns an output block of WR*2 image rows x 32 columns of one
-// image and WN*WC*16 output channels (WN = 4 / WR).  Per chunk of 32 input
-// channels it stages the block's input halo - (WR*2 + 2) rows x 34 columns
-// x 32 channels, zeros outside the image, the ReLU mask of xm applied on
-// load - in LDS, each pixel padded to 40 channels (80 bytes: the 16 lanes
-// of one MFMA row read 16 different bank groups), and every tap's A
-// fragments are 16-byte LDS reads at the shifted pixel.  Wave (wr, wn)
-// computes rows 2wr, 2wr+1 (four 16-pixel tiles) x WC channel tiles; its B
-// fragments (weights) are 16-byte global loads that the L1 shares between
-// the waves and workgroups using the same channels.  The next chunk's halo
-// is loaded into registers while the current one is consumed (two LDS
-// buffers, one barrier per chunk).
-constexpr int kHaloC = 40;   // padded channels per staged pixel
-constexpr int kHaloW = 34;   // 32 columns + one either side
+// Buffer access to one image or to the weights: a descriptor of `bytes`
+// bytes; a load at kOOB (any offset past the end) returns zeros without a
+// memory access, which is the convolution's zero padding.
+using rsrc_t = __amdgpu_buffer_rsrc_t;
+constexpr unsigned kOOB = 0x7FFFFF00u;
+constexpr int64_t kMaxBytes = (int64_t)0x7FFFFE00;  // of one descriptor
 
-template <int WR, int WC, bool MASK>
-__global__ __launch_bounds__(256) void conv_fwd_lds(const uint16_t* __restrict__ x, const uint16_t* __restrict__ xm,
-                                                    const uint16_t* __restrict__ w, const float* __restrict__ bias,
-                                                    float* __restrict__ y32, uint16_t* __restrict__ y16, int N, int H,
-                                                    int W, int Cin, int Cout, int relu) {
-    constexpr int WN = 4 / WR;
-    constexpr int BR = 2 * WR;                    // output rows of the block
-    constexpr int HR = BR + 2;                    // halo rows
-    constexpr int HP = HR * kHaloW;               // halo pixels
-    constexpr int PIECES = HP * 4;                // 16-byte pieces (8 channels) per chunk
-    constexpr int PPT = (PIECES + 255) / 256;     // pieces per thread
-    __shared__ __align__(16) uint16_t halo[2][HP * kHaloC];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wr = wave % WR, wn = wave / WR;
-    const int wblocks = (W + 31) / 32, hblocks = (H + BR - 1) / BR;
-    // logical workgroup = tile x channel block, channel blocks adjacent
-    const int ncb = (Cout + WN * WC * 16 - 1) / (WN * WC * 16);
-    const int L = xcd_band();
-    int b = L / ncb;
-    const int cb = L - b * ncb;
-    const int bw = b % wblocks;
-    b /= wblocks;
-    const int bh = b % hblocks;
-    const int n = b / hblocks;
-    const int h0 = bh * BR, w0 = bw * 32;
-    const int co0 = cb * (WN * WC * 16) + wn * (WC * 16);
-    const int K = 9 * Cin;
-    const int64_t img = (int64_t)n * H;
+__device__ __forceinline__ rsrc_t make_rsrc(const void* p, int64_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ u4v load16(rsrc_t r, unsigned voff, unsigned soff) {
+    return __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
+}
 
-    // staging: piece q = pixel q / 4 of the halo, channels 8 * (q % 4)
-    auto fetch = [&](int ci0, u4v v[PPT]) {
+__device__ __forceinline__ void store16(rsrc_t r, unsigned voff, u4v v) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)voff, 0, 0);
+}
+__device__ __forceinline__ void store8(rsrc_t r, unsigned voff, u2v v) {
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, (int)voff, 0, 0);
+}
+
+// Tile geometry shared by the two staged convolution kernels below: four
+// waves, WP of them stacked over pixel rows and 4 / WP side by side over
+// output channels; a wave computes R rows x 16 CT columns x 16 WC output
+// channels.  The weights are the MFMA's A operand (rows = output channels)
+// and the pixels its B operand, so a lane's results are output channels of
+// one pixel.  With WC even, row i of tile t of a pair holds channel
+// 8 (i / 4) + 4 (t mod 2) + i mod 4 of the pair's 32, and the lane holds
+// eight consecutive channels: one 16-byte store (bf16).  Scattered 2-byte
+// stores of the transposed assignment had cost the thin layers as much as
+// their MFMAs.
+template <int R, int CT, int WC, int WP>
+struct Tile {
+    static constexpr int WN = 4 / WP;
+    static constexpr int BR = WP * R;          // output rows of the block
+    static constexpr int BW = 16 * CT;         // output columns
+    static constexpr int BC = WN * WC * 16;    // output channels
+    static constexpr int HW = BW + 2;          // halo columns
+    static constexpr int HP = (BR + 2) * HW;   // halo pixels
+    // LDS row (A row) of the block's output channel c
+    static __device__ __forceinline__ int wrow(int c) {
+        if (WC % 2) return c;
+        return (c & ~31) + 16 * ((c >> 2) & 1) + 4 * ((c >> 3) & 3) + (c & 3);
+    }
+};
+
+struct ConvArgs {
+    const uint16_t* x;
+    const uint16_t* xm;   // ReLU mask of x applied on load (MASK)
+    const uint16_t* w;
+    const float* bias;
+    float* y32;
+    uint16_t* y16;
+    int N, H, W, Cin, Cout, relu;
+    int hb, wb;           // blocks of an image
+    int npx, ncb;         // pixel blocks in all, channel blocks
+};
+
+// Results of one wave's tile at rows h0.., columns w0.. and the block's
+// channels c0.. (co0 + c0 of the layer).  The stores are predicated by
+// offset, without a branch, and the bias comes from LDS: a branch, or a
+// load of its own here, makes the wait for the next block's prefetched
+// halo cover these stores, or these results wait for that halo.
+template <int R, int CT, int WC, bool OUT32>
+__device__ __forceinline__ void store_tile(const ConvArgs& a, const v4f (&acc)[R][CT][WC], const float* sbias, int n,
+                                           int h0, int w0, int co0, int c0) {
+    const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
+    constexpr int V = (WC % 2) ? 4 : 8;        // consecutive channels of a lane
+    constexpr int G = (WC % 2) ? WC : WC / 2;
+    constexpr int ES = OUT32 ? 4 : 2;
+    const int64_t img = (int64_t)a.H * a.W * a.Cout * ES;
+    const rsrc_t yr = make_rsrc(OUT32 ? (char*)a.y32 + n * img : (char*)a.y16 + n * img, img);
 #pragma unroll
-        for (int j = 0; j < PPT; ++j) {
-            const int q = threadIdx.x + 256 * j;
-            v[j] = u4v{0u, 0u, 0u, 0u};
-            if (q < PIECES) {
-                const int px = q >> 2, g = q & 3;
-                const int hh = h0 - 1 + px / kHaloW, ww = w0 - 1 + px % kHaloW;
-                if (hh >= 0 && hh < H && ww >= 0 && ww < W) {
-                    const int64_t o = ((img + hh) * W + ww) * Cin + ci0 + 8 * g;
-                    v[j] = *reinterpret_cast<const u4v*>(x + o);
-                    if (MASK) v[j] = relu_keep(v[j], *reinterpret_cast<const u4v*>(xm + o));
+    for (int u = 0; u < G; ++u) {
+        const int c = c0 + (V == 8 ? 32 : 16) * u + V * q, co = co0 + c;
+        float b[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) b[e] = sbias[c + e];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int k = 0; k < CT; ++k) {
+                const int h = h0 + r, w = w0 + 16 * k + j;
+                const bool in = h < a.H && w < a.W && co < a.Cout;
+                const unsigned o = in ? (unsigned)(((h * a.W + w) * a.Cout + co) * ES) : kOOB;
+                float v[V];
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    v[e] = acc[r][k][V == 8 ? 2 * u + (e >> 2) : u][e & 3] + b[e];
+                    if (a.relu) v[e] = fmaxf(v[e], 0.f);
+                }
+                if constexpr (OUT32) {
+#pragma unroll
+                    for (int e = 0; e < V; e += 4) store16(yr, o + 4 * e, __builtin_bit_cast(u4v, v4f{v[e], v[e + 1], v[e + 2], v[e + 3]}));
+                } else {
+                    unsigned p[V / 2];
+#pragma unroll
+                    for (int e = 0; e < V; e += 2)
+                        p[e / 2] = (unsigned)to_bf16(v[e]) | ((unsigned)to_bf16(v[e + 1]) << 16);
+                    if constexpr (V == 8)
+                        store16(yr, o, u4v{p[0], p[1], p[2], p[3]});
+                    else
+                        store8(yr, o, u2v{p[0], p[1]});
                 }
             }
-        }
-    };
-    auto stage = [&](int buf, const u4v v[PPT]) {
-#pragma unroll
-        for (int j = 0; j < PPT; ++j) {
-            const int q = threadIdx.x + 256 * j;
-            if (q < PIECES)
-                *reinterpret_cast<u4v*>(&halo[buf][(q >> 2) * kHaloC + 8 * (q & 3)]) = v[j];
-        }
-    };
-
-    v4f acc[4][WC];
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int t = 0; t < WC; ++t) acc[m][t] = v4f{0.f, 0.f, 0.f, 0.f};
-
-    u4v nxt[PPT];
-    fetch(0, nxt);
-    stage(0, nxt);
-    __syncthreads();
-    const int nchunks = Cin / 32;
-    for (int c = 0; c < nchunks; ++c) {
-        const int buf = c & 1;
-        if (c + 1 < nchunks) fetch(32 * (c + 1), nxt);
-        const uint16_t* hb = halo[buf];
-        // fragments of tap t + 1 are loaded while tap t's MFMAs run
-        auto load_b = [&](int tap, u4v bv[WC]) {
-            const int k0 = tap * Cin + 32 * c + 8 * (lane >> 4);
-#pragma unroll
-            for (int t = 0; t < WC; ++t) {
-                const int co = co0 + 16 * t + (lane & 15);
-                bv[t] = co < Cout ? *reinterpret_cast<const u4v*>(w + (int64_t)co * K + k0) : u4v{0u, 0u, 0u, 0u};
-            }
-        };
-        auto load_a = [&](int tap, u4v av[4]) {
-            const int dh = tap / 3, dw = tap % 3;     // halo offsets (0..2)
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                // tile m: block row 2 wr + m / 2, columns 16 (m % 2) .. + 15
-                const int hr = 2 * wr + (m >> 1) + dh;
-                const int hc = 16 * (m & 1) + (lane & 15) + dw;
-                av[m] = *reinterpret_cast<const u4v*>(&hb[(hr * kHaloW + hc) * kHaloC + 8 * (lane >> 4)]);
-            }
-        };
-        u4v bv[WC], av[4], bn[WC], an[4];
-        load_b(0, bv);
-        load_a(0, av);
-#pragma unroll 1
-        for (int tap = 0; tap < 9; ++tap) {
-            if (tap < 8) {
-                load_b(tap + 1, bn);
-                load_a(tap + 1, an);
-            }
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-#pragma unroll
-                for (int t = 0; t < WC; ++t)
-                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf8(av[m]), bf8(bv[t]), acc[m][t], 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < WC; ++t) bv[t] = bn[t];
-#pragma unroll
-            for (int m = 0; m < 4; ++m) av[m] = an[m];
-        }
-        if (c + 1 < nchunks) {
-            stage(buf ^ 1, nxt);
-            __syncthreads();
-        }
     }
+}
+
+// The block of index t: with one chunk of input channels the channel block
+// is the slow index (a workgroup's run of blocks keeps its weights in LDS),
+// else the fast one (the channel blocks of a pixel block share its halo
+// through L2).
+struct BlockPos {
+    int n, h0, w0, cb;
+};
+__device__ __forceinline__ BlockPos block_pos(const ConvArgs& a, int t, bool cb_slow, int BR, int BW) {
+    BlockPos p;
+    int px;
+    if (cb_slow) {
+        p.cb = t / a.npx;
+        px = t - p.cb * a.npx;
+    } else {
+        px = t / a.ncb;
+        p.cb = t - px * a.ncb;
+    }
+    const int row = px / a.wb;
+    p.w0 = (px - row * a.wb) * BW;
+    p.n = row / a.hb;
+    p.h0 = (row - p.n * a.hb) * BR;
+    return p;
+}
+
+// Convolution with input and weights staged in LDS, Cin a multiple of 32.
+// A workgroup walks a contiguous run of blocks.  Per block and chunk of 32
+// input channels it holds in LDS the block's input halo (zeros outside the
+// image) and the nine taps' weights, 64 bytes per pixel or channel, the
+// four 16-byte pieces of row p stored at piece ^ ((p / 2) mod 4): the
+// fragment reads of eight consecutive rows then cover all 32 banks.  The
+// next halo is loaded into registers while this one's MFMAs run (with PFW
+// the weights too); with one chunk the weights stay for the whole run.
+//
+// Bounds: the MFMA needs a fragment (1 KB of LDS reads) per two of its
+// 16-cycle issues at most; R = 4, CT = 2, WC = 4 reads 12 fragments per 32
+// MFMAs.  The kernel before this one took its weight fragments from global
+// memory, 16 rows of 64 bytes per load instruction with consecutive lanes
+// in different rows, four times the tag lookups of a contiguous load.
+// K order per output: chunk, tap, channel (as that kernel's).
+template <int R, int CT, int WC, int WP, int PF, bool MASK, bool OUT32>
+__global__ __launch_bounds__(256, 2) void conv_tile(ConvArgs a) {
+    using T = Tile<R, CT, WC, WP>;
+    constexpr int HPC = T::HP * 4;                 // 16-byte pieces of the halo
+    constexpr int PPT = (HPC + 255) / 256;
+    constexpr int WPC = 9 * T::BC * 4;             // of the weights
+    constexpr int WPT = (WPC + 255) / 256;
+    __shared__ __align__(16) u4v halo[HPC];
+    __shared__ __align__(16) u4v wlds[WPC];
+    __shared__ float sbias[T::BC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wr = wave % WP, wn = wave / WP;
+    const int j = lane & 15, q = lane >> 4;
+    const int nchunks = a.Cin / 32;
+    const int total = a.npx * a.ncb, G = (int)gridDim.x;
+    const int L = xcd_band();
+    const int tbeg = (int)((int64_t)total * L / G), tend = (int)((int64_t)total * (L + 1) / G);
+    if (tbeg >= tend) return;
+    const int64_t img_bytes = (int64_t)a.H * a.W * a.Cin * 2;
+    const int wbytes = a.Cout * 9 * a.Cin * 2;
+    const rsrc_t wres = make_rsrc(a.w, wbytes);
+    const rsrc_t bres = make_rsrc(a.bias, a.bias ? a.Cout * 4 : 0);
+    const int krow = 9 * a.Cin * 2;
+
+    u4v hv[PPT], mv[MASK ? PPT : 1], wv[PF == 2 ? WPT : 1];
+    auto fetch_halo = [&](const BlockPos& p, int c) {
+        const rsrc_t xr = make_rsrc(a.x + p.n * (img_bytes / 2), img_bytes);
+        const rsrc_t mr = make_rsrc(MASK ? a.xm + p.n * (img_bytes / 2) : a.x, MASK ? img_bytes : 0);
 #pragma unroll
-    for (int t = 0; t < WC; ++t) {
-        const int co = co0 + 16 * t + (lane & 15);
-        if (co >= Cout) continue;
-        const float bb = bias ? bias[co] : 0.f;
+        for (int i = 0; i < PPT; ++i) {
+            const int s = tid + 256 * i, px = s >> 2, g = s & 3;
+            const int hr = px / T::HW, hc = px - hr * T::HW;
+            const int hh = p.h0 - 1 + hr, ww = p.w0 - 1 + hc;
+            const bool in = s < HPC && (unsigned)hh < (unsigned)a.H && (unsigned)ww < (unsigned)a.W;
+            const unsigned vo = in ? (unsigned)(((hh * a.W + ww) * a.Cin + 8 * g) * 2) : kOOB;
+            hv[i] = load16(xr, vo, 64 * c);
+            if (MASK) mv[i] = load16(mr, vo, 64 * c);
+        }
+    };
+    auto stage_halo = [&]() {
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const int h = h0 + 2 * wr + (m >> 1);
+        for (int i = 0; i < PPT; ++i) {
+            const int s = tid + 256 * i, px = s >> 2, g = s & 3;
+            const int hr = px / T::HW, hc = px - hr * T::HW;
+            if (s < HPC) halo[px * 4 + (g ^ ((hc >> 1) & 3))] = MASK ? relu_keep(hv[i], mv[i]) : hv[i];
+        }
+    };
+    auto fetch_w = [&](int i, int cb, int c) {
+        const int s = tid + 256 * i, tap = s / (T::BC * 4), rem = s - tap * (T::BC * 4), co = rem >> 2, g = rem & 3;
+        const bool in = s < WPC && cb * T::BC + co < a.Cout;
+        return load16(wres, in ? (unsigned)((cb * T::BC + co) * krow + (tap * a.Cin + 8 * g) * 2) : kOOB, 64 * c);
+    };
+    auto stage_w = [&](int i, const u4v& v) {
+        const int s = tid + 256 * i, tap = s / (T::BC * 4), rem = s - tap * (T::BC * 4), co = rem >> 2, g = rem & 3;
+        const int row = T::wrow(co);
+        if (s < WPC) wlds[(tap * T::BC + row) * 4 + (g ^ ((row >> 1) & 3))] = v;
+    };
+
+    BlockPos p = block_pos(a, tbeg, nchunks == 1, T::BR, T::BW);
+    int t = tbeg, c = 0, wcb = -1;  // wcb: channel block whose only chunk is staged
+    if (PF) fetch_halo(p, 0);
+    if (PF == 2) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int wc = w0 + 16 * (m & 1) + 4 * (lane >> 4) + r;
-                if (h >= H || wc >= W) continue;
-                const int64_t p = (img + h) * W + wc;
-                float v = acc[m][t][r] + bb;
-                if (relu) v = fmaxf(v, 0.f);
-                if (y32) y32[p * Cout + co] = v;
-                if (y16) y16[p * Cout + co] = to_bf16(v);
+        for (int i = 0; i < WPT; ++i) wv[i] = fetch_w(i, p.cb, 0);
+    }
+    v4f acc[R][CT][WC];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int k = 0; k < CT; ++k)
+#pragma unroll
+            for (int u = 0; u < WC; ++u) acc[r][k][u] = v4f{0.f, 0.f, 0.f, 0.f};
+    // fragment addresses (in 16-byte pieces): pixel row wr R, column j + dw;
+    // rows, column tiles and taps are constant offsets from them
+    int pa[3];
+#pragma unroll
+    for (int dw = 0; dw < 3; ++dw) pa[dw] = (wr * R * T::HW + j + dw) * 4 + (q ^ (((j + dw) >> 1) & 3));
+    const int wa = (wn * WC * 16 + j) * 4 + (q ^ ((j >> 1) & 3));
+
+    for (;;) {
+        if (!PF) fetch_halo(p, c);
+        __syncthreads();  // the previous chunk's fragments have been read
+        stage_halo();
+        if (wcb != p.cb) {
+            if (tid < T::BC && c == 0)
+                sbias[tid] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(bres, (p.cb * T::BC + tid) * 4, 0, 0));
+            if (PF == 2) {
+#pragma unroll
+                for (int i = 0; i < WPT; ++i) stage_w(i, wv[i]);
+            } else {
+                u4v v[WPT];
+#pragma unroll
+                for (int i = 0; i < WPT; ++i) v[i] = fetch_w(i, p.cb, c);
+#pragma unroll
+                for (int i = 0; i < WPT; ++i) stage_w(i, v[i]);
+            }
+            wcb = nchunks == 1 ? p.cb : -1;
+        }
+        __syncthreads();
+        // the next chunk (of this block or of the next one)
+        const bool last = c + 1 == nchunks;
+        const int tn = last ? t + 1 : t, cn = last ? 0 : c + 1;
+        BlockPos pn = p;
+        if (last && tn < tend) pn = block_pos(a, tn, nchunks == 1, T::BR, T::BW);
+        if (PF && tn < tend) {
+            fetch_halo(pn, cn);
+            if (PF == 2 && wcb != pn.cb) {
+#pragma unroll
+                for (int i = 0; i < WPT; ++i) wv[i] = fetch_w(i, pn.cb, cn);
             }
         }
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) {
+            v8bf wf[WC];
+#pragma unroll
+            for (int u = 0; u < WC; ++u) wf[u] = bf8(wlds[wa + (tap * T::BC + 16 * u) * 4]);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int k = 0; k < CT; ++k) {
+                    const v8bf pf = bf8(halo[pa[tap % 3] + ((r + tap / 3) * T::HW + 16 * k) * 4]);
+#pragma unroll
+                    for (int u = 0; u < WC; ++u)
+                        acc[r][k][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], pf, acc[r][k][u], 0, 0, 0);
+                }
+        }
+        if (last) {
+            store_tile<R, CT, WC, OUT32>(a, acc, sbias, p.n, p.h0 + wr * R, p.w0, p.cb * T::BC, wn * WC * 16);
+            if (tn >= tend) break;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int k = 0; k < CT; ++k)
+#pragma unroll
+                    for (int u = 0; u < WC; ++u) acc[r][k][u] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
+        t = tn;
+        c = cn;
+        p = pn;
+    }
+}
+
+// The same for few input channels (Cin = 8 CG, 1 <= CG <= 7): the K index
+// k = tap Cin + ci runs over all nine taps in steps of 32, so a lane's
+// eight values are channels of tap k / Cin of its pixel; all channels of
+// the halo are staged at once, CG pieces per pixel (one more when CG is
+// even: an odd stride in 16-byte pieces spreads the banks), and the whole
+// weight rows, zero-padded to whole steps.
+template <int R, int CT, int WC, int CG, bool MASK, bool OUT32>
+__global__ __launch_bounds__(256, 2) void conv_tile_thin(ConvArgs a) {
+    using T = Tile<R, CT, WC, 4>;
+    constexpr int Cin = 8 * CG, K = 9 * Cin;
+    constexpr int S = (K + 31) / 32;               // MFMA steps
+    constexpr int PS = CG | 1;                     // pieces per staged pixel
+    constexpr int WS = 4 * S + 1;                  // pieces per staged weight row
+    constexpr int HPC = T::HP * CG, PPT = (HPC + 255) / 256;
+    constexpr int WPC = T::BC * 4 * S;
+    __shared__ __align__(16) u4v halo[T::HP * PS];
+    __shared__ __align__(16) u4v wlds[T::BC * WS];
+    __shared__ float sbias[T::BC];
+    const int tid = threadIdx.x, lane = tid & 63, wr = tid >> 6;
+    const int j = lane & 15, q = lane >> 4;
+    const int total = a.npx * a.ncb, G = (int)gridDim.x;
+    const int L = xcd_band();
+    const int tbeg = (int)((int64_t)total * L / G), tend = (int)((int64_t)total * (L + 1) / G);
+    if (tbeg >= tend) return;
+    const int64_t img_bytes = (int64_t)a.H * a.W * Cin * 2;
+    const rsrc_t wres = make_rsrc(a.w, (int64_t)a.Cout * K * 2);
+    const rsrc_t bres = make_rsrc(a.bias, a.bias ? a.Cout * 4 : 0);
+
+    u4v hv[PPT], mv[MASK ? PPT : 1];
+    auto fetch_halo = [&](const BlockPos& p) {
+        const rsrc_t xr = make_rsrc(a.x + p.n * (img_bytes / 2), img_bytes);
+        const rsrc_t mr = make_rsrc(MASK ? a.xm + p.n * (img_bytes / 2) : a.x, MASK ? img_bytes : 0);
+#pragma unroll
+        for (int i = 0; i < PPT; ++i) {
+            const int s = tid + 256 * i, px = s / CG, g = s - px * CG;
+            const int hr = px / T::HW, hc = px - hr * T::HW;
+            const int hh = p.h0 - 1 + hr, ww = p.w0 - 1 + hc;
+            const bool in = s < HPC && (unsigned)hh < (unsigned)a.H && (unsigned)ww < (unsigned)a.W;
+            const unsigned vo = in ? (unsigned)(((hh * a.W + ww) * Cin + 8 * g) * 2) : kOOB;
+            hv[i] = load16(xr, vo, 0);
+            if (MASK) mv[i] = load16(mr, vo, 0);
+        }
+    };
+    BlockPos p = block_pos(a, tbeg, true, T::BR, T::BW);
+    fetch_halo(p);
+    int wcb = -1;
+    for (int t = tbeg;;) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PPT; ++i) {
+            const int s = tid + 256 * i, px = s / CG, g = s - px * CG;
+            if (s < HPC) halo[px * PS + g] = MASK ? relu_keep(hv[i], mv[i]) : hv[i];
+        }
+        if (wcb != p.cb) {
+            wcb = p.cb;
+            if (tid < T::BC)
+                sbias[tid] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(bres, (p.cb * T::BC + tid) * 4, 0, 0));
+            for (int s = tid; s < WPC; s += 256) {
+                const int co = s / (4 * S), g = s - co * (4 * S);
+                const bool in = 8 * g < K && p.cb * T::BC + co < a.Cout;
+                wlds[T::wrow(co) * WS + g] =
+                    load16(wres, in ? (unsigned)(((p.cb * T::BC + co) * K + 8 * g) * 2) : kOOB, 0);
+            }
+        }
+        __syncthreads();
+        BlockPos pn = p;
+        if (t + 1 < tend) {
+            pn = block_pos(a, t + 1, true, T::BR, T::BW);
+            fetch_halo(pn);
+        }
+        v4f acc[R][CT][WC];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int k = 0; k < CT; ++k)
+#pragma unroll
+                for (int u = 0; u < WC; ++u) acc[r][k][u] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int k0 = 32 * s + 8 * q;
+            const bool kin = k0 < K;
+            const int tap = kin ? k0 / Cin : 0, g = kin ? (k0 - tap * Cin) >> 3 : 0;
+            const int po = ((wr * R + tap / 3) * T::HW + j + tap % 3) * PS + g;
+            v8bf wf[WC];
+#pragma unroll
+            for (int u = 0; u < WC; ++u) wf[u] = bf8(wlds[(16 * u + j) * WS + 4 * s + q]);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int k = 0; k < CT; ++k) {
+                    u4v v = halo[po + (r * T::HW + 16 * k) * PS];
+                    // the padding's pixels are zeros too: what they would
+                    // read could be infinite
+                    if (32 * s + 32 > K && !kin) v = u4v{0u, 0u, 0u, 0u};
+#pragma unroll
+                    for (int u = 0; u < WC; ++u)
+                        acc[r][k][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], bf8(v), acc[r][k][u], 0, 0, 0);
+                }
+        }
+        store_tile<R, CT, WC, OUT32>(a, acc, sbias, p.n, p.h0 + wr * R, p.w0, p.cb * T::BC, 0);
+        if (++t >= tend) break;
+        p = pn;
     }
 }
 
@@ -915,28 +1161,98 @@ BwdWPlan bwd_w_plan(int N, int H, int W, int Cin, int Cout) {
 }  // namespace
 
 namespace {
+// Two workgroups per CU.  With one chunk of input channels a launch has about
+// that many (the thin kernel, whose LDS is small, twice as many), each with
+// an equal run of blocks, so the weights are staged once per run: 51 us
+// against 54 for one block per workgroup (32 -> 32 channels, 64 x 128 x
+// 256).  With more chunks the weights are staged per chunk anyway, and one
+// block per workgroup balances better: 138 us against 154 (96 -> 32).
+constexpr int kRun = 512;
+
+template <int R, int CT, int WC, int WP, int PF, bool MASK>
+void launch_tile(ConvArgs a, hipStream_t st) {
+    using T = Tile<R, CT, WC, WP>;
+    a.hb = (a.H + T::BR - 1) / T::BR;
+    a.wb = (a.W + T::BW - 1) / T::BW;
+    a.npx = a.N * a.hb * a.wb;
+    a.ncb = (a.Cout + T::BC - 1) / T::BC;
+    const int total = a.npx * a.ncb, per = a.Cin == 32 ? (total + kRun - 1) / kRun : 1;
+    const dim3 grid((total + per - 1) / per);
+    if (a.y32)
+        hipLaunchKernelGGL((conv_tile<R, CT, WC, WP, PF, MASK, true>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((conv_tile<R, CT, WC, WP, PF, MASK, false>), grid, dim3(256), 0, st, a);
+}
+
+template <int R, int CT, int WC, int CG, bool MASK>
+void launch_thin(ConvArgs a, hipStream_t st) {
+    using T = Tile<R, CT, WC, 4>;
+    a.hb = (a.H + T::BR - 1) / T::BR;
+    a.wb = (a.W + T::BW - 1) / T::BW;
+    a.npx = a.N * a.hb * a.wb;
+    a.ncb = (a.Cout + T::BC - 1) / T::BC;
+    const int total = a.npx * a.ncb, per = (total + 2 * kRun - 1) / (2 * kRun);
+    const dim3 grid((total + per - 1) / per);
+    if (a.y32)
+        hipLaunchKernelGGL((conv_tile_thin<R, CT, WC, CG, MASK, true>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((conv_tile_thin<R, CT, WC, CG, MASK, false>), grid, dim3(256), 0, st, a);
+}
+
+// Blocks of one configuration.
+template <int R, int CT, int WC, int WP>
+int64_t blocks_of(const ConvArgs& a) {
+    using T = Tile<R, CT, WC, WP>;
+    return (int64_t)a.N * ((a.H + T::BR - 1) / T::BR) * ((a.W + T::BW - 1) / T::BW) * ((a.Cout + T::BC - 1) / T::BC);
+}
+
+bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
 template <bool MASK>
 void launch_fwd(const uint16_t* x, const uint16_t* xm, const uint16_t* w, const float* bias, float* y32, uint16_t* y16,
                 int N, int H, int W, int Cin, int Cout, int relu, hipStream_t st) {
     const int64_t P = (int64_t)N * H * W;
-    if (Cin % 32 == 0 && Cin >= 64 && Cout >= 32) {
-        // input staged in LDS: blocks of 4 rows x 32 columns x 128 channels
-        // (WR 2, WC 4) when Cout is a multiple of 128, 8 rows x 32 (WR 4,
-        // WC 2) for Cout < 64, else 8 rows x 64 (WR 4, WC 4); the measured
-        // per-layer times favour the direct kernel below when Cin is 32
-        const unsigned wb = (unsigned)((W + 31) / 32);
-        if (Cout < 64) {
-            const dim3 grid(wb * (unsigned)((H + 7) / 8) * (unsigned)N * (unsigned)((Cout + 31) / 32));
-            hipLaunchKernelGGL((conv_fwd_lds<4, 2, MASK>), grid, dim3(256), 0, st, x, xm, w, bias, y32, y16, N, H, W,
-                               Cin, Cout, relu);
-        } else if (Cout % 128 == 0) {
-            const dim3 grid(wb * (unsigned)((H + 3) / 4) * (unsigned)N * (unsigned)((Cout + 127) / 128));
-            hipLaunchKernelGGL((conv_fwd_lds<2, 4, MASK>), grid, dim3(256), 0, st, x, xm, w, bias, y32, y16, N, H, W,
-                               Cin, Cout, relu);
-        } else {
-            const dim3 grid(wb * (unsigned)((H + 7) / 8) * (unsigned)N * (unsigned)((Cout + 63) / 64));
-            hipLaunchKernelGGL((conv_fwd_lds<4, 4, MASK>), grid, dim3(256), 0, st, x, xm, w, bias, y32, y16, N, H, W,
-                               Cin, Cout, relu);
+    const ConvArgs a{x, xm, w, bias, y32, y16, N, H, W, Cin, Cout, relu, 0, 0, 0, 0};
+    // the staged kernels address one image and the weights by 31-bit byte
+    // offsets, count blocks in 32 bits and store 16 bytes at once
+    const bool staged = !(y32 && y16) && (int64_t)H * W * Cin * 2 < kMaxBytes &&
+                        (int64_t)H * W * Cout * (y32 ? 4 : 2) < kMaxBytes && (int64_t)Cout * 9 * Cin * 2 < kMaxBytes &&
+                        P < ((int64_t)1 << 28) && P * ((Cout + 15) / 16) < ((int64_t)1 << 31) && aligned16(x) && aligned16(xm) && aligned16(w) && aligned16(y32) &&
+                        aligned16(y16);
+    if (staged && Cin % 32 == 0) {
+        // The block shape, by what was measured at batch 64 on 128 x 256
+        // (thin layers) to 32 x 64 (wide ones), us a layer for the shape
+        // taken and the next best; the kernel before these in parentheses:
+        //   32 -> 8     35.7, 39.7 (110)    96 -> 32    138, 146 (374)
+        //   32 -> 32    51, 55 (177)        32 -> 96    137, 162 (512)
+        //   32 -> 64    23.5, 26.6 (76)     64 -> 192   113, 117 (359)
+        //   192 -> 64   106, 102 (260)      256 -> 128  69, 67 (162)
+        // Larger blocks read less LDS per MFMA and less halo; below 512 of
+        // them (two per CU; 256, one per CU, for the smaller shapes) CUs
+        // stay idle and the next smaller shape is faster, e.g. 128 -> 128
+        // on 64 x 16 x 32: 12.4 us against 14.5, and on 1 x 16 x 32: 6 us
+        // against 9 (32).  The masked kernels hold the mask in registers
+        // too and take the shapes that do not spill with it.
+        if (!MASK) {
+            if (Cout <= 16 && blocks_of<4, 2, 1, 4>(a) >= kRun) return launch_tile<4, 2, 1, 4, 1, false>(a, st);
+            if (Cout <= 32 && Cin >= 96 && blocks_of<4, 2, 2, 4>(a) >= kRun)
+                return launch_tile<4, 2, 2, 4, 1, false>(a, st);
+            if (Cout % 96 == 0 && blocks_of<2, 2, 6, 4>(a) >= kRun)
+                return Cin == 32 ? launch_tile<2, 2, 6, 4, 0, false>(a, st) : launch_tile<2, 2, 6, 4, 1, false>(a, st);
+        }
+        if (Cout > 32 && blocks_of<2, 2, 4, 4>(a) >= kRun) return launch_tile<2, 2, 4, 4, 1, MASK>(a, st);
+        if (blocks_of<2, 2, 2, 4>(a) >= kRun / 2) return launch_tile<2, 2, 2, 4, 2, MASK>(a, st);
+        if (!MASK && blocks_of<2, 1, 2, 4>(a) >= kRun / 2) return launch_tile<2, 1, 2, 4, 2, false>(a, st);
+        return launch_tile<1, 1, 2, 4, 2, MASK>(a, st);
+    }
+    if (staged && Cin <= 56) {
+        switch (Cin / 8) {
+            case 1: launch_thin<2, 2, 2, 1, MASK>(a, st); break;
+            case 2: launch_thin<2, 2, 2, 2, MASK>(a, st); break;
+            case 3: launch_thin<2, 2, 2, 3, MASK>(a, st); break;
+            case 5: launch_thin<2, 2, 2, 5, MASK>(a, st); break;
+            case 6: launch_thin<2, 2, 2, 6, MASK>(a, st); break;
+            default: launch_thin<2, 2, 2, 7, MASK>(a, st); break;
         }
         return;
     }
