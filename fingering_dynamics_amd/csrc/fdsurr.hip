@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 
 #include "fdsurr.h"
 
@@ -605,7 +606,399 @@ __global__ __launch_bounds__(256) void cast_flip(CastFlipArgs a) {
 
 // ------------------------------------------------------- weight gradient
 // dw[co][tap][ci] = sum_p dy[p][co] x[p + d(tap)][ci]: a GEMM whose
-// reduction runs over pixels, the strided dimension of both operands.  Each
+// reduction runs over pixels, the strided dimension of both operands.  Both
+// are staged in LDS as they lie in memory, [pixel][channel], and the
+// fragments are read with the transposing LDS load (ds_read_b64_tr_b16: the
+// 16 lanes of a group address 4 pixels x 4 groups of 4 channels and receive
+// 4 pixels of one channel each), two loads for the eight pixels of a lane.
+//
+// A wave computes 16 ACO output channels x 16 ACI input channels x all nine
+// taps.  It marches down the rows of a strip of 32 columns (the 32 k of an
+// MFMA step): a row of x meets the three rows of dy whose taps reach it,
+// kept as fragments in registers, so a row costs ACO fragments of dy and
+// 3 ACI of x (the tap's column shift is the address) for 9 ACO ACI MFMAs:
+// 8 for 36, far below what the LDS delivers, and x and dy are read from
+// global memory once for all taps.  The kernel before this one had one tap
+// per workgroup: nine times the loads, and each of its pixel pairs was
+// transposed by 32-bit LDS writes.
+//
+// The eight waves of a workgroup are WCO x WCI channel tiles x WK groups
+// that take different strips (k groups); groups are added through LDS at the
+// end in a fixed tree, and the workgroup writes one partial sum, which
+// reduce_slices adds in a fixed order.  Work items are (image, run of
+// `rows` rows, strip), the strips adjacent (groups that run together read
+// neighbouring columns): a run reads its rows and, of x, one row more on
+// either side, as zeros outside the image.
+//
+// A row step has few bytes and few MFMAs (576 cycles of them for 32 x 32
+// channels), so what bounds the kernel is how many rows are in flight and
+// what else a step issues: rows are loaded straight into LDS (no registers
+// are held for them), in a ring of NS stages of RS rows; a lane's offsets
+// are formed once per item; the steps that need no masks have a loop of
+// their own.  Measured with reduce_slices, us a layer at batch 64, the
+// kernels before these in parentheses: 32 -> 32 at 128 x 256 61 (161),
+// 96 -> 32 154 (409), 64 -> 64 at 64 x 128 54 (163), 192 -> 64 131 (418),
+// 256 -> 128 at 32 x 64 82 (286).  In registers, one row ahead: 83 for the
+// first; with the offsets formed per row and every step masked: 73.  The
+// 64-channel blocks keep the matrix cores busy 47 % of the time at the
+// 2.0 GHz the chip holds there.
+//
+// A staged row lies in LDS as 16-byte pieces, dy then x (then dy's ReLU
+// mask), then the two x columns beside the strip.  Its rows are permuted in
+// 32-byte granules so that the four pixels of a transposing load fall on
+// different banks: granule g of pixel p is stored at g ^ (p mod 4) with 64
+// channels, g ^ (p / 2 mod 2) with 32.
+template <int G>
+__device__ __forceinline__ int granule(int g, int p) {
+    return G >= 4 ? g ^ (p & 3) : (G == 2 ? g ^ ((p >> 1) & 1) : g);
+}
+
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef short v8s __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) v4s lds_v4s;
+typedef __attribute__((address_space(3))) char lds_char;
+
+// Fragment of 32 pixels x 16 channels: a and b address this lane's piece of
+// the first and second four pixels of its group of eight.
+__device__ __forceinline__ v8bf tr_frag(unsigned a, unsigned b) {
+    const v4s u = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds_char*)(uintptr_t)a);
+    const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds_char*)(uintptr_t)b);
+    return __builtin_bit_cast(v8bf, v8s{u[0], u[1], u[2], u[3], v[0], v[1], v[2], v[3]});
+}
+
+// One 16-byte piece per lane from a buffer straight into LDS at lds + 16 x
+// lane (zeros at kOOB).  No register is written, so nothing waits for it but
+// wait_loads; the compiler does not see it, and its own waits, which count
+// the same counter, only become stricter.
+__device__ __forceinline__ void load_lds(u4v rsrc, unsigned voff, unsigned soff, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
+}
+// All but the newest N loads of this wave have arrived.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" : : "i"(N) : "memory");
+}
+// The words of make_rsrc(p, bytes), in scalar registers.
+__device__ __forceinline__ u4v rsrc_words(const void* p, int64_t bytes) {
+    const uint64_t b = (uint64_t)p;
+    return u4v{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b),
+               (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)(b >> 32) & 0xFFFFu)), (unsigned)bytes,
+               0x00020000u};
+}
+
+struct WgradArgs {
+    const uint16_t* x;
+    const uint16_t* dy;
+    const uint16_t* dym;  // ReLU mask of dy (MASK)
+    float* part;          // [slice][Cout * 9 * Cin + Cout]
+    int with_bias;
+    int N, H, W, Cin, Cout;
+    int strips, chunks, rows;  // 32-column strips, row runs and their height
+    int items, slices, ncb, nib;
+};
+
+template <int ACO, int ACI, int WCO, int WCI, int WK, int NS, int RS, bool MASK>
+__global__ __launch_bounds__(512, 2) void conv_wgrad(WgradArgs a) {
+    static_assert(WCO * WCI * WK == 8, "eight waves");
+    constexpr int BCO = 16 * ACO * WCO, BCI = 16 * ACI * WCI;  // channels of the block
+    constexpr int WG = WCO * WCI, NT = 64 * WG;                 // waves, threads of a k group
+    constexpr int PO = BCO / 8, PI = BCI / 8;                   // 16-byte pieces per pixel
+    constexpr int GO = BCO / 16, GI = BCI / 16;                 // granules per pixel
+    constexpr int RD = 32 * PO, RX = 32 * PI, RE = 2 * PI;      // pieces of a row: dy, x, x beside the strip
+    static_assert(RD % 64 == 0 && RX % 64 == 0 && RE <= 64, "whole waves");
+    // loads of a row per wave: dy and x in 64-piece parts dealt to the
+    // group's waves, the two edge columns on its first wave
+    constexpr int PD = RD / 64, PX = RX / 64;
+    constexpr int ND = (PD + WG - 1) / WG, NX = (PX + WG - 1) / WG;
+    static_assert(PD % WG == 0 || WG % PD == 0, "");
+    static_assert(PX % WG == 0 || WG % PX == 0, "");
+    constexpr int ROW = RD + RX + (MASK ? RD : 0) + RE;         // pieces of a staged row
+    constexpr int TILES = 9 * ACO * ACI;
+    constexpr int NB = NS * RS;                                 // row buffers
+    constexpr int RED = 4 * (TILES + ACO) * 64;                 // pieces of the group sums
+    constexpr int RING = NB * WK * ROW;
+    static_assert(RING * 16 <= 160 * 1024 && RED * 16 <= 160 * 1024, "LDS");
+    __shared__ __align__(16) u4v smem[RING > RED ? RING : RED];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = wave / WG, wt = wave % WG, wco = wt % WCO, wci = wt / WCO;
+    const int j = lane & 15, q = lane >> 4;
+    const unsigned lds0 = (unsigned)(uintptr_t)(lds_char*)smem + (unsigned)(kg * NB * ROW * 16);  // the group's ring
+
+    // logical workgroup = slice x channel block, the blocks of one slice
+    // adjacent (they read the same x and dy)
+    const int L = xcd_band(), nblk = a.ncb * a.nib;
+    const int slice = L / nblk, blk = L - slice * nblk;
+    const int co0 = (blk % a.ncb) * BCO, ci0 = (blk / a.ncb) * BCI;
+
+    // the group's items, and how many every group of the workgroup runs
+    const int ngrp = a.slices * WK, gid = slice * WK + kg;
+    auto first = [&](int g) { return (int)(((int64_t)a.items * g + ngrp - 1) / ngrp); };  // low groups first
+    const int ibeg = first(gid), iend = first(gid + 1);
+    const int spi = (a.rows + 2 + RS - 1) / RS * RS;  // row steps of an item
+    const int nit = (a.items + ngrp - 1) / ngrp;
+
+    // Loads of the next row.  A lane's byte offsets within a row of the
+    // strip are formed once per item; the row is the scalar offset, and a
+    // row that is not wanted (outside the run or the image) reads a
+    // descriptor of no bytes, i.e. zeros.
+    const int64_t xb = (int64_t)a.H * a.W * a.Cin * 2, db = (int64_t)a.H * a.W * a.Cout * 2;
+    unsigned dvo[ND], xvo[NX], evo = kOOB;
+    int it = ibeg, st = 0, slot = 0;  // item and row to load, its buffer
+    int ln = 0, r0 = 0, r1 = 0;       // the item's image and rows
+    auto load = [&]() {
+        if (st == 0) {
+            const int run = it / a.strips, w0 = (it - run * a.strips) * 32;
+            const int n = run / a.chunks, chunk = run - n * a.chunks;
+            const bool live = it < iend;
+            ln = live ? n : 0;
+            r0 = live ? chunk * a.rows : a.H + 2;  // rows past the image: none is wanted
+            r1 = min(r0 + a.rows, a.H);
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                const int s = ((wt + WG * i) % PD) * 64 + lane, px = s / PO, g = s % PO;
+                const int c = co0 + 8 * (2 * granule<GO>(g >> 1, px) + (g & 1));
+                dvo[i] = w0 + px < a.W && c < a.Cout ? (unsigned)(((w0 + px) * a.Cout + c) * 2) : kOOB;
+            }
+#pragma unroll
+            for (int i = 0; i < NX; ++i) {
+                const int s = ((wt + WG * i) % PX) * 64 + lane, px = s / PI, g = s % PI;
+                const int c = ci0 + 8 * (2 * granule<GI>(g >> 1, px) + (g & 1));
+                xvo[i] = w0 + px < a.W && c < a.Cin ? (unsigned)(((w0 + px) * a.Cin + c) * 2) : kOOB;
+            }
+            const int ww = lane / PI ? w0 + 32 : w0 - 1, c = ci0 + 8 * (lane % PI);
+            evo = lane < RE && ww >= 0 && ww < a.W && c < a.Cin ? (unsigned)((ww * a.Cin + c) * 2) : kOOB;
+        }
+        const int h = r0 + st, xh = h - 1;
+        const bool drow = h < r1, xrow = xh >= 0 && xh < a.H && xh <= r1;
+        const u4v dr = rsrc_words((const char*)a.dy + ln * db, drow ? db : 0);
+        const u4v xr = rsrc_words((const char*)a.x + ln * xb, xrow ? xb : 0);
+        const unsigned ds = drow ? (unsigned)(h * a.W * a.Cout * 2) : 0u, xs = xrow ? (unsigned)(xh * a.W * a.Cin * 2) : 0u;
+        const unsigned base = lds0 + (unsigned)(slot * ROW * 16);
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            if (PD < WG && wt >= PD) break;  // waves without a part of their own
+            const unsigned part = (unsigned)((wt + WG * i) % PD) * 1024u;
+            load_lds(dr, dvo[i], ds, base + part);
+            if (MASK)
+                load_lds(rsrc_words((const char*)a.dym + ln * db, drow ? db : 0), dvo[i], ds,
+                         base + (unsigned)((RD + RX) * 16) + part);
+        }
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+            if (PX < WG && wt >= PX) break;
+            load_lds(xr, xvo[i], xs, base + (unsigned)(RD * 16) + (unsigned)((wt + WG * i) % PX) * 1024u);
+        }
+        // columns w0 - 1 and w0 + 32
+        if (wt == 0 && lane < RE) load_lds(xr, evo, xs, base + (unsigned)((ROW - RE) * 16));
+        slot = slot + 1 == NB ? 0 : slot + 1;
+        if (++st == spi) {
+            st = 0;
+            ++it;
+        }
+    };
+    // the wave's loads of the oldest stage (RS rows) in flight have arrived
+    constexpr int LW = ND * (MASK ? 2 : 1) + NX;  // of a wave other than the first
+    auto arrived = [&]() {
+        if constexpr (WG == 1) {
+            wait_loads<(NS - 2) * RS * (LW + 1)>();
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            // a wave without dy (x) parts has fewer loads in flight
+            if (PD < WG || PX < WG) {
+                constexpr int l0 = (PD >= WG ? ND * (MASK ? 2 : 1) : 0) + (PX >= WG ? NX : 0);
+                wait_loads<(NS - 2) * RS * l0>();
+            } else if (wt == 0) {
+                wait_loads<(NS - 2) * RS * (LW + 1)>();
+            } else {
+                wait_loads<(NS - 2) * RS * LW>();
+            }
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+    };
+
+    // fragment addresses in a staged row, bytes: group q of lanes takes
+    // pixels 8 q .. 8 q + 7 (x: shifted by the tap), lane j of it addresses
+    // pixel j / 4, channels 4 (j mod 4) .. + 3; the pixels -1 and 32 that a
+    // shift reaches lie in the edge columns
+    unsigned ad[ACO], ax[3][ACI], ax2[ACI];
+    const unsigned edge = (unsigned)((ROW - RE) * 16);
+#pragma unroll
+    for (int i = 0; i < ACO; ++i) {
+        const int p = 8 * q + (j >> 2);
+        ad[i] = (unsigned)(p * BCO * 2 + granule<GO>(wco * ACO + i, p) * 32 + (j & 3) * 8);
+    }
+    auto xaddr = [&](int p, int g) {
+        if (p < 0 || p > 31) return edge + (unsigned)((p > 31 ? BCI * 2 : 0) + g * 32 + (j & 3) * 8);
+        return (unsigned)(RD * 16 + p * BCI * 2 + granule<GI>(g, p) * 32 + (j & 3) * 8);
+    };
+#pragma unroll
+    for (int i = 0; i < ACI; ++i) {
+#pragma unroll
+        for (int w = 0; w < 3; ++w) ax[w][i] = xaddr(8 * q + (j >> 2) + w - 1, wci * ACI + i);
+        ax2[i] = xaddr(8 * q + 4 + (j >> 2) + 1, wci * ACI + i);
+    }
+    // second four pixels of tap column 0: past the edge column on the lanes
+    // that started in it
+    unsigned ax0[ACI];
+#pragma unroll
+    for (int i = 0; i < ACI; ++i) ax0[i] = xaddr(8 * q + 4 + (j >> 2) - 1, wci * ACI + i);
+
+    v4f acc[9][ACO][ACI], accb[ACO];
+#pragma unroll
+    for (int i = 0; i < ACO; ++i) {
+        accb[i] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int k = 0; k < ACI; ++k) acc[t][i][k] = v4f{0.f, 0.f, 0.f, 0.f};
+    }
+    const bool with_bias = a.with_bias && ci0 == 0 && wci == 0;
+    const v8bf ones = bf8(u4v{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+    int cslot = 0;          // buffer being computed
+    int rows_i = 0;         // the item's rows of dy
+    u4v keep{};             // the pixels of this lane's fragments before the image's edge
+    v8bf d1[ACO], d2[ACO];  // dy fragments of the last two rows
+#pragma unroll
+    for (int i = 0; i < ACO; ++i) d1[i] = d2[i] = bf8(u4v{0u, 0u, 0u, 0u});
+
+    // One row step: row h = first row + t of dy, x row h - 1.
+    auto row_step = [&](auto masked, int t) __attribute__((always_inline)) {
+        constexpr bool B = decltype(masked)::value;
+        const unsigned row = lds0 + (unsigned)(cslot * ROW * 16);
+        v8bf d0[ACO];
+#pragma unroll
+        for (int i = 0; i < ACO; ++i) {
+            d0[i] = tr_frag(row + ad[i], row + ad[i] + 4 * BCO * 2);
+            if (MASK) {
+                const unsigned m = row + (unsigned)((RD + RX) * 16) + ad[i];
+                d0[i] = bf8(relu_keep(__builtin_bit_cast(u4v, d0[i]), __builtin_bit_cast(u4v, tr_frag(m, m + 4 * BCO * 2))));
+            }
+        }
+        if (with_bias) {
+#pragma unroll
+            for (int i = 0; i < ACO; ++i)
+                accb[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d0[i], ones, accb[i], 0, 0, 0);
+        }
+        // x row h - 1 meets dy rows h (its taps of row -1), h - 1 and h - 2,
+        // those of the run only.  Where dy is zero beyond the run or the
+        // image's edge, x is zeroed too (it could be infinite).
+        const unsigned m0 = t < rows_i ? ~0u : 0u, m1 = t >= 1 && t <= rows_i ? ~0u : 0u,
+                       m2 = t >= 2 && t <= rows_i + 1 ? ~0u : 0u;
+#pragma unroll
+        for (int w = 0; w < 3; ++w)
+#pragma unroll
+            for (int m = 0; m < ACI; ++m) {
+                const unsigned p = row + ax[w][m];
+                u4v xf = __builtin_bit_cast(
+                    u4v, tr_frag(p, w == 0 ? row + ax0[m] : (w == 2 ? row + ax2[m] : p + 4 * BCI * 2)));
+                if (B && w == 0) xf &= keep;
+                const v8bf x0 = bf8(B ? xf & m0 : xf), x1 = bf8(B ? xf & m1 : xf), x2 = bf8(B ? xf & m2 : xf);
+#pragma unroll
+                for (int i = 0; i < ACO; ++i) {
+                    acc[w][i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d0[i], x0, acc[w][i][m], 0, 0, 0);
+                    acc[3 + w][i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1[i], x1, acc[3 + w][i][m], 0, 0, 0);
+                    acc[6 + w][i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d2[i], x2, acc[6 + w][i][m], 0, 0, 0);
+                }
+            }
+#pragma unroll
+        for (int i = 0; i < ACO; ++i) {
+            d2[i] = d1[i];
+            d1[i] = d0[i];
+        }
+        cslot = cslot + 1 == NB ? 0 : cslot + 1;
+    };
+    // A stage: RS rows between two barriers.
+    auto step = [&](auto masked, int t) __attribute__((always_inline)) {
+        arrived();
+        // into the buffers read in the stage before (rows past the last one
+        // are zeros, so every stage issues the same number of loads)
+#pragma unroll
+        for (int k = 0; k < RS; ++k) load();
+#pragma unroll
+        for (int k = 0; k < RS; ++k) row_step(masked, t + k);
+    };
+#pragma unroll 1
+    for (int i = 0; i < NB - RS; ++i) load();
+#pragma unroll 1
+    for (int i = 0; i < nit; ++i) {
+        const int cit = ibeg + i, run = cit / a.strips, chunk = run % a.chunks;
+        const int left = a.W - (cit - run * a.strips) * 32;
+        rows_i = cit < iend ? min(a.rows, a.H - chunk * a.rows) : 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            keep[e] = (8 * q + 2 * e < left ? 0x0000FFFFu : 0u) | (8 * q + 2 * e + 1 < left ? 0xFFFF0000u : 0u);
+        // the steps that need no mask in a loop of their own (as branches of
+        // one loop they would copy the accumulators)
+        int t = 0;
+#pragma unroll 1
+        for (; t < 2; t += RS) step(std::integral_constant<bool, true>(), t);
+        if (left >= 32) {
+#pragma unroll 1
+            for (; t + RS - 1 < rows_i; t += RS) step(std::integral_constant<bool, false>(), t);
+        }
+#pragma unroll 1
+        for (; t < spi; t += RS) step(std::integral_constant<bool, true>(), t);
+    }
+    // the ring becomes the group sums' memory: no load may land in it later
+    wait_loads<0>();
+    __syncthreads();
+
+    // sum of the k groups: groups [h, 2 h) hand their tiles to groups [0, h)
+    v4f* red = reinterpret_cast<v4f*>(smem);
+#pragma unroll
+    for (int h = WK / 2; h >= 1; h /= 2) {
+        // nothing to add where no group from h on had an item
+        if (first(slice * WK + h) == first((slice + 1) * WK)) continue;
+        v4f* sl = red + (int64_t)((kg % h) * WG + wt) * (TILES + ACO) * 64 + lane;
+        if (kg >= h && kg < 2 * h) {
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+#pragma unroll
+                for (int i = 0; i < ACO; ++i)
+#pragma unroll
+                    for (int m = 0; m < ACI; ++m) sl[((k * ACO + i) * ACI + m) * 64] = acc[k][i][m];
+#pragma unroll
+            for (int i = 0; i < ACO; ++i) sl[(TILES + i) * 64] = accb[i];
+        }
+        __syncthreads();
+        if (kg < h) {
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+#pragma unroll
+                for (int i = 0; i < ACO; ++i)
+#pragma unroll
+                    for (int m = 0; m < ACI; ++m) acc[k][i][m] += sl[((k * ACO + i) * ACI + m) * 64];
+#pragma unroll
+            for (int i = 0; i < ACO; ++i) accb[i] += sl[(TILES + i) * 64];
+        }
+        __syncthreads();
+    }
+    if (kg) return;
+    const int64_t K = 9 * (int64_t)a.Cin, nw = a.Cout * K;
+    float* out = a.part + slice * (nw + a.Cout);
+#pragma unroll
+    for (int i = 0; i < ACO; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int co = co0 + 16 * (wco * ACO + i) + 4 * q + r;
+            if (co >= a.Cout) continue;
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+#pragma unroll
+                for (int m = 0; m < ACI; ++m) {
+                    const int ci = ci0 + 16 * (wci * ACI + m) + j;
+                    if (ci < a.Cin) out[co * K + k * a.Cin + ci] = acc[k][i][m][r];
+                }
+            if (with_bias && j == 0) out[nw + co] = accb[i][r];
+        }
+}
+
+// The general weight gradient, for operands that conv_wgrad does not
+// take (unaligned, or an image beyond its 31-bit offsets).  Each
 // 64-pixel step loads dy (64 px x 64 co) and the shifted x (64 px x 64 ci)
 // with 16-byte loads (8 channels of one pixel) and stores them TRANSPOSED
 // in LDS, [channel][pixel] with rows padded to 72 elements, so that every
@@ -801,197 +1194,29 @@ __global__ __launch_bounds__(256) void conv_bwd_w(const uint16_t* __restrict__ x
     }
 }
 
-// Weight gradient of thin layers (Cout <= 32): one workgroup owns a block
-// of up to 32 input channels, all output channels and all 9 taps, and a
-// slice of row segments (64 consecutive pixels of one image row).  Per
-// segment it stages dy (transposed, [co][pixel]) and the three x rows the
-// taps reach, each in three copies shifted by dw = -1, 0, +1
-// ([dh][dw][ci][pixel]), so every tap's fragments are aligned 16-byte LDS
-// reads and x is read once for all taps.  Staging writes pixel pairs as
-// 32-bit words, 32 consecutive pairs of two channel rows 8 apart per wave
-// instruction.  Wave v computes taps v, v+4, v+8
-// (< 9), 16 x 16 tiles skipped where the channels end; wave 3 of the first
-// channel block also forms the bias sums (ones operand).  Partial sums per
-// slice, added by reduce_slices.
-constexpr int kSmallCo = 32, kSmallCi = 32;
-
-__global__ __launch_bounds__(256) void conv_bwd_w_small(const uint16_t* __restrict__ x,
-                                                        const uint16_t* __restrict__ dy,
-                                                        const uint16_t* __restrict__ dym, float* __restrict__ part,
-                                                        float* __restrict__ bpart, int N, int H, int W, int Cin,
-                                                        int Cout, int64_t segs_per_slice) {
-    __shared__ __align__(16) uint16_t sdy[kSmallCo][kLds];
-    __shared__ __align__(16) uint16_t sx[9][kSmallCi][kLds];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // logical workgroup = slice x ci block, the ci blocks of one slice adjacent
-    const int nb = (Cin + kSmallCi - 1) / kSmallCi;
-    const int L = xcd_band();
-    const int slice = L / nb, ib = L - slice * nb;
-    const int ci0 = ib * kSmallCi;
-    const int wsegs = (W + 63) / 64;
-    const int64_t nseg = (int64_t)N * H * wsegs;
-    const int64_t sbeg = (int64_t)slice * segs_per_slice;
-    const int64_t send = std::min<int64_t>(nseg, sbeg + segs_per_slice);
-    const bool co2 = Cout > 16, ci2 = ci0 + 16 < Cin;
-    const bool with_bias = bpart != nullptr && ib == 0 && wave == 3;
-    const u4v ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
-    v4f acc[3][2][2];
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc[j][a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-    v4f accb[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
-    // The next segment's operands are loaded once this segment's are in LDS,
-    // so the loads run during the barrier and the MFMAs.
-    // dy: 32 pixel pairs x 4 groups of 8 output channels on threads 0..127,
-    // lane t of group g taking pixels 2t, 2t + 1.
-    // x: 3 rows x 32 pixel pairs x 4 groups of 8 input channels, items
-    // i = (r, g, t) = thread and thread + 256 (threads 0..127); item i loads
-    // columns w0 + 2t - 1 .. w0 + 2t + 2 and writes pixels 2t, 2t + 1 of the
-    // three copies (copy dw holds column pp + dw at pixel pp), each
-    // channel's pair as one 32-bit write.
-    const bool low = threadIdx.x < 128;  // stages dy and takes a second x item
-    u4v ldy[2], lm[2], lx[2][4];
-    auto load = [&](int64_t sg) {
-        const int w0 = (int)(sg % wsegs) * 64;
-        const int64_t nh = sg / wsegs;
-        const int h = (int)(nh % H);
-        const int64_t n = nh / H;
-        if (low) {
-            const int t = threadIdx.x & 31, g = threadIdx.x >> 5;
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                ldy[k] = u4v{0u, 0u, 0u, 0u};
-                lm[k] = u4v{~0u, ~0u, ~0u, ~0u};
-                if (w0 + 2 * t + k < W && 8 * g < Cout) {
-                    const int64_t o = ((n * H + h) * W + w0 + 2 * t + k) * Cout + 8 * g;
-                    ldy[k] = *reinterpret_cast<const u4v*>(dy + o);
-                    if (dym) lm[k] = *reinterpret_cast<const u4v*>(dym + o);
-                }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            if (it == 1 && !low) break;
-            const int i = threadIdx.x + 256 * it;
-            const int t = i & 31, g = (i >> 5) & 3, r = i >> 7;
-            const int hh = h + r - 1;
-            const bool rowok = hh >= 0 && hh < H && ci0 + 8 * g < Cin;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int ww = w0 + 2 * t - 1 + k;
-                lx[it][k] = u4v{0u, 0u, 0u, 0u};
-                if (rowok && ww >= 0 && ww < W)
-                    lx[it][k] = *reinterpret_cast<const u4v*>(x + ((n * H + hh) * W + ww) * Cin + ci0 + 8 * g);
-            }
-        }
-    };
-    if (sbeg < send) load(sbeg);
-    for (int64_t sg = sbeg; sg < send; ++sg) {
-        u4v vdy[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) vdy[k] = dym ? relu_keep(ldy[k], lm[k]) : ldy[k];
-        if (low) {
-            const int t = threadIdx.x & 31, g = threadIdx.x >> 5;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int sh = 16 * (e & 1);
-                *reinterpret_cast<unsigned*>(&sdy[8 * g + e][2 * t]) =
-                    ((vdy[0][e >> 1] >> sh) & 0xFFFFu) | (((vdy[1][e >> 1] >> sh) & 0xFFFFu) << 16);
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            if (it == 1 && !low) break;
-            const int i = threadIdx.x + 256 * it;
-            const int t = i & 31, g = (i >> 5) & 3, r = i >> 7;
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int sh = 16 * (e & 1);
-                    *reinterpret_cast<unsigned*>(&sx[3 * r + d][8 * g + e][2 * t]) =
-                        ((lx[it][d][e >> 1] >> sh) & 0xFFFFu) | (((lx[it][d + 1][e >> 1] >> sh) & 0xFFFFu) << 16);
-                }
-        }
-        if (sg + 1 < send) load(sg + 1);
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const int kp = 32 * kk + 8 * (lane >> 4);
-            v8bf a[2];
-            a[0] = bf8(*reinterpret_cast<const u4v*>(&sdy[lane & 15][kp]));
-            a[1] = bf8(*reinterpret_cast<const u4v*>(&sdy[16 + (lane & 15)][kp]));
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int tap = wave + 4 * j;
-                if (tap >= 9) continue;
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    if (b == 1 && !ci2) continue;
-                    const v8bf bv = bf8(*reinterpret_cast<const u4v*>(&sx[tap][16 * b + (lane & 15)][kp]));
-                    acc[j][0][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bv, acc[j][0][b], 0, 0, 0);
-                    if (co2) acc[j][1][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], bv, acc[j][1][b], 0, 0, 0);
-                }
-            }
-            if (with_bias) {
-                accb[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bf8(ones), accb[0], 0, 0, 0);
-                if (co2) accb[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], bf8(ones), accb[1], 0, 0, 0);
-            }
-        }
-        __syncthreads();
-    }
-    const int64_t K = 9 * (int64_t)Cin;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const int tap = wave + 4 * j;
-        if (tap >= 9) continue;
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const int ci = ci0 + 16 * b + (lane & 15);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int co = 16 * a + 4 * (lane >> 4) + r;
-                    if (co < Cout && ci < Cin && ci < ci0 + kSmallCi)
-                        part[((int64_t)slice * Cout + co) * K + tap * Cin + ci] = acc[j][a][b][r];
-                }
-            }
-    }
-    if (with_bias && (lane & 15) == 0) {
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int co = 16 * a + 4 * (lane >> 4) + r;
-                if (co < Cout) bpart[(int64_t)slice * Cout + co] = accb[a][r];
-            }
-    }
-}
-
 // out[i] = sum over s of part[s][i]: eight interleaved partial sums a_j
 // (slices s = j mod 8 in ascending order, from 0), then a fixed tree of the
 // eight; the order is the same on every call.  A workgroup takes 32
 // consecutive outputs, thread t the partial sum j = t >> 5 of output t & 31
 // (eight times the threads of one per output: the sums are long, the
-// outputs few), and the tree runs from LDS.
-__global__ __launch_bounds__(256) void reduce_slices(const float* __restrict__ part, float* __restrict__ out,
-                                                     int64_t n, int S) {
+// outputs few), and the tree runs from LDS.  A slice is `stride` values: n1
+// for out, the rest up to n for out2 (weights and bias in one launch).
+__global__ __launch_bounds__(256) void reduce_slices(const float* __restrict__ part, int64_t stride, int S, int64_t n,
+                                                     float* __restrict__ out, int64_t n1, float* __restrict__ out2) {
     __shared__ float sa[8][33];
     const int j = threadIdx.x >> 5, ii = threadIdx.x & 31;
     const int64_t i = (int64_t)blockIdx.x * 32 + ii;
     float a = 0.f;
     if (i < n) {
 #pragma unroll 4
-        for (int s = j; s < S; s += 8) a += part[(int64_t)s * n + i];
+        for (int s = j; s < S; s += 8) a += part[(int64_t)s * stride + i];
     }
     sa[j][ii] = a;
     __syncthreads();
-    if (j == 0 && i < n)
-        out[i] = ((sa[0][ii] + sa[1][ii]) + (sa[2][ii] + sa[3][ii])) + ((sa[4][ii] + sa[5][ii]) + (sa[6][ii] + sa[7][ii]));
+    if (j == 0 && i < n) {
+        const float v = ((sa[0][ii] + sa[1][ii]) + (sa[2][ii] + sa[3][ii])) + ((sa[4][ii] + sa[5][ii]) + (sa[6][ii] + sa[7][ii]));
+        if (i < n1) out[i] = v; else out2[i - n1] = v;
+    }
 }
 
 // ------------------------------------------------------ U-Net plumbing
@@ -1125,37 +1350,70 @@ int check(int N, int H, int W, int Cin, int Cout) {
     return FDS_OK;
 }
 
-// Work split of the weight gradient.  Thin layers (Cout <= 32) go to
-// conv_bwd_w_small with slices of row segments, about 768 workgroups in all
-// (three per CU fit its LDS); the others to conv_bwd_w with pixel slices of
-// whole 64-pixel steps, about 2048 workgroups (1..256 slices), at least 512
-// pixels each.  chunk counts segments or pixels.
+// Work split of the weight gradient: the channel block by the layer's
+// channels, then row runs and slices, at most one workgroup per CU.  The
+// split with the least cost of the busiest k group is taken, in row steps
+// (about 1 us each with every CU busy): a run of `rows` rows costs rows + 2,
+// and the partial sum of a block, written and read back, 10/256 for 64 x 64
+// channels (256 of them, 38 MB: 7 us to write, 2.5 more in reduce_slices).
+// Too few slices show: 128 -> 128 channels at 64 x 16 x 32 take 32 us with
+// 64 slices of 10 steps and 37 with 32 of 18.
 struct BwdWPlan {
-    bool small;
-    int64_t chunk;
-    int S;
+    int kind;       // instantiation, launch_wgrad
+    int bco, bci, wk;
+    int ncb, nib;
+    int strips, chunks, rows, items, slices;
 };
 
 BwdWPlan bwd_w_plan(int N, int H, int W, int Cin, int Cout) {
     BwdWPlan pl{};
-    if (Cout <= kSmallCo) {
-        const int64_t nseg = (int64_t)N * H * ((W + 63) / 64);
-        const int64_t nb = (Cin + kSmallCi - 1) / kSmallCi;
-        const int64_t want = std::min<int64_t>(nseg, std::max<int64_t>(1, (768 + nb - 1) / nb));
-        pl.small = true;
-        pl.chunk = (nseg + want - 1) / want;
-        pl.S = (int)((nseg + pl.chunk - 1) / pl.chunk);
-        return pl;
+    if (Cout <= 16) pl = BwdWPlan{5, 16, 32, 8};
+    else if (Cin <= 16) pl = BwdWPlan{4, 32, 16, 8};
+    else if (Cout > 32 && Cin > 32) pl = BwdWPlan{0, 64, 64, 2};
+    else if (Cout > 32) pl = BwdWPlan{1, 64, 32, 4};
+    else if (Cin > 32 && Cin % 64 == 0) pl = BwdWPlan{2, 32, 64, 4};
+    else pl = BwdWPlan{3, 32, 32, 8};
+    pl.ncb = (Cout + pl.bco - 1) / pl.bco;
+    pl.nib = (Cin + pl.bci - 1) / pl.bci;
+    pl.strips = (W + 31) / 32;
+    const int64_t nblk = (int64_t)pl.ncb * pl.nib;
+    const int64_t cap = std::max<int64_t>(1, 256 / nblk);
+    const int64_t sum = nblk * pl.bco * pl.bci * 5 / 8;  // 65536ths of a step per slice
+    int64_t best = -1;
+    for (int c = 1; c <= H && c <= 256; c = c < 4 ? c + 1 : c + c / 2) {
+        const int rows = (H + c - 1) / c, chunks = (H + rows - 1) / rows;
+        const int64_t items = (int64_t)N * pl.strips * chunks;
+        int64_t per = (items + cap * pl.wk - 1) / (cap * pl.wk);  // items of the busiest group
+        for (int k = 0; k < 8; ++k, per += (per + 1) / 2) {
+            const int64_t slices = (items + per * pl.wk - 1) / (per * pl.wk);
+            const int64_t cost = per * (rows + 2) * 65536 + slices * sum;
+            if (best < 0 || cost < best) {
+                best = cost;
+                pl.chunks = chunks;
+                pl.rows = rows;
+                pl.items = (int)items;
+                pl.slices = (int)slices;
+            }
+            if (slices == 1) break;
+        }
     }
+    return pl;
+}
+
+// The general kernel's split: pixel slices of whole 64-pixel steps, about
+// 2048 workgroups (1..256 slices), at least 512 pixels each.
+struct BwdWGeneral {
+    int64_t chunk;
+    int S;
+};
+
+BwdWGeneral bwd_w_general(int N, int H, int W, int Cin, int Cout) {
     const int64_t P = (int64_t)N * H * W;
     const int64_t per_slice = (int64_t)((Cout + 63) / 64) * 9 * ((Cin + 63) / 64);
     const int64_t want = std::min<int64_t>(256, std::max<int64_t>(1, (2048 + per_slice - 1) / per_slice));
     int64_t c = (P + want - 1) / want;
     c = std::max<int64_t>((c + kStep - 1) / kStep * kStep, 512);
-    pl.small = false;
-    pl.chunk = c;
-    pl.S = (int)((P + c - 1) / c);
-    return pl;
+    return BwdWGeneral{c, (int)((P + c - 1) / c)};
 }
 
 }  // namespace
@@ -1272,6 +1530,27 @@ void launch_fwd(const uint16_t* x, const uint16_t* xm, const uint16_t* w, const 
     }
 }
 
+// conv_wgrad addresses one image of each operand by 31-bit byte offsets and
+// counts its work items in 32 bits.
+bool wgrad_fits(int N, int H, int W, int Cin, int Cout) {
+    return (int64_t)H * W * Cin * 2 < kMaxBytes && (int64_t)H * W * Cout * 2 < kMaxBytes &&
+           (int64_t)N * H * ((W + 31) / 32) < ((int64_t)1 << 30) &&
+           (int64_t)((Cout + 15) / 16) * ((Cin + 15) / 16) < ((int64_t)1 << 20);
+}
+
+template <bool MASK>
+void launch_wgrad(const WgradArgs& a, const BwdWPlan& pl, hipStream_t st) {
+    const dim3 grid(a.slices * a.ncb * a.nib), block(512);
+    switch (pl.kind) {
+        case 0: hipLaunchKernelGGL((conv_wgrad<2, 2, 2, 2, 2, MASK ? 3 : 4, 2, MASK>), grid, block, 0, st, a); break;
+        case 1: hipLaunchKernelGGL((conv_wgrad<2, 2, 2, 1, 4, 3, MASK ? 1 : 2, MASK>), grid, block, 0, st, a); break;
+        case 2: hipLaunchKernelGGL((conv_wgrad<2, 2, 1, 2, 4, MASK ? 4 : 3, MASK ? 1 : 2, MASK>), grid, block, 0, st, a); break;
+        case 3: hipLaunchKernelGGL((conv_wgrad<2, 2, 1, 1, 8, MASK ? 3 : 4, 1, MASK>), grid, block, 0, st, a); break;
+        case 4: hipLaunchKernelGGL((conv_wgrad<2, 1, 1, 1, 8, MASK ? 3 : 5, 1, MASK>), grid, block, 0, st, a); break;
+        default: hipLaunchKernelGGL((conv_wgrad<1, 2, 1, 1, 8, MASK ? 4 : 5, 1, MASK>), grid, block, 0, st, a); break;
+    }
+}
+
 int conv_fwd_checked(const uint16_t* x, const uint16_t* xm, const uint16_t* w, const float* bias, float* y32,
                      uint16_t* y16, int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout, int32_t relu,
                      void* stream) {
@@ -1337,8 +1616,9 @@ int fds_conv3x3_bwd_data(const uint16_t* dy, const uint16_t* wt, const uint16_t*
 }
 
 int64_t fds_bwd_weight_scratch(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
-    const BwdWPlan pl = bwd_w_plan(N, H, W, Cin, Cout);
-    return (int64_t)pl.S * Cout * (9 * (int64_t)Cin + 1);
+    int64_t S = bwd_w_general(N, H, W, Cin, Cout).S;
+    if (wgrad_fits(N, H, W, Cin, Cout)) S = std::max<int64_t>(S, bwd_w_plan(N, H, W, Cin, Cout).slices);
+    return S * Cout * (9 * (int64_t)Cin + 1);
 }
 
 int fds_conv3x3_bwd_weight(const uint16_t* x, const uint16_t* dy, const uint16_t* relu_y, float* dw, float* dbias,
@@ -1347,26 +1627,33 @@ int fds_conv3x3_bwd_weight(const uint16_t* x, const uint16_t* dy, const uint16_t
     if (rc) return rc;
     if (Cout % 8) return fail(FDS_E_ARG, "Cout must be a multiple of 8");
     if (!x || !dy || !dw || !scratch) return fail(FDS_E_ARG, "NULL pointer");
-    const BwdWPlan pl = bwd_w_plan(N, H, W, Cin, Cout);
-    const int S = pl.S;
     hipStream_t st = (hipStream_t)stream;
     const int64_t nw = (int64_t)Cout * 9 * Cin;
-    float* bp = dbias ? scratch + (int64_t)S * nw : nullptr;
-    if (pl.small) {
-        const dim3 grid((unsigned)S * (unsigned)((Cin + kSmallCi - 1) / kSmallCi));
-        hipLaunchKernelGGL(conv_bwd_w_small, grid, dim3(256), 0, st, x, dy, relu_y, scratch, bp, N, H, W, Cin, Cout,
-                           pl.chunk);
-    } else {
-        const dim3 grid((unsigned)S * (unsigned)(((Cout + 63) / 64) * 9 * ((Cin + 63) / 64)));
-        hipLaunchKernelGGL(conv_bwd_w, grid, dim3(256), 0, st, x, dy, relu_y, scratch, bp, N, H, W, Cin, Cout,
-                           pl.chunk);
+    if (wgrad_fits(N, H, W, Cin, Cout) && aligned16(x) && aligned16(dy) && aligned16(relu_y)) {
+        const BwdWPlan pl = bwd_w_plan(N, H, W, Cin, Cout);
+        const WgradArgs a{x, dy, relu_y, scratch, dbias != nullptr, N, H, W, Cin, Cout, pl.strips, pl.chunks, pl.rows,
+                          pl.items, pl.slices, pl.ncb, pl.nib};
+        if (relu_y) launch_wgrad<true>(a, pl, st);
+        else launch_wgrad<false>(a, pl, st);
+        FDS_HIP(hipGetLastError());
+        const int64_t n = dbias ? nw + Cout : nw;
+        hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, st, scratch, nw + Cout,
+                           pl.slices, n, dw, nw, dbias);
+        FDS_HIP(hipGetLastError());
+        return FDS_OK;
     }
+    const BwdWGeneral pl = bwd_w_general(N, H, W, Cin, Cout);
+    const int S = pl.S;
+    float* bp = dbias ? scratch + (int64_t)S * nw : nullptr;
+    const dim3 grid((unsigned)S * (unsigned)(((Cout + 63) / 64) * 9 * ((Cin + 63) / 64)));
+    hipLaunchKernelGGL(conv_bwd_w, grid, dim3(256), 0, st, x, dy, relu_y, scratch, bp, N, H, W, Cin, Cout, pl.chunk);
     FDS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((nw + 31) / 32)), dim3(256), 0, st, scratch, dw, nw, S);
+    hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((nw + 31) / 32)), dim3(256), 0, st, scratch, nw, S, nw, dw, nw,
+                       dbias);
     FDS_HIP(hipGetLastError());
     if (dbias) {
-        hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((Cout + 31) / 32)), dim3(256), 0, st, bp, dbias,
-                           (int64_t)Cout, S);
+        hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((Cout + 31) / 32)), dim3(256), 0, st, bp, (int64_t)Cout, S,
+                           (int64_t)Cout, dbias, (int64_t)Cout, dbias);
         FDS_HIP(hipGetLastError());
     }
     return FDS_OK;
