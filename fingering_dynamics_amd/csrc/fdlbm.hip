@@ -81,9 +81,19 @@ struct KBufs {
     const float* __restrict__ side_in; // [4][H] P of the previous psi
     float* __restrict__ side_out;
     const float* __restrict__ uprof;   // [H] inlet/outlet velocity
-    float* __restrict__ fields;        // [4][H][Wp] psi, rho, ux, uy
-    double* __restrict__ partials;     // per wave [3]
+    float* out[4];                     // psi, rho, ux, uy, rows opitch floats apart (NULL: not wanted)
+    int opitch;
+    double* __restrict__ partials;     // per wave [4] (NULL: no sums)
 };
+
+// Node o's fields to the wanted outputs (row y, column x).
+__device__ __forceinline__ void put_fields(const KBufs& b, int y, int x, float psi, float rho, float ux, float uy) {
+    const size_t o = (size_t)y * b.opitch + x;
+    if (b.out[0]) b.out[0][o] = psi;
+    if (b.out[1]) b.out[1][o] = rho;
+    if (b.out[2]) b.out[2][o] = ux;
+    if (b.out[3]) b.out[3][o] = uy;
+}
 
 __device__ __forceinline__ int wrap(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
 
@@ -393,12 +403,9 @@ __device__ __forceinline__ void finish_node(const KParams& k, const KBufs& b, rs
             rho = m.rho;
             ux = m.ux;
             uy = m.uy;
-            red4_add(red, rho, pc, fdn::tau_excess(rho, pc, k.c));
+            if (b.partials) red4_add(red, rho, pc, fdn::tau_excess(rho, pc, k.c));
         }
-        b.fields[o] = pc;
-        b.fields[k.Q + o] = rho;
-        b.fields[2 * k.Q + o] = ux;
-        b.fields[3 * k.Q + o] = uy;
+        put_fields(b, y, (int)ln.x, pc, rho, ux, uy);
         if (b.dst) {
             // inert solid nodes carry no populations (they were not pulled: zeros)
 #pragma unroll
@@ -467,8 +474,9 @@ __device__ __forceinline__ PsiRow psi_row_of(float pcen, float halo, int lane) {
 }
 
 // MODE 0: one iteration (collide and store the next post-collision state).
-// MODE 1: moments only - fields psi/rho/ux/uy, FP64 partial sums, and (if
-//         b.dst) the post-stream populations; the state is not advanced.
+// MODE 1: moments only - the wanted fields of psi/rho/ux/uy, FP64 partial
+//         sums (if b.partials), and (if b.dst) the post-stream populations;
+//         the state is not advanced.
 // Workgroups of WPB waves cover WPB adjacent strips of one chunk of k.rows
 // rows.  Blocks are numbered so that each XCD (workgroups are dealt
 // round-robin over the eight XCDs) gets a contiguous band of chunks:
@@ -490,10 +498,10 @@ __device__ __forceinline__ void march_block(const KParams& k, const KBufs& b, in
     const int wave = threadIdx.x >> 6;
     const int chunk = L / k.nsb;
     const int strip = (k.sb0 + L - chunk * k.nsb) * WPB + wave;
-    double* part = b.partials + 4 * (WPB * L + wave);
+    double* part = b.partials ? b.partials + 4 * (WPB * L + wave) : nullptr;
     const int x0 = strip * 64;
     if (x0 >= k.W) {
-        if (MODE == 1 && lane == 0) put_red4(part, red4_init());
+        if (MODE == 1 && part && lane == 0) put_red4(part, red4_init());
         return;
     }
     const int xcol = x0 + lane;
@@ -565,7 +573,7 @@ __device__ __forceinline__ void march_block(const KParams& k, const KBufs& b, in
         fla = fl2;
         flah = fl2h;
     }
-    if (MODE == 1) {
+    if (MODE == 1 && part) {
         red = wave_red4(red);
         if (lane == 0) put_red4(part, red);
     }
@@ -1350,18 +1358,26 @@ __global__ __launch_bounds__(256) void zero_inert_solids(float* __restrict__ pop
 
 // Initial state (fingering_periodic.py:90-121, or fingering.py:95-127 with
 // the walled init), one thread per node.
-//   PRE = 1: pre-collision populations f0/g0 into b.dst and the N = 0
-//            fields + partial sums.
+//   PRE = 1: pre-collision populations f0/g0 into b.dst (if not NULL) and
+//            the N = 0 fields + partial sums, as wanted.
 //   PRE = 0: post-collision populations of iteration 0 into b.dst and the
 //            side buffer P of the initial psi into b.side_out.
-//   ux0/uy0 (may be NULL): restart from given fields - the velocity is
+//   in.ux/in.uy (may be NULL): restart from given fields - the velocity is
 //            taken as given and mu from psi, so a running flow continues
 //            (fd_init_fields); with PRE = 1 the N = 0 state of such a start.
+//   in.keep  (may be NULL): the handle's own copies of the four fields
+//            (rows Wp apart), written from the caller's as they are read.
+struct InitFields {
+    const float* __restrict__ psi;
+    const float* __restrict__ rho;
+    const float* __restrict__ ux;
+    const float* __restrict__ uy;
+    int pitch;  // floats between rows
+    float* keep[4];
+};
+
 template <int PRE>
-__global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, const float* __restrict__ psi0,
-                                                   const float* __restrict__ rho0, int walled_init,
-                                                   const float* __restrict__ ux0 = nullptr,
-                                                   const float* __restrict__ uy0 = nullptr) {
+__global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, InitFields in, int walled_init) {
     const int x = blockIdx.x * 64 + threadIdx.x;
     const int y = blockIdx.y * 4 + threadIdx.y;
     Red4 red = red4_init();
@@ -1374,7 +1390,7 @@ __global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, const flo
                 xx = wrap(xx, k.W);
             }
             const int o = yy * k.Wp + xx;
-            return (b.flags[o] & kSolid) ? k.c.psi_wall : psi0[o];
+            return (b.flags[o] & kSolid) ? k.c.psi_wall : in.psi[(size_t)yy * in.pitch + xx];
         };
         const float n[9] = {P(y, x),         P(y, x + 1),     P(y + 1, x),
                             P(y, x - 1),     P(y - 1, x),     P(y + 1, x + 1),
@@ -1383,6 +1399,13 @@ __global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, const flo
         fdn::stencil(n, dpx, dpy, lap);
         const float psi = n[0];
         const int o = y * k.Wp + x;
+        const size_t oi = (size_t)y * in.pitch + x;
+        if (in.keep[0]) {
+            in.keep[0][o] = in.psi[oi];
+            in.keep[1][o] = in.rho[oi];
+            in.keep[2][o] = in.ux[oi];
+            in.keep[3][o] = in.uy[oi];
+        }
         const bool solid = (b.flags[o] & kSolid) != 0;
         float f[9], g[9];
         fdn::Mom<float> m{};
@@ -1390,7 +1413,7 @@ __global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, const flo
 #pragma unroll
             for (int i = 0; i < 9; ++i) f[i] = g[i] = 0.f;
         } else {
-            m.rho = rho0[o];
+            m.rho = in.rho[oi];
             m.psi = psi;
             m.mu = walled_init ? fdn::chem_pot(psi, lap, k.c) : 0.f;
             m.fx = m.mu * dpx + k.c.gx;
@@ -1398,28 +1421,27 @@ __global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, const flo
             m.ux = 0.f;
             m.uy = walled_init ? (0.5f * m.fy) / m.rho : 0.f;
             m.p = m.rho * (1.f / 3.f);  // evaluated before mu (both inits)
-            if (ux0) {
+            if (in.ux) {
                 m.mu = fdn::chem_pot(psi, lap, k.c);
                 m.fx = m.mu * dpx + k.c.gx;
                 m.fy = m.mu * dpy + k.c.gy;
-                m.ux = ux0[o];
-                m.uy = uy0[o];
+                m.ux = in.ux[oi];
+                m.uy = in.uy[oi];
                 m.p = m.rho * (1.f / 3.f) + psi * m.mu;
             }
             m.itau = fdn::inv_tau_mix(m.rho, psi, k.c);
             fdn::equilibria(m, k.c, f, g);
             if (!PRE) fdn::collide(f, g, m, k.c);
         }
+        if (!PRE || b.dst) {
 #pragma unroll
-        for (int i = 0; i < 9; ++i) {
-            b.dst[i * k.Q + o] = f[i];
-            b.dst[(9 + i) * k.Q + o] = g[i];
+            for (int i = 0; i < 9; ++i) {
+                b.dst[i * k.Q + o] = f[i];
+                b.dst[(9 + i) * k.Q + o] = g[i];
+            }
         }
         if (PRE) {
-            b.fields[o] = psi;
-            b.fields[k.Q + o] = solid ? 0.f : m.rho;
-            b.fields[2 * k.Q + o] = solid ? 0.f : m.ux;
-            b.fields[3 * k.Q + o] = solid ? 0.f : m.uy;
+            put_fields(b, y, x, psi, solid ? 0.f : m.rho, solid ? 0.f : m.ux, solid ? 0.f : m.uy);
             if (!solid) red4_add(red, m.rho, psi, fdn::tau_excess(m.rho, psi, k.c));
         } else if (!k.x_periodic && (x == 0 || x == k.W - 1)) {
             const float mu = fdn::chem_pot(psi, lap, k.c);
@@ -1428,14 +1450,14 @@ __global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, const flo
             b.side_out[(s + 1) * k.H + y] = dpy * mu;
         }
     }
-    if (PRE) block_red4<256>(red, b.partials + 4 * (blockIdx.y * gridDim.x + blockIdx.x));
+    if (PRE && b.partials) block_red4<256>(red, b.partials + 4 * (blockIdx.y * gridDim.x + blockIdx.x));
 }
 
 // State from given post-stream populations of iteration N (what
 // fd_get_populations returns: after bounce-back, walls and Zou-He), one
 // thread per node.  `staged` holds them as 18 planes [H][Wp].
 //   COLLIDE = 0: fields (psi, rho, ux, uy) and FP64 partial sums of
-//                iteration N into b.fields / b.partials.
+//                iteration N into b.out / b.partials, as wanted.
 //   COLLIDE = 1: the collision of iteration N into b.dst (the post-collision
 //                state the next launch pulls from) and P = d psi * mu of
 //                columns 0 and W-1 into b.side_out; on inert solid nodes the
@@ -1510,13 +1532,10 @@ __global__ __launch_bounds__(256) void restage_kernel(KParams k, KBufs b, float*
                 uy = m.uy;
                 red4_add(red, rho, psi, fdn::tau_excess(rho, psi, k.c));
             }
-            b.fields[o] = psi;
-            b.fields[k.Q + o] = rho;
-            b.fields[2 * k.Q + o] = ux;
-            b.fields[3 * k.Q + o] = uy;
+            put_fields(b, y, x, psi, rho, ux, uy);
         }
     }
-    if (!COLLIDE) block_red4<256>(red, b.partials + 4 * (blockIdx.y * gridDim.x + blockIdx.x));
+    if (!COLLIDE && b.partials) block_red4<256>(red, b.partials + 4 * (blockIdx.y * gridDim.x + blockIdx.x));
 }
 
 // Streaming copy, the HBM yardstick: grid-stride 16-byte non-temporal
@@ -1913,32 +1932,56 @@ int ensure_partials(fd_handle* h, int n) {
     return FD_OK;
 }
 
-// Fields (and optionally post-stream populations into `pops`) of the current
-// iteration, plus the FP64 sums in h->mass.  With populations staged by
-// fd_set_populations the post-stream populations already sit in
+// Where compute_fields puts the four fields: rows `pitch` floats apart, NULL
+// where one is not wanted.
+struct FieldsOut {
+    float* p[4];
+    int pitch;
+};
+
+// The handle's own padded planes (for the copies to the host).
+FieldsOut own_fields(const fd_handle* h) {
+    return FieldsOut{{h->fields, h->fields + h->Q, h->fields + 2 * h->Q, h->fields + 3 * h->Q}, h->Wp};
+}
+
+// The staged state of a handle that fd_init / fd_init_fields has started.
+InitFields staged_fields(const fd_handle* h) {
+    const bool u = h->init_u;
+    return InitFields{h->psi0, h->rho0, u ? h->fields + 2 * h->Q : nullptr, u ? h->fields + 3 * h->Q : nullptr, h->Wp,
+                      {nullptr, nullptr, nullptr, nullptr}};
+}
+
+// What `want` asks for of the current iteration - its fields into `out`, its
+// post-stream populations into `pops`, the FP64 sums in h->mass - in one pass
+// over the state (and a small reduction for the sums).  With populations
+// staged by fd_set_populations the post-stream populations already sit in
 // pop[1 - cur]: `pops` may then only be that buffer (or NULL).
-int compute_fields(fd_handle* h, float* pops, double* scratch = nullptr, int scratch_slots = 0) {
+int compute_fields(fd_handle* h, const FieldsOut* out, float* pops, bool sums, double* scratch = nullptr,
+                   int scratch_slots = 0) {
     if (!h->inited) return fail(FD_E_STATE, "fd_init has not been called");
     KBufs b{};
     b.flags = h->flags;
     b.uprof = h->uprof;
-    b.fields = h->fields;
+    if (out) {
+        for (int i = 0; i < 4; ++i) b.out[i] = out->p[i];
+        b.opitch = out->pitch;
+    }
     b.dst = pops;
     int nblk;
     // FP64 partial sums: the handle's buffer (grown on demand), or a
     // caller-provided fixed scratch area
-    double* part = nullptr;
     auto take_partials = [&](int n) -> int {
+        if (!sums) return FD_OK;
         if (scratch) {
             if (n > scratch_slots)
                 return fail(FD_E_ARG, "this launch shape needs " + std::to_string(n) +
                                           " partial-sum slots; the fixed scratch holds " +
                                           std::to_string(scratch_slots));
-            part = scratch;
+            b.partials = scratch;
             return FD_OK;
         }
         int rc = ensure_partials(h, n);
-        part = h->partials;
+        b.partials = h->partials;
         return rc;
     };
     const dim3 ngrid((h->p.W + 63) / 64, (h->p.H + 3) / 4);
@@ -1946,52 +1989,47 @@ int compute_fields(fd_handle* h, float* pops, double* scratch = nullptr, int scr
         nblk = ngrid.x * ngrid.y;
         int rc = take_partials(nblk);
         if (rc) return rc;
-        b.partials = part;
-        if (!pops) b.dst = h->pop[1 - h->cur];
         // after fd_init_fields the staged velocity (fields planes 2, 3) is
         // part of the N = 0 state; each node reads its own value before
         // writing the same one back
-        const float* ux0 = h->init_u ? h->fields + 2 * h->Q : nullptr;
-        const float* uy0 = h->init_u ? h->fields + 3 * h->Q : nullptr;
-        hipLaunchKernelGGL((init_kernel<1>), ngrid, dim3(64, 4), 0, h->stream, h->k, b, h->psi0, h->rho0,
-                           h->p.init_mode == FD_INIT_WALLED ? 1 : 0, ux0, uy0);
+        hipLaunchKernelGGL((init_kernel<1>), ngrid, dim3(64, 4), 0, h->stream, h->k, b, staged_fields(h),
+                           h->p.init_mode == FD_INIT_WALLED ? 1 : 0);
         FD_HIP(hipGetLastError());
     } else if (h->stage == kStagePops) {
         if (pops && pops != h->pop[1 - h->cur]) return fail(FD_E_STATE, "internal: staged populations elsewhere");
         nblk = ngrid.x * ngrid.y;
         int rc = take_partials(nblk);
         if (rc) return rc;
-        b.partials = part;
         hipLaunchKernelGGL((restage_kernel<0>), ngrid, dim3(64, 4), 0, h->stream, h->k, b, h->pop[1 - h->cur]);
         FD_HIP(hipGetLastError());
     } else {
         nblk = moments_grid_blocks(h);
         int rc = take_partials(nblk);
         if (rc) return rc;
-        b.partials = part;
         b.src = h->pop[h->cur];
         b.side_in = h->side[h->sc];
         rc = launch_step(h, 1, b);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(reduce_partials, dim3(1), dim3(256), 0, h->stream, part, nblk, h->mass);
-    FD_HIP(hipGetLastError());
+    if (sums) {
+        hipLaunchKernelGGL(reduce_partials, dim3(1), dim3(256), 0, h->stream, b.partials, nblk, h->mass);
+        FD_HIP(hipGetLastError());
+    }
     return FD_OK;
 }
 
 // Fields of columns [x0, x1) only (the moments pass over the strips that
-// hold them; no FP64 sums).  At N = 0 the full initial fields are used.
+// hold them).  At N = 0 the full initial fields are used.
 int compute_fields_window(fd_handle* h, int x0, int x1) {
     if (!h->inited) return fail(FD_E_STATE, "fd_init has not been called");
-    if (h->stage) return compute_fields(h, nullptr);
+    const FieldsOut out = own_fields(h);
+    if (h->stage) return compute_fields(h, &out, nullptr, false);
     const int sb_lo = (x0 / 64) / h->wx, sb_hi = ((x1 - 1) / 64) / h->wx + 1;
-    int rc = ensure_partials(h, h->wx * step_grid(h, nullptr, sb_lo, sb_hi));
-    if (rc) return rc;
     KBufs b{};
     b.flags = h->flags;
     b.uprof = h->uprof;
-    b.fields = h->fields;
-    b.partials = h->partials;
+    for (int i = 0; i < 4; ++i) b.out[i] = out.p[i];
+    b.opitch = out.pitch;
     b.src = h->pop[h->cur];
     b.side_in = h->side[h->sc];
     return launch_step(h, 1, b, sb_lo, sb_hi);
@@ -2163,8 +2201,9 @@ int init_impl(fd_handle* h, const double* psi0, const double* rho0, const double
         dux = h->fields + 2 * h->Q;
         duy = h->fields + 3 * h->Q;
     }
-    hipLaunchKernelGGL((init_kernel<0>), grid, dim3(64, 4), 0, h->stream, h->k, b, h->psi0, h->rho0,
-                       h->p.init_mode == FD_INIT_WALLED ? 1 : 0, dux, duy);
+    hipLaunchKernelGGL((init_kernel<0>), grid, dim3(64, 4), 0, h->stream, h->k, b,
+                       InitFields{h->psi0, h->rho0, dux, duy, h->Wp, {nullptr, nullptr, nullptr, nullptr}},
+                       h->p.init_mode == FD_INIT_WALLED ? 1 : 0);
     FD_HIP(hipGetLastError());
     FD_HIP(hipStreamSynchronize(h->stream));  // host staging vectors go out of scope
     h->cur = 0;
@@ -2351,9 +2390,12 @@ int fd_set_tile(fd_handle* h, int32_t waves_x, int32_t rows) {
 int fd_get_fields(fd_handle* h, float* psi, float* rho, float* ux, float* uy) {
     if (!h) return fail(FD_E_ARG, "handle is NULL");
     FD_HIP(hipSetDevice(h->device));
-    int rc = compute_fields(h, nullptr);
-    if (rc) return rc;
     float* outs[4] = {psi, rho, ux, uy};
+    FieldsOut want = own_fields(h);
+    for (int i = 0; i < 4; ++i)
+        if (!outs[i]) want.p[i] = nullptr;
+    int rc = compute_fields(h, &want, nullptr, false);
+    if (rc) return rc;
     for (int i = 0; i < 4; ++i)
         if (outs[i] && (rc = copy_plane_out(h, outs[i], h->fields + i * h->Q))) return rc;
     FD_HIP(hipStreamSynchronize(h->stream));
@@ -2382,7 +2424,7 @@ int fd_get_populations(fd_handle* h, float* f, float* g) {
     // The idle ping-pong set receives the post-stream copy; the next launch
     // overwrites it anyway.
     float* tmp = h->pop[1 - h->cur];
-    int rc = compute_fields(h, tmp);
+    int rc = compute_fields(h, nullptr, tmp, false);
     if (rc) return rc;
     for (int i = 0; i < 9; ++i) {
         if (f && (rc = copy_plane_out(h, f + (size_t)i * h->p.H * h->p.W, tmp + i * h->Q))) return rc;
@@ -2395,7 +2437,7 @@ int fd_get_populations(fd_handle* h, float* f, float* g) {
 int fd_phase_mass(fd_handle* h, double out[3]) {
     if (!h || !out) return fail(FD_E_ARG, "handle/out is NULL");
     FD_HIP(hipSetDevice(h->device));
-    int rc = compute_fields(h, nullptr);
+    int rc = compute_fields(h, nullptr, nullptr, true);
     if (rc) return rc;
     FD_HIP(hipMemcpyAsync(out, h->mass, sizeof(double) * 3, hipMemcpyDeviceToHost, h->stream));
     FD_HIP(hipStreamSynchronize(h->stream));
@@ -2444,7 +2486,7 @@ int fd_phase_mass_noalloc(fd_handle* h, double out[3]) {
     double* sp = nullptr;
     int rc = scratch_of(h->device, &sp);
     if (rc) return rc;
-    rc = compute_fields(h, nullptr, sp, kScratchSlots);
+    rc = compute_fields(h, nullptr, nullptr, true, sp, kScratchSlots);
     if (rc) return rc;
     FD_HIP(hipMemcpyAsync(out, h->mass, sizeof(double) * 3, hipMemcpyDeviceToHost, h->stream));
     FD_HIP(hipStreamSynchronize(h->stream));
@@ -2532,7 +2574,7 @@ int fd_set_populations(fd_handle* h, const float* f, const float* g) {
 int fd_watchdog(fd_handle* h, double out[2]) {
     if (!h || !out) return fail(FD_E_ARG, "handle/out is NULL");
     FD_HIP(hipSetDevice(h->device));
-    int rc = compute_fields(h, nullptr);
+    int rc = compute_fields(h, nullptr, nullptr, true);
     if (rc) return rc;
     FD_HIP(hipMemcpyAsync(out, h->mass + 2, sizeof(double) * 2, hipMemcpyDeviceToHost, h->stream));
     FD_HIP(hipStreamSynchronize(h->stream));
@@ -2612,12 +2654,24 @@ int fd_fields_device(fd_handle* h, float* psi, float* rho, float* ux, float* uy)
     FD_HIP(hipSetDevice(h->device));
     int rc = check_device_ptrs(h, {psi, rho, ux, uy});
     if (rc) return rc;
-    rc = compute_fields(h, nullptr);
-    if (rc) return rc;
     float* outs[4] = {psi, rho, ux, uy};
+    const size_t plane = (size_t)h->p.H * h->p.W;
+    bool apart = true;
+    for (int i = 0; i < 4; ++i)
+        for (int j = 0; j < i; ++j)
+            if (outs[i] && outs[j] && outs[i] < outs[j] + plane && outs[j] < outs[i] + plane) apart = false;
+    if (apart) {
+        // straight into the caller's arrays: no padded copy, no sums
+        const FieldsOut out{{psi, rho, ux, uy}, h->p.W};
+        return compute_fields(h, &out, nullptr, false);
+    }
+    // arrays that overlap are written one after the other
+    const FieldsOut own = own_fields(h);
+    rc = compute_fields(h, &own, nullptr, false);
+    if (rc) return rc;
     for (int i = 0; i < 4; ++i)
         if (outs[i])
-            FD_HIP(hipMemcpy2DAsync(outs[i], sizeof(float) * h->p.W, h->fields + i * h->Q, sizeof(float) * h->Wp,
+            FD_HIP(hipMemcpy2DAsync(outs[i], sizeof(float) * h->p.W, own.p[i], sizeof(float) * h->Wp,
                                     sizeof(float) * h->p.W, h->p.H, hipMemcpyDeviceToDevice, h->stream));
     return FD_OK;
 }
@@ -2628,21 +2682,17 @@ int fd_init_fields_device(fd_handle* h, const float* psi, const float* rho, cons
     FD_HIP(hipSetDevice(h->device));
     int rc = check_device_ptrs(h, {psi, rho, ux, uy});
     if (rc) return rc;
-    // Padding columns x >= W of the staging planes are never read by the
-    // initialisation (it covers x < W only).
-    const float* src[4] = {psi, rho, ux, uy};
-    float* dst[4] = {h->psi0, h->rho0, h->fields + 2 * h->Q, h->fields + 3 * h->Q};
-    for (int i = 0; i < 4; ++i)
-        FD_HIP(hipMemcpy2DAsync(dst[i], sizeof(float) * h->Wp, src[i], sizeof(float) * h->p.W,
-                                sizeof(float) * h->p.W, h->p.H, hipMemcpyDeviceToDevice, h->stream));
+    // one pass reads the caller's fields, starts the state and keeps the
+    // copies that the reads of N = 0 need
     KBufs b{};
     b.flags = h->flags;
     b.dst = h->pop[0];
     b.side_out = h->side[0];
     b.uprof = h->uprof;
     const dim3 grid((h->p.W + 63) / 64, (h->p.H + 3) / 4);
-    hipLaunchKernelGGL((init_kernel<0>), grid, dim3(64, 4), 0, h->stream, h->k, b, h->psi0, h->rho0,
-                       h->p.init_mode == FD_INIT_WALLED ? 1 : 0, dst[2], dst[3]);
+    hipLaunchKernelGGL((init_kernel<0>), grid, dim3(64, 4), 0, h->stream, h->k, b,
+                       InitFields{psi, rho, ux, uy, h->p.W, {h->psi0, h->rho0, h->fields + 2 * h->Q, h->fields + 3 * h->Q}},
+                       h->p.init_mode == FD_INIT_WALLED ? 1 : 0);
     FD_HIP(hipGetLastError());
     h->cur = 0;
     h->sc = 0;
