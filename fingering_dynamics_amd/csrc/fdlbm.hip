@@ -1269,6 +1269,247 @@ __global__ __launch_bounds__(64 * WPB) void fused3_kernel(KParams k, KBufs b) {
         fused3_march<WPB, true>(k, b, chunk, strip, rings);
 }
 
+// ---------------------------------------------------- tiles in LDS
+// Several iterations per launch on a tile that lives in LDS, for domains too
+// small to fill the device with marching waves: a march is a serial chain of
+// rows (about 3 us a row of the two-iteration kernel when its waves run
+// alone), while here every node of a tile is updated at once.
+//
+// A workgroup loads the post-collision populations of its tile of TW x TH
+// nodes and a margin of 2 T nodes around it (one iteration reaches two
+// nodes: one for the pull, one more for the psi stencil), runs up to T
+// iterations on them in LDS, each on a region two nodes smaller on every
+// side, and stores the tile.  Per iteration: psi of the region and a ring
+// around it (pulled g, Zou-He), then moments and collision of the region
+// from pulled f and g into registers, then the new populations over the old
+// ones, with a barrier after each.  The shape is a compile-time constant, so
+// LDS addresses are a lane's own plus immediates.
+//
+// Rows of the margin are the domain's rows, wrapped (np.roll); with walls,
+// psi across the seam between rows H-1 and 0 is psi_wall both ways, as the
+// ghost rows are.  So walls on any rows are covered, also those of
+// fingering.py:573 on rows 1 and H-2, whose rows 0 and H-1 do pull across
+// the seam.  Columns beyond Zou-He columns are ghosts: psi +1 / -1, no
+// populations (what column 0 or W-1 pulls from them is rewritten).  Columns
+// wrap when x is periodic.  Every node runs the single-iteration kernel's
+// arithmetic in the same order: results are bit for bit the same.
+__device__ __forceinline__ int wrap_far(int v, int n) {
+    while (v < 0) v += n;
+    while (v >= n) v -= n;
+    return v;
+}
+
+// Nodes a region of TW x TH nodes and T iterations holds, and its LDS words:
+// 18 populations, psi, flags (16 bits each), P of columns 0 and W-1.
+template <int TW, int TH, int T>
+struct TileDim {
+    static constexpr int RW = TW + 4 * T, RH = TH + 4 * T, NS = RW * RH;
+    static constexpr int BYTES = 4 * (NS * 19 + (NS + 1) / 2 + RH * 4);
+    static constexpr int MOST = (RW - 4) * (RH - 4);  // nodes of the first iteration's region
+};
+
+// Region node j of a w-wide rectangle with margin m, as (column, row).
+template <int w, int m>
+__device__ __forceinline__ void tile_node(int j, int& lx, int& ly) {
+    const int r = (int)(((float)j + 0.5f) * (1.0f / (float)w));
+    lx = __mul24(r, -w) + j + m;
+    ly = r + m;
+}
+
+// The shapes, by tiles of a domain (TileRule below): a domain of at most one
+// tile per CU takes the smallest shape that covers it so, larger ones the
+// last, whose LDS lets three workgroups share a CU.  Us per iteration,
+// measured, against the fastest marching kernel at its best launch shape:
+//   droplet 320 x 128      24 x 8 x 4 iterations  3.1   march 6.1
+//   channel 400 x 100      24 x 8 x 4             4.0         7.3
+//   walls on rows 1, H-2, 601 x 151   20 x 20 x 3  5.0        8.7
+//   bed 600 x 300          40 x 18 x 3            6.4        10.1
+//   flow 512 x 256         40 x 18 x 3            6.2        10.0
+//   flow 1024 x 512        24 x 13 x 2           14.1        16.3
+//   bed 1400 x 700         24 x 13 x 2           22.2        22.2
+//   flow 2048 x 1024       24 x 13 x 2           49.7        45.7
+// What bounds a tile: the latency of an iteration's two passes (LDS reads,
+// about 350 VALU operations a node in one dependent chain, three barriers)
+// and about 4 us of launch, load and store per launch.
+template <int TW, int TH, int T, int NT>
+struct TileRun {
+    using D = TileDim<TW, TH, T>;
+    static constexpr int RW = D::RW, RH = D::RH, NS = D::NS;
+    const KParams& k;
+    const KBufs& b;
+    float* pop;        // [18][NS]
+    float* psi;        // [NS]
+    float* side;       // [2 columns][RH][P_x, P_y]
+    uint16_t* flg;     // [NS]
+    int ox, oy;        // the region's first column and row
+    bool cols, rows;   // it holds a Zou-He column; a wall seam
+
+    // Pull of one distribution (P0 = 0: f, 9: g) at node i, bounced-back
+    // links applied: both candidates are read and the value selected (an
+    // address select would cost two more operations per direction).
+    __device__ __forceinline__ void pull_at(int P0, int i, unsigned links, float v[9]) const {
+        v[0] = pop[P0 * NS + i];
+#pragma unroll
+        for (int d = 1; d < 9; ++d)
+            v[d] = sel_bit(links, d - 1, pop[(P0 + fdn::OPP[d]) * NS + i],
+                           pop[(P0 + d) * NS + i - (fdn::EY[d] * RW + fdn::EX[d])]);
+    }
+
+    template <int it>
+    __device__ __forceinline__ void psi_pass() {
+        constexpr int m = 2 * it - 1, w = RW - 2 * m, n = w * (RH - 2 * m);
+#pragma unroll 1
+        for (int j = threadIdx.x; j < n; j += NT) {
+            int lx, ly;
+            tile_node<w, m>(j, lx, ly);
+            const int i = __mul24(ly, RW) + lx;
+            const unsigned fl = flg[i];
+            float g[9];
+            pull_at(9, i, fl & kLinks, g);
+            const int x = ox + lx;
+            if (cols && (x == 0 || x == k.W - 1) && !((fl & kSolid) && k.inert)) bc_g(k, wrap_far(oy + ly, k.H), x, g);
+            const float sum = g[0] + g[1] + g[2] + g[3] + g[4] + g[5] + g[6] + g[7] + g[8];
+            float v = (fl & kSolid) ? k.c.psi_wall : sum;
+            if (cols) v = x < 0 ? 1.0f : (x >= k.W ? -1.0f : v);
+            psi[i] = v;
+        }
+    }
+
+    template <int it>
+    __device__ __forceinline__ void collide_pass() {
+        constexpr int m = 2 * it, w = RW - 2 * m, n = w * (RH - 2 * m), K = (n + NT - 1) / NT;
+        float rf[K][9], rg[K][9], rp[K][2];
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            const int j = threadIdx.x + kk * NT;
+            if (j < n) {
+                int lx, ly;
+                tile_node<w, m>(j, lx, ly);
+                const int i = __mul24(ly, RW) + lx;
+                const unsigned fl = flg[i];
+                float f[9], g[9];
+                pull_at(0, i, fl & kLinks, f);
+                pull_at(9, i, fl & kLinks, g);
+                float n9[9] = {psi[i],          psi[i + 1],      psi[i + RW],     psi[i - 1],     psi[i - RW],
+                               psi[i + RW + 1], psi[i + RW - 1], psi[i - RW - 1], psi[i - RW + 1]};
+                const int x = ox + lx;
+                if (rows) {
+                    const int y = wrap_far(oy + ly, k.H);
+                    if (y == 0) n9[4] = n9[7] = n9[8] = k.c.psi_wall;
+                    if (y == k.H - 1) n9[2] = n9[5] = n9[6] = k.c.psi_wall;
+                }
+                float dpx, dpy, lap;
+                fdn::stencil(n9, dpx, dpy, lap);
+                if (cols && (x == 0 || x == k.W - 1)) {
+                    const int y = wrap_far(oy + ly, k.H);
+                    if (!((fl & kSolid) && k.inert)) bc_g(k, y, x, g);
+                    float rho_nb = 0.f;
+                    if (x == 0 && k.y_walls && (y == 0 || y == k.H - 1)) {
+                        // walled inlet corner: the adjacent row's inlet density
+                        const int d = y == 0 ? 1 : -1, ib = i + d * RW;
+                        float fb[9];
+                        pull_at(0, ib, flg[ib] & kLinks, fb);
+                        rho_nb = fdn::inlet_rho(fb, b.uprof[y + d], side[2 * (ly + d)]);
+                    }
+                    const float* sp = side + 2 * ((x == 0 ? 0 : RH) + ly);
+                    reg_bc_f(k, b, y, x, f, sp[0], sp[1], rho_nb);
+                }
+                const float mu = collide_node(k, f, g, n9[0], dpx, dpy, lap, (fl & kSolid) != 0);
+#pragma unroll
+                for (int d = 0; d < 9; ++d) {
+                    rf[kk][d] = f[d];
+                    rg[kk][d] = g[d];
+                }
+                rp[kk][0] = dpx * mu;
+                rp[kk][1] = dpy * mu;
+            }
+        }
+        if constexpr (it < T) __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            const int j = threadIdx.x + kk * NT;
+            if (j >= n) continue;
+            int lx, ly;
+            tile_node<w, m>(j, lx, ly);
+            const int x = ox + lx;
+            if constexpr (it < T) {
+                const int i = __mul24(ly, RW) + lx;
+#pragma unroll
+                for (int d = 0; d < 9; ++d) {
+                    pop[d * NS + i] = rf[kk][d];
+                    pop[(9 + d) * NS + i] = rg[kk][d];
+                }
+                if (cols && (x == 0 || x == k.W - 1)) {
+                    float* sp = side + 2 * ((x == 0 ? 0 : RH) + ly);
+                    sp[0] = rp[kk][0];
+                    sp[1] = rp[kk][1];
+                }
+            } else {
+                const int y = oy + ly;  // the tile itself: not wrapped
+                if (x >= k.W || y >= k.H) continue;
+                const int o = y * k.Wp + x;
+#pragma unroll
+                for (int d = 0; d < 9; ++d) {
+                    b.dst[d * k.Q + o] = rf[kk][d];
+                    b.dst[(9 + d) * k.Q + o] = rg[kk][d];
+                }
+                if (cols && (x == 0 || x == k.W - 1)) {
+                    const int sd = x == 0 ? 0 : 2;
+                    b.side_out[sd * k.H + y] = rp[kk][0];
+                    b.side_out[(sd + 1) * k.H + y] = rp[kk][1];
+                }
+            }
+        }
+    }
+
+    // iterations T - iters + 1 .. T of the region (fewer than T: the outer
+    // part of the margin is not needed)
+    template <int it>
+    __device__ __forceinline__ void run(int iters) {
+        if (iters >= T - it + 1) {
+            psi_pass<it>();
+            __syncthreads();
+            collide_pass<it>();
+            if constexpr (it < T) __syncthreads();
+        }
+        if constexpr (it < T) run<it + 1>(iters);
+    }
+};
+
+template <int TW, int TH, int T, int NT>
+__global__ __launch_bounds__(NT) void tile_kernel(KParams k, KBufs b, int ntx, int iters) {
+    using D = TileDim<TW, TH, T>;
+    __shared__ float tile_mem[D::BYTES / 4];
+    const int L = banded_block();
+    const int ty = L / ntx, tx = L - ty * ntx;
+    float* const psi = tile_mem + 18 * D::NS;
+    TileRun<TW, TH, T, NT> r{k, b, tile_mem, psi, psi + D::NS, nullptr, tx * TW - 2 * T, ty * TH - 2 * T, false, false};
+    r.flg = reinterpret_cast<uint16_t*>(r.side + 4 * D::RH);
+    r.cols = !k.x_periodic && (r.ox <= 0 || r.ox + D::RW >= k.W);
+    r.rows = k.y_walls && (r.oy <= 0 || r.oy + D::RH >= k.H);
+    for (int i = threadIdx.x; i < D::NS; i += NT) {
+        int lx, ly;
+        tile_node<D::RW, 0>(i, lx, ly);
+        int x = r.ox + lx;
+        if (k.x_periodic) x = wrap_far(x, k.W);
+        const bool in = x >= 0 && x < k.W;
+        const int o = wrap_far(r.oy + ly, k.H) * k.Wp + (in ? x : 0);
+        r.flg[i] = in ? b.flags[o] : (uint16_t)kSolid;
+#pragma unroll
+        for (int p = 0; p < 18; ++p) r.pop[p * D::NS + i] = b.src[p * k.Q + o];
+    }
+    if (r.cols)
+        for (int i = threadIdx.x; i < D::RH; i += NT) {
+            const int y = wrap_far(r.oy + i, k.H);
+            r.side[2 * i] = b.side_in[y];
+            r.side[2 * i + 1] = b.side_in[k.H + y];
+            r.side[2 * (D::RH + i)] = b.side_in[2 * k.H + y];
+            r.side[2 * (D::RH + i) + 1] = b.side_in[3 * k.H + y];
+        }
+    __syncthreads();
+    r.template run<1>(iters);
+}
+
 // One domain of a batched launch (an ensemble): its constants, flags,
 // inlet profile, both population and side-buffer sets, the parity of its
 // handle when the table was built, and its first logical workgroup.
@@ -1620,11 +1861,13 @@ struct fd_handle {
     int fuse = 2;   // iterations per launch of fd_step (1, 2: fused_kernel, 3: fused3_kernel)
     bool use_graph = false;            // fd_step replays captured launch pairs
     hipGraphExec_t gexec = nullptr;    // the captured pair
-    int gkey[5] = {0, 0, 0, 0, 0};     // its launch configuration
+    int gkey[6] = {0, 0, 0, 0, 0, 0};  // its launch configuration
     int fwx = 1;    // fused_kernel: waves per workgroup
     int frows = 12; // fused_kernel: output rows per wave
     int f3wx = 1;   // fused3_kernel: waves per workgroup
     int f3rows = kFuse3Rows; // fused3_kernel: output rows per wave
+    int tile = 0;   // tile shape fd_step runs (kTileShapes; 0: the marching kernels)
+    int auto_tile = 0; // the shape fd_create chose for the domain
     int timed_launches = 0;
     bool have_timing = false;
     int ens_refs = 0;  // ensembles holding this handle: fd_destroy refuses while > 0
@@ -1842,6 +2085,13 @@ int launch_fused(fd_handle* h, const KBufs& b, hipStream_t stream = nullptr, int
     return FD_OK;
 }
 
+// The fewest rows per wave, at most `most`, with which `strips` strips of H
+// rows make no more than `waves` waves.
+int rows_for(int strips, int H, int64_t waves, int most) {
+    const int64_t chunks = std::max<int64_t>(1, waves / strips);
+    return (int)std::min<int64_t>(most, (H + chunks - 1) / chunks);
+}
+
 // Waves of the three-iteration kernel the device holds at once (one-wave
 // workgroups): the quantum of its launch rounds.
 int fused3_slots(int dev, const hipDeviceProp_t& prop, int* slots) {
@@ -1873,8 +2123,51 @@ int launch_fused3(fd_handle* h, const KBufs& b, hipStream_t stream = nullptr) {
     return FD_OK;
 }
 
-// One launch of `it` iterations (1, 2 or 3) from the buffers b.
+// The tile shapes, smallest first (0: no tiles): TW, TH, iterations,
+// threads.  The rule (tile_for): the smallest shape that covers the domain
+// with at most one tile per CU, else the last up to kTileNodes nodes, where
+// the marching kernels have caught up (a flow of 1024 x 512: 14.1 us per
+// iteration against 16.3; a bed of 1400 x 700: 22.2 both).
+constexpr int kTileShapes[][4] = {{0, 0, 0, 0},      {8, 8, 4, 512},    {24, 8, 4, 1024},
+                                  {20, 20, 3, 1024}, {40, 18, 3, 1024}, {24, 13, 2, 512}};
+constexpr int kTiles = 5;
+constexpr int64_t kTileNodes = 700000;
+
+int64_t tiles_of(int H, int W, int shape) {
+    const int* t = kTileShapes[shape];
+    return (int64_t)((W + t[0] - 1) / t[0]) * ((H + t[1] - 1) / t[1]);
+}
+
+int tile_for(int H, int W, int cus) {
+    for (int i = 1; i < kTiles; ++i)
+        if (tiles_of(H, W, i) <= cus) return i;
+    return (int64_t)H * W <= kTileNodes ? kTiles : 0;
+}
+
+// One launch of tile shape h->tile: `it` iterations, at most the shape's.
+int launch_tile(fd_handle* h, int it, const KBufs& b) {
+    const int* t = kTileShapes[h->tile];
+    const int ntx = (h->p.W + t[0] - 1) / t[0];
+    const dim3 grid((unsigned)tiles_of(h->p.H, h->p.W, h->tile)), block(t[3]);
+    switch (h->tile) {
+        case 1: hipLaunchKernelGGL((tile_kernel<8, 8, 4, 512>), grid, block, 0, h->stream, h->k, b, ntx, it); break;
+        case 2: hipLaunchKernelGGL((tile_kernel<24, 8, 4, 1024>), grid, block, 0, h->stream, h->k, b, ntx, it); break;
+        case 3: hipLaunchKernelGGL((tile_kernel<20, 20, 3, 1024>), grid, block, 0, h->stream, h->k, b, ntx, it); break;
+        case 4: hipLaunchKernelGGL((tile_kernel<40, 18, 3, 1024>), grid, block, 0, h->stream, h->k, b, ntx, it); break;
+        default: hipLaunchKernelGGL((tile_kernel<24, 13, 2, 512>), grid, block, 0, h->stream, h->k, b, ntx, it); break;
+    }
+    FD_HIP(hipGetLastError());
+    return FD_OK;
+}
+
+// Iterations of one launch of fd_step.
+int launch_depth(const fd_handle* h) {
+    return h->tile ? kTileShapes[h->tile][2] : (fusable(h) ? h->fuse : 1);
+}
+
+// One launch of `it` iterations (1 .. launch_depth) from the buffers b.
 int launch_iterations(fd_handle* h, int it, const KBufs& b) {
+    if (h->tile) return launch_tile(h, it, b);
     return it == 3 ? launch_fused3(h, b) : (it == 2 ? launch_fused(h, b) : launch_step(h, 0, b));
 }
 
@@ -1893,7 +2186,7 @@ KBufs step_bufs(const fd_handle* h, int c, int sc) {
 // The captured pair of launches of `per` iterations each, from parity 0:
 // (re)captured when the launch configuration changed since the last one.
 int step_graph(fd_handle* h, int per) {
-    const int key[5] = {per, per == 3 ? h->f3wx : h->fwx, per == 3 ? h->f3rows : h->frows, h->wx, h->rows};
+    const int key[6] = {per, per == 3 ? h->f3wx : h->fwx, per == 3 ? h->f3rows : h->frows, h->wx, h->rows, h->tile};
     if (h->gexec && std::memcmp(key, h->gkey, sizeof key) == 0) return FD_OK;
     if (h->gexec) {
         (void)hipGraphExecDestroy(h->gexec);
@@ -2097,28 +2390,40 @@ int fd_create(const fd_params* p, const uint8_t* solid, const uint8_t* links, fd
     std::vector<uint16_t> fl;
     h->inert = pack_flags(*p, solid, links, h->Wp, fl);
     fill_kparams(h);
-    // Launch shapes: rows per wave chosen so that a launch has enough waves
-    // to fill the device (about 8192 for one iteration per launch, 12288 for
-    // two; measured on MI355X: 4 x 16 and 1 x 8 on 4096 x 2048, 1 row per
-    // wave on 400 x 100).  fd_set_tile / fd_set_fusion override them.
+    // Launch shapes.  The device holds 4096 waves of the one-iteration
+    // kernel, 3072 of the two-iteration and 2048 of the three-iteration one
+    // at once (its rounds); fd_set_tile / fd_set_fusion override them.
     {
-        const int64_t strips64 = (p->W + 63) / 64, strips58 = (p->W + kFuseCols - 1) / kFuseCols;
+        const int64_t strips64 = (p->W + 63) / 64;
         h->wx = strips64 >= 16 ? 4 : 1;
         h->rows = (int)std::min<int64_t>(16, std::max<int64_t>(1, (strips64 * p->H + 4096) / 8192));
         h->fwx = 1;
-        h->frows = (int)std::min<int64_t>(8, std::max<int64_t>(1, (strips58 * p->H + 6144) / 12288));
+        // Two iterations per launch: the fewest rows (at most 8) that make one
+        // round.  Us per iteration at one round and at other heights: 1400 x
+        // 700 22.2 at 6 rows (29.7 at 2, 23.3 at 8), 1024 x 512 16.3 at 4 (18.6
+        // at 3, 17.7 at 6), 600 x 300 10.1 at 2 (13.5 at 1, 12.3 at 4).
+        const int slots2 = 12 * prop.multiProcessorCount;
+        h->frows = rows_for((p->W + kFuseCols - 1) / kFuseCols, p->H, slots2, 8);
         int slots = 0;
         if ((rc = fused3_slots(dev, prop, &slots))) {
             delete h;
             return rc;
         }
+        // Three iterations per launch where ten rows per wave fill one round
+        // (1.05 M nodes; below, two iterations are as fast: 1024 x 1024 25.2
+        // us against 25.4), with the fewest rounds that leave at most 16 rows:
+        // 2048 x 1024 45.7 us at 10 rows and two rounds (48.1 at 20 and one,
+        // 50.5 two iterations at 8), 3000 x 1500 87.6 at 14, 4096 x 2048 144
+        // at 16 (kFuse3Rows).
+        const int strips3 = (p->W + kFuse3Cols - 1) / kFuse3Cols;
         h->f3rows = kFuse3Rows;
-        // three iterations per launch on domains that fill the device at
-        // least twice over with waves of 16 rows (measured on 4096 x 2048:
-        // 0.1455 ms per iteration at 1 x 16 against 0.175 with two)
-        if (geom_fusable(*p) &&
-            (int64_t)((p->W + kFuse3Cols - 1) / kFuse3Cols) * ((p->H + h->f3rows - 1) / h->f3rows) >= 2 * (int64_t)slots)
+        if (geom_fusable(*p) && (int64_t)strips3 * p->H >= 10 * (int64_t)slots) {
             h->fuse = 3;
+            int rows = kFuse3Rows + 1;
+            for (int q = 1; rows > kFuse3Rows; ++q) rows = rows_for(strips3, p->H, q * slots, p->H);
+            h->f3rows = rows;
+        }
+        h->tile = h->auto_tile = tile_for(p->H, p->W, prop.multiProcessorCount);
     }
 
     const size_t Q = h->Q, H = p->H;
@@ -2256,9 +2561,9 @@ int fd_step(fd_handle* h, int32_t nsteps) {
         return FD_OK;
     };
     if (nl > 0) FD_HIP(hipEventRecord(h->ev0, h->stream));
-    // groups of iterations go to the two- or three-iteration kernel; long
+    // groups of iterations go to the tile, two- or three-iteration kernel; long
     // loops replay a captured pair of launches (buffer parity 0 -> 1 -> 0)
-    const int per = fusable(h) ? h->fuse : 1;
+    const int per = launch_depth(h);
     int rc = FD_OK;
     if (h->use_graph && h->cur == h->sc && nl >= 4 * per) {
         if (h->cur != 0 && (rc = issue(per))) return failed(rc);
@@ -2358,6 +2663,7 @@ int fd_set_fusion(fd_handle* h, int32_t depth, int32_t waves_x, int32_t rows) {
     if (waves_x > 0 && waves_x != 1 && waves_x != 2 && waves_x != 4)
         return fail(FD_E_ARG, "waves_x must be 1, 2 or 4 (or <= 0 to keep)");
     h->fuse = depth;
+    h->tile = 0;
     if (depth == 3) {
         if (waves_x > 0) h->f3wx = waves_x;
         if (rows > 0) h->f3rows = rows;
@@ -2365,6 +2671,13 @@ int fd_set_fusion(fd_handle* h, int32_t depth, int32_t waves_x, int32_t rows) {
         if (waves_x > 0) h->fwx = waves_x;
         if (rows > 0) h->frows = rows;
     }
+    return FD_OK;
+}
+
+int fd_auto_launch(fd_handle* h, int32_t* tiles) {
+    if (!h) return fail(FD_E_ARG, "handle is NULL");
+    h->tile = h->auto_tile;
+    if (tiles) *tiles = h->tile ? 1 : 0;
     return FD_OK;
 }
 

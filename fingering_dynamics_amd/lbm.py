@@ -131,13 +131,22 @@ class Compute:
         """Iterations per launch: 3 or 2 keep the intermediate states of
         each group of iterations on chip; 1 runs one launch per iteration.
         Identical results.  waves_x / rows (> 0) set that depth's launch
-        shape.  The default depends on the domain size (``fusion``)."""
+        shape.  The default depends on the domain size (``fusion``; small
+        domains run tiles held on chip until this is called,
+        ``auto_launch``)."""
         _native.check(self._lib.fd_set_fusion(self._h, int(depth), int(waves_x), int(rows)))
+
+    def auto_launch(self):
+        """Back to the kernel chosen for the domain's size.  True if that
+        runs tiles held on chip, False if it is the one of ``fusion``."""
+        tiles = _native.ctypes.c_int32()
+        _native.check(self._lib.fd_auto_launch(self._h, _native.ctypes.byref(tiles)))
+        return bool(tiles.value)
 
     @property
     def fusion(self):
         """(iterations per launch, waves per workgroup, rows per wave) that
-        step() uses now."""
+        step() uses now, unless it runs tiles (``auto_launch``)."""
         d, w, r = (_native.ctypes.c_int32() for _ in range(3))
         _native.check(self._lib.fd_get_fusion(self._h, _native.ctypes.byref(d), _native.ctypes.byref(w),
                                               _native.ctypes.byref(r)))
@@ -150,11 +159,17 @@ class Compute:
     def autotune(self, candidates=TUNE_CANDIDATES, steps=20):
         """Time ``steps`` real iterations per launch configuration
         (depth, waves, rows) and keep the fastest; the results do not depend
-        on it, so the trial iterations are part of the run.  Returns
-        {(depth, waves, rows): ms per iteration}."""
+        on it, so the trial iterations are part of the run.  Where the
+        domain's default is tiles held on chip (``auto_launch``), that is a
+        candidate too, with the key (0, 0, 0).  Returns {(depth, waves,
+        rows): ms per iteration}."""
         times = {}
         steps -= steps % 6
         steps = max(steps, 6)
+        if self.auto_launch():
+            self.step(12)
+            self.step(steps + steps % 12)        # whole launches of any tile shape
+            times[(0, 0, 0)] = self.last_step_ms()
         for depth, wx, rows in candidates:
             if depth == 1:
                 self.set_fusion(1)
@@ -165,7 +180,9 @@ class Compute:
             self.step(steps)
             times[(depth, wx, rows)] = self.last_step_ms()
         best = min(times, key=times.get)
-        if best[0] == 1:
+        if best[0] == 0:
+            self.auto_launch()
+        elif best[0] == 1:
             self.set_fusion(1)
             self.set_tile(*best[1:])
         else:

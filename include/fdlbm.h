@@ -237,19 +237,28 @@ int fd_set_tile(fd_handle* h, int32_t waves_x, int32_t rows);
  * for triples (two intermediate states on chip); depth 1 runs one launch
  * per iteration.  The results are identical bit for bit.  waves_x (1, 2 or
  * 4; depth 3 uses 1 or 2) and rows set the launch shape of that depth's
- * kernel (<= 0 keeps the current one).  Defaults: depth 3 at 1 wave x 16
- * rows on domains that fill the device at least twice over with such waves
- * (4096 x 2048 does), else depth 2 at 1 wave x 8 rows,
- * fewer rows on domains too small to fill the device.  Domains with H < 8,
- * and walled domains whose walls are not the edge rows (the rows 1 and H-2
- * of fingering.py:573), always run depth 1.  No reference counterpart (a
- * launch control of this implementation). */
+ * kernel (<= 0 keeps the current one).  Defaults: depth 3 from about a
+ * million nodes on, at 1 wave x 10 to 16 rows, else depth 2 at 1 wave and
+ * at most 8 rows, fewer on domains too small to fill the device.  Domains
+ * with H < 8, and walled domains whose walls are not the edge rows (the rows
+ * 1 and H-2 of fingering.py:573), always run depth 1.
+ * A domain too small for these kernels to fill the device (up to about
+ * 700,000 nodes) runs tiles held in LDS instead, two to four iterations per
+ * launch, walls on any rows, until this call chooses depth and shape;
+ * fd_auto_launch returns to them.  No reference counterpart (a launch
+ * control of this implementation). */
 int fd_set_fusion(fd_handle* h, int32_t depth, int32_t waves_x, int32_t rows);
 
-/* The iterations per launch fd_step uses now (1 when the domain does not
- * allow more) and that kernel's launch shape; NULL outputs are skipped.
+/* The depth that fd_set_fusion chose, or would take by default (1 when the
+ * domain does not allow more), and that kernel's launch shape; NULL outputs
+ * are skipped.  What fd_step uses now, unless it runs tiles.
  * No reference counterpart. */
 int fd_get_fusion(const fd_handle* h, int32_t* depth, int32_t* waves_x, int32_t* rows);
+
+/* Back to the kernel that fd_create chose for the domain; *tiles (if not
+ * NULL): 1 if that runs tiles, 0 if it is the kernel of fd_get_fusion.
+ * Results are identical bit for bit.  No reference counterpart. */
+int fd_auto_launch(fd_handle* h, int32_t* tiles);
 
 /* 1 if the handle runs with inert solid nodes, 0 if solid nodes stream
  * their populations on (store-and-forward, fingering_periodic.py:455-466),
