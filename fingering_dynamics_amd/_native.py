@@ -68,6 +68,8 @@ EXPORTS = {
     "fd_ens_step_sequential": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32]),
     "fd_ens_set_tile": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32]),
     "fd_ens_set_fusion": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]),
+    "fd_ens_get_fusion": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32),
+                                         ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]),
     "fd_ens_use_graph": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32]),
     "fd_ens_synchronize": (ctypes.c_int, [ctypes.c_void_p]),
     "fd_ens_last_step_ms": (ctypes.c_double, [ctypes.c_void_p]),

@@ -3073,11 +3073,11 @@ struct fd_ensemble {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, evd = nullptr;
     EnsDomain* table = nullptr;      // single-iteration launch
-    EnsDomain* ftable = nullptr;     // two- or three-iteration launch (fdepth)
-    int nblocks = 0, fnblocks = 0, fdepth = 0;
+    EnsDomain* ftable[4] = {nullptr, nullptr, nullptr, nullptr};  // [2], [3]: that many iterations
+    int nblocks = 0, fnblocks[4] = {0, 0, 0, 0}, fdepth = 0;
     int wx = 4, rows = 16;           // single-iteration launch shape
     int fuse = 3, fwx = 1, frows = 8;  // iterations per launch, two-iteration launch shape
-    int f3wx = 1, f3rows = 26;       // three-iteration launch shape
+    int f3wx = 1, f3rows = 0;        // three-iteration launch shape (0 rows: ens_rows3)
     bool table_ok = false;
     int64_t flips = 0;               // launches since the table was built
     bool use_graph = true;
@@ -3098,17 +3098,35 @@ int ens_depth(const fd_ensemble* e) {
     return e->fuse;
 }
 
+// Rows per wave of the three-iteration batch unless set: the fewest, from 6
+// to 20, that make at most two and a half rounds of the device's 2,048
+// waves.  Us per iteration at the rule's height and at the 26 rows before:
+// 4 domains (0.57 M nodes) 23 and 52, 12 domains (3.3 M) 82 and 97, 24 (4.6
+// M) 111 and 120, 8 flows of 2048 x 256 94 and 99, 64 domains 278 and 277,
+// 48 flows 417 and 416.
+int ens_rows3(const fd_ensemble* e) {
+    if (e->f3rows > 0) return e->f3rows;
+    int r = 6;
+    for (; r < 20; ++r) {
+        int64_t waves = 0;
+        for (const fd_handle* h : e->hs)
+            waves += (int64_t)((h->p.W + kFuse3Cols - 1) / kFuse3Cols) * ((h->p.H + r - 1) / r);
+        if (waves <= 5200) break;
+    }
+    return r;
+}
+
 int ens_build(fd_ensemble* e) {
     for (hipGraphExec_t* x : {&e->exec, &e->fexec})
         if (*x) {
             (void)hipGraphExecDestroy(*x);
             *x = nullptr;
         }
-    std::vector<EnsDomain> t(e->hs.size()), ft;
-    int64_t blk = 0, fblk = 0;
-    const int depth = ens_depth(e);
-    const bool fused = depth > 1;
-    if (fused) ft.resize(e->hs.size());
+    std::vector<EnsDomain> t(e->hs.size()), ft[4];
+    int64_t blk = 0, fblk[4] = {0, 0, 0, 0};
+    const int depth = ens_depth(e), rows3 = ens_rows3(e);
+    // three iterations per launch leave remainders of two
+    for (int d = 2; d <= depth; ++d) ft[d].resize(e->hs.size());
     for (size_t i = 0; i < e->hs.size(); ++i) {
         fd_handle* h = e->hs[i];
         EnsDomain& d = t[i];
@@ -3128,50 +3146,52 @@ int ens_build(fd_ensemble* e) {
         d.blk0 = (int)blk;
         e->cur0[i] = h->cur;
         blk += (int64_t)d.k.nsb * ((h->p.H + e->rows - 1) / e->rows);
-        if (fused) {
-            EnsDomain& fd = ft[i];
+        for (int it = 2; it <= depth; ++it) {
+            EnsDomain& fd = ft[it][i];
             fd = d;
-            const int frows = depth == 3 ? e->f3rows : e->frows;
+            const int frows = it == 3 ? rows3 : e->frows;
             fd.k.rows = frows;
-            fd.k.nsb = depth == 3 ? ((h->p.W + kFuse3Cols - 1) / kFuse3Cols + e->f3wx - 1) / e->f3wx
-                                  : fused_strip_groups(h->p.W, e->fwx);
-            fd.blk0 = (int)fblk;
-            fblk += (int64_t)fd.k.nsb * ((h->p.H + frows - 1) / frows);
+            fd.k.nsb = it == 3 ? ((h->p.W + kFuse3Cols - 1) / kFuse3Cols + e->f3wx - 1) / e->f3wx
+                               : fused_strip_groups(h->p.W, e->fwx);
+            fd.blk0 = (int)fblk[it];
+            fblk[it] += (int64_t)fd.k.nsb * ((h->p.H + frows - 1) / frows);
         }
     }
-    if (blk >= ((int64_t)1 << 31) || fblk >= ((int64_t)1 << 31))
+    if (blk >= ((int64_t)1 << 31) || fblk[2] >= ((int64_t)1 << 31) || fblk[3] >= ((int64_t)1 << 31))
         return fail(FD_E_ARG, "ensemble too large for one launch");
     FD_HIP(hipMemcpyAsync(e->table, t.data(), sizeof(EnsDomain) * t.size(), hipMemcpyHostToDevice, e->stream));
-    if (fused)
-        FD_HIP(hipMemcpyAsync(e->ftable, ft.data(), sizeof(EnsDomain) * ft.size(), hipMemcpyHostToDevice,
+    for (int it = 2; it <= depth; ++it)
+        FD_HIP(hipMemcpyAsync(e->ftable[it], ft[it].data(), sizeof(EnsDomain) * ft[it].size(), hipMemcpyHostToDevice,
                               e->stream));
     FD_HIP(hipStreamSynchronize(e->stream));
     e->nblocks = (int)blk;
-    e->fnblocks = fused ? (int)fblk : 0;
+    for (int it = 2; it <= 3; ++it) e->fnblocks[it] = it <= depth ? (int)fblk[it] : 0;
     e->fdepth = depth;
     e->flips = 0;
     e->table_ok = true;
     return FD_OK;
 }
 
-// One batched launch of `it` iterations (1, or the table's depth).
+// One batched launch of `it` iterations (1 .. the table's depth).
 int ens_launch(fd_ensemble* e, int parity, int it = 1) {
     const int n = (int)e->hs.size();
     if (it == 3) {
-        const dim3 grid(e->fnblocks), block(64 * e->f3wx);
+        const dim3 grid(e->fnblocks[3]), block(64 * e->f3wx);
+        const EnsDomain* ft = e->ftable[3];
         if (e->f3wx == 2)
-            hipLaunchKernelGGL((ens_fused_kernel<2, 3>), grid, block, 0, e->stream, e->ftable, n, parity);
+            hipLaunchKernelGGL((ens_fused_kernel<2, 3>), grid, block, 0, e->stream, ft, n, parity);
         else
-            hipLaunchKernelGGL((ens_fused_kernel<1, 3>), grid, block, 0, e->stream, e->ftable, n, parity);
+            hipLaunchKernelGGL((ens_fused_kernel<1, 3>), grid, block, 0, e->stream, ft, n, parity);
         FD_HIP(hipGetLastError());
         return FD_OK;
     }
     if (it == 2) {
-        const dim3 grid(e->fnblocks), block(64 * e->fwx);
+        const dim3 grid(e->fnblocks[2]), block(64 * e->fwx);
+        const EnsDomain* ft = e->ftable[2];
         switch (e->fwx) {
-            case 1: hipLaunchKernelGGL((ens_fused_kernel<1, 2>), grid, block, 0, e->stream, e->ftable, n, parity); break;
-            case 4: hipLaunchKernelGGL((ens_fused_kernel<4, 2>), grid, block, 0, e->stream, e->ftable, n, parity); break;
-            default: hipLaunchKernelGGL((ens_fused_kernel<2, 2>), grid, block, 0, e->stream, e->ftable, n, parity); break;
+            case 1: hipLaunchKernelGGL((ens_fused_kernel<1, 2>), grid, block, 0, e->stream, ft, n, parity); break;
+            case 4: hipLaunchKernelGGL((ens_fused_kernel<4, 2>), grid, block, 0, e->stream, ft, n, parity); break;
+            default: hipLaunchKernelGGL((ens_fused_kernel<2, 2>), grid, block, 0, e->stream, ft, n, parity); break;
         }
         FD_HIP(hipGetLastError());
         return FD_OK;
@@ -3236,18 +3256,18 @@ int ens_step(fd_ensemble* e, int32_t nsteps, bool sequential) {
         }
         FD_HIP(hipEventRecord(e->ev0, e->stream));
         // iterations per launch: groups go to the two- or three-iteration
-        // kernel, a shorter remainder to the single-iteration one
+        // kernel, a shorter remainder to the kernel of that many
         const int per = e->fdepth > 1 ? e->fdepth : 1;
         if (sequential) {
             // the baseline: one launch per domain per launch step, one stream
             for (int64_t i = 0; i < nl;) {
-                const int it = nl - i >= per ? per : 1;
+                const int it = (int)std::min<int64_t>(per, nl - i);
                 for (fd_handle* h : e->hs) {
                     const KBufs b = step_bufs(h, h->cur, h->sc);
                     if (it == 3) {
                         const int wx3 = h->f3wx, rows3 = h->f3rows;
                         h->f3wx = e->f3wx;
-                        h->f3rows = e->f3rows;
+                        h->f3rows = ens_rows3(e);
                         rc = launch_fused3(h, b, e->stream);
                         h->f3wx = wx3;
                         h->f3rows = rows3;
@@ -3280,14 +3300,14 @@ int ens_step(fd_ensemble* e, int32_t nsteps, bool sequential) {
                 }
                 return r;
             };
-            if ((e->flips & 1) != 0 && (rc = one(nl >= per ? per : 1))) return rc;
+            if ((e->flips & 1) != 0 && (rc = one((int)std::min<int64_t>(per, nl)))) return rc;
             if (e->use_graph && nl - i >= 2 * per) {
                 if ((rc = ens_graph(e, per))) return rc;
                 for (; nl - i >= 2 * per; i += 2 * per, e->flips += 2, launches += 2)
                     FD_HIP(hipGraphLaunch(per > 1 ? e->fexec : e->exec, e->stream));
             }
             while (i < nl)
-                if ((rc = one(nl - i >= per ? per : 1))) return rc;
+                if ((rc = one((int)std::min<int64_t>(per, nl - i)))) return rc;
             for (fd_handle* h : e->hs) {
                 h->cur ^= (int)(launches & 1);
                 h->sc ^= (int)(launches & 1);
@@ -3342,7 +3362,7 @@ int fd_ens_create(fd_handle* const* hs, int32_t n, fd_ensemble** out) {
     FD_HIP_E(hipEventCreate(&e->ev1));
     FD_HIP_E(hipEventCreateWithFlags(&e->evd, hipEventDisableTiming));
     FD_HIP_E(hipMalloc(&e->table, sizeof(EnsDomain) * (size_t)n));
-    FD_HIP_E(hipMalloc(&e->ftable, sizeof(EnsDomain) * (size_t)n));
+    for (int it = 2; it <= 3; ++it) FD_HIP_E(hipMalloc(&e->ftable[it], sizeof(EnsDomain) * (size_t)n));
 #undef FD_HIP_E
     for (fd_handle* h : e->hs) ++h->ens_refs;
     e->counted = true;
@@ -3382,6 +3402,14 @@ int fd_ens_set_fusion(fd_ensemble* e, int32_t depth, int32_t waves_x, int32_t ro
     return FD_OK;
 }
 
+int fd_ens_get_fusion(const fd_ensemble* e, int32_t* depth, int32_t* waves_x, int32_t* rows) {
+    if (!e) return fail(FD_E_ARG, "ensemble is NULL");
+    if (depth) *depth = e->fuse;
+    if (waves_x) *waves_x = e->fuse == 3 ? e->f3wx : e->fwx;
+    if (rows) *rows = e->fuse == 3 ? ens_rows3(e) : e->frows;
+    return FD_OK;
+}
+
 int fd_ens_use_graph(fd_ensemble* e, int32_t on) {
     if (!e) return fail(FD_E_ARG, "ensemble is NULL");
     e->use_graph = on != 0;
@@ -3412,7 +3440,8 @@ void fd_ens_destroy(fd_ensemble* e) {
     if (e->exec) (void)hipGraphExecDestroy(e->exec);
     if (e->fexec) (void)hipGraphExecDestroy(e->fexec);
     if (e->table) (void)hipFree(e->table);
-    if (e->ftable) (void)hipFree(e->ftable);
+    for (EnsDomain* f : e->ftable)
+        if (f) (void)hipFree(f);
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     if (e->evd) (void)hipEventDestroy(e->evd);

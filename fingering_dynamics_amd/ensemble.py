@@ -54,8 +54,11 @@ class Ensemble:
         _native.check(self._lib.fd_ens_create(arr, len(self.computes), _native.ctypes.byref(h)))
         self._h = h
         self.tile = (4, 16)
-        self.fusion = (3, 1, 26)
-        self._shapes = {2: (1, 8), 3: (1, 26)}
+        d, w, r = (_native.ctypes.c_int32() for _ in range(3))
+        _native.check(self._lib.fd_ens_get_fusion(h, _native.ctypes.byref(d), _native.ctypes.byref(w),
+                                                  _native.ctypes.byref(r)))
+        self.fusion = (d.value, w.value, r.value)
+        self._shapes = {2: (1, 8), 3: self.fusion[1:]}
         # the device table points at every member's buffers: a member may not
         # be closed while the ensemble exists (Compute.close raises)
         for c in self.computes:

@@ -317,13 +317,17 @@ int fd_ens_set_tile(fd_ensemble* e, int32_t waves_x, int32_t rows);
  * advances triples of iterations of every domain with one launch of the
  * three-iteration kernel, depth 2 pairs with the two-iteration kernel,
  * depth 1 one iteration per launch.  waves_x and rows set that depth's
- * launch shape (<= 0 keeps the current one; defaults 1 x 26 for depth 3,
- * 1 x 8 for depth 2; depth 3 takes 1 or 2 waves).  Groups run batched only
+ * launch shape (<= 0 keeps the current one; defaults 1 x 6 to 20 rows by the
+ * ensemble's size for depth 3, 1 x 8 for depth 2; depth 3 takes 1 or 2
+ * waves).  A remainder of two iterations runs the two-iteration kernel.  Groups run batched only
  * when every domain's geometry allows the fused kernels (fd_set_fusion);
  * otherwise every launch is of one iteration.  Results are identical bit
  * for bit in every case.
  * No reference counterpart (the reference runs one domain per process). */
 int fd_ens_set_fusion(fd_ensemble* e, int32_t depth, int32_t waves_x, int32_t rows);
+
+/* The depth and the launch shape of its kernel; NULL outputs are skipped. */
+int fd_ens_get_fusion(const fd_ensemble* e, int32_t* depth, int32_t* waves_x, int32_t* rows);
 
 /* 1: replay step loops from a captured graph (default); 0: launch eagerly. */
 int fd_ens_use_graph(fd_ensemble* e, int32_t on);

@@ -126,3 +126,24 @@ def test_large_domains_march():
     assert not cm.auto_launch()
     cm.close()
 
+
+@pytest.mark.parametrize("sizes", [[(40, 90)], [(64, 200), (33, 131), (128, 70)]])
+@pytest.mark.parametrize("n", [2, 3, 5, 8, 14])
+def test_ensemble_remainders(sizes, n):
+    """A batched remainder of two iterations runs the two-iteration kernel."""
+    from fingering_dynamics_amd.ensemble import Ensemble
+    a = [_solver("walled_edge", H, W, True) for H, W in sizes]
+    b = [_solver("walled_edge", H, W, False) for H, W in sizes]
+    ens = Ensemble(a)
+    assert ens.depth == 3
+    for _ in range(2):
+        ens.step(n)
+        for c in b:
+            c.step(n)
+    ens.step_sequential(n)
+    for x, y in zip(a, b):
+        y.step(n)
+        _same(x, y)
+    ens.close()
+    for c in a + b:
+        c.close()
