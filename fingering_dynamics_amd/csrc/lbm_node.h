@@ -40,6 +40,16 @@ FD_HD float rcp(float x) {
 }
 FD_HD double rcp(double x) { return 1.0 / x; }
 
+// x between -b and b (b > 0); one v_med3_f32 in FP32 device code.
+FD_HD float clampv(float x, float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_fmed3f(x, -b, b);
+#else
+    return x < -b ? -b : (x > b ? b : x);
+#endif
+}
+FD_HD double clampv(double x, double b) { return x < -b ? -b : (x > b ? b : x); }
+
 // D2Q9 order of fingering_periodic.py:50-89.
 constexpr int EX[9] = {0, 1, 0, -1, 0, 1, -1, -1, 1};
 constexpr int EY[9] = {0, 0, 1, 0, -1, 1, 1, -1, -1};
@@ -67,8 +77,9 @@ struct Consts {
 // n[0]=C n[1]=E n[2]=N n[3]=W n[4]=S n[5]=NE n[6]=NW n[7]=SW n[8]=SE
 template <typename T>
 FD_HD void stencil(const T n[9], T& dx, T& dy, T& lap) {
-    dx = (T(4) * (n[1] - n[3]) + n[5] - n[6] - n[7] + n[8]) * (T(1) / T(12));
-    dy = (T(4) * (n[2] - n[4]) + n[5] + n[6] - n[7] - n[8]) * (T(1) / T(12));
+    const T a = n[5] - n[7], b = n[8] - n[6];
+    dx = (T(4) * (n[1] - n[3]) + (a + b)) * (T(1) / T(12));
+    dy = (T(4) * (n[2] - n[4]) + (a - b)) * (T(1) / T(12));
     lap = (T(-20) * n[0] + T(4) * (n[2] + n[4] + n[1] + n[3]) + n[5] + n[6] + n[7] + n[8]) *
           (T(1) / T(6));
 }
@@ -86,9 +97,11 @@ FD_HD T inv_tau_mix(T rho, T psi, const Consts<T>& c) {
     // wetting solids reach; with c.psi_visc = 1 the interpolation uses psi
     // clamped to the pure phases.  With the default huge bound both
     // comparisons fail and psi passes unchanged.
-    const T pv = psi < -c.psi_visc ? -c.psi_visc : (psi > c.psi_visc ? c.psi_visc : psi);
-    const T tau = T(6) * c.M * c.eta_n * rcp(rho * ((T(1) - pv) + c.M * (T(1) + pv))) + T(0.5);
-    return rcp(tau);
+    // 1/tau = y / (6 M eta + y/2) with y the denominator: one reciprocal, and
+    // 0 at the pole.
+    const T pv = clampv(psi, c.psi_visc);
+    const T y = rho * (T(2) + (c.M - T(1)) * (T(1) + pv));
+    return y * rcp(T(6) * c.M * c.eta_n + T(0.5) * y);
 }
 
 // tau_mix - 1/2 = 6 M eta / (rho ((1-psi) + M (1+psi))), with the same psi
@@ -112,8 +125,9 @@ template <typename T>
 FD_HD Mom<T> moments(const T f[9], T psi, T dpx, T dpy, T lap, const Consts<T>& c) {
     Mom<T> m;
     m.rho = f[0] + f[1] + f[2] + f[3] + f[4] + f[5] + f[6] + f[7] + f[8];
-    const T jx = f[1] - f[3] + f[5] - f[6] - f[7] + f[8];
-    const T jy = f[2] - f[4] + f[5] + f[6] - f[7] - f[8];
+    const T d57 = f[5] - f[7], d86 = f[8] - f[6];
+    const T jx = (f[1] - f[3]) + (d57 + d86);
+    const T jy = (f[2] - f[4]) + (d57 - d86);
     m.psi = psi;
     m.mu = chem_pot(psi, lap, c);
     m.fx = m.mu * dpx + c.gx;
@@ -144,51 +158,66 @@ FD_HD void equilibria(const Mom<T>& m, const Consts<T>& c, T feq[9], T geq[9]) {
     }
 }
 
-// In-place BGK collision of both distributions with Guo forcing, written
-// over the direction pairs (i, opp(i)) that share |e.u| and |e.F|:
-//   f*_i = f_i - (f_i - feq_i)/tau_mix + F_i,  g*_i = g_i - (g_i - geq_i)/tau
-//   feq_i = w_i (A_i + rho Q_i),  geq_i = w_i (B_i + psi Q_i)
-//   Q_{i,opp} = S +- 3 eu,             S = 4.5 eu^2 - 1.5 u.u
-//   F_{i,opp} = w_i fac (T +- 3 eF),   T = 9 eu eF - 3 u.F
+// In-place BGK collision of both distributions with Guo forcing:
+//   f*_i = (1 - s) f_i + s feq_i + F_i,  s = 1/tau_mix,  F_i = w_i (1 - s/2) [...]
+//   g*_i = (1 - t) g_i + t geq_i,        t = 1/tau
+// written over the direction pairs (i, opp(i)).  With the vectors
+//   J = 3 w1 (s rho u + (1 - s/2) F),  K = J + 3 w1 (1 - s/2) F
+// the part of s feq_i + F_i that is odd in e_i is (w_i/w1) e.J and the even
+// part is (w_i/w1) (s w1 A_i - u.K/2 + 3/2 (e.u)(e.K)), so that px = ux Kx,
+// py = uy Ky and the cross term ux Ky + uy Kx serve all nine directions; the
+// same for g with H = 3 w1 t psi u in place of both.  The kernels spend most
+// of their time issuing vector instructions; this form and the moments'
+// shared differences and reciprocals take 75 fewer of them per node than
+// equilibria formed for each pair (350 -> 275): 100 x 400 on tiles 8.0 ->
+// 7.7 us per iteration, 2048 x 1024 45.7 -> 43.9, 24 domains of an ensemble
+// 343 -> 325 per launch of three.  Against the FP64 oracle the error is 0.88
+// of the other form's in the mean over 30 domains (0.55 ... 1.17).
+// The factors 1 - s and s have to add up to 1 exactly or the sum of a node's
+// populations drifts: rest() rounds 1 - s and s is taken back from it, which
+// is exact (for 0 <= s <= 2).
+template <typename T>
+FD_HD T rest(T s) {
+    return T(1) - s;
+}
+
+template <typename T>
+FD_HD void relax(T f[9], T om, T a0, T a1, T px, T py, T cross, T jx, T jy) {
+    const T sp = px + py;
+    const T s13 = (a1 + px) - T(0.5) * py, s24 = (a1 + py) - T(0.5) * px;
+    const T q = T(0.25) * (a1 + sp);
+    const T s57 = q + T(0.375) * cross, s68 = q - T(0.375) * cross;
+    const T j57 = jx + jy, j68 = jy - jx;
+    f[0] = om * f[0] + (a0 - T(2) * sp);
+    f[1] = om * f[1] + (s13 + jx);
+    f[3] = om * f[3] + (s13 - jx);
+    f[2] = om * f[2] + (s24 + jy);
+    f[4] = om * f[4] + (s24 - jy);
+    f[5] = om * f[5] + (s57 + T(0.25) * j57);
+    f[7] = om * f[7] + (s57 - T(0.25) * j57);
+    f[6] = om * f[6] + (s68 + T(0.25) * j68);
+    f[8] = om * f[8] + (s68 - T(0.25) * j68);
+}
+
 template <typename T>
 FD_HD void collide(T f[9], T g[9], const Mom<T>& m, const Consts<T>& c) {
-    const T usq = m.ux * m.ux + m.uy * m.uy;
-    const T uF = m.ux * m.fx + m.uy * m.fy;
-    const T it = m.itau, ig = c.inv_tau_g;
-    const T fac = T(1) - T(0.5) * it;
-    const T A = T(3) * m.p;
-    const T B = T(3) * c.gamma * m.mu;
-    // rest direction: Q0 = -1.5 u.u, F_0 = w0 fac (-3 u.F)
     {
-        const T A0 = (m.rho - T(5) / T(3) * m.p) * T(2.25);
-        const T B0 = (m.psi - T(5) / T(3) * c.gamma * m.mu) * T(2.25);
-        const T q0 = T(-1.5) * usq;
-        const T w = W9<T>::w0;
-        const T feq = w * (A0 + m.rho * q0);
-        const T geq = w * (B0 + m.psi * q0);
-        f[0] = f[0] - (f[0] - feq) * it + w * fac * (T(-3) * uF);
-        g[0] = g[0] - (g[0] - geq) * ig;
+        const T om = rest(m.itau), s = T(1) - om;
+        const T s3 = s * (T(1) / T(3)), sr = s3 * m.rho;       // 3 w1 = 1/3
+        const T f3 = T(1) / T(3) - T(0.5) * s3;                // 3 w1 (1 - s/2)
+        const T jx = sr * m.ux + f3 * m.fx, jy = sr * m.uy + f3 * m.fy;
+        const T kx = jx + f3 * m.fx, ky = jy + f3 * m.fy;
+        // w1 A = p/3;  w0 A_0 = rho - 5/3 p
+        relax(f, om, s * (m.rho - T(5) / T(3) * m.p), s3 * m.p, m.ux * kx, m.uy * ky, m.ux * ky + m.uy * kx, jx,
+              jy);
     }
-    // pairs (1,3) (2,4) (5,7) (6,8): e = (1,0) (0,1) (1,1) (-1,1)
-    constexpr int PI[4] = {1, 2, 5, 6};
-    constexpr int PO[4] = {3, 4, 7, 8};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int i = PI[k], o = PO[k];
-        const T ex = T(EX[i]), ey = T(EY[i]);
-        const T w = W9<T>::w(i);
-        const T eu = ex * m.ux + ey * m.uy;
-        const T eF = ex * m.fx + ey * m.fy;
-        const T S = T(4.5) * eu * eu - T(1.5) * usq;
-        const T a3 = T(3) * eu;
-        const T Fs = w * fac * (T(9) * eu * eF - T(3) * uF);
-        const T Fa = w * fac * (T(3) * eF);
-        const T fp = w * (A + m.rho * (S + a3)), fm = w * (A + m.rho * (S - a3));
-        const T gp = w * (B + m.psi * (S + a3)), gm = w * (B + m.psi * (S - a3));
-        f[i] = f[i] - (f[i] - fp) * it + (Fs + Fa);
-        f[o] = f[o] - (f[o] - fm) * it + (Fs - Fa);
-        g[i] = g[i] - (g[i] - gp) * ig;
-        g[o] = g[o] - (g[o] - gm) * ig;
+    {
+        const T om = rest(c.inv_tau_g), t = T(1) - om;
+        const T t3 = t * (T(1) / T(3));
+        const T b = c.gamma * m.mu, h = t3 * m.psi;
+        const T hx = h * m.ux, hy = h * m.uy;
+        // w1 B = gamma mu / 3;  w0 B_0 = psi - 5/3 gamma mu
+        relax(g, om, t * (m.psi - T(5) / T(3) * b), t3 * b, m.ux * hx, m.uy * hy, T(2) * (m.ux * hy), hx, hy);
     }
 }
 
