@@ -127,14 +127,20 @@ __device__ __forceinline__ rsrc_t make_rsrc(const float* p, unsigned bytes) {
 // wrapped in x when x is periodic (np.roll semantics).  For Zou-He x the
 // column -1 / W reads of the first / last column land inside the
 // allocation (planes >= 1, padding columns) and are rewritten by Zou-He.
+// All ones where links bit b is set, else 0.
+__device__ __forceinline__ unsigned bit_mask(unsigned links, int b) {
+    unsigned m;
+    asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(m) : "v"(links), "i"(b));
+    return m;
+}
+
 // (links bit b set) ? a : c, as a sign-extended one-bit field extract and
 // a bitfield insert: two VALU operations and no compare into VCC (the
 // compiler turns the same expression written in C into and + compare +
 // select).
 __device__ __forceinline__ unsigned sel_bit(unsigned links, int b, unsigned a, unsigned c) {
-    unsigned m, r;
-    asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(m) : "v"(links), "i"(b));
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(c));
+    unsigned r;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(bit_mask(links, b)), "v"(a), "v"(c));
     return r;
 }
 __device__ __forceinline__ float sel_bit(unsigned links, int b, float a, float c) {
@@ -654,34 +660,58 @@ __device__ __forceinline__ void reg_pull(const float lo[9], const float mid[9], 
 // lanes 0 and 63 (their values are never used).
 constexpr int kRingSlot = 9 * 64;
 constexpr int kRingRegion = 4 * kRingSlot + 2;
+// Where plane i of the row in slot sl lies in a ring.
+struct RingAll {
+    static __device__ __forceinline__ constexpr int at(int i, int sl) { return (sl & 3) * kRingSlot + i * 64; }
+};
+// The same with the space of rows nothing reads any more left out: planes
+// pulled from the row below (2, 5, 6) are read two rows on and keep four
+// slots, the others two.  Every pull has to come before the row two above
+// it is written.
+constexpr int kRingTight = 24 * 64;
+struct RingTight {
+    static __device__ __forceinline__ constexpr int at(int i, int sl) {
+        constexpr int base[9] = {0, 2, 12, 4, 6, 16, 20, 8, 10};
+        return (base[i] + (sl & (fdn::EY[i] > 0 ? 3 : 1))) * 64;
+    }
+};
 
-// Stage B's pull of f for the node of row y at this lane from the ring:
+// Stage B's pull of f for the node of a row at this lane from the ring, sl
+// the row's slot (the rows below and above it are in the slots either side):
 // direction i from row y - e_iy at lane - e_ix, or, linked, the node's own
 // opposite population of row y (half-way bounce-back) - one LDS read at one
 // of two addresses.  Inert solid nodes pull zeros (see reg_pull).
-__device__ __forceinline__ void lds_pull(const float* ring, int y, int lane, unsigned links, float v[9]) {
+template <typename Ring = RingAll>
+__device__ __forceinline__ void lds_pull(const float* ring, int sl, int lane, unsigned links, float v[9]) {
+    const char* const at = reinterpret_cast<const char*>(ring + lane - 1);
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
-        int idx = ((y - fdn::EY[i]) & 3) * kRingSlot + i * 64 + lane - fdn::EX[i];
-        if (i > 0) idx = (int)sel_bit(links, i - 1, (unsigned)((y & 3) * kRingSlot + fdn::OPP[i] * 64 + lane), (unsigned)idx);
-        v[i] = ring[idx];
+        // the difference of the two addresses under the link's mask: with sl
+        // a constant everything but the mask is an immediate, so no address
+        // is kept in a register
+        const int c = (Ring::at(i, sl - fdn::EY[i]) + 1 - fdn::EX[i]) * 4;
+        const int own = (Ring::at(fdn::OPP[i], sl) + 1) * 4;
+        const char* p = at + c;
+        if (i > 0) p += bit_mask(links, i - 1) & (unsigned)(own - c);
+        v[i] = *reinterpret_cast<const float*>(p);
     }
 }
 
-// Inlet density (fingering_periodic.py:276-277) of the node of row y at
-// column 0 from stage A's rows y-1, y, y+1 in the ring: the adjacent-row
-// density of the walled inlet corners (fingering.py:334-364).
-__device__ __forceinline__ float ring_inlet_rho(const float* ring, int y, int lane, unsigned links, float u,
+// Inlet density (fingering_periodic.py:276-277) of the node of the row in
+// slot sl at column 0 from stage A's rows y-1, y, y+1 in the ring: the
+// adjacent-row density of the walled inlet corners (fingering.py:334-364).
+__device__ __forceinline__ float ring_inlet_rho(const float* ring, int sl, int lane, unsigned links, float u,
                                                 float px) {
     float f[9];
-    lds_pull(ring, y, lane, links, f);
+    lds_pull(ring, sl, lane, links, f);
     return fdn::inlet_rho(f, u, px);
 }
 
 // Stage B's Zou-He / walled-corner update of f at node (y, x): as bc_f,
-// with the side values P (of stage A's psi) and the corner density given.
-__device__ __forceinline__ void reg_bc_f(const KParams& k, const KBufs& b, int y, int x, float f[9], float px,
-                                         float py, float rho_nb) {
+// with the inlet profile u of the row, the side values P (of stage A's psi)
+// and the corner density given.
+__device__ __forceinline__ void reg_bc_f(const KParams& k, int y, int x, float f[9], float u, float px, float py,
+                                         float rho_nb) {
     if (k.x_periodic) return;
     if (x == 0) {
         const bool bot = k.y_walls && y == 0;
@@ -689,16 +719,94 @@ __device__ __forceinline__ void reg_bc_f(const KParams& k, const KBufs& b, int y
         float n[9], cb[9], ct[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) n[i] = cb[i] = ct[i] = f[i];
-        fdn::inlet_f(n, b.uprof[y], px, py);
+        fdn::inlet_f(n, u, px, py);
         fdn::inlet_corner_bottom_f(cb, rho_nb);
         fdn::inlet_corner_top_f(ct, rho_nb);
 #pragma unroll
         for (int i = 0; i < 9; ++i) f[i] = bot ? cb[i] : (top ? ct[i] : n[i]);
     }
     if (x == k.W - 1) {
-        fdn::outlet_f(f, b.uprof[y], px, py, k.pressure != 0, k.rho_out, k.c3);
+        fdn::outlet_f(f, u, px, py, k.pressure != 0, k.rho_out, k.c3);
         const float f2 = (k.y_walls && y == 0) ? f[4] : f[2];
         const float f4 = (k.y_walls && y == k.H - 1) ? f[2] : f[4];
+        f[2] = f2;
+        f[4] = f4;
+    }
+}
+
+// The Zou-He columns of a wave that marches along y: whether its lanes hold
+// column 0 / W-1 at all (the same for every lane), and whether this one does.
+struct ZouHe {
+    bool in, out, lane_in, lane_out;
+};
+
+// bc_g and reg_bc_f for such a wave.  Row and strip are the wave's, so only
+// the lane of the column is a select, of the three populations that the
+// formulas write; as branches over lanes with copies of all nine they cost a
+// wave at the domain's edge as many instructions again as its two collisions.
+__device__ __forceinline__ void zou_he_g(const KParams& k, const ZouHe& z, int y, float g[9]) {
+    const bool bot = k.y_walls && y == 0, top = k.y_walls && y == k.H - 1;
+    if (z.in && !(bot || top)) {
+        float n[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) n[i] = g[i];
+        fdn::inlet_g(n);
+        g[1] = z.lane_in ? n[1] : g[1];
+        g[5] = z.lane_in ? n[5] : g[5];
+        g[8] = z.lane_in ? n[8] : g[8];
+    }
+    if (z.in && (bot || top)) {
+        float cb[9], ct[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) cb[i] = ct[i] = g[i];
+        fdn::inlet_corner_bottom_g(cb);
+        fdn::inlet_corner_top_g(ct);
+#pragma unroll
+        for (int i = 1; i < 9; ++i) g[i] = z.lane_in ? (bot ? cb[i] : ct[i]) : g[i];
+    }
+    if (z.out) {
+        float n[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) n[i] = g[i];
+        fdn::outlet_g(n);
+        g[3] = z.lane_out ? n[3] : g[3];
+        g[6] = z.lane_out ? n[6] : g[6];
+        g[7] = z.lane_out ? n[7] : g[7];
+        const float g2 = bot && z.lane_out ? g[4] : g[2], g4 = top && z.lane_out ? g[2] : g[4];
+        g[2] = g2;
+        g[4] = g4;
+    }
+}
+__device__ __forceinline__ void zou_he_f(const KParams& k, const ZouHe& z, int y, float f[9], float u, float px,
+                                         float py, float rho_nb) {
+    const bool bot = k.y_walls && y == 0, top = k.y_walls && y == k.H - 1;
+    if (z.in && !(bot || top)) {
+        float n[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) n[i] = f[i];
+        fdn::inlet_f(n, u, px, py);
+        f[1] = z.lane_in ? n[1] : f[1];
+        f[5] = z.lane_in ? n[5] : f[5];
+        f[8] = z.lane_in ? n[8] : f[8];
+    }
+    if (z.in && (bot || top)) {
+        float cb[9], ct[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) cb[i] = ct[i] = f[i];
+        fdn::inlet_corner_bottom_f(cb, rho_nb);
+        fdn::inlet_corner_top_f(ct, rho_nb);
+#pragma unroll
+        for (int i = 1; i < 9; ++i) f[i] = z.lane_in ? (bot ? cb[i] : ct[i]) : f[i];
+    }
+    if (z.out) {
+        float n[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) n[i] = f[i];
+        fdn::outlet_f(n, u, px, py, k.pressure != 0, k.rho_out, k.c3);
+        f[3] = z.lane_out ? n[3] : f[3];
+        f[6] = z.lane_out ? n[6] : f[6];
+        f[7] = z.lane_out ? n[7] : f[7];
+        const float f2 = bot && z.lane_out ? f[4] : f[2], f4 = top && z.lane_out ? f[2] : f[4];
         f[2] = f2;
         f[4] = f4;
     }
@@ -863,20 +971,20 @@ __device__ __forceinline__ void fused_march(const KParams& k, const KBufs& b, in
         // walled inlet corners need the inlet density of the adjacent row:
         // the row behind stage B's first row is one it has not marched
         if (j == 3 && has_in && k.y_walls && yf - d >= 0 && yf - d < k.H)
-            rho_prev = ring_inlet_rho(fring, yf - d, lane, fr2 & kLinks, b.uprof[yf - d], pxc);
+            rho_prev = ring_inlet_rho(fring, (yf - d) & 3, lane, fr2 & kLinks, b.uprof[yf - d], pxc);
         if (j >= 4) {
             // ------------ stage B: collision of row y = r-2d
             const int y = r - 2 * d;
             const unsigned fl = fr2;
             const bool solid = (fl & kSolid) != 0;
             float f[9];
-            lds_pull(fring, y, lane, fl & kLinks, f);
+            lds_pull(fring, y & 3, lane, fl & kLinks, f);
             float rho_nb = rho_prev;
             if (has_in) {
                 // the corner met first (row 0 marching up, H-1 marching
                 // down) takes its neighbour row (ahead) from the ring
                 if (k.y_walls && y == (d > 0 ? 0 : k.H - 1))
-                    rho_nb = ring_inlet_rho(fring, y + d, lane, fr1 & kLinks, b.uprof[y + d], pxb);
+                    rho_nb = ring_inlet_rho(fring, (y + d) & 3, lane, fr1 & kLinks, b.uprof[y + d], pxb);
                 rho_prev = fdn::inlet_rho(f, b.uprof[y], pxc);
             }
             const PsiRow qa = d > 0 ? qn : qs;  // row y + 1
@@ -884,7 +992,7 @@ __device__ __forceinline__ void fused_march(const KParams& k, const KBufs& b, in
             const float nb9[9] = {qc.c, qc.r, qa.c, qc.l, qb.c, qa.r, qa.l, qb.l, qb.r};
             float dpx, dpy, lap;
             fdn::stencil(nb9, dpx, dpy, lap);
-            reg_bc_f(k, b, y, (int)ln.x, f, pxc, pyc, rho_nb);
+            reg_bc_f(k, y, (int)ln.x, f, b.uprof[y], pxc, pyc, rho_nb);
             float g[9];
 #pragma unroll
             for (int i = 0; i < 9; ++i) g[i] = gq[i];
@@ -921,15 +1029,24 @@ __global__ __launch_bounds__(64 * WPB) void fused_kernel(KParams k, KBufs b) {
 // as above; stage B (two rows behind A) keeps S_n+2 on chip - g in a second
 // register ring, f in a second LDS ring - instead of storing it; stage C
 // (two rows behind B) pulls S_n+2 from them, collides and stores S_n+3.
-// Each stage needs two columns more of the stage before it, so the 64
-// lanes hold columns x0 - 5 ... x0 + 58 and stage C's 54 output columns
-// are lanes 5..58.  For the chunk [y0, y1) stage A runs rows y0-4 ... y1+3
-// (upwards) and stage B rows y0-2 ... y1+1, which may lie beyond a walled domain's
-// edge rows (ghost rows: psi_wall, no populations) or wrap around a
-// periodic one.  The arithmetic of every node is the single-iteration
-// kernel's, in the same order, so the result equals three single-iteration
-// launches bit for bit.
-constexpr int kFuse3Cols = 54;
+// Every stage pulls from a column either side, and its psi stencil from one
+// more, so the 64 lanes hold columns x0 - 6 ... x0 + 57 and stage C's 52
+// output columns are lanes 6..57: a multiple of four, so that a row of them
+// is whole 16-byte pieces.  For the chunk [y0, y1) stage A runs rows y0-4 ...
+// y1+3 (upwards) and stage B rows y0-2 ... y1+1, which may lie beyond a
+// walled domain's edge rows (ghost rows: psi_wall, no populations) or wrap
+// around a periodic one.  The arithmetic of every node is the
+// single-iteration kernel's, in the same order, so the result equals three
+// single-iteration launches bit for bit.
+//
+// A launch of it is bound by issuing vector instructions while its waves are
+// all there (81 % of the cycles of two waves per SIMD).  What it took to get
+// there, 2048 x 1024 and 4096 x 2048, us per iteration: 43.9 and 143 before;
+// per-row values in rings of four slots, no moves, every wait exact, the
+// state's rows through LDS by 16-byte pieces (a row of 64 columns at an odd
+// offset keeps the address unit busy for 22 cycles), stores too, and edge
+// strips without branches over lanes or loads inside them: 39.0 and 132.
+constexpr int kFuse3Cols = 52;
 
 // Rows per wave of the three-iteration kernel.  Measured on 4096 x 2048 (76
 // strips, 2,048 concurrent waves), ms per iteration: 12 rows 0.153, 14
@@ -938,16 +1055,58 @@ constexpr int kFuse3Cols = 54;
 // chunk but run slower per row; shorter ones pay more extra rows.
 constexpr int kFuse3Rows = 16;
 
-// rings_all: the workgroup's LDS rings, WPB * 2 * kRingRegion floats,
-// declared by the kernel (one array whatever copies of the march it holds).
+// Rows of the state staged for a wave of the inner march: 64 columns of each
+// of the 18 planes, in pieces of four columns (16 bytes) that load straight
+// into LDS, one piece a lane: a plane's row is 17 pieces from column x0 - 8.
+constexpr int kPieces = 17;
+constexpr int kStageLoads = (9 * kPieces + 63) / 64;
+constexpr int kStageRow = 4 * kPieces;              // floats
+constexpr int kStage = 2 * kStageLoads * 256;        // floats, with the idle lanes' pieces
+// The output rows of one distribution on their way from a column per lane to
+// a piece per lane, nine planes of 13 pieces.
+constexpr int kOutPieces = kFuse3Cols / 4;
+constexpr int kOut = 9 * kFuse3Cols;                // floats
+// LDS floats of a wave: both rings and, in the inner march, the staged rows
+constexpr int kWave3 = std::max((2 * kRingRegion + 3) / 4 * 4, kStage + kOut + 2 * kRingTight + 4);
+static_assert(8 * kWave3 * 4 <= 160 * 1024, "eight waves per CU");
+
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
+// 16 bytes a lane from buffer offset voff + soff to LDS bytes lds + 16 lane
+__device__ __forceinline__ void load_to_lds(unsigned lds, unsigned voff, u4v rsrc, unsigned soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
+}
+
+__device__ __forceinline__ unsigned lds_bytes(const float* p) {
+    return (unsigned)__builtin_amdgcn_readfirstlane(
+        (int)(unsigned)(uintptr_t)(__attribute__((address_space(3))) const float*)p);
+}
+// The words of make_rsrc(p, bytes), in scalar registers.
+__device__ __forceinline__ u4v rsrc_words(const void* p, unsigned bytes) {
+    const uint64_t b = (uint64_t)p;
+    return u4v{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b),
+               (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)(b >> 32) & 0xFFFFu)), bytes,
+               (unsigned)kRsrcWord3};
+}
+
+// The wave's index in its workgroup, in a scalar register: what follows from
+// it (strip, branches) then needs no lane masks.
+__device__ __forceinline__ int uniform_wave() {
+    return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+}
+
+// rings_all: the workgroup's LDS, WPB * kWave3 floats, declared by the
+// kernel (one array whatever copies of the march it holds).
 template <int WPB, bool EDGE>
 __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, int chunk, int strip,
                                              float* rings_all) {
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = uniform_wave();
     const int xc0 = strip * kFuse3Cols;
     if (xc0 >= k.W) return;
-    const int xa = xc0 - 5 + lane;
+    const int xa = xc0 - 6 + lane;
     // !EDGE: every lane is a domain column other than 0 and W-1 (no ghost
     // column, no wrap, no Zou-He column), so the lane predicates are
     // constant and the Zou-He code is left out
@@ -957,7 +1116,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
         ln.x = (unsigned)xa;
         ln.ghost = 0.f;
     }
-    const bool cout = lane >= 5 && lane < 5 + kFuse3Cols && (!EDGE || xa < k.W);   // stage C stores this lane
+    const bool cout = lane >= 6 && lane < 6 + kFuse3Cols && (!EDGE || xa < k.W);   // stage C stores this lane
     const bool zx = !k.x_periodic;
     const bool has_in = EDGE && zx && xc0 == 0;                                     // column 0 among the outputs
     const int y0 = chunk * k.rows;
@@ -966,288 +1125,320 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
     const unsigned bytes = 18u * (unsigned)k.Q * 4u;
     const rsrc_t src = make_rsrc(b.src, bytes);
     const rsrc_t dst = make_rsrc(b.dst, bytes);
-    const PullOff po = pull_offsets(k, ln.x);
-    float* const fring = rings_all + wave * 2 * kRingRegion + 1;    // A -> B
-    float* const fring2 = fring + kRingRegion;                       // B -> C
+    using Ring = std::conditional_t<EDGE, RingAll, RingTight>;
+    float* const lds = rings_all + wave * kWave3;
+    float* const out = lds + kStage;
+    float* const fring = lds + (EDGE ? 1 : kStage + kOut + 1);               // A -> B
+    float* const fring2 = fring + (EDGE ? kRingRegion : kRingTight);         // B -> C
 
-    // Every chunk marches up.  This kernel is bound by its arithmetic, not
-    // by HBM, so the L2 reuse that alternating directions buy the
-    // two-iteration kernel is worth less here than the direction selects
-    // it costs (measured on 4096 x 2048 at 1 x 26: 0.1617 ms per iteration
-    // up-only, 0.1641 alternating).  The row expressions keep d for the
-    // reading.
-    constexpr int d = 1;
-    const int ys = d > 0 ? y0 - 4 : y1 + 3;   // stage A's first row
-    const int yfb = ys + 2 * d;               // stage B's first row
-    const int yfc = ys + 4 * d;               // stage C's first row
+    const ZouHe zh{has_in, EDGE && zx && xc0 + 57 >= k.W - 1, ln.x == 0u, ln.x == (unsigned)k.W - 1u};
+    auto ghost_row = [&](int y) { return k.y_walls && (y < 0 || y >= k.H); };
+    // flags of a row: ghost rows and columns are solid without links
+    auto flags_at = [&](int y) { return flags_of(k, b, ln, y); };
+    auto psi_at = [&](int y, unsigned fl, float g[9]) {
+        // (no column of Zou-He holds an inert solid)
+        if (EDGE && !ghost_row(y)) zou_he_g(k, zh, wrap(y, k.H), g);
+        const float s = g[0] + g[1] + g[2] + g[3] + g[4] + g[5] + g[6] + g[7] + g[8];
+        const float v = (fl & kSolid) ? k.c.psi_wall : s;
+        return lane_row(EDGE && !ln.inside && !ghost_row(y) ? ln.ghost : v);
+    };
 
-    // ---- stage A prologue: psi_n+1 of rows ys-d, ys and g of row ys
-    // GA: g pulled by stage A, two slots: at a step of phase P (= j mod 2),
-    // slot P holds row r (for the collision) and slot 1-P row r+d (for psi);
-    // the pulls of row r+2d go to slot P once its row r is consumed, so the
-    // loads in flight are never moved between registers.
-    float GA[2][9];
-    PsiRow pb, pc;
-    {
-        const int yb = ys - d;
-        const unsigned fb = flags_of(k, b, ln, yb);
-        const bool on = g_on(k, ln, yb, fb);
-        pull(src, k, 9, rows_of(k, wrap(yb, k.H)), po, fb & kLinks, on, GA[0]);
-        pb = lane_row(finish_g(k, ln, yb, fb, EDGE && on, GA[0]));
+    // Every chunk marches up: the L2 reuse that alternating directions buy
+    // the two-iteration kernel is worth less here than the direction selects
+    // it costs.
+    const int ys = y0 - 4;   // stage A's first row; stage B's is ys + 2, stage C's ys + 4
+
+    // Row y of every per-row value below lives in slot (y - ys) & 3 of its
+    // ring, in registers and in LDS, and the march is unrolled over the four
+    // phases, so nothing is moved from one row to the next: g pulled into a
+    // slot is collided there and read there by the stage behind.
+    // RG, RF: the state as stored, g of rows r ... r + 2 and f of rows r - 1
+    // ... r + 1.  G, PA, PX, PY: stage A's g (pulled, then post-collision),
+    // psi and side values; H, PB, QX, QY: stage B's; U, PC: stage C's g and
+    // psi.  FL: flags of rows r ... r + 3, FR: of rows r - 1 ... r - 4.
+    float RG[4][9], RF[4][9], G[4][9], H[4][9], U[2][9];
+    PsiRow PA[4], PB[4], PC[4];
+    float PX[4], PY[4], QX[4], QY[4];
+    unsigned FL[4], FR[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        PB[s] = PC[s] = PsiRow{0.f, 0.f, 0.f};
+        PX[s] = PY[s] = QX[s] = QY[s] = 0.f;
+        FR[s] = kSolid;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) G[s][i] = H[s][i] = U[s & 1][i] = 0.f;
     }
-    unsigned flc = flags_of(k, b, ln, ys);
-    {
-        const bool on = g_on(k, ln, ys, flc);
-        pull(src, k, 9, rows_of(k, wrap(ys, k.H)), po, flc & kLinks, on, GA[0]);
-        pc = lane_row(finish_g(k, ln, ys, flc, EDGE && on, GA[0]));
-    }
-    unsigned fla = flags_of(k, b, ln, ys + d);
-    // Flags are loaded two rows ahead: the pulls issued after stage A need
-    // the flags of row r + 2d, and a flag load issued at the top of the same
-    // step would be younger than stage C's stores of the step before, which
-    // the wait for it would then cover too (0.1543 -> 0.1455 ms per iteration
-    // on 4096 x 2048 at 1 x 16).
-    unsigned flb = flags_of(k, b, ln, ys + 2 * d);
-    // Stage A's pulls run one row ahead: the loads for row r + d are issued
-    // right after stage A of row r, so stages B and C of this row cover
-    // their latency.  The first row's are issued here.
-    float f_n[9];
-    pull(src, k, 9, rows_of(k, wrap(ys + d, k.H)), po, fla & kLinks, true, GA[1]);
-    pull(src, k, 0, rows_of(k, wrap(ys, k.H)), po, flc & kLinks, true, f_n);
-    // Stages B and C read their f rings one row ahead as well (the rows
-    // they read are complete one row earlier).
-    float fb_n[9], fc_n[9];
+    // Stages B and C read their f rings one row ahead (the rows they read
+    // are complete one row earlier).
+    float f_n[9], fb_n[9], fc_n[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) fb_n[i] = fc_n[i] = 0.f;
+    float rho_prev = 0.f, rho_prev_c = 0.f;
 
-    // A -> B: g of A's rows r (Ga), r-d (Gb), r-2d (Gc); side values P of
-    // the same rows.  Flags of rows r, r-d, ..., r-4d (ghost rows solid).
-    float Ga[9], Gb[9], Gc[9];
+    // ---- loads of the state: g of row y and f of row y - 1.  !EDGE: by
+    // pieces into LDS, and from there into registers in stage_read; EDGE:
+    // a column per lane (ghost lanes load column 0, which nothing uses),
+    // straight into registers.  Every lane loads: what inert solids and
+    // ghost rows load is never used by a node of the domain (psi and the
+    // collision of those lanes do not depend on it, and every pull of a
+    // domain node from them is a bounce-back link or rewritten by Zou-He),
+    // and inert solid nodes hold zeros in memory, which they keep.
+    const unsigned x4 = ln.inside ? ln.x * 4u : 0u;
+    u4v srsrc{};
+    unsigned sv[kStageLoads], ov[2];
+    if (!EDGE) {
+        srsrc = rsrc_words(b.src, bytes);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) Ga[i] = Gb[i] = Gc[i] = 0.f;
-    unsigned fr0 = kSolid, fr1 = kSolid, fr2 = kSolid, fr3 = kSolid, fr4 = kSolid;
-    float pxa = 0.f, pya = 0.f, pxb = 0.f, pyb = 0.f, pxc = 0.f, pyc = 0.f;
-    // stage B: psi_n+2 of rows behind (qs) and current (qc), g of the current row
-    PsiRow qs{}, qc{};
-    float gq[9];
+        for (int q = 0; q < kStageLoads; ++q) {
+            const int c = q * 64 + lane;   // lanes beyond the last piece get zeros
+            sv[q] = c < 9 * kPieces ? (unsigned)(c / kPieces * k.Q + xc0 - 8 + 4 * (c % kPieces)) * 4u : kOOB;
+        }
 #pragma unroll
-    for (int i = 0; i < 9; ++i) gq[i] = 0.f;
-    float rho_prev = 0.f;
-    // B -> C: g of B's rows r-2d (Ha), r-3d (Hb), r-4d (Hc) and their P
-    float Ha[9], Hb[9], Hc[9];
+        for (int q = 0; q < 2; ++q) {
+            const int c = q * 64 + lane;
+            ov[q] = c < 9 * kOutPieces ? (unsigned)(c / kOutPieces * k.Q + xc0 + 4 * (c % kOutPieces)) * 4u : kOOB;
+        }
+    }
+    auto row_load = [&](int P0, int y, bool all, float v[9]) {
+        const int row = wrap(y, k.H) * k.Wp + P0 * k.Q;
 #pragma unroll
-    for (int i = 0; i < 9; ++i) Ha[i] = Hb[i] = Hc[i] = 0.f;
-    float qxa = 0.f, qya = 0.f, qxb = 0.f, qyb = 0.f, qxc = 0.f, qyc = 0.f;
-    // stage C: psi_n+3 of rows behind (us) and current (uc), g of the current row
-    PsiRow us{}, uc{};
-    float gu[9];
+        for (int i = 0; i < 9; ++i)
+            if (all || fdn::EY[i] > 0)
+                v[i] = __builtin_bit_cast(float,
+                                          __builtin_amdgcn_raw_buffer_load_b32(src, x4, (row + i * k.Q) * 4, 0));
+    };
+    auto state_load = [&](int y, float g[9], float f[9]) {
+        if (EDGE) {
+            row_load(9, y, true, g);
+            row_load(0, y - 1, true, f);
+        } else {
+            const unsigned to = lds_bytes(lds), rf = (unsigned)(wrap(y - 1, k.H) * k.Wp) * 4u;
+            const unsigned rg = (unsigned)(wrap(y, k.H) * k.Wp + 9 * k.Q) * 4u;
 #pragma unroll
-    for (int i = 0; i < 9; ++i) gu[i] = 0.f;
-    float rho_prev_c = 0.f;
+            for (int q = 0; q < kStageLoads; ++q) load_to_lds(to + q * 1024, sv[q], srsrc, rf);
+#pragma unroll
+            for (int q = 0; q < kStageLoads; ++q) load_to_lds(to + (kStageLoads + q) * 1024, sv[q], srsrc, rg);
+        }
+    };
+    // Waits for every load and store of this wave so far: the loads were
+    // issued two stages ago, the last stores before them, so neither is
+    // waited for long, and later waits (which the compiler would have to
+    // make cover both on some paths) find nothing outstanding.
+    auto stage_read = [&](float g[9], float f[9]) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        asm volatile("" ::: "memory");
+        if (EDGE) return;
+        const float* const at = lds + 2 + lane;   // pieces start at column xc0 - 8
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            f[i] = at[i * kStageRow];
+            g[i] = at[kStageLoads * 256 + i * kStageRow];
+        }
+    };
+
+    // ---- stage C's stores.  EDGE: a column per lane; !EDGE: through LDS, 16
+    // bytes a lane, two instructions for nine planes (LDS serves one wave in
+    // order)
+    const float* const out_at = out + 4 * lane;
+    auto store_row = [&](const float v[9], unsigned vo, int row) {
+        if (EDGE) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[i]), dst, vo,
+                                                      (row + i * k.Q) * 4, 0);
+            return;
+        }
+        if (cout) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i) out[i * kFuse3Cols + lane - 6] = v[i];
+        }
+        asm volatile("" ::: "memory");  // other lanes' writes: the compiler keeps the order
+        float4 piece[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) piece[q] = *reinterpret_cast<const float4*>(out_at + 256 * q);
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, piece[q]), dst, ov[q], row * 4, 0);
+    };
+
+    // ---- EDGE: the inlet profile of rows r ... r - 4 (up1 ... up5) and, for stage A's
+    // Zou-He, the side values of row r of the lane's column, loaded a row
+    // ahead
+    float up0 = 0.f, up1 = 0.f, up2 = 0.f, up3 = 0.f, up4 = 0.f, up5 = 0.f, sx = 0.f, sy = 0.f;
+    const unsigned side = (zh.lane_in ? 0u : 2u) * (unsigned)k.H * 4u;   // of side_in and side_out
+    const rsrc_t sin = make_rsrc(b.side_in, 16u * (unsigned)k.H), sout = make_rsrc(b.side_out, 16u * (unsigned)k.H);
+    const rsrc_t uprof = make_rsrc(b.uprof, 4u * (unsigned)k.H);
+    // a value of column 0 (lane 6 of strip 0), kept in a scalar register
+    auto of_inlet = [](float v) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 6));
+    };
+    auto side_load = [&](int y) {
+        const int yw = wrap(y, k.H) * 4;
+        up0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(uprof, 0, yw, 0));
+        sx = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sin, side, yw, 0));
+        sy = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sin, side, yw + k.H * 4, 0));
+    };
+
+    // ---- prologue: the state's rows of the first step, psi_n+1 of rows ys -
+    // 1, ys and g of row ys.  Flags are loaded three rows ahead, of use two.
+    {
+        const unsigned fb = flags_at(ys - 1);
+#pragma unroll
+        for (int s = 0; s < 3; ++s) FL[s] = flags_at(ys + s);
+        if (EDGE) side_load(ys);
+        state_load(ys + 2, RG[2], RF[1]);
+        float lo[9];
+        row_load(9, ys - 2, false, lo);
+        row_load(9, ys - 1, true, RG[3]);
+        row_load(9, ys, true, RG[0]);
+        row_load(9, ys + 1, true, RG[1]);
+        row_load(0, ys - 1, false, RF[3]);
+        row_load(0, ys, true, RF[0]);
+        reg_pull(lo, RG[3], RG[0], fb & kLinks, G[3]);
+        PA[3] = psi_at(ys - 1, fb, G[3]);
+        reg_pull(RG[3], RG[0], RG[1], FL[0] & kLinks, G[0]);
+        PA[0] = psi_at(ys, FL[0], G[0]);
+        stage_read(RG[2], RF[1]);
+    }
 
     const int nj = (y1 - y0) + 8;
     auto step = [&](auto phase, const int j) __attribute__((always_inline)) {
-        constexpr int P = decltype(phase)::value;
-        const int r = ys + j * d;    // stage A row
-        const bool arow = !(k.y_walls && (r < 0 || r >= k.H));
-        const int rw = wrap(r, k.H);
+        constexpr int p0 = decltype(phase)::value, p1 = (p0 + 1) & 3, p2 = (p0 + 2) & 3, p3 = (p0 + 3) & 3;
+        const int r = ys + j;    // stage A row, slot p0
         // ---------------- stage A, row r
-        float Gn[9], pxn = 0.f, pyn = 0.f;
+        reg_pull(RG[p0], RG[p1], RG[p2], FL[p1] & kLinks, G[p1]);
+        reg_pull(RF[p3], RF[p0], RF[p1], FL[p0] & kLinks, f_n);
+        // what stage_read took from LDS is in registers: the next row's loads
+        if (!EDGE) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        FL[p3] = flags_at(r + 3);
+        state_load(r + 3, RG[p3], RF[p2]);
         {
-            const int ya = r + d;
-            const unsigned fl3 = flags_of(k, b, ln, ya + 2 * d);
-            // every lane loads: what inert solids, ghost rows and lanes
-            // beyond the domain load is never used by a node of the domain
-            // (psi and the collision of those lanes do not depend on it, and
-            // every pull of a domain node from them is a bounce-back link or
-            // rewritten by Zou-He), and inert solid nodes hold zeros in
-            // memory, which they keep; so no load needs a mask here
-            float (&ga)[9] = GA[1 - P];   // g pulled at row ya (issued one row ahead)
-            float (&f)[9] = f_n;          // f pulled at row r
-            const bool ga_on = g_on(k, ln, ya, fla);
-            const PsiRow pa = lane_row(finish_g(k, ln, ya, fla, EDGE && ga_on, ga));
-            const PsiRow pn = d > 0 ? pa : pb;  // row r + 1
-            const PsiRow ps = d > 0 ? pb : pa;  // row r - 1
+            const PsiRow pn = PA[p1] = psi_at(r + 1, FL[p1], G[p1]);
+            const PsiRow pc = PA[p0], ps = PA[p3];
             const float nb9[9] = {pc.c, pc.r, pn.c, pc.l, ps.c, pn.r, pn.l, ps.l, ps.r};
             float dpx, dpy, lap;
             fdn::stencil(nb9, dpx, dpy, lap);
-            if (EDGE && arow) bc_f(k, b, src, rw, (int)ln.x, f);
-#pragma unroll
-            for (int i = 0; i < 9; ++i) Gn[i] = GA[P][i];
-            const bool solid = !arow || !ln.inside || (flc & kSolid) != 0;
-            const float mu = collide_node(k, f, Gn, pc.c, dpx, dpy, lap, solid);
-            float* const slot = fring + (r & 3) * kRingSlot + lane;
-#pragma unroll
-            for (int i = 0; i < 9; ++i) slot[i * 64] = f[i];
-            pxn = dpx * mu;
-            pyn = dpy * mu;
-            pb = pc;
-            pc = pa;
-            fr4 = fr3;
-            fr3 = fr2;
-            fr2 = fr1;
-            fr1 = fr0;
-            fr0 = arow && ln.inside ? flc : kSolid;
-            flc = fla;
-            fla = flb;
-            flb = fl3;
-            // the next row's pulls (rows wrap, so the loads past the
-            // chunk's last row stay inside the allocation; they are unused)
-            pull(src, k, 9, rows_of(k, wrap(ya + d, k.H)), po, fla & kLinks, true, GA[P]);
-            pull(src, k, 0, rows_of(k, wrap(r + d, k.H)), po, flc & kLinks, true, f_n);
-        }
-#pragma unroll
-        for (int i = 0; i < 9; ++i) {
-            Gc[i] = Gb[i];
-            Gb[i] = Ga[i];
-            Ga[i] = Gn[i];
-        }
-        pxc = pxb;
-        pyc = pyb;
-        pxb = pxa;
-        pyb = pya;
-        pxa = pxn;
-        pya = pyn;
-        if (j < 2) return;
-        // ---------------- stage B: psi_n+2 and g of row r-d
-        {
-            PsiRow qn;
-            float gn[9];
-            {
-                const int yq = r - d;
-                const bool on = ln.inside && !(k.y_walls && (yq < 0 || yq >= k.H)) && !((fr1 & kSolid) && k.inert);
-                float lo[9], hi[9];
-#pragma unroll
-                for (int i = 0; i < 9; ++i) {
-                    lo[i] = d > 0 ? Gc[i] : Ga[i];
-                    hi[i] = d > 0 ? Ga[i] : Gc[i];
-                }
-                reg_pull(lo, Gb, hi, fr1 & kLinks, gn);
-                qn = lane_row(finish_g(k, ln, yq, fr1, EDGE && on, gn));
+            if (EDGE && !ghost_row(r)) {
+                const int rw = wrap(r, k.H);
+                float rho_nb = 0.f;
+                if (has_in && k.y_walls && (r == 0 || r == k.H - 1))
+                    rho_nb = inlet_rho_row(k, b, src, r == 0 ? 1 : k.H - 2);
+                zou_he_f(k, zh, rw, f_n, up0, sx, sy, rho_nb);
             }
-            if (j == 3 && has_in && k.y_walls && yfb - d >= 0 && yfb - d < k.H)
-                rho_prev = ring_inlet_rho(fring, yfb - d, lane, fr2 & kLinks, b.uprof[yfb - d], pxc);
-            float Hn[9], qxn = 0.f, qyn = 0.f;
+            const float mu = collide_node(k, f_n, G[p0], pc.c, dpx, dpy, lap, (FL[p0] & kSolid) != 0);
+            float* const slot = fring + lane;
+#pragma unroll
+            for (int i = 0; i < 9; ++i) slot[Ring::at(i, p0)] = f_n[i];
+            PX[p0] = dpx * mu;
+            PY[p0] = dpy * mu;
+            if (EDGE) {
+                up5 = up4;
+                up4 = up3;
+                up3 = up2;
+                up2 = up1;
+                up1 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, up0)));
+                side_load(r + 1);
+            }
+        }
+        const unsigned fr1 = FR[p3], fr2 = FR[p2], fr3 = FR[p1], fr4 = FR[p0];
+        FR[p0] = FL[p0];
+        if (j >= 2) {
+            // -------- stage B: psi_n+2 and g of row r - 1
+            reg_pull(G[p2], G[p3], G[p0], fr1 & kLinks, H[p3]);
+            PB[p3] = psi_at(r - 1, fr1, H[p3]);
+            // walled inlet corners need the inlet density of the adjacent
+            // row: the row behind the first row is one not marched
+            if (j == 3 && has_in && k.y_walls && ys + 1 >= 0 && ys + 1 < k.H)
+                rho_prev = of_inlet(ring_inlet_rho(fring, p2, lane, fr2 & kLinks, b.uprof[ys + 1], PX[p2]));
             if (j >= 4) {
-                // -------- stage B: collision of row y = r-2d into the rings
-                const int y = r - 2 * d;
-                const bool brow = !(k.y_walls && (y < 0 || y >= k.H));
-                const int yw = wrap(y, k.H);
-                const unsigned fl = fr2;
-                const bool solid = (fl & kSolid) != 0;
+                // -------- stage B: collision of row y = r - 2 into the rings
+                const int y = r - 2;
                 float f[9];
 #pragma unroll
                 for (int i = 0; i < 9; ++i) f[i] = fb_n[i];
-                float rho_nb = rho_prev;
-                if (has_in && brow) {
-                    if (k.y_walls && y == (d > 0 ? 0 : k.H - 1))
-                        rho_nb = ring_inlet_rho(fring, y + d, lane, fr1 & kLinks, b.uprof[y + d], pxb);
-                    rho_prev = fdn::inlet_rho(f, b.uprof[yw], pxc);
-                }
-                const PsiRow qa = d > 0 ? qn : qs;
-                const PsiRow qb = d > 0 ? qs : qn;
-                const float nb9[9] = {qc.c, qc.r, qa.c, qc.l, qb.c, qa.r, qa.l, qb.l, qb.r};
+                const PsiRow qn = PB[p3], qc = PB[p2], qs = PB[p1];
+                const float nb9[9] = {qc.c, qc.r, qn.c, qc.l, qs.c, qn.r, qn.l, qs.l, qs.r};
                 float dpx, dpy, lap;
                 fdn::stencil(nb9, dpx, dpy, lap);
-                if (EDGE && brow) reg_bc_f(k, b, yw, (int)ln.x, f, pxc, pyc, rho_nb);
+                if (EDGE && !ghost_row(y)) {
+                    float rho_nb = rho_prev;
+                    if (has_in) {
+                        if (k.y_walls && y == 0)
+                            rho_nb = ring_inlet_rho(fring, p3, lane, fr1 & kLinks, b.uprof[1], PX[p3]);
+                        rho_prev = of_inlet(fdn::inlet_rho(f, up3, PX[p2]));
+                    }
+                    zou_he_f(k, zh, wrap(y, k.H), f, up3, PX[p2], PY[p2], rho_nb);
+                }
+                const float mu = collide_node(k, f, H[p2], qc.c, dpx, dpy, lap, (fr2 & kSolid) != 0);
+                float* const slot = fring2 + lane;
 #pragma unroll
-                for (int i = 0; i < 9; ++i) Hn[i] = gq[i];
-                const float mu = collide_node(k, f, Hn, qc.c, dpx, dpy, lap, solid || !ln.inside);
-                float* const slot = fring2 + (y & 3) * kRingSlot + lane;
-#pragma unroll
-                for (int i = 0; i < 9; ++i) slot[i * 64] = f[i];
-                qxn = dpx * mu;
-                qyn = dpy * mu;
-            } else {
-#pragma unroll
-                for (int i = 0; i < 9; ++i) Hn[i] = 0.f;
+                for (int i = 0; i < 9; ++i) slot[Ring::at(i, p2)] = f[i];
+                QX[p2] = dpx * mu;
+                QY[p2] = dpy * mu;
             }
-            qs = qc;
-            qc = qn;
-#pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                gq[i] = gn[i];
-                Hc[i] = Hb[i];
-                Hb[i] = Ha[i];
-                Ha[i] = Hn[i];
-            }
-            qxc = qxb;
-            qyc = qyb;
-            qxb = qxa;
-            qyb = qya;
-            qxa = qxn;
-            qya = qyn;
-            // B's pull of the next row, r - d: rows r - 2d .. r are in the ring
-            lds_pull(fring, r - d, lane, fr1 & kLinks, fb_n);
+            // B's pull of the next row, r - 1: rows r - 2 .. r are in the ring
+            lds_pull<Ring>(fring, p3, lane, fr1 & kLinks, fb_n);
         }
-        if (j < 6) return;
-        // ---------------- stage C: psi_n+3 and g of row r-3d
-        PsiRow un;
-        float gv[9];
-        {
-            const int yq = r - 3 * d;
-            const bool on = ln.inside && !(k.y_walls && (yq < 0 || yq >= k.H)) && !((fr3 & kSolid) && k.inert);
-            float lo[9], hi[9];
+        // the state's next row, loaded during stages A and B
+        stage_read(RG[p3], RF[p2]);
+        // ---------------- stage C: psi_n+3 and g of row r - 3
+        if (j >= 6) {
+            reg_pull(H[p0], H[p1], H[p2], fr3 & kLinks, U[p1 & 1]);
+            PC[p1] = psi_at(r - 3, fr3, U[p1 & 1]);
+            if (j == 6 && has_in && k.y_walls && ys + 3 >= 0 && ys + 3 < k.H)
+                rho_prev_c = of_inlet(ring_inlet_rho(fring2, p1, lane, fr3 & kLinks, b.uprof[ys + 3], QX[p1]));
+            if (j >= 8) {
+                // ------------ stage C: collision of row y = r - 4, stored
+                const int y = r - 4;
+                float f[9], (&g)[9] = U[p0 & 1];
 #pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                lo[i] = d > 0 ? Hc[i] : Ha[i];
-                hi[i] = d > 0 ? Ha[i] : Hc[i];
+                for (int i = 0; i < 9; ++i) f[i] = fc_n[i];
+                const PsiRow un = PC[p1], uc = PC[p0], us = PC[p3];
+                const float nb9[9] = {uc.c, uc.r, un.c, uc.l, us.c, un.r, un.l, us.l, us.r};
+                float dpx, dpy, lap;
+                fdn::stencil(nb9, dpx, dpy, lap);
+                if (EDGE) {
+                    float rho_nb = rho_prev_c;
+                    if (has_in) {
+                        if (k.y_walls && y == 0)
+                            rho_nb = ring_inlet_rho(fring2, p1, lane, fr3 & kLinks, b.uprof[1], QX[p1]);
+                        rho_prev_c = of_inlet(fdn::inlet_rho(f, up5, QX[p0]));
+                    }
+                    zou_he_f(k, zh, y, f, up5, QX[p0], QY[p0], rho_nb);
+                }
+                const float mu = collide_node(k, f, g, uc.c, dpx, dpy, lap, (fr4 & kSolid) != 0);
+                if (EDGE && zx) {
+                    const unsigned so = cout && (zh.lane_in || zh.lane_out) ? side : kOOB;
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dpx * mu), sout, so, y * 4, 0);
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dpy * mu), sout, so,
+                                                          (y + k.H) * 4, 0);
+                }
+                const unsigned vo = cout && !(fr4 & kDeadPiece) ? ln.x * 4u : kOOB;
+                store_row(f, vo, y * k.Wp);
+                store_row(g, vo, y * k.Wp + 9 * k.Q);
             }
-            reg_pull(lo, Hb, hi, fr3 & kLinks, gv);
-            un = lane_row(finish_g(k, ln, yq, fr3, EDGE && on, gv));
+            // C's pull of the next row, r - 3: B wrote row r - 2 above
+            lds_pull<Ring>(fring2, p1, lane, fr3 & kLinks, fc_n);
         }
-        if (j == 6 && has_in && k.y_walls && yfc - d >= 0 && yfc - d < k.H)
-            rho_prev_c = ring_inlet_rho(fring2, yfc - d, lane, fr3 & kLinks, b.uprof[yfc - d], qxb);
-        if (j >= 8) {
-            // ------------ stage C: collision of row y = r-4d, stored
-            const int y = r - 4 * d;
-            const unsigned fl = fr4;
-            const bool solid = (fl & kSolid) != 0;
-            float f[9];
-#pragma unroll
-            for (int i = 0; i < 9; ++i) f[i] = fc_n[i];
-            float rho_nb = rho_prev_c;
-            if (has_in) {
-                if (k.y_walls && y == (d > 0 ? 0 : k.H - 1))
-                    rho_nb = ring_inlet_rho(fring2, y + d, lane, fr3 & kLinks, b.uprof[y + d], qxb);
-                rho_prev_c = fdn::inlet_rho(f, b.uprof[y], qxc);
-            }
-            const PsiRow ua = d > 0 ? un : us;
-            const PsiRow ub = d > 0 ? us : un;
-            const float nb9[9] = {uc.c, uc.r, ua.c, uc.l, ub.c, ua.r, ua.l, ub.l, ub.r};
-            float dpx, dpy, lap;
-            fdn::stencil(nb9, dpx, dpy, lap);
-            if (EDGE) reg_bc_f(k, b, y, (int)ln.x, f, qxc, qyc, rho_nb);
-            float g[9];
-#pragma unroll
-            for (int i = 0; i < 9; ++i) g[i] = gu[i];
-            const float mu = collide_node(k, f, g, uc.c, dpx, dpy, lap, solid || !ln.inside);
-            if (EDGE && cout && zx && (ln.x == 0 || ln.x == (unsigned)k.W - 1)) {
-                const int sd = (ln.x == 0) ? 0 : 2;
-                b.side_out[sd * k.H + y] = dpx * mu;
-                b.side_out[(sd + 1) * k.H + y] = dpy * mu;
-            }
-            const unsigned vo = (cout && !(fl & kDeadPiece)) ? ln.x * 4u : kOOB;
-            const int rc = y * k.Wp;
-#pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, f[i]), dst, vo, (rc + i * k.Q) * 4,
-                                                      0);
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, g[i]), dst, vo,
-                                                      (rc + (9 + i) * k.Q) * 4, 0);
-            }
-        }
-        us = uc;
-        uc = un;
-#pragma unroll
-        for (int i = 0; i < 9; ++i) gu[i] = gv[i];
-        // C's pull of the next row, r - 3d: B wrote row r - 2d above
-        lds_pull(fring2, r - 3 * d, lane, fr3 & kLinks, fc_n);
     };
-    for (int j = 0; j < nj; j += 2) {
+    for (int j = 0;; j += 4) {
         step(std::integral_constant<int, 0>(), j);
-        if (j + 1 < nj) step(std::integral_constant<int, 1>(), j + 1);
+        if (j + 1 == nj) break;
+        step(std::integral_constant<int, 1>(), j + 1);
+        if (j + 2 == nj) break;
+        step(std::integral_constant<int, 2>(), j + 2);
+        if (j + 3 == nj) break;
+        step(std::integral_constant<int, 3>(), j + 3);
+        if (j + 4 == nj) break;
     }
+}
+
+// Whether every column the march of a strip reads is an inner one: no Zou-He
+// or ghost column, no wrap.
+__device__ __forceinline__ bool fused3_inner(const KParams& k, int strip) {
+    const int x0 = strip * kFuse3Cols;
+    return x0 >= 8 && x0 + 60 <= k.W;
 }
 
 // The launch of the three-iteration march, one wave per (chunk, strip).
@@ -1257,13 +1448,12 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
 // 4096 x 2048 at 1 x 26: 0.149 ms per iteration against 0.156 with the full
 // copy everywhere.  Both copies share the workgroup's one LDS ring array.
 template <int WPB>
-__global__ __launch_bounds__(64 * WPB) void fused3_kernel(KParams k, KBufs b) {
-    __shared__ float rings[WPB * 2 * kRingRegion];
+__global__ __launch_bounds__(64 * WPB, 2) void fused3_kernel(KParams k, KBufs b) {
+    __shared__ __align__(16) float rings[WPB * kWave3];
     const int L = banded_block();
     const int chunk = L / k.nsb;
-    const int strip = (L - chunk * k.nsb) * WPB + (int)(threadIdx.x >> 6);
-    const int x0 = strip * kFuse3Cols;
-    if (x0 >= 6 && x0 + 60 <= k.W)
+    const int strip = (L - chunk * k.nsb) * WPB + uniform_wave();
+    if (fused3_inner(k, strip))
         fused3_march<WPB, false>(k, b, chunk, strip, rings);
     else
         fused3_march<WPB, true>(k, b, chunk, strip, rings);
@@ -1412,7 +1602,7 @@ struct TileRun {
                         rho_nb = fdn::inlet_rho(fb, b.uprof[y + d], side[2 * (ly + d)]);
                     }
                     const float* sp = side + 2 * ((x == 0 ? 0 : RH) + ly);
-                    reg_bc_f(k, b, y, x, f, sp[0], sp[1], rho_nb);
+                    reg_bc_f(k, y, x, f, b.uprof[y], sp[0], sp[1], rho_nb);
                 }
                 const float mu = collide_node(k, f, g, n9[0], dpx, dpy, lap, (fl & kSolid) != 0);
 #pragma unroll
@@ -1572,10 +1762,9 @@ __global__ __launch_bounds__(64 * WPB) void ens_fused_kernel(const EnsDomain* __
     b.uprof = e.uprof;
     if (DEPTH == 3) {
         const int Ld = L - e.blk0, chunk = Ld / e.k.nsb;
-        __shared__ float rings[WPB * 2 * kRingRegion];
-        const int strip = (Ld - chunk * e.k.nsb) * WPB + (int)(threadIdx.x >> 6);
-        const int x0 = strip * kFuse3Cols;
-        if (x0 >= 6 && x0 + 60 <= e.k.W)
+        __shared__ __align__(16) float rings[WPB * kWave3];
+        const int strip = (Ld - chunk * e.k.nsb) * WPB + uniform_wave();
+        if (fused3_inner(e.k, strip))
             fused3_march<WPB, false>(e.k, b, chunk, strip, rings);
         else
             fused3_march<WPB, true>(e.k, b, chunk, strip, rings);
