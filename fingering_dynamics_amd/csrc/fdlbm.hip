@@ -68,6 +68,9 @@ struct KParams {
     int rows;       // rows per wave
     int nsb;        // workgroups across x in this launch (each covers WPB strips of 64 columns)
     int sb0;        // first workgroup column of this launch (0 unless a column window)
+    // the three-iteration launch: inner strips, edge strips, rows per wave of
+    // the latter and the workgroups that run them (the first ones)
+    int nin, nes, rows_e, blk_e;
     int y_walls, x_periodic, pressure;
     int inert;      // solid nodes are never read (leak-free geometry)
     float rho_out, c3;
@@ -492,10 +495,11 @@ __device__ __forceinline__ PsiRow psi_row_of(float pcen, float halo, int lane) {
 // XCD-banded logical index of this workgroup: workgroups are dealt
 // round-robin over the eight XCDs, so XCD j runs blocks j, j+8, ...; they
 // are renumbered to one contiguous range per XCD.
-__device__ __forceinline__ int banded_block() {
-    const int nb = gridDim.x, q = nb >> 3, rem = nb & 7, xcd = blockIdx.x & 7;
-    return xcd * q + min(xcd, rem) + (blockIdx.x >> 3);
+__device__ __forceinline__ int banded(int blk, int nb) {
+    const int q = nb >> 3, rem = nb & 7, xcd = blk & 7;
+    return xcd * q + min(xcd, rem) + (blk >> 3);
 }
+__device__ __forceinline__ int banded_block() { return banded(blockIdx.x, gridDim.x); }
 
 // The march of logical workgroup L of one domain (see step_kernel).
 template <int WPB, int MODE>
@@ -1048,13 +1052,6 @@ __global__ __launch_bounds__(64 * WPB) void fused_kernel(KParams k, KBufs b) {
 // strips without branches over lanes or loads inside them: 39.0 and 132.
 constexpr int kFuse3Cols = 52;
 
-// Rows per wave of the three-iteration kernel.  Measured on 4096 x 2048 (76
-// strips, 2,048 concurrent waves), ms per iteration: 12 rows 0.153, 14
-// 0.151, 15 0.150, 16 0.1455, 17 0.148, 18 0.148, 20 0.148, 22 0.152, 24
-// 0.155, 26 0.154, 32 0.156.  Taller chunks save stage A's 8 extra rows per
-// chunk but run slower per row; shorter ones pay more extra rows.
-constexpr int kFuse3Rows = 16;
-
 // Rows of the state staged for a wave of the inner march: 64 columns of each
 // of the 18 planes, in pieces of four columns (16 bytes) that load straight
 // into LDS, one piece a lane: a plane's row is 17 pieces from column x0 - 8.
@@ -1100,12 +1097,11 @@ __device__ __forceinline__ int uniform_wave() {
 // rings_all: the workgroup's LDS, WPB * kWave3 floats, declared by the
 // kernel (one array whatever copies of the march it holds).
 template <int WPB, bool EDGE>
-__device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, int chunk, int strip,
+__device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, int y0, int rows, int strip,
                                              float* rings_all) {
     const int lane = threadIdx.x & 63;
     const int wave = uniform_wave();
     const int xc0 = strip * kFuse3Cols;
-    if (xc0 >= k.W) return;
     const int xa = xc0 - 6 + lane;
     // !EDGE: every lane is a domain column other than 0 and W-1 (no ghost
     // column, no wrap, no Zou-He column), so the lane predicates are
@@ -1119,8 +1115,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
     const bool cout = lane >= 6 && lane < 6 + kFuse3Cols && (!EDGE || xa < k.W);   // stage C stores this lane
     const bool zx = !k.x_periodic;
     const bool has_in = EDGE && zx && xc0 == 0;                                     // column 0 among the outputs
-    const int y0 = chunk * k.rows;
-    const int y1 = min(y0 + k.rows, k.H);
+    const int y1 = min(y0 + rows, k.H);
 
     const unsigned bytes = 18u * (unsigned)k.Q * 4u;
     const rsrc_t src = make_rsrc(b.src, bytes);
@@ -1434,29 +1429,34 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
     }
 }
 
-// Whether every column the march of a strip reads is an inner one: no Zou-He
-// or ghost column, no wrap.
-__device__ __forceinline__ bool fused3_inner(const KParams& k, int strip) {
-    const int x0 = strip * kFuse3Cols;
-    return x0 >= 8 && x0 + 60 <= k.W;
+// Workgroup L (of k.blk_e edge workgroups and then the inner ones) of the
+// three-iteration launch over a domain.  Inner strips are those whose lanes
+// are all columns 1 ... W-2: no Zou-He or ghost column, no wrap; they run a
+// copy of the march without that code.  Strip 0 and the last one or two run
+// the full copy, whose rows take longer, in chunks of fewer rows
+// (fuse3_grid), and start first: a launch ends with its slowest wave.
+template <int WPB>
+__device__ __forceinline__ void fused3_block(const KParams& k, const KBufs& b, int L, float* rings) {
+    const int wave = uniform_wave();
+    const bool edge = L < k.blk_e;
+    if (!edge) L -= k.blk_e;
+    const int n = edge ? k.nes : k.nin, rows = edge ? k.rows_e : k.rows;
+    const int per = (n + WPB - 1) / WPB, chunk = L / per;
+    const int s = (L - chunk * per) * WPB + wave, y0 = chunk * rows;
+    if (s >= n || y0 >= k.H) return;
+    if (edge)
+        fused3_march<WPB, true>(k, b, y0, rows, s ? k.nin + s : 0, rings);
+    else
+        fused3_march<WPB, false>(k, b, y0, rows, s + 1, rings);
 }
 
-// The launch of the three-iteration march, one wave per (chunk, strip).
-// Interior strips (all 64 lanes are columns 1 ... W-2: no Zou-He column,
-// ghost column or periodic wrap) run a copy of the march without the edge
-// code; strip 0 and the last one or two run the full copy.  Measured on
-// 4096 x 2048 at 1 x 26: 0.149 ms per iteration against 0.156 with the full
-// copy everywhere.  Both copies share the workgroup's one LDS ring array.
+// Each XCD gets a contiguous band of either kind (blk_e is a multiple of 8).
 template <int WPB>
 __global__ __launch_bounds__(64 * WPB, 2) void fused3_kernel(KParams k, KBufs b) {
     __shared__ __align__(16) float rings[WPB * kWave3];
-    const int L = banded_block();
-    const int chunk = L / k.nsb;
-    const int strip = (L - chunk * k.nsb) * WPB + uniform_wave();
-    if (fused3_inner(k, strip))
-        fused3_march<WPB, false>(k, b, chunk, strip, rings);
-    else
-        fused3_march<WPB, true>(k, b, chunk, strip, rings);
+    const int blk = blockIdx.x;
+    fused3_block<WPB>(k, b, blk < k.blk_e ? banded(blk, k.blk_e) : k.blk_e + banded(blk - k.blk_e, gridDim.x - k.blk_e),
+                      rings);
 }
 
 // ---------------------------------------------------- tiles in LDS
@@ -1761,13 +1761,8 @@ __global__ __launch_bounds__(64 * WPB) void ens_fused_kernel(const EnsDomain* __
     b.side_out = e.side[ps ^ 1];
     b.uprof = e.uprof;
     if (DEPTH == 3) {
-        const int Ld = L - e.blk0, chunk = Ld / e.k.nsb;
         __shared__ __align__(16) float rings[WPB * kWave3];
-        const int strip = (Ld - chunk * e.k.nsb) * WPB + uniform_wave();
-        if (fused3_inner(e.k, strip))
-            fused3_march<WPB, false>(e.k, b, chunk, strip, rings);
-        else
-            fused3_march<WPB, true>(e.k, b, chunk, strip, rings);
+        fused3_block<WPB>(e.k, b, L - e.blk0, rings);
     }
     else
         fused_march<WPB>(e.k, b, L - e.blk0);
@@ -2054,7 +2049,8 @@ struct fd_handle {
     int fwx = 1;    // fused_kernel: waves per workgroup
     int frows = 12; // fused_kernel: output rows per wave
     int f3wx = 1;   // fused3_kernel: waves per workgroup
-    int f3rows = kFuse3Rows; // fused3_kernel: output rows per wave
+    int f3rows = 16; // fused3_kernel: output rows per wave of inner strips
+    int f3slots = 2048; // waves of it the device holds
     int tile = 0;   // tile shape fd_step runs (kTileShapes; 0: the marching kernels)
     int auto_tile = 0; // the shape fd_create chose for the domain
     int timed_launches = 0;
@@ -2292,17 +2288,48 @@ int fused3_slots(int dev, const hipDeviceProp_t& prop, int* slots) {
     return FD_OK;
 }
 
+// Edge strips' rows per wave for `rows` of the inner ones: a row of theirs
+// takes 1.4 to 1.7 times as long.  With 22 rows in both kinds of strip 2048 x
+// 1024 takes 39.0 us per iteration, with 12 in the edge strips 29.2 (45 to 65
+// % of the rows 29.2 ... 29.3, 80 % 30.6).
+int fuse3_edge_rows(int rows) { return std::max(3, rows * 5 / 8 - 1); }
+
+// Fills the parameters of a three-iteration launch over the domain of k with
+// chunks of `rows` rows and wx waves per workgroup; the edge workgroups are
+// padded to a multiple of `pad`.  Returns the number of workgroups.
+int fuse3_grid(KParams& k, int rows, int wx, int pad) {
+    k.rows = rows;
+    k.rows_e = fuse3_edge_rows(rows);
+    k.nin = k.W >= kFuse3Cols + 60 ? (k.W - 60) / kFuse3Cols : 0;
+    k.nes = (k.W + kFuse3Cols - 1) / kFuse3Cols - k.nin;
+    const int e = (k.nes + wx - 1) / wx * ((k.H + k.rows_e - 1) / k.rows_e);
+    k.blk_e = (e + pad - 1) / pad * pad;
+    return k.blk_e + (k.nin + wx - 1) / wx * ((k.H + rows - 1) / rows);
+}
+
+// Rows per wave of the three-iteration kernel: the fewest that make one round
+// of the device's `slots` waves, or, where those are more than kFuse3Tall,
+// the fewest rounds.  Rows cost a wave 3 R + 12 stage rows, so tall chunks
+// save work, and a launch that just exceeds a round pays a whole one more:
+// 2048 x 1024 takes 29.2 us per iteration at 22 rows (one round), 38.9 at 20,
+// 32.8 at 11 (two); 1024 x 1024 15.2 at 11, 21.0 at 10; 1400 x 700 14.6 at
+// 10.  From 4 M nodes on it matters little, the clock falls with the power
+// drawn: 4096 x 2048 takes 122.5 at 86, 121.6 at 42, 120.5 at 28, 128 at 16.
+constexpr int kFuse3Tall = 64;
+
+int fuse3_rows(const KParams& k0, int H, int64_t slots) {
+    KParams k = k0;
+    for (int64_t q = 1;; ++q)
+        for (int rows = 3; rows <= kFuse3Tall; ++rows)
+            if (fuse3_grid(k, rows, 1, 8) <= q * slots - 7 || rows >= H) return rows;
+}
+
 // One launch of the three-iteration kernel (one or two waves per
 // workgroup).
 int launch_fused3(fd_handle* h, const KBufs& b, hipStream_t stream = nullptr) {
     const int wx = h->f3wx >= 2 ? 2 : 1;
     KParams k = h->k;
-    k.rows = h->f3rows;
-    const int nstrips = (h->p.W + kFuse3Cols - 1) / kFuse3Cols;
-    k.nsb = (nstrips + wx - 1) / wx;
-    k.sb0 = 0;
-    const int nchunks = (h->p.H + h->f3rows - 1) / h->f3rows;
-    const dim3 grid(k.nsb * nchunks), block(64 * wx);
+    const dim3 grid(fuse3_grid(k, h->f3rows, wx, 8)), block(64 * wx);
     if (!stream) stream = h->stream;
     if (wx == 2)
         hipLaunchKernelGGL((fused3_kernel<2>), grid, block, 0, stream, k, b);
@@ -2314,23 +2341,25 @@ int launch_fused3(fd_handle* h, const KBufs& b, hipStream_t stream = nullptr) {
 
 // The tile shapes, smallest first (0: no tiles): TW, TH, iterations,
 // threads.  The rule (tile_for): the smallest shape that covers the domain
-// with at most one tile per CU, else the last up to kTileNodes nodes, where
-// the marching kernels have caught up (a flow of 1024 x 512: 14.1 us per
-// iteration against 16.3; a bed of 1400 x 700: 22.2 both).
+// with at most one tile per CU, else the last up to the nodes where the march
+// has caught up: 240,000 where three iterations per launch are allowed (600 x
+// 300 6.2 us per iteration against 8.7, 700 x 350 9.2 against 8.8, 800 x 400
+// 10.7 against 9.0), 700,000 where it is one (walls of fingering.py:573).
 constexpr int kTileShapes[][4] = {{0, 0, 0, 0},      {8, 8, 4, 512},    {24, 8, 4, 1024},
                                   {20, 20, 3, 1024}, {40, 18, 3, 1024}, {24, 13, 2, 512}};
 constexpr int kTiles = 5;
-constexpr int64_t kTileNodes = 700000;
+constexpr int64_t kTileNodes = 240000, kTileNodes1 = 700000;
 
 int64_t tiles_of(int H, int W, int shape) {
     const int* t = kTileShapes[shape];
     return (int64_t)((W + t[0] - 1) / t[0]) * ((H + t[1] - 1) / t[1]);
 }
 
-int tile_for(int H, int W, int cus) {
+int tile_for(int H, int W, int cus, bool fusable) {
+    const int64_t most = fusable ? kTileNodes : kTileNodes1;
     for (int i = 1; i < kTiles; ++i)
-        if (tiles_of(H, W, i) <= cus) return i;
-    return (int64_t)H * W <= kTileNodes ? kTiles : 0;
+        if (tiles_of(H, W, i) <= cus && (int64_t)H * W <= most) return i;
+    return (int64_t)H * W <= most ? kTiles : 0;
 }
 
 // One launch of tile shape h->tile: `it` iterations, at most the shape's.
@@ -2598,21 +2627,13 @@ int fd_create(const fd_params* p, const uint8_t* solid, const uint8_t* links, fd
             delete h;
             return rc;
         }
-        // Three iterations per launch where ten rows per wave fill one round
-        // (1.05 M nodes; below, two iterations are as fast: 1024 x 1024 25.2
-        // us against 25.4), with the fewest rounds that leave at most 16 rows:
-        // 2048 x 1024 45.7 us at 10 rows and two rounds (48.1 at 20 and one,
-        // 50.5 two iterations at 8), 3000 x 1500 87.6 at 14, 4096 x 2048 144
-        // at 16 (kFuse3Rows).
-        const int strips3 = (p->W + kFuse3Cols - 1) / kFuse3Cols;
-        h->f3rows = kFuse3Rows;
-        if (geom_fusable(*p) && (int64_t)strips3 * p->H >= 10 * (int64_t)slots) {
-            h->fuse = 3;
-            int rows = kFuse3Rows + 1;
-            for (int q = 1; rows > kFuse3Rows; ++q) rows = rows_for(strips3, p->H, q * slots, p->H);
-            h->f3rows = rows;
-        }
-        h->tile = h->auto_tile = tile_for(p->H, p->W, prop.multiProcessorCount);
+        // Three iterations per launch wherever the geometry allows it and no
+        // tiles are used: 1400 x 700 14.6 us per iteration against 20.3 with
+        // two, 1000 x 500 10.7 against 14.1.
+        h->f3slots = slots;
+        h->f3rows = fuse3_rows(h->k, p->H, slots);
+        if (geom_fusable(*p)) h->fuse = 3;
+        h->tile = h->auto_tile = tile_for(p->H, p->W, prop.multiProcessorCount, geom_fusable(*p));
     }
 
     const size_t Q = h->Q, H = p->H;
@@ -3287,22 +3308,26 @@ int ens_depth(const fd_ensemble* e) {
     return e->fuse;
 }
 
-// Rows per wave of the three-iteration batch unless set: the fewest, from 6
-// to 20, that make at most two and a half rounds of the device's 2,048
-// waves.  Us per iteration at the rule's height and at the 26 rows before:
-// 4 domains (0.57 M nodes) 23 and 52, 12 domains (3.3 M) 82 and 97, 24 (4.6
-// M) 111 and 120, 8 flows of 2048 x 256 94 and 99, 64 domains 278 and 277,
-// 48 flows 417 and 416.
+// Rows per wave of the three-iteration batch unless set: the fewest that make
+// one round of the device's waves up to 64 rows, or two rounds up to 32, or
+// 20 (domains of different heights: a tall chunk that starts late ends the
+// launch).  Us per iteration at the rule's height and others: 4 domains (0.57
+// M nodes) 14.0 at 7 rows, 21 at 4; 12 (3.3 M) 53.8 at 40, 54.6 at 18 (two
+// rounds), 65 at 9; 24 (4.6 M) 80.1 at 26, 91 at 9; 8 flows of 2048 x 256
+// 61.6 at 44, 74 at 12; 64 domains (13.6 M) 214 at 20, 209 at 16, 235 at 64;
+// 48 flows 380 at 20, 372 at 32.
 int ens_rows3(const fd_ensemble* e) {
     if (e->f3rows > 0) return e->f3rows;
-    int r = 6;
-    for (; r < 20; ++r) {
-        int64_t waves = 0;
-        for (const fd_handle* h : e->hs)
-            waves += (int64_t)((h->p.W + kFuse3Cols - 1) / kFuse3Cols) * ((h->p.H + r - 1) / r);
-        if (waves <= 5200) break;
-    }
-    return r;
+    for (int q = 1, most = 64; q <= 2; ++q, most = 32)
+        for (int rows = 4; rows <= most; ++rows) {
+            int64_t waves = 0;
+            for (const fd_handle* h : e->hs) {
+                KParams k = h->k;
+                waves += fuse3_grid(k, rows, 1, 1);
+            }
+            if (waves <= (int64_t)q * (e->hs[0]->f3slots - 7)) return rows;
+        }
+    return 20;
 }
 
 int ens_build(fd_ensemble* e) {
@@ -3340,10 +3365,13 @@ int ens_build(fd_ensemble* e) {
             fd = d;
             const int frows = it == 3 ? rows3 : e->frows;
             fd.k.rows = frows;
-            fd.k.nsb = it == 3 ? ((h->p.W + kFuse3Cols - 1) / kFuse3Cols + e->f3wx - 1) / e->f3wx
-                               : fused_strip_groups(h->p.W, e->fwx);
             fd.blk0 = (int)fblk[it];
-            fblk[it] += (int64_t)fd.k.nsb * ((h->p.H + frows - 1) / frows);
+            if (it == 3) {
+                fblk[3] += fuse3_grid(fd.k, rows3, e->f3wx, 1);
+            } else {
+                fd.k.nsb = fused_strip_groups(h->p.W, e->fwx);
+                fblk[2] += (int64_t)fd.k.nsb * ((h->p.H + frows - 1) / frows);
+            }
         }
     }
     if (blk >= ((int64_t)1 << 31) || fblk[2] >= ((int64_t)1 << 31) || fblk[3] >= ((int64_t)1 << 31))

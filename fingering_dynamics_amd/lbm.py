@@ -159,9 +159,10 @@ class Compute:
     def autotune(self, candidates=TUNE_CANDIDATES, steps=20):
         """Time ``steps`` real iterations per launch configuration
         (depth, waves, rows) and keep the fastest; the results do not depend
-        on it, so the trial iterations are part of the run.  Where the
-        domain's default is tiles held on chip (``auto_launch``), that is a
-        candidate too, with the key (0, 0, 0).  Returns {(depth, waves,
+        on it, so the trial iterations are part of the run.  The current
+        marching configuration is a candidate too, or, where the domain's
+        default is tiles held on chip (``auto_launch``), those, with the key
+        (0, 0, 0).  Returns {(depth, waves,
         rows): ms per iteration}."""
         times = {}
         steps -= steps % 6
@@ -170,6 +171,8 @@ class Compute:
             self.step(12)
             self.step(steps + steps % 12)        # whole launches of any tile shape
             times[(0, 0, 0)] = self.last_step_ms()
+        elif self.fusion[0] > 1:
+            candidates = (self.fusion,) + tuple(candidates)
         for depth, wx, rows in candidates:
             if depth == 1:
                 self.set_fusion(1)

@@ -19,13 +19,13 @@ def _domain(kind, H, W):
                                               outlet=OUTLET_PRESSURE, psi_visc_bound=1.0)
     mask, bits, _ = rect_domain(H, W, max(2, H * W // 500), size=4, seed=W, x_min=14)
     if kind == "x_periodic":
-        return mask, bits, LbmParams.periodic(H, W, M=5.0, psi_wall=0.0, x_bc=X_PERIODIC, gx=1e-6)
-    if kind == "gauss":
-        return mask, bits, LbmParams.periodic(H, W, M=5.0, psi_wall=0.0, n_inv_cols=10)
+        return mask, bits, LbmParams.periodic(H, W, M=5.0, psi_wall=0.0, x_bc=X_PERIODIC, gx=1e-6, profile=PROFILE_CONST)
+    if kind == "rects":
+        return mask, bits, LbmParams.periodic(H, W, M=5.0, psi_wall=0.0, n_inv_cols=10, profile=PROFILE_CONST)
     return mask, bits, LbmParams.walled(H, W, shipped_walls=False, M=20.0, psi_wall=-0.5, gamma=1.0027)
 
 
-@pytest.mark.parametrize("kind", ["gauss", "circles", "walled", "x_periodic"])
+@pytest.mark.parametrize("kind", ["rects", "circles", "walled", "x_periodic"])
 @pytest.mark.parametrize("H,W,waves,rows", [(23, 111, 1, 5), (23, 112, 1, 7), (40, 113, 2, 40), (31, 156, 1, 1),
                                             (31, 163, 2, 3), (64, 164, 1, 16), (64, 165, 1, 22), (50, 320, 2, 9),
                                             (97, 333, 1, 80)])

@@ -61,7 +61,7 @@ CASES = [("open", 3, 3), ("open", 4, 5), ("open", 9, 37), ("open_x", 3, 4), ("op
          ("circles", 60, 131), ("walled_edge", 40, 150), ("walled_shipped", 41, 99), ("x_periodic", 30, 70),
          ("gauss", 100, 401), ("walled_shipped", 99, 400), ("circles", 151, 601), ("walled_edge", 163, 515),
          ("walled_shipped", 151, 601), ("x_periodic", 150, 450), ("gauss", 300, 599), ("walled_edge", 299, 560),
-         ("circles", 418, 703), ("walled_shipped", 399, 801), ("x_periodic", 420, 700)]
+         ("circles", 330, 703), ("walled_shipped", 399, 801), ("x_periodic", 330, 700)]
 
 
 @pytest.mark.parametrize("kind,H,W", CASES)
