@@ -598,6 +598,7 @@ __global__ __launch_bounds__(256) void cast_flip(CastFlipArgs a) {
     const int Cin = a.cin[l], Cout = a.cout[l];
     const uint16_t v = to_bf16(a.w[l][j]);
     a.w16[l][j] = v;
+    if (!a.wt[l]) return;
     const int ci = (int)(j % Cin);
     const int tap = (int)((j / Cin) % 9);
     const int co = (int)(j / (9 * (int64_t)Cin));
@@ -1343,6 +1344,48 @@ __global__ __launch_bounds__(256) void pool_skip_bwd(const uint16_t* __restrict_
     reinterpret_cast<u4v*>(out)[i] = r;
 }
 
+// y[n][h][w][c] = the mean of x over each 2 x 2 block: the four values added
+// in the order of torch's mean over those two axes (row by row, in float),
+// times 1/4, rounded to bf16.  One 8-channel piece per thread; at batch 64
+// the three pools of the network take 55 us (torch's mean 97).
+__global__ __launch_bounds__(256) void avg_pool2(const uint16_t* __restrict__ x, uint16_t* __restrict__ y, int W, int G,
+                                                 int64_t n8) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n8) return;
+    const int64_t q = i / G;               // output pixel
+    const int g = (int)(i - q * G), w2 = W / 2;
+    const int64_t row = q / w2;            // output row of the batch: input rows 2 row, 2 row + 1
+    const int w = (int)(q - row * w2);
+    const u4v* const d = reinterpret_cast<const u4v*>(x) + (2 * row * W + 2 * w) * G + g;
+    const u4v a = d[0], b = d[G], c = d[(int64_t)W * G], e = d[(int64_t)(W + 1) * G];
+    u4v r;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float lo = ((bf_lo(a[k]) + bf_lo(b[k])) + bf_lo(c[k])) + bf_lo(e[k]);
+        const float hi = ((bf_hi(a[k]) + bf_hi(b[k])) + bf_hi(c[k])) + bf_hi(e[k]);
+        r[k] = (unsigned)to_bf16(lo * 0.25f) | ((unsigned)to_bf16(hi * 0.25f) << 16);
+    }
+    reinterpret_cast<u4v*>(y)[i] = r;
+}
+
+// The network's input: per pixel psi, ux s, uy s, solid, lm, th and two
+// zeros, each rounded to bf16 (s the reciprocal of the velocity scale, lm and
+// th one value per sample or for all).  One 16-byte store per thread, where
+// ten tensor operations each made a pass over 4-byte channels.
+__global__ __launch_bounds__(256) void net_inputs(const float* __restrict__ psi, const float* __restrict__ ux,
+                                                  const float* __restrict__ uy, const float* __restrict__ solid,
+                                                  const float* __restrict__ lm, const float* __restrict__ th, float s,
+                                                  uint16_t* __restrict__ out, int64_t cells, int64_t solid_n,
+                                                  int lm_n, int th_n, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int64_t smp = i / cells;
+    const float so = solid[solid_n == n ? i : i - smp * cells];
+    auto two = [](float a, float b) { return (unsigned)to_bf16(a) | ((unsigned)to_bf16(b) << 16); };
+    reinterpret_cast<u4v*>(out)[i] = u4v{two(psi[i], ux[i] * s), two(uy[i] * s, so),
+                                         two(lm[lm_n > 1 ? smp : 0], th[th_n > 1 ? smp : 0]), 0u};
+}
+
 int check(int N, int H, int W, int Cin, int Cout) {
     if (N < 1 || H < 1 || W < 1 || Cin < 8 || Cout < 1) return fail(FDS_E_ARG, "bad shape");
     if (Cin % 8) return fail(FDS_E_ARG, "Cin must be a multiple of 8");
@@ -1565,6 +1608,71 @@ int conv_fwd_checked(const uint16_t* x, const uint16_t* xm, const uint16_t* w, c
     FDS_HIP(hipGetLastError());
     return FDS_OK;
 }
+// w16 (and, where wt[l] is given, the flipped copy) of n layers.
+int cast_layers(int n, const float* const* w, uint16_t* const* w16, uint16_t* const* wt, const int32_t* cin,
+                const int32_t* cout, hipStream_t stream) {
+    CastFlipArgs a{};
+    a.n = n;
+    a.start[0] = 0;
+    for (int l = 0; l < n; ++l) {
+        if (!w[l] || !w16[l]) return fail(FDS_E_ARG, "NULL pointer");
+        if (cin[l] < 1 || cout[l] < 1) return fail(FDS_E_ARG, "bad arguments");
+        a.w[l] = w[l];
+        a.w16[l] = w16[l];
+        a.wt[l] = wt ? wt[l] : nullptr;
+        a.cin[l] = cin[l];
+        a.cout[l] = cout[l];
+        a.start[l + 1] = a.start[l] + (int64_t)cout[l] * 9 * cin[l];
+    }
+    hipLaunchKernelGGL(cast_flip, dim3((unsigned)((a.start[n] + 255) / 256)), dim3(256), 0, stream, a);
+    FDS_HIP(hipGetLastError());
+    return FDS_OK;
+}
+
+// The U-Net's 15 layers in the order of their weights (e0a e0b e1a e1b e2a
+// e2b e3a e3b d2a d2b d1a d1b d0a d0b head) for level widths c[0..3].
+constexpr int kNetLayers = 15;
+struct NetPlan {
+    int32_t cin[kNetLayers], cout[kNetLayers];
+    // elements (bf16) of the workspace: skips of the three upper levels, two
+    // buffers that every other activation alternates between, the weights
+    int64_t skip[3], buf, w[kNetLayers], total;
+};
+
+int net_plan(int N, int H, int W, const int32_t* c, NetPlan* p) {
+    if (!c || N < 1 || H < 8 || W < 8 || (H % 8) || (W % 8)) return fail(FDS_E_ARG, "H and W must be multiples of 8");
+    for (int l = 0; l < 4; ++l)
+        if (c[l] < 8 || (c[l] % 8)) return fail(FDS_E_ARG, "level widths must be positive multiples of 8");
+    if ((int64_t)N * H * W >= ((int64_t)1 << 40)) return fail(FDS_E_ARG, "too many pixels");
+    const int32_t in[kNetLayers] = {8,           c[0], c[0],        c[1], c[1],        c[2], c[2], c[3],
+                                    c[3] + c[2], c[2], c[2] + c[1], c[1], c[1] + c[0], c[0], c[0]};
+    const int32_t out[kNetLayers] = {c[0], c[0], c[1], c[1], c[2], c[2], c[3], c[3],
+                                     c[2], c[2], c[1], c[1], c[0], c[0], 8};
+    const auto up = [](int64_t n) { return (n + 127) / 128 * 128; };   // 256-byte pieces
+    const int64_t P = (int64_t)N * H * W;
+    p->total = 0;
+    p->buf = 0;
+    for (int l = 0; l < 3; ++l) {
+        p->skip[l] = p->total;
+        p->total += up((P >> (2 * l)) * c[l]);
+    }
+    for (int l = 0; l < kNetLayers; ++l) {
+        p->cin[l] = in[l];
+        p->cout[l] = out[l];
+        p->w[l] = p->total;
+        p->total += up((int64_t)9 * in[l] * out[l]);
+        const int lv = l < 8 ? l / 2 : (l < 14 ? 2 - (l - 8) / 2 : 0);
+        p->buf = std::max(p->buf, up((P >> (2 * lv)) * std::max(in[l], out[l])));
+    }
+    return FDS_OK;
+}
+
+int pool_launch(const uint16_t* x, uint16_t* y, int N, int H, int W, int C, hipStream_t stream) {
+    const int64_t n8 = (int64_t)N * (H / 2) * (W / 2) * (C / 8);
+    hipLaunchKernelGGL(avg_pool2, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, stream, x, y, W, C / 8, n8);
+    FDS_HIP(hipGetLastError());
+    return FDS_OK;
+}
 }  // namespace
 
 extern "C" {
@@ -1590,22 +1698,9 @@ int fds_cast_flip(int32_t n, const float* const* w, uint16_t* const* w16, uint16
                   const int32_t* cout, void* stream) {
     if (n < 1 || n > kCastLayers) return fail(FDS_E_ARG, "1 to 16 layers expected");
     if (!w || !w16 || !wt || !cin || !cout) return fail(FDS_E_ARG, "NULL pointer");
-    CastFlipArgs a{};
-    a.n = n;
-    a.start[0] = 0;
-    for (int l = 0; l < n; ++l) {
-        if (!w[l] || !w16[l] || !wt[l]) return fail(FDS_E_ARG, "NULL pointer");
-        if (cin[l] < 1 || cout[l] < 1) return fail(FDS_E_ARG, "bad arguments");
-        a.w[l] = w[l];
-        a.w16[l] = w16[l];
-        a.wt[l] = wt[l];
-        a.cin[l] = cin[l];
-        a.cout[l] = cout[l];
-        a.start[l + 1] = a.start[l] + (int64_t)cout[l] * 9 * cin[l];
-    }
-    hipLaunchKernelGGL(cast_flip, dim3((unsigned)((a.start[n] + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a);
-    FDS_HIP(hipGetLastError());
-    return FDS_OK;
+    for (int l = 0; l < n; ++l)
+        if (!wt[l]) return fail(FDS_E_ARG, "NULL pointer");
+    return cast_layers(n, w, w16, wt, cin, cout, (hipStream_t)stream);
 }
 
 int fds_conv3x3_bwd_data(const uint16_t* dy, const uint16_t* wt, const uint16_t* relu_y, float* dx32,
@@ -1709,6 +1804,70 @@ int fds_pool_skip_bwd(const uint16_t* dp, const uint16_t* dskip, int32_t dskip_l
                        dskip, dskip_ld / 8, s, out, H, W, C / 8, n8);
     FDS_HIP(hipGetLastError());
     return FDS_OK;
+}
+
+int fds_avg_pool2(const uint16_t* x, uint16_t* y, int32_t N, int32_t H, int32_t W, int32_t C, void* stream) {
+    if (!x || !y) return fail(FDS_E_ARG, "NULL pointer");
+    if (N < 1 || H < 2 || W < 2 || (H % 2) || (W % 2)) return fail(FDS_E_ARG, "N >= 1 and even H, W >= 2 expected");
+    if (C < 8 || (C % 8)) return fail(FDS_E_ARG, "C must be a positive multiple of 8");
+    return pool_launch(x, y, N, H, W, C, (hipStream_t)stream);
+}
+
+int fds_net_inputs(const float* psi, const float* ux, const float* uy, const float* solid, int32_t solid_per_sample,
+                   const float* lm, int32_t lm_n, const float* th, int32_t th_n, float scale, uint16_t* out, int32_t N,
+                   int32_t H, int32_t W, void* stream) {
+    if (!psi || !ux || !uy || !solid || !lm || !th || !out) return fail(FDS_E_ARG, "NULL pointer");
+    if (N < 1 || H < 1 || W < 1) return fail(FDS_E_ARG, "bad shape");
+    if ((lm_n != 1 && lm_n != N) || (th_n != 1 && th_n != N)) return fail(FDS_E_ARG, "one value or one per sample");
+    const int64_t cells = (int64_t)H * W, n = N * cells;
+    hipLaunchKernelGGL(net_inputs, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, psi, ux, uy,
+                       solid, lm, th, scale, out, cells, solid_per_sample ? n : cells, lm_n, th_n, n);
+    FDS_HIP(hipGetLastError());
+    return FDS_OK;
+}
+
+int64_t fds_unet_scratch(int32_t N, int32_t H, int32_t W, const int32_t* c) {
+    NetPlan p;
+    if (net_plan(N, H, W, c, &p)) return -1;
+    return 2 * (p.total + 2 * p.buf);
+}
+
+int fds_unet_fwd(const uint16_t* x, const float* const* w, const float* const* bias, float* y, void* scratch,
+                 int32_t N, int32_t H, int32_t W, const int32_t* c, void* stream) {
+    NetPlan p;
+    int rc = net_plan(N, H, W, c, &p);
+    if (rc) return rc;
+    if (!x || !w || !bias || !y || !scratch) return fail(FDS_E_ARG, "NULL pointer");
+    uint16_t* const base = (uint16_t*)scratch;
+    uint16_t* const X = base + p.total;
+    uint16_t* const Y = X + p.buf;
+    uint16_t* w16[kNetLayers];
+    for (int l = 0; l < kNetLayers; ++l) w16[l] = base + p.w[l];
+    rc = cast_layers(kNetLayers, w, w16, nullptr, p.cin, p.cout, (hipStream_t)stream);
+    if (rc) return rc;
+    int layer = 0;
+    const auto conv = [&](const uint16_t* in, uint16_t* out, int lv) {
+        const int l = layer++;
+        return conv_fwd_checked(in, nullptr, w16[l], bias[l], l == 14 ? y : nullptr, l == 14 ? nullptr : out, N,
+                                H >> lv, W >> lv, p.cin[l], p.cout[l], l == 14 ? 0 : 1, stream);
+    };
+    const uint16_t* in = x;
+    for (int lv = 0; lv < 3; ++lv) {
+        uint16_t* const skip = base + p.skip[lv];
+        if ((rc = conv(in, X, lv)) || (rc = conv(X, skip, lv)) ||
+            (rc = pool_launch(skip, Y, N, H >> lv, W >> lv, c[lv], (hipStream_t)stream)))
+            return rc;
+        in = Y;
+    }
+    if ((rc = conv(Y, X, 3)) || (rc = conv(X, Y, 3))) return rc;
+    uint16_t *a = Y, *b = X;   // the coarser level's output and a free buffer
+    for (int lv = 2; lv >= 0; --lv) {
+        if ((rc = fds_up_cat(a, base + p.skip[lv], b, N, H >> lv, W >> lv, c[lv + 1], c[lv], stream)) ||
+            (rc = conv(b, a, lv)) || (rc = conv(a, b, lv)))
+            return rc;
+        std::swap(a, b);
+    }
+    return conv(a, nullptr, 0);
 }
 
 }  // extern "C"

@@ -27,6 +27,10 @@ EXPORTS = {
     "fds_up_cat_bwd_masked": (ctypes.c_int, [_VP] * 4 + [_I32] * 5 + [_VP]),
     "fds_relu_mask": (ctypes.c_int, [_VP, _VP, _VP, ctypes.c_int64, _VP]),
     "fds_pool_skip_bwd": (ctypes.c_int, [_VP, _VP, _I32, _VP, _VP] + [_I32] * 4 + [_VP]),
+    "fds_avg_pool2": (ctypes.c_int, [_VP, _VP] + [_I32] * 4 + [_VP]),
+    "fds_net_inputs": (ctypes.c_int, [_VP] * 4 + [_I32, _VP, _I32, _VP, _I32, ctypes.c_float, _VP] + [_I32] * 3 + [_VP]),
+    "fds_unet_scratch": (ctypes.c_int64, [_I32] * 3 + [_VP]),
+    "fds_unet_fwd": (ctypes.c_int, [_VP] * 5 + [_I32] * 3 + [_VP, _VP]),
     "fds_last_error": (ctypes.c_char_p, []),
 }
 
@@ -56,11 +60,11 @@ def _check(rc):
 
 
 def _p(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _nhwc(x, dtype):
@@ -258,3 +262,69 @@ def pool_skip_bwd(dp, dskip, s):
     out = torch.empty_like(s)
     _check(load().fds_pool_skip_bwd(_p(dp), _p(dskip), ld, _p(s), _p(out), N, H, W, C, _stream()))
     return out
+
+
+def avg_pool2(x):
+    """x.view(N, H/2, 2, W/2, 2, C).mean(dim=(2, 4)) for bf16 NHWC x with
+    even H, W and C a multiple of 8, bit for bit, in one kernel."""
+    N, H, W, C = _nhwc(x, torch.bfloat16)
+    if H % 2 or W % 2 or C % 8 or C < 8 or N < 1 or H < 2 or W < 2:
+        raise ValueError("x must be [N, H, W, C] with H, W even and C a multiple of 8")
+    _same_device(x)
+    y = torch.empty((N, H // 2, W // 2, C), dtype=torch.bfloat16, device=x.device)
+    _check(load().fds_avg_pool2(_p(x), _p(y), N, H, W, C, _stream()))
+    return y
+
+
+def plain(*ts):
+    """Whether a call on ts may go to native code in one piece, past autograd
+    and PyTorch's dispatcher: no gradient is asked for, nothing transforms,
+    traces or intercepts operations, and every tensor is an ordinary one on
+    the current GPU."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    if (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None):
+        return False
+    if not ts[0].is_cuda:
+        return False
+    dev, kinds, strided = torch.cuda.current_device(), (torch.Tensor, torch.nn.Parameter), torch.strided
+    return all(type(t) in kinds and t.layout is strided and t.get_device() == dev for t in ts)
+
+
+def net_inputs(psi, ux, uy, solid, lm, th, scale):
+    """The network's input [N, H, W, 8] bf16 in one kernel: channels psi, ux *
+    scale, uy * scale, solid, lm, th, 0, 0.  psi, ux, uy [N, H, W], solid the
+    same or [H, W] or [1, H, W], lm and th of 1 or N values; contiguous
+    float32."""
+    N, H, W = psi.shape
+    ts = (psi, ux, uy, solid, lm, th)
+    if (any(t.dtype != torch.float32 or not t.is_contiguous() for t in ts) or ux.shape != psi.shape
+            or uy.shape != psi.shape or tuple(solid.shape) not in ((N, H, W), (H, W), (1, H, W))
+            or lm.numel() not in (1, N) or th.numel() not in (1, N) or psi.numel() < 1):
+        raise ValueError("expected contiguous float32 fields of one shape")
+    _same_device(*ts)
+    x = torch.empty((N, H, W, 8), dtype=torch.bfloat16, device=psi.device)
+    _check(load().fds_net_inputs(_p(psi), _p(ux), _p(uy), _p(solid), 1 if solid.numel() == psi.numel() else 0, _p(lm),
+                                 lm.numel(), _p(th), th.numel(), scale, _p(x), N, H, W, _stream()))
+    return x
+
+
+def unet_fwd(x, ws, bs, channels):
+    """The U-Net's forward pass in one native call: [N, H, W, 8] float32 from
+    x [N, H, W, 8] bf16 and the 15 layers' FP32 weights and biases."""
+    N, H, W, _ = _nhwc(x, torch.bfloat16)
+    dev = x.get_device()
+    if dev < 0 or any(t.get_device() != dev for t in (*ws, *bs)):
+        raise ValueError("every tensor must be on the same GPU device")
+    c = (ctypes.c_int32 * 4)(*channels)
+    lib = load()
+    n = int(lib.fds_unet_scratch(N, H, W, c))
+    if n < 0:
+        raise FdsError(lib.fds_last_error().decode())
+    scratch = torch.empty(n, dtype=torch.uint8, device=x.device)
+    y = torch.empty((N, H, W, 8), dtype=torch.float32, device=x.device)
+    ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+    _check(lib.fds_unet_fwd(_p(x), ptrs(ws), ptrs(bs), _p(y), _p(scratch), N, H, W, c, _stream()))
+    return y

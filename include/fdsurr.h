@@ -101,6 +101,30 @@ int fds_relu_mask(const uint16_t* dy, const uint16_t* y, uint16_t* out, int64_t 
 int fds_pool_skip_bwd(const uint16_t* dp, const uint16_t* dskip, int32_t dskip_ld, const uint16_t* s, uint16_t* out,
                       int32_t N, int32_t H, int32_t W, int32_t C, void* stream);
 
+/* y = the mean of x over each 2 x 2 block (x N x H x W x C, H and W even, C a
+ * multiple of 8; y N x H/2 x W/2 x C; bf16): the four values added in float,
+ * row by row, times 1/4, rounded - torch's mean over the two axes. */
+int fds_avg_pool2(const uint16_t* x, uint16_t* y, int32_t N, int32_t H, int32_t W, int32_t C, void* stream);
+
+/* The U-Net's input, N x H x W x 8 bf16: psi, ux * scale, uy * scale, solid,
+ * lm, th, 0, 0.  psi, ux, uy: N x H x W floats; solid the same, or H x W for
+ * every sample (solid_per_sample 0); lm and th: lm_n, th_n = 1 or N floats. */
+int fds_net_inputs(const float* psi, const float* ux, const float* uy, const float* solid, int32_t solid_per_sample,
+                   const float* lm, int32_t lm_n, const float* th, int32_t th_n, float scale, uint16_t* out, int32_t N,
+                   int32_t H, int32_t W, void* stream);
+
+/* Bytes of scratch fds_unet_fwd needs (-1: bad arguments). */
+int64_t fds_unet_scratch(int32_t N, int32_t H, int32_t W, const int32_t* c);
+
+/* Forward pass of the whole U-Net in one call: y (N x H x W x 8 floats, the
+ * head's output) from x (N x H x W x 8 bf16; H and W multiples of 8).  c:
+ * the widths of the four levels (multiples of 8); w and bias: device pointers
+ * of the FP32 weights and biases of the 15 layers, encoder then decoder then
+ * head (e0a e0b e1a e1b e2a e2b e3a e3b d2a d2b d1a d1b d0a d0b head), in
+ * host arrays.  The same kernels as the calls above, launch by launch. */
+int fds_unet_fwd(const uint16_t* x, const float* const* w, const float* const* bias, float* y, void* scratch,
+                 int32_t N, int32_t H, int32_t W, const int32_t* c, void* stream);
+
 /* Message of the last failed call on this thread. */
 const char* fds_last_error(void);
 

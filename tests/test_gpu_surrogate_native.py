@@ -1,0 +1,124 @@
+"""The surrogate's native calls against the PyTorch operations they stand
+for, bit for bit: the 2 x 2 mean, the input channels, and the forward pass
+of the whole network in one call; and that whatever asks autograd or
+PyTorch's dispatcher for more still goes through them."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _spread(shape, gen):
+    """bf16 values over about 60 binades with both signs and zeros, so that
+    rounding and the order of a sum show."""
+    v = torch.randn(shape, generator=gen) * torch.pow(2.0, torch.randint(-30, 30, shape, generator=gen).float())
+    v[torch.rand(shape, generator=gen) < 0.05] = 0.0
+    return v.to(torch.bfloat16).cuda()
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 2, 8), (3, 8, 8, 128), (2, 16, 32, 32), (64, 64, 128, 32), (5, 6, 10, 24)])
+def test_mean_pool_is_torch_mean(shape):
+    from fingering_dynamics_amd import surrogate as sg, surrogate_ops as so
+    x = _spread(shape, torch.Generator().manual_seed(sum(shape)))
+    x.view(-1)[0], x.view(-1)[-1] = float("inf"), float("nan")
+    got, want = so.avg_pool2(x), sg._pool(x)
+    assert torch.equal(got.view(torch.int16)[~got.isnan()], want.view(torch.int16)[~got.isnan()])
+    assert torch.equal(got.isnan(), want.isnan())
+
+
+@pytest.mark.parametrize("N,H,W", [(1, 8, 16), (3, 17, 5), (8, 128, 256)])
+@pytest.mark.parametrize("solid_shape", ["full", "shared", "one"])
+def test_inputs_are_torchs(monkeypatch, N, H, W, solid_shape):
+    from fingering_dynamics_amd import surrogate as sg, surrogate_ops as so
+    g = torch.Generator(device="cuda").manual_seed(N * H + W)
+    psi, ux, uy = [torch.randn(N, H, W, device="cuda", generator=g) for _ in range(3)]
+    solid = torch.rand(*dict(full=(N, H, W), shared=(H, W), one=(1, H, W))[solid_shape], device="cuda", generator=g)
+    for M, theta in ((torch.rand(N, device="cuda", generator=g) * 20 + 0.1, torch.rand(N, device="cuda") * 180),
+                     (15.0, 135.0), ([7.5], np.array([60.0]))):
+        called = []
+        with monkeypatch.context() as m:
+            m.setattr(so, "net_inputs", lambda *a, f=so.net_inputs: called.append(1) or f(*a))
+            got = sg.inputs(psi, ux, uy, solid, M, theta)
+            m.setattr(so, "plain", lambda *a: False)
+            want = sg.inputs(psi, ux, uy, solid, M, theta)
+        assert called == [1] and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("N,H,W,channels", [(1, 8, 8, (32, 64, 128, 128)), (2, 64, 128, (32, 64, 128, 128)),
+                                            (3, 24, 40, (8, 16, 24, 40)), (1, 128, 256, (32, 64, 128, 128))])
+def test_native_forward_is_the_layers(monkeypatch, N, H, W, channels):
+    from fingering_dynamics_amd import surrogate as sg, surrogate_ops as so
+    g = torch.Generator(device="cuda").manual_seed(N * H + W)
+    model = sg.UNet(channels=channels, seed=3).cuda()
+    with torch.no_grad():
+        for n in model.names:
+            getattr(model, "b_" + n).normal_(0.0, 0.05, generator=g)
+    x = torch.randn(N, H, W, 8, device="cuda", generator=g).to(torch.bfloat16)
+    called = []
+    native = so.unet_fwd
+    monkeypatch.setattr(so, "unet_fwd", lambda *a: called.append(1) or native(*a))
+    want = model(x)
+    assert want.requires_grad and not called
+    with torch.no_grad():
+        got = model(x)
+        assert called == [1] and torch.equal(got, want)
+        off = torch.empty(x.numel() + 1, dtype=x.dtype, device="cuda")[1:].view_as(x).copy_(x)   # unaligned input
+        assert torch.equal(model(off), want)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            other = model(x)
+        torch.cuda.current_stream().wait_stream(side)
+        assert torch.equal(other, want)
+    model.requires_grad_(False)
+    assert torch.equal(model(x), want) and len(called) == 4
+    x.requires_grad_(True)
+    assert model(x).requires_grad and len(called) == 4
+
+
+def test_native_forward_in_a_graph():
+    from fingering_dynamics_amd import surrogate as sg
+    model = sg.UNet(seed=1).cuda()
+    x = torch.randn(1, 32, 64, 8, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            model(x)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = model(x)
+        for k in range(3):
+            x.copy_(torch.randn(1, 32, 64, 8, device="cuda"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, model(x))
+
+
+def test_what_is_not_plain_goes_the_general_way(monkeypatch):
+    from fingering_dynamics_amd import surrogate as sg, surrogate_ops as so
+    model = sg.UNet(seed=1).cuda()
+    x = torch.randn(1, 16, 16, 8, device="cuda").to(torch.bfloat16)
+    monkeypatch.setattr(so, "unet_fwd", lambda *a: pytest.fail("native call"))
+
+    class Mode(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        with Mode():
+            model(x)
+        with torch.autograd.forward_ad.dual_level():
+            model(x)
+        model(torch.randn(1, 16, 16, 16, device="cuda").to(torch.bfloat16)[..., ::2].contiguous().as_subclass(
+            type("Sub", (torch.Tensor,), {})))
+        with pytest.raises(Exception):
+            model(torch.zeros(1, 12, 16, 8, device="cuda", dtype=torch.bfloat16))
+        with pytest.raises(Exception):
+            model(x.float())
+        with pytest.raises(Exception):
+            model(x.cpu())
