@@ -619,11 +619,14 @@ __global__ __launch_bounds__(64 * WPB) void step_kernel(KParams k, KBufs b) {
 // single-iteration launches bit for bit.
 constexpr int kFuseCols = 58;
 
+// The lane without a neighbour gets 0 from the instruction itself (bound
+// control); as the value it keeps, the 0 would be a move of its own before
+// each shift.
 __device__ __forceinline__ float lane_from_left(float v) {  // lane l <- lane l-1 (DPP wave_shr:1)
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xF, 0xF, false));
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x138, 0xF, 0xF, true));
 }
 __device__ __forceinline__ float lane_from_right(float v) {  // lane l <- lane l+1 (DPP wave_shl:1)
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xF, 0xF, false));
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x130, 0xF, 0xF, true));
 }
 // psi of a row at this lane and its left / right neighbour lanes (lanes 0
 // and 63 get 0 for the missing neighbour; their stencils are not used)
@@ -1034,33 +1037,39 @@ __global__ __launch_bounds__(64 * WPB) void fused_kernel(KParams k, KBufs b) {
 // register ring, f in a second LDS ring - instead of storing it; stage C
 // (two rows behind B) pulls S_n+2 from them, collides and stores S_n+3.
 // Every stage pulls from a column either side, and its psi stencil from one
-// more, so the 64 lanes hold columns x0 - 6 ... x0 + 57 and stage C's 52
-// output columns are lanes 6..57: a multiple of four, so that a row of them
-// is whole 16-byte pieces.  For the chunk [y0, y1) stage A runs rows y0-4 ...
-// y1+3 (upwards) and stage B rows y0-2 ... y1+1, which may lie beyond a
-// walled domain's edge rows (ghost rows: psi_wall, no populations) or wrap
-// around a periodic one.  The arithmetic of every node is the
+// more: six columns either side of an output column.  The 64 lanes hold
+// columns x0 - 8 ... x0 + 55 and stage C's 48 output columns are lanes
+// 8..55, so that a row of them is whole 64-byte sectors.  For the chunk
+// [y0, y1) stage A runs rows y0-4 ... y1+3 (upwards) and stage B rows y0-2
+// ... y1+1, which may lie beyond a walled domain's edge rows (ghost rows:
+// psi_wall, no populations) or wrap around a periodic one.  The arithmetic of every node is the
 // single-iteration kernel's, in the same order, so the result equals three
 // single-iteration launches bit for bit.
 //
-// A launch of it is bound by issuing vector instructions while its waves are
-// all there (81 % of the cycles of two waves per SIMD).  What it took to get
-// there, 2048 x 1024 and 4096 x 2048, us per iteration: 43.9 and 143 before;
-// per-row values in rings of four slots, no moves, every wait exact, the
-// state's rows through LDS by 16-byte pieces (a row of 64 columns at an odd
-// offset keeps the address unit busy for 22 cycles), stores too, and edge
-// strips without branches over lanes or loads inside them: 39.0 and 132.
-constexpr int kFuse3Cols = 52;
+// What bounds a launch, 2048 x 1024: its vector instructions, 86 % of the
+// cycles of two waves per SIMD while they are there, and that waves differ by
+// 20 %; 4096 x 2048: its stores.  With all of them to one row it takes 87 us
+// per iteration instead of 123, and 52 output columns (208 bytes, sectors
+// shared by neighbouring strips), which leave less margin, take 118 instead
+// of 107; 3000 x 1500 68.4 and 59.8, 2048 x 1024 29.4 and 29.5, 1024 x 1024
+// 16.5 and 17.0.  What it took to get there, 2048 x 1024 and 4096 x 2048 with
+// 16-row chunks: 43.9 and 143 before; per-row values in rings of four slots,
+// no moves, every wait exact, the state's rows through LDS by 16-byte pieces
+// (a row of 64 columns at an odd offset keeps the address unit busy for 22
+// cycles), stores too, and edge strips without branches over lanes or loads
+// inside them: 39.0 and 132; then chunk heights (fuse3_rows).
+constexpr int kFuse3Cols = 48;
+constexpr int kHalo3 = (64 - kFuse3Cols) / 2;   // lanes either side of the output columns
 
 // Rows of the state staged for a wave of the inner march: 64 columns of each
 // of the 18 planes, in pieces of four columns (16 bytes) that load straight
-// into LDS, one piece a lane: a plane's row is 17 pieces from column x0 - 8.
-constexpr int kPieces = 17;
+// into LDS, one piece a lane: a plane's row is 16 pieces from column x0 - 8.
+constexpr int kPieces = 16;
 constexpr int kStageLoads = (9 * kPieces + 63) / 64;
 constexpr int kStageRow = 4 * kPieces;              // floats
 constexpr int kStage = 2 * kStageLoads * 256;        // floats, with the idle lanes' pieces
 // The output rows of one distribution on their way from a column per lane to
-// a piece per lane, nine planes of 13 pieces.
+// a piece per lane, nine planes of 12 pieces.
 constexpr int kOutPieces = kFuse3Cols / 4;
 constexpr int kOut = 9 * kFuse3Cols;                // floats
 // LDS floats of a wave: both rings and, in the inner march, the staged rows
@@ -1102,7 +1111,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
     const int lane = threadIdx.x & 63;
     const int wave = uniform_wave();
     const int xc0 = strip * kFuse3Cols;
-    const int xa = xc0 - 6 + lane;
+    const int xa = xc0 - kHalo3 + lane;
     // !EDGE: every lane is a domain column other than 0 and W-1 (no ghost
     // column, no wrap, no Zou-He column), so the lane predicates are
     // constant and the Zou-He code is left out
@@ -1112,7 +1121,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
         ln.x = (unsigned)xa;
         ln.ghost = 0.f;
     }
-    const bool cout = lane >= 6 && lane < 6 + kFuse3Cols && (!EDGE || xa < k.W);   // stage C stores this lane
+    const bool cout = lane >= kHalo3 && lane < kHalo3 + kFuse3Cols && (!EDGE || xa < k.W);   // stage C stores this lane
     const bool zx = !k.x_periodic;
     const bool has_in = EDGE && zx && xc0 == 0;                                     // column 0 among the outputs
     const int y1 = min(y0 + rows, k.H);
@@ -1126,7 +1135,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
     float* const fring = lds + (EDGE ? 1 : kStage + kOut + 1);               // A -> B
     float* const fring2 = fring + (EDGE ? kRingRegion : kRingTight);         // B -> C
 
-    const ZouHe zh{has_in, EDGE && zx && xc0 + 57 >= k.W - 1, ln.x == 0u, ln.x == (unsigned)k.W - 1u};
+    const ZouHe zh{has_in, EDGE && zx && xc0 + 63 - kHalo3 >= k.W - 1, ln.x == 0u, ln.x == (unsigned)k.W - 1u};
     auto ghost_row = [&](int y) { return k.y_walls && (y < 0 || y >= k.H); };
     // flags of a row: ghost rows and columns are solid without links
     auto flags_at = [&](int y) { return flags_of(k, b, ln, y); };
@@ -1186,7 +1195,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
 #pragma unroll
         for (int q = 0; q < kStageLoads; ++q) {
             const int c = q * 64 + lane;   // lanes beyond the last piece get zeros
-            sv[q] = c < 9 * kPieces ? (unsigned)(c / kPieces * k.Q + xc0 - 8 + 4 * (c % kPieces)) * 4u : kOOB;
+            sv[q] = c < 9 * kPieces ? (unsigned)(c / kPieces * k.Q + xc0 - kHalo3 + 4 * (c % kPieces)) * 4u : kOOB;
         }
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -1223,7 +1232,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
         asm volatile("" ::: "memory");
         if (EDGE) return;
-        const float* const at = lds + 2 + lane;   // pieces start at column xc0 - 8
+        const float* const at = lds + lane;
 #pragma unroll
         for (int i = 0; i < 9; ++i) {
             f[i] = at[i * kStageRow];
@@ -1245,7 +1254,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
         }
         if (cout) {
 #pragma unroll
-            for (int i = 0; i < 9; ++i) out[i * kFuse3Cols + lane - 6] = v[i];
+            for (int i = 0; i < 9; ++i) out[i * kFuse3Cols + lane - kHalo3] = v[i];
         }
         asm volatile("" ::: "memory");  // other lanes' writes: the compiler keeps the order
         float4 piece[2];
@@ -1266,7 +1275,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
     const rsrc_t uprof = make_rsrc(b.uprof, 4u * (unsigned)k.H);
     // a value of column 0 (lane 6 of strip 0), kept in a scalar register
     auto of_inlet = [](float v) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 6));
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), kHalo3));
     };
     auto side_load = [&](int y) {
         const int yw = wrap(y, k.H) * 4;
@@ -2305,10 +2314,10 @@ int fused3_slots(int dev, const hipDeviceProp_t& prop, int* slots) {
 }
 
 // Edge strips' rows per wave for `rows` of the inner ones: a row of theirs
-// takes 1.4 to 1.7 times as long.  With 22 rows in both kinds of strip 2048 x
-// 1024 takes 39.0 us per iteration, with 12 in the edge strips 29.2 (45 to 65
-// % of the rows 29.2 ... 29.3, 80 % 30.6).
-int fuse3_edge_rows(int rows) { return std::max(3, rows * 5 / 8 - 1); }
+// takes 1.4 to 1.7 times as long.  With 22 rows in both kinds of strip (of 52
+// columns then) 2048 x 1024 took 39.0 us per iteration, with 12 in the edge
+// strips 29.2 (45 to 65 % of the rows 29.2 ... 29.3, 80 % 30.6).
+int fuse3_edge_rows(int rows) { return std::max(4, rows * 5 / 8 - 1); }
 
 // Fills the parameters of a three-iteration launch over the domain of k with
 // chunks of `rows` rows and wx waves per workgroup; the edge workgroups are
@@ -2316,7 +2325,8 @@ int fuse3_edge_rows(int rows) { return std::max(3, rows * 5 / 8 - 1); }
 int fuse3_grid(KParams& k, int rows, int wx, int pad) {
     k.rows = rows;
     k.rows_e = fuse3_edge_rows(rows);
-    k.nin = k.W >= kFuse3Cols + 60 ? (k.W - 60) / kFuse3Cols : 0;
+const int last = 64 - kHalo3 + 1;   // an inner strip's lanes end at column W - 2
+    k.nin = k.W >= kFuse3Cols + last ? (k.W - last) / kFuse3Cols : 0;
     k.nes = (k.W + kFuse3Cols - 1) / kFuse3Cols - k.nin;
     const int e = (k.nes + wx - 1) / wx * ((k.H + k.rows_e - 1) / k.rows_e);
     k.blk_e = (e + pad - 1) / pad * pad;
@@ -2327,16 +2337,15 @@ int fuse3_grid(KParams& k, int rows, int wx, int pad) {
 // of the device's `slots` waves, or, where those are more than kFuse3Tall,
 // the fewest rounds.  Rows cost a wave 3 R + 12 stage rows, so tall chunks
 // save work, and a launch that just exceeds a round pays a whole one more:
-// 2048 x 1024 takes 29.2 us per iteration at 22 rows (one round), 38.9 at 20,
-// 32.8 at 11 (two); 1024 x 1024 15.2 at 11, 21.0 at 10; 1400 x 700 14.6 at
-// 10.  From 4 M nodes on it matters little, the clock falls with the power
-// drawn: 4096 x 2048 takes 122.5 at 86, 121.6 at 42, 120.5 at 28, 128 at 16.
-constexpr int kFuse3Tall = 64;
+// 2048 x 1024 takes 29.5 us per iteration at 23 rows (one round), 39.3 at 22;
+// 1024 x 1024 17.0 at 13, 23 at 12; 3000 x 1500 59.8 at 51 (one round), 64.9
+// at 26 (two); 4096 x 2048 107 at 94, 110 at 46, 114 at 31.
+constexpr int kFuse3Tall = 96;
 
 int fuse3_rows(const KParams& k0, int H, int64_t slots) {
     KParams k = k0;
     for (int64_t q = 1;; ++q)
-        for (int rows = 3; rows <= kFuse3Tall; ++rows)
+        for (int rows = 4; rows <= kFuse3Tall; ++rows)
             if (fuse3_grid(k, rows, 1, 8) <= q * slots - 7 || rows >= H) return rows;
 }
 
@@ -2358,13 +2367,13 @@ int launch_fused3(fd_handle* h, const KBufs& b, hipStream_t stream = nullptr) {
 // The tile shapes, smallest first (0: no tiles): TW, TH, iterations,
 // threads.  The rule (tile_for): the smallest shape that covers the domain
 // with at most one tile per CU, else the last up to the nodes where the march
-// has caught up: 240,000 where three iterations per launch are allowed (600 x
-// 300 6.2 us per iteration against 8.7, 700 x 350 9.2 against 8.8, 800 x 400
-// 10.7 against 9.0), 700,000 where it is one (walls of fingering.py:573).
+// has caught up: 320,000 where three iterations per launch are allowed (600 x
+// 300 5.6 us per iteration against 9.4, 800 x 400 9.7 and 9.8, 1024 x 512
+// 12.8 against 11.6), 700,000 where it is one (walls of fingering.py:573).
 constexpr int kTileShapes[][4] = {{0, 0, 0, 0},      {8, 8, 4, 512},    {24, 8, 4, 1024},
                                   {20, 20, 3, 1024}, {40, 18, 3, 1024}, {24, 13, 2, 512}};
 constexpr int kTiles = 5;
-constexpr int64_t kTileNodes = 240000, kTileNodes1 = 700000;
+constexpr int64_t kTileNodes = 320000, kTileNodes1 = 700000;
 
 int64_t tiles_of(int H, int W, int shape) {
     const int* t = kTileShapes[shape];
@@ -2645,7 +2654,7 @@ int fd_create(const fd_params* p, const uint8_t* solid, const uint8_t* links, fd
         }
         // Three iterations per launch wherever the geometry allows it and no
         // tiles are used: 1400 x 700 14.6 us per iteration against 20.3 with
-        // two, 1000 x 500 10.7 against 14.1.
+        // two, 1024 x 512 11.6 against 15.0.
         h->f3slots = slots;
         h->f3rows = fuse3_rows(h->k, p->H, slots);
         if (geom_fusable(*p)) h->fuse = 3;
@@ -3326,12 +3335,12 @@ int ens_depth(const fd_ensemble* e) {
 
 // Rows per wave of the three-iteration batch unless set: the fewest that make
 // one round of the device's waves up to 64 rows, or two rounds up to 32, or
-// 20 (domains of different heights: a tall chunk that starts late ends the
+// 32 (domains of different heights: a tall chunk that starts late ends the
 // launch).  Us per iteration at the rule's height and others: 4 domains (0.57
-// M nodes) 14.0 at 7 rows, 21 at 4; 12 (3.3 M) 53.8 at 40, 54.6 at 18 (two
-// rounds), 65 at 9; 24 (4.6 M) 80.1 at 26, 91 at 9; 8 flows of 2048 x 256
-// 61.6 at 44, 74 at 12; 64 domains (13.6 M) 214 at 20, 209 at 16, 235 at 64;
-// 48 flows 380 at 20, 372 at 32.
+// M nodes) 13.9 at 7 rows, 21 at 6 (more than a round); 12 (3.3 M) 48.9 at
+// 40, 53.5 at 20 (two rounds), 61 at 10; 24 (4.6 M) 69 at 56, 72 at 28, 88 at
+// 10; 8 flows of 2048 x 256 56.8 at 52, 64 at 24; 64 domains (13.6 M) 195 at
+// 32, 203 at 20, 206 at 64; 48 flows 334 at 32, 356 at 20.
 int ens_rows3(const fd_ensemble* e) {
     if (e->f3rows > 0) return e->f3rows;
     for (int q = 1, most = 64; q <= 2; ++q, most = 32)
@@ -3343,7 +3352,7 @@ int ens_rows3(const fd_ensemble* e) {
             }
             if (waves <= (int64_t)q * (e->hs[0]->f3slots - 7)) return rows;
         }
-    return 20;
+    return 32;
 }
 
 int ens_build(fd_ensemble* e) {

@@ -26,8 +26,8 @@ def _domain(kind, H, W):
 
 
 @pytest.mark.parametrize("kind", ["rects", "circles", "walled", "x_periodic"])
-@pytest.mark.parametrize("H,W,waves,rows", [(23, 111, 1, 5), (23, 112, 1, 7), (40, 113, 2, 40), (31, 156, 1, 1),
-                                            (31, 163, 2, 3), (64, 164, 1, 16), (64, 165, 1, 22), (50, 320, 2, 9),
+@pytest.mark.parametrize("H,W,waves,rows", [(23, 104, 1, 5), (23, 105, 1, 7), (40, 106, 2, 40), (31, 152, 1, 1),
+                                            (31, 153, 2, 3), (64, 154, 1, 16), (64, 193, 1, 22), (50, 320, 2, 9),
                                             (97, 333, 1, 80)])
 def test_strips_equal_one_iteration_per_launch(kind, H, W, waves, rows):
     from fingering_dynamics_amd.lbm import Compute
