@@ -493,6 +493,47 @@ def batch(data, items, d, flip=None):
     return x, p0, p1, v0, v1, 1.0 - sol
 
 
+def _mse(out, psi0, psi1, v0, v1, wfluid, w):
+    lp = ((psi0 + out[..., 0] - psi1) ** 2 * wfluid).sum() / w
+    lu = (((v0 + out[..., 1:3] - v1) ** 2).sum(dim=-1) * wfluid).sum() / w
+    return lp + LAMBDA_U * lu
+
+
+class _Mse(torch.autograd.Function):
+    """_mse on one kernel each way: the same gradient bit for bit, the sums
+    added in double."""
+
+    @staticmethod
+    def forward(ctx, out, psi0, psi1, v0, v1, wfluid, w):
+        ctx.save_for_backward(out, psi0, psi1, v0, v1, wfluid, w)
+        ctx.lam = LAMBDA_U
+        return so.net_loss(out, psi0, psi1, v0, v1, wfluid, w, ctx.lam)
+
+    @staticmethod
+    def backward(ctx, g):
+        out, psi0, psi1, v0, v1, wfluid, w = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            # the gradient is to be differentiated again: tensor operations
+            gp, gu = g / w * wfluid, (g * ctx.lam / w * wfluid).unsqueeze(-1)
+            return (torch.cat([(gp * (2.0 * (psi0 + out[..., 0] - psi1))).unsqueeze(-1),
+                               gu * (2.0 * (v0 + out[..., 1:3] - v1))], dim=-1),) + (None,) * 6
+        return (so.net_loss_bwd(out, psi0, psi1, v0, v1, wfluid, w, ctx.lam, g.contiguous()),) + (None,) * 6
+
+
+def _mse_native(out, psi0, psi1, v0, v1, wfluid):
+    """Whether _mse can run on its kernels: ordinary tensors of the shapes
+    that batch() makes, gradients asked for of the network only."""
+    rest = (psi0, psi1, v0, v1, wfluid)
+    if not all(isinstance(t, torch.Tensor) for t in rest) or any(t.requires_grad for t in rest):
+        return False
+    if not so.plain(out, *rest, grad=True) or so.pixel_ld(out) is None or not out.numel():
+        return False
+    shape = out.shape[:3]
+    return (all(t.dtype == torch.float32 and t.is_contiguous() for t in rest)
+            and psi0.shape == psi1.shape == wfluid.shape == shape and v0.shape == v1.shape == (*shape, 2)
+            and (v0.data_ptr() | v1.data_ptr()) % 8 == 0)
+
+
 def loss_fn(model, x, psi0, psi1, v0, v1, wfluid):
     """Fluid-weighted MSE of psi(t + K), plus LAMBDA_U times that of the
     velocity / U_REF, plus LAMBDA_S times the cross-entropy of the phase
@@ -506,11 +547,8 @@ def loss_fn(model, x, psi0, psi1, v0, v1, wfluid):
     if LOSS_BAND > 0:
         wfluid = wfluid * near_interface(psi0, LOSS_BAND)
     w = wfluid.sum().clamp(min=1.0)
-    pred = psi0 + out[..., 0]
-    lp = ((pred - psi1) ** 2 * wfluid).sum() / w
-    lu = (((v0 + out[..., 1:3] - v1) ** 2).sum(dim=-1) * wfluid).sum() / w
-    band = ((psi0.abs() < 0.9) | (psi1.abs() < 0.9)).float() * wfluid
-    loss = lp + LAMBDA_U * lu
+    mse = _Mse.apply if _mse_native(out, psi0, psi1, v0, v1, wfluid) else _mse
+    loss = mse(out, psi0, psi1, v0, v1, wfluid, w)
     if LAMBDA_V > 0.0:
         # networks whose jumps add too little volume lag in the coupled run
         # (the mass correction scales their smeared increments up instead)
@@ -519,8 +557,9 @@ def loss_fn(model, x, psi0, psi1, v0, v1, wfluid):
         loss = loss + LAMBDA_V * (((gp - gt) / gt.abs().mean().clamp(min=1e-6)) ** 2).mean()
     if LAMBDA_S == 0.0:
         return loss
+    band = ((psi0.abs() < 0.9) | (psi1.abs() < 0.9)).float() * wfluid
     ls = torch.nn.functional.binary_cross_entropy_with_logits(
-        SIGN_GAIN * pred, (psi1 > 0).float(), weight=band, reduction="sum") / band.sum().clamp(min=1.0)
+        SIGN_GAIN * (psi0 + out[..., 0]), (psi1 > 0).float(), weight=band, reduction="sum") / band.sum().clamp(min=1.0)
     return loss + LAMBDA_S * ls
 
 

@@ -31,6 +31,9 @@ EXPORTS = {
     "fds_net_inputs": (ctypes.c_int, [_VP] * 4 + [_I32, _VP, _I32, _VP, _I32, ctypes.c_float, _VP] + [_I32] * 3 + [_VP]),
     "fds_unet_scratch": (ctypes.c_int64, [_I32] * 3 + [_VP]),
     "fds_unet_fwd": (ctypes.c_int, [_VP] * 5 + [_I32] * 3 + [_VP, _VP]),
+    "fds_net_loss_scratch": (ctypes.c_int64, []),
+    "fds_net_loss": (ctypes.c_int, [_VP, _I32] + [_VP] * 6 + [ctypes.c_float, _VP, _VP, ctypes.c_int64, _VP]),
+    "fds_net_loss_bwd": (ctypes.c_int, [_VP, _I32] + [_VP] * 6 + [ctypes.c_float, _VP, _VP, ctypes.c_int64, _VP]),
     "fds_last_error": (ctypes.c_char_p, []),
 }
 
@@ -276,12 +279,12 @@ def avg_pool2(x):
     return y
 
 
-def plain(*ts):
+def plain(*ts, grad=False):
     """Whether a call on ts may go to native code in one piece, past autograd
-    and PyTorch's dispatcher: no gradient is asked for, nothing transforms,
-    traces or intercepts operations, and every tensor is an ordinary one on
-    the current GPU."""
-    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+    and PyTorch's dispatcher: no gradient is asked for (unless grad: the
+    caller is an autograd function), nothing transforms, traces or intercepts
+    operations, and every tensor is an ordinary one on the current GPU."""
+    if not grad and torch.is_grad_enabled() and any(t.requires_grad for t in ts):
         return False
     if (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0
             or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
@@ -328,3 +331,46 @@ def unet_fwd(x, ws, bs, channels):
     ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
     _check(lib.fds_unet_fwd(_p(x), ptrs(ws), ptrs(bs), _p(y), _p(scratch), N, H, W, c, _stream()))
     return y
+
+
+def pixel_ld(out):
+    """Floats between the pixels of out [N, H, W, 3] float32 when its channels
+    are contiguous and its pixels evenly spaced (a channel slice of a
+    contiguous tensor); None otherwise."""
+    if out.dtype != torch.float32 or out.dim() != 4 or out.shape[3] != 3:
+        return None
+    N, H, W, _ = out.shape
+    ld = out.stride(2)
+    return ld if out.stride() == (H * W * ld, W * ld, ld, 1) and ld >= 3 else None
+
+
+def _loss_ptrs(out, psi0, psi1, v0, v1, wf, w):
+    ld = pixel_ld(out)
+    shape = tuple(out.shape[:3])
+    if (ld is None or any(t.dtype != torch.float32 or not t.is_contiguous() for t in (psi0, psi1, v0, v1, wf, w))
+            or any(tuple(t.shape) != shape for t in (psi0, psi1, wf)) or w.numel() != 1
+            or any(tuple(t.shape) != shape + (2,) for t in (v0, v1))):
+        raise ValueError("expected contiguous float32 tensors shaped like the network's output")
+    _same_device(out, psi0, psi1, v0, v1, wf, w)
+    return [_p(out), ld] + [_p(t) for t in (psi0, psi1, v0, v1, wf, w)]
+
+
+def net_loss(out, psi0, psi1, v0, v1, wf, w, lam):
+    """sum(d^2 wf) / w + lam sum(|x|^2 wf) / w with d = psi0 + out[..., 0] -
+    psi1 and x = v0 + out[..., 1:3] - v1: a 0-d float32 tensor."""
+    ptrs = _loss_ptrs(out, psi0, psi1, v0, v1, wf, w)
+    scratch = torch.empty(load().fds_net_loss_scratch(), dtype=torch.float64, device=out.device)
+    loss = torch.empty((), dtype=torch.float32, device=out.device)
+    _check(load().fds_net_loss(*ptrs, lam, _p(scratch), _p(loss), wf.numel(), _stream()))
+    return loss
+
+
+def net_loss_bwd(out, psi0, psi1, v0, v1, wf, w, lam, g):
+    """g times the gradient of net_loss in out, [N, H, W, 3] float32."""
+    ptrs = _loss_ptrs(out, psi0, psi1, v0, v1, wf, w)
+    if g.dtype != torch.float32 or g.numel() != 1:
+        raise ValueError("g must be one float32 value")
+    _same_device(out, g)
+    dout = torch.empty(tuple(out.shape), dtype=torch.float32, device=out.device)
+    _check(load().fds_net_loss_bwd(*ptrs, lam, _p(g), _p(dout), wf.numel(), _stream()))
+    return dout

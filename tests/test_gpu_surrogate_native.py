@@ -122,3 +122,33 @@ def test_what_is_not_plain_goes_the_general_way(monkeypatch):
             model(x.float())
         with pytest.raises(Exception):
             model(x.cpu())
+
+
+@pytest.mark.parametrize("N,H,W", [(1, 1, 1), (3, 17, 5), (2, 64, 128), (64, 32, 64)])
+def test_loss_is_torchs(N, H, W):
+    """The loss within the rounding of a float sum, its gradient bit for
+    bit; a gradient of the gradient; targets that ask for one."""
+    from fingering_dynamics_amd import surrogate as sg
+    g = torch.Generator(device="cuda").manual_seed(N * H + W)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    psi0, psi1, v0, v1, wf = rnd(N, H, W), rnd(N, H, W), rnd(N, H, W, 2), rnd(N, H, W, 2), rnd(N, H, W).abs()
+    head = rnd(N, H, W, 8).requires_grad_(True)
+    args = (None, psi0, psi1, v0, v1, wf)
+    w = wf.sum().clamp(min=1.0)
+    for scale in (1.0, 0.37):
+        got = sg.loss_fn(lambda x: head[..., :3], *args)
+        want = sg._mse(head[..., :3], *args[1:], w)
+        assert type(got.grad_fn).__name__ == "_MseBackward" and got.dtype == want.dtype and got.shape == want.shape
+        # want adds N H W positive floats in a tree, got in double: at most
+        # log2(N H W) + 4 roundings of 2^-24 each
+        tol = (math.log2(N * H * W + 1) + 4) * 2.0 ** -24 * 2
+        assert abs(float(got.detach()) - float(want.detach())) <= tol * float(want.detach())
+        assert torch.equal(*[torch.autograd.grad(scale * v, head)[0] for v in (got, want)])
+    got = sg.loss_fn(lambda x: head[..., :3], *args)
+    (first,) = torch.autograd.grad(got, head, create_graph=True)
+    (second,) = torch.autograd.grad(first.sum(), head)
+    (ref,) = torch.autograd.grad(sg._mse(head[..., :3], *args[1:], w), head, create_graph=True)
+    (ref2,) = torch.autograd.grad(ref.sum(), head)
+    assert torch.equal(first, ref) and torch.equal(second, ref2)
+    psi1.requires_grad_(True)
+    assert torch.autograd.grad(sg.loss_fn(lambda x: head[..., :3], *args), psi1)[0].abs().sum() > 0
