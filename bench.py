@@ -12,9 +12,9 @@ Prints ONE JSON line.  ``value`` is MLUPS over all H*W nodes.  ``roofline``
 prices the dominant kernel at 144 algorithmic bytes per fluid-node update
 (9 f + 9 g FP32 read and written) against 8 TB/s, using the kernel's average
 launch time from HIP events on the solver's stream.  By default one launch
-advances two iterations (the intermediate state stays in registers), so a
-launch carries 2 x 144 algorithmic bytes per fluid node while moving the
-populations through HBM once.  ``cpu_baseline`` times
+advances three iterations (the intermediate states stay on chip), so a launch
+carries 3 x 144 algorithmic bytes per fluid node while moving the populations
+through HBM once.  ``cpu_baseline`` times
 the FP64 numpy restatement (the oracle, one core) on a few iterations of the
 same workload.
 
@@ -138,7 +138,7 @@ def cpu_baseline(mask, bits, params, steps):
 def ensemble_bench(n, steps, warmup):
     """Aggregate MLUPS of n independent domains (the seeded many-domain
     workload of fingering_dynamics_amd.ensemble.domain_spec) advanced by
-    graph-replayed batched launches of two iterations each, against one
+    graph-replayed batched launches of three iterations each, against one
     launch per domain per launch step on the same stream, and against
     batched launches of one iteration.  Prints one JSON line."""
     from fingering_dynamics_amd.ensemble import Ensemble, domain_spec, build_domain
@@ -190,9 +190,9 @@ def ensemble_bench(n, steps, warmup):
 def cfg1_bench(steps):
     """The 400 x 100 channel of the reference-faithful configuration
     (periodic y, Gaussian Zou-He inlet/outlet, 56 seeded 6x6 squares, M = 5,
-    psi_wall = 0): `steps` iterations, one launch per iteration or two, eager
-    or replayed from a captured graph, each at the library's default launch
-    shape for this size (one row per wave).  Its state (6 MB) stays in the
+    psi_wall = 0): `steps` iterations, at the library's default for this size
+    (tiles held on chip, four iterations per launch) or one launch per
+    iteration, eager or replayed from a captured graph.  Its state (6 MB) stays in the
     caches, so this measures launch overhead and latency, not HBM.  Prints
     one JSON line."""
     from fingering_dynamics_amd.lbm import Compute
@@ -205,7 +205,7 @@ def cfg1_bench(steps):
     bits = geometry.Bounce_back(h, w).link_bits_rec(corners)
     params = LbmParams.periodic(h, w, M=5.0, psi_wall=0.0, n_inv_cols=40)
     res = {}
-    for depth in (2, 1):
+    for depth in (None, 1):
         for graph in (True, False):
             cm = Compute(mask, bits, params)
             if depth == 1:
@@ -217,7 +217,7 @@ def cfg1_bench(steps):
             cm.step(steps)
             cm.synchronize()
             dt = time.perf_counter() - t0
-            res["%s_%s" % ("two_per_launch" if depth == 2 else "one_per_launch", "graph" if graph else "eager")] = {
+            res["%s_%s" % ("default" if depth is None else "one_per_launch", "graph" if graph else "eager")] = {
                 "us_per_iteration": round(dt * 1e6 / steps, 3), "device_us_per_iteration": round(cm.last_step_ms() * 1e3, 3),
                 "mlups": round(h * w * steps / dt / 1e6, 1)}
             bad = cm.mass()[2]
@@ -233,7 +233,7 @@ def cfg1_bench(steps):
     print(json.dumps({
         "metric": "MLUPS of the 400x100 channel (%d iterations), by launch mode" % steps,
         "value": res[best]["mlups"], "unit": "MLUPS", "best_mode": best, "modes": res,
-        "graph_speedup_two_per_launch": round(res["two_per_launch_graph"]["mlups"] / res["two_per_launch_eager"]["mlups"], 2),
+        "graph_speedup_default": round(res["default_graph"]["mlups"] / res["default_eager"]["mlups"], 2),
         "non_finite_after": bad,
         "cpu_baseline": {"value": round(h * w * n_cpu / cpu_dt / 1e6, 3), "unit": "MLUPS", "cores": 1, "kind": "port",
                          "sample": "%d iterations of the same channel, FP64 numpy restatement, %.1f s" % (n_cpu, cpu_dt)},

@@ -1516,21 +1516,19 @@ __device__ __forceinline__ void tile_node(int j, int& lx, int& ly) {
     ly = r + m;
 }
 
-// The shapes, by tiles of a domain (TileRule below): a domain of at most one
-// tile per CU takes the smallest shape that covers it so, larger ones the
-// last, whose LDS lets three workgroups share a CU.  Us per iteration,
-// measured, against the fastest marching kernel at its best launch shape:
-//   droplet 320 x 128      24 x 8 x 4 iterations  3.1   march 6.1
-//   channel 400 x 100      24 x 8 x 4             4.0         7.3
-//   walls on rows 1, H-2, 601 x 151   20 x 20 x 3  5.0        8.7
-//   bed 600 x 300          40 x 18 x 3            6.4        10.1
-//   flow 512 x 256         40 x 18 x 3            6.2        10.0
-//   flow 1024 x 512        24 x 13 x 2           14.1        16.3
-//   bed 1400 x 700         24 x 13 x 2           22.2        22.2
-//   flow 2048 x 1024       24 x 13 x 2           49.7        45.7
+// The shapes (tile_for): a domain of at most one tile per CU takes the
+// smallest shape that covers it so, larger ones the last, whose LDS lets three
+// workgroups share a CU.  Us per iteration, measured, against the three-iteration march at its best launch shape:
+//   flow 256 x 128         24 x 8 x 4 iterations  3.2   march 8.0
+//   droplet 320 x 128      24 x 8 x 4             2.6         -
+//   channel 400 x 100      24 x 8 x 4             3.4         -
+//   walls on rows 1, H-2, 601 x 151   20 x 20 x 3  4.4  (one iteration) 8.7
+//   bed 600 x 300          40 x 18 x 3            5.4         9.4
+//   bed 800 x 400          24 x 13 x 2            9.7         9.7
+//   flow 1024 x 512        24 x 13 x 2           12.8        11.6
 // What bounds a tile: the latency of an iteration's two passes (LDS reads,
-// about 350 VALU operations a node in one dependent chain, three barriers)
-// and about 4 us of launch, load and store per launch.
+// about 275 VALU operations a node in one dependent chain, three barriers)
+// and about 3 us of launch, load and store per launch.
 template <int TW, int TH, int T, int NT>
 struct TileRun {
     using D = TileDim<TW, TH, T>;

@@ -1347,7 +1347,7 @@ __global__ __launch_bounds__(256) void pool_skip_bwd(const uint16_t* __restrict_
 // y[n][h][w][c] = the mean of x over each 2 x 2 block: the four values added
 // in the order of torch's mean over those two axes (row by row, in float),
 // times 1/4, rounded to bf16.  One 8-channel piece per thread; at batch 64
-// the three pools of the network take 55 us (torch's mean 97).
+// the three pools of the network take 46 us (torch's mean 97).
 __global__ __launch_bounds__(256) void avg_pool2(const uint16_t* __restrict__ x, uint16_t* __restrict__ y, int W, int G,
                                                  int64_t n8) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1392,8 +1392,8 @@ __global__ __launch_bounds__(256) void net_inputs(const float* __restrict__ psi,
 // net_loss adds in double (a partial sum per workgroup, added in a fixed
 // order by net_loss_sum); net_loss_bwd forms the products in the order of
 // autograd's backward of that expression, so the gradients are its bits.  As
-// some forty tensor operations these were 290 us of a training step at batch
-// 64 (2.1 M pixels); both kernels take 45, bound by reading 126 MB.
+// some forty tensor operations these were 250 us of a training step at batch
+// 64 (2.1 M pixels); both kernels take 44, bound by reading 126 MB.
 struct LossArgs {
     const float *out, *psi0, *psi1, *v0, *v1, *wf, *w;
     int64_t n;

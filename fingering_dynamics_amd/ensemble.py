@@ -38,7 +38,7 @@ from .params import LbmParams, PROFILE_CONST, OUTLET_PRESSURE, Y_WALLS
 
 TILE_CANDIDATES = ((4, 16), (4, 8), (4, 32), (8, 16), (2, 16), (1, 16))
 FUSED_CANDIDATES = ((1, 8), (1, 6), (1, 12), (1, 16), (2, 8), (4, 8))
-FUSED3_CANDIDATES = ((1, 16), (1, 20), (1, 26), (1, 32), (1, 12), (2, 16))
+FUSED3_CANDIDATES = ((1, 16), (1, 20), (1, 26), (1, 32), (1, 48), (2, 16))
 
 
 class Ensemble:
@@ -123,11 +123,13 @@ class Ensemble:
 
     def autotune(self, candidates=None, steps=20):
         """Time ``steps`` real iterations per launch shape of the kernel that
-        runs (two-iteration when ``fused``) and keep the fastest.  Returns
+        runs, the current one among them, and keep the fastest.  Returns
         {shape: ms per iteration}."""
         depth = self.depth
         if candidates is None:
             candidates = {3: FUSED3_CANDIDATES, 2: FUSED_CANDIDATES}.get(depth, TILE_CANDIDATES)
+            if depth >= 2:
+                candidates = (self.fusion[1:],) + tuple(candidates)   # the current shape
         steps = max(6, steps - steps % 6)
         times = {}
         for wx, rows in candidates:

@@ -152,7 +152,7 @@ class Compute:
                                               _native.ctypes.byref(r)))
         return d.value, w.value, r.value
 
-    TUNE_CANDIDATES = tuple((3, 1, r) for r in (16, 20, 26, 39)) + \
+    TUNE_CANDIDATES = tuple((3, 1, r) for r in (16, 24, 32, 48)) + \
         tuple((2, 1, r) for r in (1, 2, 4, 8, 12, 16, 24)) + ((2, 4, 16),) + \
         tuple((1, wx, r) for wx, r in ((1, 1), (4, 1), (4, 4), (4, 16)))
 

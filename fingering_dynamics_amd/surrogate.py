@@ -87,11 +87,10 @@ class _Conv(torch.autograd.Function):
             dw, db = so.conv3x3_bwd_weight(x, dy, relu_y=y if mask else None)
             return None, dw, db, None, None, None, None, None
         if mask:
-            # one masking pass: measured faster here than the kernels'
-            # mask-on-load (relu_y), which adds a load per operand fragment,
-            # and than a mask in the input-gradient epilogue of the
-            # convolution consuming y, whose scattered 2-byte mask loads
-            # slowed those kernels by more than the pass costs
+            # one masking pass: faster here than the kernels' mask-on-load
+            # (relu_y), which both gradients would pay, and than a mask in the
+            # input-gradient epilogue of the convolution consuming y, whose
+            # loads wait behind the next block's prefetched input
             dy = so.relu_mask(dy, y)
         dx = so.conv3x3_bwd_data(dy, wt)
         dw, db = so.conv3x3_bwd_weight(x, dy)

@@ -237,14 +237,15 @@ int fd_set_tile(fd_handle* h, int32_t waves_x, int32_t rows);
  * for triples (two intermediate states on chip); depth 1 runs one launch
  * per iteration.  The results are identical bit for bit.  waves_x (1, 2 or
  * 4; depth 3 uses 1 or 2) and rows set the launch shape of that depth's
- * kernel (<= 0 keeps the current one).  Defaults: depth 3 from about a
- * million nodes on, at 1 wave x 10 to 16 rows, else depth 2 at 1 wave and
- * at most 8 rows, fewer on domains too small to fill the device.  Domains
- * with H < 8, and walled domains whose walls are not the edge rows (the rows
- * 1 and H-2 of fingering.py:573), always run depth 1.
- * A domain too small for these kernels to fill the device (up to about
- * 700,000 nodes) runs tiles held in LDS instead, two to four iterations per
- * launch, walls on any rows, until this call chooses depth and shape;
+ * kernel (<= 0 keeps the current one).  Defaults: depth 3, with the fewest
+ * rows per wave that make one round of the device's waves, up to 96 (depth 3
+ * counts the rows of strips without a Zou-He column or wrap; the others take
+ * fewer); depth 2 at 1 wave and at most 8 rows.  Domains with H < 8, and
+ * walled domains whose walls are not the edge rows (the rows 1 and H-2 of
+ * fingering.py:573), always run depth 1.
+ * A domain too small for these kernels (up to 320,000 nodes; up to 700,000
+ * where only depth 1 is allowed) runs tiles held in LDS instead, two to four
+ * iterations per launch, walls on any rows, until this call chooses depth and shape;
  * fd_auto_launch returns to them.  No reference counterpart (a launch
  * control of this implementation). */
 int fd_set_fusion(fd_handle* h, int32_t depth, int32_t waves_x, int32_t rows);
@@ -317,7 +318,7 @@ int fd_ens_set_tile(fd_ensemble* e, int32_t waves_x, int32_t rows);
  * advances triples of iterations of every domain with one launch of the
  * three-iteration kernel, depth 2 pairs with the two-iteration kernel,
  * depth 1 one iteration per launch.  waves_x and rows set that depth's
- * launch shape (<= 0 keeps the current one; defaults 1 x 6 to 20 rows by the
+ * launch shape (<= 0 keeps the current one; defaults 1 x 4 to 64 rows by the
  * ensemble's size for depth 3, 1 x 8 for depth 2; depth 3 takes 1 or 2
  * waves).  A remainder of two iterations runs the two-iteration kernel.  Groups run batched only
  * when every domain's geometry allows the fused kernels (fd_set_fusion);
