@@ -1261,9 +1261,14 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
 #pragma unroll
         for (int q = 0; q < 2; ++q) piece[q] = *reinterpret_cast<const float4*>(out_at + 256 * q);
         asm volatile("" ::: "memory");
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, piece[q]), dst, ov[q], row * 4, 0);
+        // A store of more than eight bytes reads its registers after it was issued, and the link masks that
+        // the next phase makes by inline asm are no writes that the compiler's hazard table sees: without
+        // these wait states, with the registers as operands to keep them whole, the last store of a phase
+        // put masks into memory wherever the allocator had reused its registers at once.
+        const u4v piece0 = __builtin_bit_cast(u4v, piece[0]), piece1 = __builtin_bit_cast(u4v, piece[1]);
+        __builtin_amdgcn_raw_buffer_store_b128(piece0, dst, ov[0], row * 4, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(piece1, dst, ov[1], row * 4, 0);
+        asm volatile("s_nop 7" ::"v"(piece0), "v"(piece1));
     };
 
     // ---- EDGE: the inlet profile of rows r ... r - 4 (up1 ... up5) and, for stage A's

@@ -45,3 +45,25 @@ def test_strips_equal_one_iteration_per_launch(kind, H, W, waves, rows):
             assert np.array_equal(x, y, equal_nan=True)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("depth", [2, 3])
+@pytest.mark.parametrize("H,W,rows", [(2048, 1500, 90), (1023, 2050, 31)])
+def test_a_full_device_equals_one_iteration_per_launch(depth, H, W, rows):
+    """Several waves on every SIMD: a store's data registers are read late, so a kernel that writes them too soon
+    after it issued the store (the link masks of the next phase) stores other values here and not on small grids."""
+    from fingering_dynamics_amd.lbm import Compute
+    mask, bits, _ = rect_domain(H, W, 150, size=8, seed=W, x_min=14)
+    params = LbmParams.periodic(H, W, M=5.0, psi_wall=0.0, n_inv_cols=10, profile=PROFILE_CONST)
+    psi0 = np.full((H, W), -1.0)
+    psi0[:, :W // 5] = 1.0
+    a, b = Compute(mask, bits, params, psi0=psi0), Compute(mask, bits, params, psi0=psi0)
+    a.set_fusion(depth, 1, rows)
+    b.set_fusion(1)
+    for _ in range(3):
+        a.step(2 * depth)
+        b.step(2 * depth)
+        for x, y in zip(a.populations(), b.populations()):
+            assert np.array_equal(x, y, equal_nan=True)
+    a.close()
+    b.close()
