@@ -594,31 +594,12 @@ __global__ __launch_bounds__(64 * WPB) void step_kernel(KParams k, KBufs b) {
     march_block<WPB, MODE>(k, b, banded_block());
 }
 
-// ---------------------------------------------------- two-iteration march
-// One launch advances the state by two iterations: S_n -> S_n+2, with
-// S_n+1 kept in registers and never written to HBM, so each iteration moves
-// half the bytes of a single-iteration launch.
+// ------------------------------------------------- fused marches: lane shifts
+// The marches of two and three iterations per launch keep a strip of 64
+// columns in the lanes of a wave.  A population that moves in x comes from the
+// neighbouring lane by a DPP lane shift (wave_shr:1 / wave_shl:1), or, f of
+// the stage before, from a ring of rows in LDS read at the shifted lane.
 //
-// A wave owns a strip of kFuseCols output columns [xb0, xb0 + 58) and its
-// 64 lanes hold columns a0 = xb0 - 3 ... xb0 + 60.  Stage A is the
-// single-iteration march (S_n from HBM -> S_n+1 of the strip, P_n+1 of the
-// Zou-He columns), valid on lanes 1..62 (its psi stencil takes the
-// neighbours' psi from the neighbouring lanes); stage B marches two rows behind it
-// and pulls S_n+1 from A's last rows: g from registers, where a population
-// moving in x comes from the neighbouring lane by a DPP lane shift
-// (wave_shr:1 / wave_shl:1), f from a four-row ring in LDS read at the
-// shifted lane.  B needs A's output two columns either side of a node (one
-// for the f pull, one more for the g pulls of the psi stencil), so it is
-// valid on lanes 3..60: strips overlap by six columns of stage-A work.
-// For the chunk of output rows [y0, y1) stage A runs rows y0-2 ... y1+1,
-// upwards in even chunks and downwards in odd ones (B then lags two rows
-// behind in the march direction).
-//
-// Every node of either stage runs the single-iteration kernel's arithmetic
-// on the same values in the same order, so the result equals two
-// single-iteration launches bit for bit.
-constexpr int kFuseCols = 58;
-
 // The lane without a neighbour gets 0 from the instruction itself (bound
 // control); as the value it keeps, the 0 would be a move of its own before
 // each shift.
@@ -714,40 +695,14 @@ __device__ __forceinline__ float ring_inlet_rho(const float* ring, int sl, int l
     return fdn::inlet_rho(f, u, px);
 }
 
-// Stage B's Zou-He / walled-corner update of f at node (y, x): as bc_f,
-// with the inlet profile u of the row, the side values P (of stage A's psi)
-// and the corner density given.
-__device__ __forceinline__ void reg_bc_f(const KParams& k, int y, int x, float f[9], float u, float px, float py,
-                                         float rho_nb) {
-    if (k.x_periodic) return;
-    if (x == 0) {
-        const bool bot = k.y_walls && y == 0;
-        const bool top = k.y_walls && y == k.H - 1;
-        float n[9], cb[9], ct[9];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) n[i] = cb[i] = ct[i] = f[i];
-        fdn::inlet_f(n, u, px, py);
-        fdn::inlet_corner_bottom_f(cb, rho_nb);
-        fdn::inlet_corner_top_f(ct, rho_nb);
-#pragma unroll
-        for (int i = 0; i < 9; ++i) f[i] = bot ? cb[i] : (top ? ct[i] : n[i]);
-    }
-    if (x == k.W - 1) {
-        fdn::outlet_f(f, u, px, py, k.pressure != 0, k.rho_out, k.c3);
-        const float f2 = (k.y_walls && y == 0) ? f[4] : f[2];
-        const float f4 = (k.y_walls && y == k.H - 1) ? f[2] : f[4];
-        f[2] = f2;
-        f[4] = f4;
-    }
-}
-
 // The Zou-He columns of a wave that marches along y: whether its lanes hold
 // column 0 / W-1 at all (the same for every lane), and whether this one does.
 struct ZouHe {
     bool in, out, lane_in, lane_out;
 };
 
-// bc_g and reg_bc_f for such a wave.  Row and strip are the wave's, so only
+// bc_g, and bc_f given the inlet profile u of the row, the side values P and
+// the corner density, for such a wave.  Row and strip are the wave's, so only
 // the lane of the column is a select, of the three populations that the
 // formulas write; as branches over lanes with copies of all nine they cost a
 // wave at the domain's edge as many instructions again as its two collisions.
@@ -834,208 +789,14 @@ __device__ __forceinline__ float collide_node(const KParams& k, float f[9], floa
     return mu;
 }
 
-// Two iterations of logical workgroup L of a launch over one domain.
-template <int WPB>
-__device__ __forceinline__ void fused_march(const KParams& k, const KBufs& b, int L) {
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int chunk = L / k.nsb;
-    const int strip = (L - chunk * k.nsb) * WPB + wave;
-    const int xb0 = strip * kFuseCols;
-    if (xb0 >= k.W) return;
-    const int a0 = xb0 - 3;
-    const int xa = a0 + lane;
-    const Lane ln = lane_of(k, xa);
-    const bool bout = lane >= 3 && lane < 3 + kFuseCols && xa < k.W;   // stage B stores this lane
-    const bool zx = !k.x_periodic;
-    const bool has_in = zx && xb0 == 0;                                  // column 0 among the outputs
-    const int y0 = chunk * k.rows;
-    const int y1 = min(y0 + k.rows, k.H);
-
-    const unsigned bytes = 18u * (unsigned)k.Q * 4u;
-    const rsrc_t src = make_rsrc(b.src, bytes);
-    const rsrc_t dst = make_rsrc(b.dst, bytes);
-    const PullOff po = pull_offsets(k, ln.x);
-    __shared__ float fring_all[WPB * kRingRegion];
-    float* const fring = fring_all + wave * kRingRegion + 1;
-
-    // Even chunks march up (d = 1), odd chunks down (d = -1).  Stage A's
-    // rows beyond the chunk (two on either side) are read by both chunks
-    // beside a boundary; with alternating directions both read them at the
-    // same time (both first or both last), so the second read hits the L2.
-    const int d = (chunk & 1) ? -1 : 1;
-    const int ys = d > 0 ? y0 - 2 : y1 + 1;   // stage A's first row
-    const int yf = d > 0 ? y0 : y1 - 1;       // stage B's first row
-
-    // ---- stage A prologue: psi_n+1 of rows ys-d, ys and g of row ys
-    float gc[9];
-    PsiRow pb, pc;
-    {
-        const int yb = ys - d;
-        const unsigned fb = flags_of(k, b, ln, yb);
-        const bool on = g_on(k, ln, yb, fb);
-        pull(src, k, 9, rows_of(k, wrap(yb, k.H)), po, fb & kLinks, on, gc);
-        pb = lane_row(finish_g(k, ln, yb, fb, on, gc));
-    }
-    unsigned flc = flags_of(k, b, ln, ys);
-    {
-        const bool on = g_on(k, ln, ys, flc);
-        pull(src, k, 9, rows_of(k, wrap(ys, k.H)), po, flc & kLinks, on, gc);
-        pc = lane_row(finish_g(k, ln, ys, flc, on, gc));
-    }
-    unsigned fla = flags_of(k, b, ln, ys + d);
-
-    // ---- the hand-over: A's post-collision f of rows r, r-d, r-2d, r-3d
-    // in the LDS ring (slot row & 3); its g of rows r (Ga), r-d (Gb), r-2d
-    // (Gc: only the three directions pulled from two rows back are read) in
-    // registers; A's flags of rows r, r-d, r-2d; A's side values P of the
-    // same rows
-    float Ga[9], Gb[9], Gc[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Ga[i] = Gb[i] = Gc[i] = 0.f;
-    unsigned fr0 = kSolid, fr1 = kSolid, fr2 = kSolid;
-    float pxa = 0.f, pya = 0.f, pxb = 0.f, pyb = 0.f, pxc = 0.f, pyc = 0.f;
-    // ---- stage B state: psi_n+2 of rows y-d (qs), y (qc); g of row y (gq);
-    // inlet density of the row behind (walled inlet corners)
-    PsiRow qs{}, qc{};
-    float gq[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) gq[i] = 0.f;
-    float rho_prev = 0.f;
-
-    const int nj = (y1 - y0) + 4;
-    for (int j = 0; j < nj; ++j) {
-        const int r = ys + j * d;    // stage A row
-        const bool arow = !(k.y_walls && (r < 0 || r >= k.H));
-        const int rw = wrap(r, k.H);
-        // ---------------- stage A, row r
-        float Gn[9], pxn = 0.f, pyn = 0.f;
-        {
-            const int ya = r + d;
-            const unsigned fl2 = flags_of(k, b, ln, ya + d);
-            float ga[9], f[9];
-            const bool ga_on = g_on(k, ln, ya, fla);
-            pull(src, k, 9, rows_of(k, wrap(ya, k.H)), po, fla & kLinks, ga_on, ga);
-            const bool f_on = arow && ln.inside && !((flc & kSolid) && k.inert);
-            pull(src, k, 0, rows_of(k, rw), po, flc & kLinks, f_on, f);
-            const PsiRow pa = lane_row(finish_g(k, ln, ya, fla, ga_on, ga));
-            const PsiRow pn = d > 0 ? pa : pb;  // row r + 1
-            const PsiRow ps = d > 0 ? pb : pa;  // row r - 1
-            const float nb9[9] = {pc.c, pc.r, pn.c, pc.l, ps.c, pn.r, pn.l, ps.l, ps.r};
-            float dpx, dpy, lap;
-            fdn::stencil(nb9, dpx, dpy, lap);
-            if (arow) bc_f(k, b, src, rw, (int)ln.x, f);
-#pragma unroll
-            for (int i = 0; i < 9; ++i) Gn[i] = gc[i];
-            const bool solid = !arow || !ln.inside || (flc & kSolid) != 0;
-            const float mu = collide_node(k, f, Gn, pc.c, dpx, dpy, lap, solid);
-            float* const slot = fring + (r & 3) * kRingSlot + lane;
-#pragma unroll
-            for (int i = 0; i < 9; ++i) slot[i * 64] = f[i];
-            // P = d psi * mu of this row's psi at the Zou-He columns (the
-            // value the next iteration's Zou-He reads)
-            pxn = dpx * mu;
-            pyn = dpy * mu;
-            pb = pc;
-            pc = pa;
-#pragma unroll
-            for (int i = 0; i < 9; ++i) gc[i] = ga[i];
-            fr2 = fr1;
-            fr1 = fr0;
-            fr0 = arow && ln.inside ? flc : kSolid;
-            flc = fla;
-            fla = fl2;
-        }
-        // ---------------- hand-over
-#pragma unroll
-        for (int i = 0; i < 9; ++i) {
-            Gc[i] = Gb[i];
-            Gb[i] = Ga[i];
-            Ga[i] = Gn[i];
-        }
-        pxc = pxb;
-        pyc = pyb;
-        pxb = pxa;
-        pyb = pya;
-        pxa = pxn;
-        pya = pyn;
-        if (j < 2) continue;
-        // ---------------- stage B: psi_n+2 and g of row r-d
-        PsiRow qn;
-        float gn[9];
-        {
-            const int yq = r - d;
-            const bool on = ln.inside && !(k.y_walls && (yq < 0 || yq >= k.H)) && !((fr1 & kSolid) && k.inert);
-            float lo[9], hi[9];  // A's rows yq - 1 and yq + 1
-#pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                lo[i] = d > 0 ? Gc[i] : Ga[i];
-                hi[i] = d > 0 ? Ga[i] : Gc[i];
-            }
-            reg_pull(lo, Gb, hi, fr1 & kLinks, gn);
-            qn = lane_row(finish_g(k, ln, yq, fr1, on, gn));
-        }
-        // walled inlet corners need the inlet density of the adjacent row:
-        // the row behind stage B's first row is one it has not marched
-        if (j == 3 && has_in && k.y_walls && yf - d >= 0 && yf - d < k.H)
-            rho_prev = ring_inlet_rho(fring, (yf - d) & 3, lane, fr2 & kLinks, b.uprof[yf - d], pxc);
-        if (j >= 4) {
-            // ------------ stage B: collision of row y = r-2d
-            const int y = r - 2 * d;
-            const unsigned fl = fr2;
-            const bool solid = (fl & kSolid) != 0;
-            float f[9];
-            lds_pull(fring, y & 3, lane, fl & kLinks, f);
-            float rho_nb = rho_prev;
-            if (has_in) {
-                // the corner met first (row 0 marching up, H-1 marching
-                // down) takes its neighbour row (ahead) from the ring
-                if (k.y_walls && y == (d > 0 ? 0 : k.H - 1))
-                    rho_nb = ring_inlet_rho(fring, (y + d) & 3, lane, fr1 & kLinks, b.uprof[y + d], pxb);
-                rho_prev = fdn::inlet_rho(f, b.uprof[y], pxc);
-            }
-            const PsiRow qa = d > 0 ? qn : qs;  // row y + 1
-            const PsiRow qb = d > 0 ? qs : qn;  // row y - 1
-            const float nb9[9] = {qc.c, qc.r, qa.c, qc.l, qb.c, qa.r, qa.l, qb.l, qb.r};
-            float dpx, dpy, lap;
-            fdn::stencil(nb9, dpx, dpy, lap);
-            reg_bc_f(k, y, (int)ln.x, f, b.uprof[y], pxc, pyc, rho_nb);
-            float g[9];
-#pragma unroll
-            for (int i = 0; i < 9; ++i) g[i] = gq[i];
-            const float mu = collide_node(k, f, g, qc.c, dpx, dpy, lap, solid || !ln.inside);
-            if (bout && zx && (ln.x == 0 || ln.x == (unsigned)k.W - 1)) {
-                const int sd = (ln.x == 0) ? 0 : 2;
-                b.side_out[sd * k.H + y] = dpx * mu;
-                b.side_out[(sd + 1) * k.H + y] = dpy * mu;
-            }
-            const unsigned vo = (bout && !(fl & kDeadPiece)) ? ln.x * 4u : kOOB;
-            const int rc = y * k.Wp;
-#pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, f[i]), dst, vo, (rc + i * k.Q) * 4,
-                                                      0);
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, g[i]), dst, vo,
-                                                      (rc + (9 + i) * k.Q) * 4, 0);
-            }
-        }
-        qs = qc;
-        qc = qn;
-#pragma unroll
-        for (int i = 0; i < 9; ++i) gq[i] = gn[i];
-    }
-}
-
-template <int WPB>
-__global__ __launch_bounds__(64 * WPB) void fused_kernel(KParams k, KBufs b) {
-    fused_march<WPB>(k, b, banded_block());
-}
-
-// ---------------------------------------------------- three-iteration march
-// One launch advances the state by three iterations, S_n -> S_n+3: stage A
-// as above; stage B (two rows behind A) keeps S_n+2 on chip - g in a second
-// register ring, f in a second LDS ring - instead of storing it; stage C
-// (two rows behind B) pulls S_n+2 from them, collides and stores S_n+3.
+// --------------------------------------- march of two or three iterations
+// One launch advances the state by DEPTH iterations, S_n -> S_n+DEPTH, and
+// moves it through HBM once.  Of three: stage A is the single-iteration march,
+// S_n -> S_n+1 and the side values P_n+1; stage B, two rows behind A, pulls
+// S_n+1 - g from a register ring of A's rows, f from an LDS ring - and keeps
+// S_n+2 in rings of its own; stage C, two rows behind B, pulls S_n+2 from them,
+// collides and stores S_n+3.  Of two: stage B stores, C is left out (and the
+// chunk's rows are two fewer either side).
 // Every stage pulls from a column either side, and its psi stencil from one
 // more: six columns either side of an output column.  The 64 lanes hold
 // columns x0 - 8 ... x0 + 55 and stage C's 48 output columns are lanes
@@ -1072,9 +833,11 @@ constexpr int kStage = 2 * kStageLoads * 256;        // floats, with the idle la
 // a piece per lane, nine planes of 12 pieces.
 constexpr int kOutPieces = kFuse3Cols / 4;
 constexpr int kOut = 9 * kFuse3Cols;                // floats
-// LDS floats of a wave: both rings and, in the inner march, the staged rows
-constexpr int kWave3 = std::max((2 * kRingRegion + 3) / 4 * 4, kStage + kOut + 2 * kRingTight + 4);
-static_assert(8 * kWave3 * 4 <= 160 * 1024, "eight waves per CU");
+// LDS floats of a wave: a ring between two stages and, in the inner march,
+// the staged rows
+template <int DEPTH>
+constexpr int kWave = std::max(((DEPTH - 1) * kRingRegion + 3) / 4 * 4, kStage + kOut + (DEPTH - 1) * kRingTight + 4);
+static_assert(8 * kWave<3> * 4 <= 160 * 1024, "eight waves per CU");
 
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
 // 16 bytes a lane from buffer offset voff + soff to LDS bytes lds + 16 lane
@@ -1103,11 +866,12 @@ __device__ __forceinline__ int uniform_wave() {
     return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
-// rings_all: the workgroup's LDS, WPB * kWave3 floats, declared by the
+// rings_all: the workgroup's LDS, WPB * kWave<DEPTH> floats, declared by the
 // kernel (one array whatever copies of the march it holds).
-template <int WPB, bool EDGE>
+template <int WPB, bool EDGE, int DEPTH>
 __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, int y0, int rows, int strip,
                                              float* rings_all) {
+    constexpr int lag = 2 * (DEPTH - 1);   // rows the last stage is behind stage A
     const int lane = threadIdx.x & 63;
     const int wave = uniform_wave();
     const int xc0 = strip * kFuse3Cols;
@@ -1130,7 +894,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
     const rsrc_t src = make_rsrc(b.src, bytes);
     const rsrc_t dst = make_rsrc(b.dst, bytes);
     using Ring = std::conditional_t<EDGE, RingAll, RingTight>;
-    float* const lds = rings_all + wave * kWave3;
+    float* const lds = rings_all + wave * kWave<DEPTH>;
     float* const out = lds + kStage;
     float* const fring = lds + (EDGE ? 1 : kStage + kOut + 1);               // A -> B
     float* const fring2 = fring + (EDGE ? kRingRegion : kRingTight);         // B -> C
@@ -1147,10 +911,9 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
         return lane_row(EDGE && !ln.inside && !ghost_row(y) ? ln.ghost : v);
     };
 
-    // Every chunk marches up: the L2 reuse that alternating directions buy
-    // the two-iteration kernel is worth less here than the direction selects
-    // it costs.
-    const int ys = y0 - 4;   // stage A's first row; stage B's is ys + 2, stage C's ys + 4
+    // Every chunk marches up: the L2 reuse that alternating directions buy is
+    // worth less than the direction selects cost.
+    const int ys = y0 - lag;   // stage A's first row; stage B's is ys + 2, stage C's ys + 4
 
     // Row y of every per-row value below lives in slot (y - ys) & 3 of its
     // ring, in registers and in LDS, and the march is unrolled over the four
@@ -1289,6 +1052,14 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
         sy = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sin, side, yw + k.H * 4, 0));
     };
 
+    // the last stage's side values, for the next launch's Zou-He
+    auto store_sides = [&](int y, float px, float py) {
+        if (!EDGE || !zx) return;
+        const unsigned so = cout && (zh.lane_in || zh.lane_out) ? side : kOOB;
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, px), sout, so, y * 4, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, py), sout, so, (y + k.H) * 4, 0);
+    };
+
     // ---- prologue: the state's rows of the first step, psi_n+1 of rows ys -
     // 1, ys and g of row ys.  Flags are loaded three rows ahead, of use two.
     {
@@ -1311,7 +1082,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
         stage_read(RG[2], RF[1]);
     }
 
-    const int nj = (y1 - y0) + 8;
+    const int nj = (y1 - y0) + 2 * lag;
     auto step = [&](auto phase, const int j) __attribute__((always_inline)) {
         constexpr int p0 = decltype(phase)::value, p1 = (p0 + 1) & 3, p2 = (p0 + 2) & 3, p3 = (p0 + 3) & 3;
         const int r = ys + j;    // stage A row, slot p0
@@ -1363,9 +1134,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
             if (j >= 4) {
                 // -------- stage B: collision of row y = r - 2 into the rings
                 const int y = r - 2;
-                float f[9];
-#pragma unroll
-                for (int i = 0; i < 9; ++i) f[i] = fb_n[i];
+                float (&f)[9] = fb_n;
                 const PsiRow qn = PB[p3], qc = PB[p2], qs = PB[p1];
                 const float nb9[9] = {qc.c, qc.r, qn.c, qc.l, qs.c, qn.r, qn.l, qs.l, qs.r};
                 float dpx, dpy, lap;
@@ -1380,17 +1149,27 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
                     zou_he_f(k, zh, wrap(y, k.H), f, up3, PX[p2], PY[p2], rho_nb);
                 }
                 const float mu = collide_node(k, f, H[p2], qc.c, dpx, dpy, lap, (fr2 & kSolid) != 0);
-                float* const slot = fring2 + lane;
+                if (DEPTH == 3) {
+                    float* const slot = fring2 + lane;
 #pragma unroll
-                for (int i = 0; i < 9; ++i) slot[Ring::at(i, p2)] = f[i];
-                QX[p2] = dpx * mu;
-                QY[p2] = dpy * mu;
+                    for (int i = 0; i < 9; ++i) slot[Ring::at(i, p2)] = f[i];
+                    QX[p2] = dpx * mu;
+                    QY[p2] = dpy * mu;
+                } else {
+                    store_sides(y, dpx * mu, dpy * mu);
+                }
             }
-            // B's pull of the next row, r - 1: rows r - 2 .. r are in the ring
-            lds_pull<Ring>(fring, p3, lane, fr1 & kLinks, fb_n);
         }
-        // the state's next row, loaded during stages A and B
+        // the state's next row, loaded during stage A and, of three stages, B
         stage_read(RG[p3], RF[p2]);
+        if (DEPTH == 2 && j >= 4) {
+            const unsigned vo = cout && !(fr2 & kDeadPiece) ? ln.x * 4u : kOOB;
+            store_row(fb_n, vo, (r - 2) * k.Wp);
+            store_row(H[p2], vo, (r - 2) * k.Wp + 9 * k.Q);
+        }
+        // B's pull of the next row, r - 1: rows r - 2 .. r are in the ring
+        if (j >= 2) lds_pull<Ring>(fring, p3, lane, fr1 & kLinks, fb_n);
+        if (DEPTH == 2) return;
         // ---------------- stage C: psi_n+3 and g of row r - 3
         if (j >= 6) {
             reg_pull(H[p0], H[p1], H[p2], fr3 & kLinks, U[p1 & 1]);
@@ -1417,12 +1196,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
                     zou_he_f(k, zh, y, f, up5, QX[p0], QY[p0], rho_nb);
                 }
                 const float mu = collide_node(k, f, g, uc.c, dpx, dpy, lap, (fr4 & kSolid) != 0);
-                if (EDGE && zx) {
-                    const unsigned so = cout && (zh.lane_in || zh.lane_out) ? side : kOOB;
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dpx * mu), sout, so, y * 4, 0);
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dpy * mu), sout, so,
-                                                          (y + k.H) * 4, 0);
-                }
+                store_sides(y, dpx * mu, dpy * mu);
                 const unsigned vo = cout && !(fr4 & kDeadPiece) ? ln.x * 4u : kOOB;
                 store_row(f, vo, y * k.Wp);
                 store_row(g, vo, y * k.Wp + 9 * k.Q);
@@ -1449,7 +1223,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
 // copy of the march without that code.  Strip 0 and the last one or two run
 // the full copy, whose rows take longer, in chunks of fewer rows
 // (fuse3_grid), and start first: a launch ends with its slowest wave.
-template <int WPB>
+template <int WPB, int DEPTH>
 __device__ __forceinline__ void fused3_block(const KParams& k, const KBufs& b, int L, float* rings) {
     const int wave = uniform_wave();
     const bool edge = L < k.blk_e;
@@ -1459,24 +1233,34 @@ __device__ __forceinline__ void fused3_block(const KParams& k, const KBufs& b, i
     const int s = (L - chunk * per) * WPB + wave, y0 = chunk * rows;
     if (s >= n || y0 >= k.H) return;
     if (edge)
-        fused3_march<WPB, true>(k, b, y0, rows, s ? k.nin + s : 0, rings);
+        fused3_march<WPB, true, DEPTH>(k, b, y0, rows, s ? k.nin + s : 0, rings);
     else
-        fused3_march<WPB, false>(k, b, y0, rows, s + 1, rings);
+        fused3_march<WPB, false, DEPTH>(k, b, y0, rows, s + 1, rings);
 }
 
 // Each XCD gets a contiguous band of either kind (blk_e is a multiple of 8).
+template <int WPB, int DEPTH>
+__device__ __forceinline__ void fused_launch(const KParams& k, const KBufs& b, float* rings) {
+    const int blk = blockIdx.x;
+    fused3_block<WPB, DEPTH>(
+        k, b, blk < k.blk_e ? banded(blk, k.blk_e) : k.blk_e + banded(blk - k.blk_e, gridDim.x - k.blk_e), rings);
+}
 template <int WPB>
 __global__ __launch_bounds__(64 * WPB, 2) void fused3_kernel(KParams k, KBufs b) {
-    __shared__ __align__(16) float rings[WPB * kWave3];
-    const int blk = blockIdx.x;
-    fused3_block<WPB>(k, b, blk < k.blk_e ? banded(blk, k.blk_e) : k.blk_e + banded(blk - k.blk_e, gridDim.x - k.blk_e),
-                      rings);
+    __shared__ __align__(16) float rings[WPB * kWave<3>];
+    fused_launch<WPB, 3>(k, b, rings);
+}
+// Two iterations per launch: the same march without stage C.
+template <int WPB>
+__global__ __launch_bounds__(64 * WPB, 2) void fused_kernel(KParams k, KBufs b) {
+    __shared__ __align__(16) float rings[WPB * kWave<2>];
+    fused_launch<WPB, 2>(k, b, rings);
 }
 
 // ---------------------------------------------------- tiles in LDS
 // Several iterations per launch on a tile that lives in LDS, for domains too
 // small to fill the device with marching waves: a march is a serial chain of
-// rows (about 3 us a row of the two-iteration kernel when its waves run
+// rows (about 2 us a row of the three-iteration kernel when its waves run
 // alone), while here every node of a tile is updated at once.
 //
 // A workgroup loads the post-collision populations of its tile of TW x TH
@@ -1771,7 +1555,7 @@ __global__ __launch_bounds__(64 * WPB) void ens_kernel(const EnsDomain* __restri
 // ensemble in one launch: as ens_kernel, over a table laid out for that
 // march.
 template <int WPB, int DEPTH>
-__global__ __launch_bounds__(64 * WPB) void ens_fused_kernel(const EnsDomain* __restrict__ doms, int ndom,
+__global__ __launch_bounds__(64 * WPB, 2) void ens_fused_kernel(const EnsDomain* __restrict__ doms, int ndom,
                                                              int parity) {
     const int L = banded_block();
     int lo = 0, hi = ndom - 1;
@@ -1788,12 +1572,8 @@ __global__ __launch_bounds__(64 * WPB) void ens_fused_kernel(const EnsDomain* __
     b.side_in = e.side[ps];
     b.side_out = e.side[ps ^ 1];
     b.uprof = e.uprof;
-    if (DEPTH == 3) {
-        __shared__ __align__(16) float rings[WPB * kWave3];
-        fused3_block<WPB>(e.k, b, L - e.blk0, rings);
-    }
-    else
-        fused_march<WPB>(e.k, b, L - e.blk0);
+    __shared__ __align__(16) float rings[WPB * kWave<DEPTH>];
+    fused3_block<WPB, DEPTH>(e.k, b, L - e.blk0, rings);
 }
 
 // Zeros on every solid node of an inert-solid handle's population set:
@@ -2075,7 +1855,7 @@ struct fd_handle {
     hipGraphExec_t gexec = nullptr;    // the captured pair
     int gkey[6] = {0, 0, 0, 0, 0, 0};  // its launch configuration
     int fwx = 1;    // fused_kernel: waves per workgroup
-    int frows = 12; // fused_kernel: output rows per wave
+    int frows = 16; // fused_kernel: output rows per wave of inner strips
     int f3wx = 1;   // fused3_kernel: waves per workgroup
     int f3rows = 16; // fused3_kernel: output rows per wave of inner strips
     int f3slots = 2048; // waves of it the device holds
@@ -2275,36 +2055,6 @@ bool geom_fusable(const fd_params& p) {
 
 bool fusable(const fd_handle* h) { return h->fuse >= 2 && geom_fusable(h->p); }
 
-// Workgroups across x and chunks of the two-iteration kernel on a domain of
-// width W and height H with launch shape wx x rows.
-int fused_strip_groups(int W, int wx) { return ((W + kFuseCols - 1) / kFuseCols + wx - 1) / wx; }
-
-int launch_fused(fd_handle* h, const KBufs& b, hipStream_t stream = nullptr, int wx = 0, int rows = 0) {
-    if (wx <= 0) wx = h->fwx;
-    if (rows <= 0) rows = h->frows;
-    KParams k = h->k;
-    k.rows = rows;
-    k.nsb = fused_strip_groups(h->p.W, wx);
-    k.sb0 = 0;
-    const int nchunks = (h->p.H + rows - 1) / rows;
-    const dim3 grid(k.nsb * nchunks), block(64 * wx);
-    if (!stream) stream = h->stream;
-    switch (wx) {
-        case 1: hipLaunchKernelGGL((fused_kernel<1>), grid, block, 0, stream, k, b); break;
-        case 4: hipLaunchKernelGGL((fused_kernel<4>), grid, block, 0, stream, k, b); break;
-        default: hipLaunchKernelGGL((fused_kernel<2>), grid, block, 0, stream, k, b); break;
-    }
-    FD_HIP(hipGetLastError());
-    return FD_OK;
-}
-
-// The fewest rows per wave, at most `most`, with which `strips` strips of H
-// rows make no more than `waves` waves.
-int rows_for(int strips, int H, int64_t waves, int most) {
-    const int64_t chunks = std::max<int64_t>(1, waves / strips);
-    return (int)std::min<int64_t>(most, (H + chunks - 1) / chunks);
-}
-
 // Waves of the three-iteration kernel the device holds at once (one-wave
 // workgroups): the quantum of its launch rounds.
 int fused3_slots(int dev, const hipDeviceProp_t& prop, int* slots) {
@@ -2363,6 +2113,25 @@ int launch_fused3(fd_handle* h, const KBufs& b, hipStream_t stream = nullptr) {
         hipLaunchKernelGGL((fused3_kernel<2>), grid, block, 0, stream, k, b);
     else
         hipLaunchKernelGGL((fused3_kernel<1>), grid, block, 0, stream, k, b);
+    FD_HIP(hipGetLastError());
+    return FD_OK;
+}
+
+// One launch of the two-iteration kernel.  As a march of its own, of 58
+// columns, one-row-ahead loads and alternating directions, it took 174 us per
+// iteration on 4096 x 2048 at its best height (158 now, at 90 rows), 49 on
+// 2048 x 1024 (40.8), 23.4 on 1024 x 1024 (18.0).
+int launch_fused(fd_handle* h, const KBufs& b, hipStream_t stream = nullptr, int wx = 0, int rows = 0) {
+    if (wx <= 0) wx = h->fwx;
+    if (rows <= 0) rows = h->frows;
+    KParams k = h->k;
+    if (!stream) stream = h->stream;
+    const int grid = fuse3_grid(k, rows, wx == 1 || wx == 4 ? wx : 2, 8);
+    switch (wx) {
+        case 1: hipLaunchKernelGGL((fused_kernel<1>), dim3(grid), dim3(64), 0, stream, k, b); break;
+        case 4: hipLaunchKernelGGL((fused_kernel<4>), dim3(grid), dim3(256), 0, stream, k, b); break;
+        default: hipLaunchKernelGGL((fused_kernel<2>), dim3(grid), dim3(128), 0, stream, k, b); break;
+    }
     FD_HIP(hipGetLastError());
     return FD_OK;
 }
@@ -2636,30 +2405,25 @@ int fd_create(const fd_params* p, const uint8_t* solid, const uint8_t* links, fd
     std::vector<uint16_t> fl;
     h->inert = pack_flags(*p, solid, links, h->Wp, fl);
     fill_kparams(h);
-    // Launch shapes.  The device holds 4096 waves of the one-iteration
-    // kernel, 3072 of the two-iteration and 2048 of the three-iteration one
-    // at once (its rounds); fd_set_tile / fd_set_fusion override them.
+    // Launch shapes.  The device holds 4096 waves of the one-iteration kernel
+    // and 2048 of the two- and three-iteration ones at once (its rounds);
+    // fd_set_tile / fd_set_fusion override them.
     {
         const int64_t strips64 = (p->W + 63) / 64;
         h->wx = strips64 >= 16 ? 4 : 1;
         h->rows = (int)std::min<int64_t>(16, std::max<int64_t>(1, (strips64 * p->H + 4096) / 8192));
         h->fwx = 1;
-        // Two iterations per launch: the fewest rows (at most 8) that make one
-        // round.  Us per iteration at one round and at other heights: 1400 x
-        // 700 22.2 at 6 rows (29.7 at 2, 23.3 at 8), 1024 x 512 16.3 at 4 (18.6
-        // at 3, 17.7 at 6), 600 x 300 10.1 at 2 (13.5 at 1, 12.3 at 4).
-        const int slots2 = 12 * prop.multiProcessorCount;
-        h->frows = rows_for((p->W + kFuseCols - 1) / kFuseCols, p->H, slots2, 8);
         int slots = 0;
         if ((rc = fused3_slots(dev, prop, &slots))) {
             delete h;
             return rc;
         }
         // Three iterations per launch wherever the geometry allows it and no
-        // tiles are used: 1400 x 700 14.6 us per iteration against 20.3 with
-        // two, 1024 x 512 11.6 against 15.0.
+        // tiles are used, with the same rows as two (remainders): 1400 x 700
+        // 15.8 us per iteration against 16.9 with two, 2048 x 1024 29.5 against
+        // 40.8, 4096 x 2048 105 against 158.
         h->f3slots = slots;
-        h->f3rows = fuse3_rows(h->k, p->H, slots);
+        h->frows = h->f3rows = fuse3_rows(h->k, p->H, slots);
         if (geom_fusable(*p)) h->fuse = 3;
         h->tile = h->auto_tile = tile_for(p->H, p->W, prop.multiProcessorCount, geom_fusable(*p));
     }
@@ -3314,8 +3078,8 @@ struct fd_ensemble {
     EnsDomain* ftable[4] = {nullptr, nullptr, nullptr, nullptr};  // [2], [3]: that many iterations
     int nblocks = 0, fnblocks[4] = {0, 0, 0, 0}, fdepth = 0;
     int wx = 4, rows = 16;           // single-iteration launch shape
-    int fuse = 3, fwx = 1, frows = 8;  // iterations per launch, two-iteration launch shape
-    int f3wx = 1, f3rows = 0;        // three-iteration launch shape (0 rows: ens_rows3)
+    int fuse = 3, fwx = 1, frows = 0;  // iterations per launch, two-iteration launch shape (0 rows: ens_rows)
+    int f3wx = 1, f3rows = 0;        // three-iteration launch shape (0 rows: ens_rows)
     bool table_ok = false;
     int64_t flips = 0;               // launches since the table was built
     bool use_graph = true;
@@ -3336,7 +3100,7 @@ int ens_depth(const fd_ensemble* e) {
     return e->fuse;
 }
 
-// Rows per wave of the three-iteration batch unless set: the fewest that make
+// Rows per wave of the two- and three-iteration batches unless set: the fewest that make
 // one round of the device's waves up to 64 rows, or two rounds up to 32, or
 // 32 (domains of different heights: a tall chunk that starts late ends the
 // launch).  Us per iteration at the rule's height and others: 4 domains (0.57
@@ -3344,8 +3108,8 @@ int ens_depth(const fd_ensemble* e) {
 // 40, 53.5 at 20 (two rounds), 61 at 10; 24 (4.6 M) 69 at 56, 72 at 28, 88 at
 // 10; 8 flows of 2048 x 256 56.8 at 52, 64 at 24; 64 domains (13.6 M) 195 at
 // 32, 203 at 20, 206 at 64; 48 flows 334 at 32, 356 at 20.
-int ens_rows3(const fd_ensemble* e) {
-    if (e->f3rows > 0) return e->f3rows;
+int ens_rows(const fd_ensemble* e, int set) {
+    if (set > 0) return set;
     for (int q = 1, most = 64; q <= 2; ++q, most = 32)
         for (int rows = 4; rows <= most; ++rows) {
             int64_t waves = 0;
@@ -3366,7 +3130,7 @@ int ens_build(fd_ensemble* e) {
         }
     std::vector<EnsDomain> t(e->hs.size()), ft[4];
     int64_t blk = 0, fblk[4] = {0, 0, 0, 0};
-    const int depth = ens_depth(e), rows3 = ens_rows3(e);
+    const int depth = ens_depth(e), rows3 = ens_rows(e, e->f3rows), rows2 = ens_rows(e, e->frows);
     // three iterations per launch leave remainders of two
     for (int d = 2; d <= depth; ++d) ft[d].resize(e->hs.size());
     for (size_t i = 0; i < e->hs.size(); ++i) {
@@ -3391,15 +3155,8 @@ int ens_build(fd_ensemble* e) {
         for (int it = 2; it <= depth; ++it) {
             EnsDomain& fd = ft[it][i];
             fd = d;
-            const int frows = it == 3 ? rows3 : e->frows;
-            fd.k.rows = frows;
             fd.blk0 = (int)fblk[it];
-            if (it == 3) {
-                fblk[3] += fuse3_grid(fd.k, rows3, e->f3wx, 1);
-            } else {
-                fd.k.nsb = fused_strip_groups(h->p.W, e->fwx);
-                fblk[2] += (int64_t)fd.k.nsb * ((h->p.H + frows - 1) / frows);
-            }
+            fblk[it] += it == 3 ? fuse3_grid(fd.k, rows3, e->f3wx, 1) : fuse3_grid(fd.k, rows2, e->fwx, 1);
         }
     }
     if (blk >= ((int64_t)1 << 31) || fblk[2] >= ((int64_t)1 << 31) || fblk[3] >= ((int64_t)1 << 31))
@@ -3512,12 +3269,12 @@ int ens_step(fd_ensemble* e, int32_t nsteps, bool sequential) {
                     if (it == 3) {
                         const int wx3 = h->f3wx, rows3 = h->f3rows;
                         h->f3wx = e->f3wx;
-                        h->f3rows = ens_rows3(e);
+                        h->f3rows = ens_rows(e, e->f3rows);
                         rc = launch_fused3(h, b, e->stream);
                         h->f3wx = wx3;
                         h->f3rows = rows3;
                     } else if (it == 2) {
-                        rc = launch_fused(h, b, e->stream, e->fwx, e->frows);
+                        rc = launch_fused(h, b, e->stream, e->fwx, ens_rows(e, e->frows));
                     } else {
                         const int wx = h->wx, rows = h->rows;
                         h->wx = e->wx;
@@ -3651,7 +3408,7 @@ int fd_ens_get_fusion(const fd_ensemble* e, int32_t* depth, int32_t* waves_x, in
     if (!e) return fail(FD_E_ARG, "ensemble is NULL");
     if (depth) *depth = e->fuse;
     if (waves_x) *waves_x = e->fuse == 3 ? e->f3wx : e->fwx;
-    if (rows) *rows = e->fuse == 3 ? ens_rows3(e) : e->frows;
+    if (rows) *rows = ens_rows(e, e->fuse == 3 ? e->f3rows : e->frows);
     return FD_OK;
 }
 

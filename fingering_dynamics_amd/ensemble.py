@@ -37,7 +37,7 @@ from . import _native, geometry, wetting
 from .params import LbmParams, PROFILE_CONST, OUTLET_PRESSURE, Y_WALLS
 
 TILE_CANDIDATES = ((4, 16), (4, 8), (4, 32), (8, 16), (2, 16), (1, 16))
-FUSED_CANDIDATES = ((1, 8), (1, 6), (1, 12), (1, 16), (2, 8), (4, 8))
+FUSED_CANDIDATES = ((1, 8), (1, 12), (1, 16), (1, 24), (1, 40), (2, 16))
 FUSED3_CANDIDATES = ((1, 16), (1, 20), (1, 26), (1, 32), (1, 48), (2, 16))
 
 
@@ -58,7 +58,7 @@ class Ensemble:
         _native.check(self._lib.fd_ens_get_fusion(h, _native.ctypes.byref(d), _native.ctypes.byref(w),
                                                   _native.ctypes.byref(r)))
         self.fusion = (d.value, w.value, r.value)
-        self._shapes = {2: (1, 8), 3: self.fusion[1:]}
+        self._shapes = {2: self.fusion[1:], 3: self.fusion[1:]}
         # the device table points at every member's buffers: a member may not
         # be closed while the ensemble exists (Compute.close raises)
         for c in self.computes:

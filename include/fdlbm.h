@@ -240,7 +240,7 @@ int fd_set_tile(fd_handle* h, int32_t waves_x, int32_t rows);
  * kernel (<= 0 keeps the current one).  Defaults: depth 3, with the fewest
  * rows per wave that make one round of the device's waves, up to 96 (depth 3
  * counts the rows of strips without a Zou-He column or wrap; the others take
- * fewer); depth 2 at 1 wave and at most 8 rows.  Domains with H < 8, and
+ * fewer); depth 2 the same.  Domains with H < 8, and
  * walled domains whose walls are not the edge rows (the rows 1 and H-2 of
  * fingering.py:573), always run depth 1.
  * A domain too small for these kernels (up to 320,000 nodes; up to 700,000
@@ -319,8 +319,7 @@ int fd_ens_set_tile(fd_ensemble* e, int32_t waves_x, int32_t rows);
  * three-iteration kernel, depth 2 pairs with the two-iteration kernel,
  * depth 1 one iteration per launch.  waves_x and rows set that depth's
  * launch shape (<= 0 keeps the current one; defaults 1 x 4 to 64 rows by the
- * ensemble's size for depth 3, 1 x 8 for depth 2; depth 3 takes 1 or 2
- * waves).  A remainder of two iterations runs the two-iteration kernel.  Groups run batched only
+ * ensemble's size; depth 3 takes 1 or 2 waves).  A remainder of two iterations runs the two-iteration kernel.  Groups run batched only
  * when every domain's geometry allows the fused kernels (fd_set_fusion);
  * otherwise every launch is of one iteration.  Results are identical bit
  * for bit in every case.
