@@ -2,14 +2,13 @@
 
 libfdlbm.so     HIP kernels + C ABI for gfx950 (hipcc)
 libfdsurr.so    BF16 MFMA convolutions of the phase-field surrogate (hipcc)
-libfdnode.so    host FP64 build of the per-node arithmetic (g++), loaded only
-                by the CPU tests
+libfdnode.so    host build of the per-node arithmetic (hipcc's clang++, the
+                kernels' FMA contraction), loaded only by the CPU tests
 
 Run ``python -m fingering_dynamics_amd.build`` (or ``__graft_entry__.build()``).
 Every call compiles: a stale library is never reused.
 """
 import os
-import shutil
 import subprocess
 import sys
 
@@ -62,8 +61,8 @@ def build_node_host():
     os.makedirs(LIBDIR, exist_ok=True)
     out = os.path.join(LIBDIR, "libfdnode.so")
     tmp = out + ".tmp"
-    cxx = shutil.which("g++") or "g++"
-    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-I" + CSRC,
+    cxx = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(HIPCC))), "lib", "llvm", "bin", "clang++")
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-mfma", "-ffp-contract=on", "-I" + CSRC,
           os.path.join(CSRC, "node_host.cpp"), "-o", tmp])
     os.replace(tmp, out)
     return out

@@ -384,7 +384,7 @@ __device__ __forceinline__ void finish_node(const KParams& k, const KBufs& b, rs
             fdn::Mom<float> m = fdn::moments(f, pc, dpx, dpy, lap, k.c);
             fdn::Consts<float> cl = k.c;
             if (solid) {
-                m.rho = m.psi = m.mu = m.ux = m.uy = m.p = m.itau = m.fx = m.fy = 0.f;
+                m.rho = m.psi = m.mu3 = m.ux = m.uy = m.p3 = m.itau = m.fx = m.fy = 0.f;
                 cl.inv_tau_g = 0.f;
             }
             fdn::collide(f, g, m, cl);
@@ -782,7 +782,7 @@ __device__ __forceinline__ float collide_node(const KParams& k, float f[9], floa
     const float mu = m.mu;
     fdn::Consts<float> cl = k.c;
     if (solid) {
-        m.rho = m.psi = m.mu = m.ux = m.uy = m.p = m.itau = m.fx = m.fy = 0.f;
+        m.rho = m.psi = m.mu3 = m.ux = m.uy = m.p3 = m.itau = m.fx = m.fy = 0.f;
         cl.inv_tau_g = 0.f;
     }
     fdn::collide(f, g, m, cl);
@@ -1654,6 +1654,7 @@ __global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, InitField
             m.ux = 0.f;
             m.uy = walled_init ? (0.5f * m.fy) / m.rho : 0.f;
             m.p = m.rho * (1.f / 3.f);  // evaluated before mu (both inits)
+            float mu_p = 0.f;
             if (in.ux) {
                 m.mu = fdn::chem_pot(psi, lap, k.c);
                 m.fx = m.mu * dpx + k.c.gx;
@@ -1661,7 +1662,9 @@ __global__ __launch_bounds__(256) void init_kernel(KParams k, KBufs b, InitField
                 m.ux = in.ux[oi];
                 m.uy = in.uy[oi];
                 m.p = m.rho * (1.f / 3.f) + psi * m.mu;
+                mu_p = m.mu;
             }
+            fdn::thirds(m, mu_p);
             m.itau = fdn::inv_tau_mix(m.rho, psi, k.c);
             fdn::equilibria(m, k.c, f, g);
             if (!PRE) fdn::collide(f, g, m, k.c);

@@ -95,8 +95,8 @@ FD_HD T inv_tau_mix(T rho, T psi, const Consts<T>& c) {
     // = 2 M eta / (rho ((1-psi) + M (1+psi))).  The denominator vanishes at
     // psi = -(1+M)/(M-1) (-1.14 for M = 15), which overshoots past -1 near
     // wetting solids reach; with c.psi_visc = 1 the interpolation uses psi
-    // clamped to the pure phases.  With the default huge bound both
-    // comparisons fail and psi passes unchanged.
+    // clamped to the pure phases.  With the default huge bound the clamp
+    // leaves psi as it is.
     // 1/tau = y / (6 M eta + y/2) with y the denominator: one reciprocal, and
     // 0 at the pole.
     const T pv = clampv(psi, c.psi_visc);
@@ -114,11 +114,21 @@ FD_HD T tau_excess(T rho, T psi, const Consts<T>& c) {
     return T(6) * c.M * c.eta_n * rcp(rho * ((T(1) - pv) + c.M * (T(1) + pv)));
 }
 
-// Moments the collision of one node uses.
+// Moments the collision of one node uses.  p3 and mu3 are thirds of the
+// pressure and of mu, each rounded once.
 template <typename T>
 struct Mom {
-    T rho, psi, mu, ux, uy, p, itau, fx, fy;
+    T rho, psi, mu, ux, uy, p, itau, fx, fy, p3, mu3;
 };
+
+// p3 and mu3 of a pressure rho/3 + psi mu_p (mu_p is mu, or 0 where the
+// pressure is evaluated before mu).
+template <typename T>
+FD_HD void thirds(Mom<T>& m, T mu_p) {
+    m.mu3 = m.mu * (T(1) / T(3));
+    const T e = m.psi * (mu_p * (T(1) / T(3)));
+    m.p3 = m.rho * (T(1) / T(9)) + e;
+}
 
 // Moments from the node's post-stream populations (fingering_periodic.py:470-479).
 template <typename T>
@@ -136,6 +146,7 @@ FD_HD Mom<T> moments(const T f[9], T psi, T dpx, T dpy, T lap, const Consts<T>& 
     m.ux = (jx + T(0.5) * m.fx) * ir;
     m.uy = (jy + T(0.5) * m.fy) * ir;
     m.p = m.rho * (T(1) / T(3)) + psi * m.mu;
+    thirds(m, m.mu);
     m.itau = inv_tau_mix(m.rho, psi, c);
     return m;
 }
@@ -171,11 +182,27 @@ FD_HD void equilibria(const Mom<T>& m, const Consts<T>& c, T feq[9], T geq[9]) {
 // shared differences and reciprocals take 75 fewer of them per node than
 // equilibria formed for each pair (350 -> 275): 100 x 400 on tiles 8.0 ->
 // 7.7 us per iteration, 2048 x 1024 45.7 -> 43.9, 24 domains of an ensemble
-// 343 -> 325 per launch of three.  Against the FP64 oracle the error is 0.88
-// of the other form's in the mean over 30 domains (0.55 ... 1.17).
-// The factors 1 - s and s have to add up to 1 exactly or the sum of a node's
-// populations drifts: rest() rounds 1 - s and s is taken back from it, which
-// is exact (for 0 <= s <= 2).
+// 343 -> 325 per launch of three.
+// Conservation.  A collision keeps the sums of f and of g if every rounded
+// constant and product enters the rest population as it enters the others:
+//   - 1 - s and s have to add up to 1: rest() rounds 1 - s and s is taken back
+//     from it, which is exact (for 0 <= s <= 2).  For s < 1/2 (tau > 2) that
+//     puts s on a grid of 2^-24, an error of at most 2^-25; what it multiplies
+//     is f - feq, and with s in full at the price of an addition a population
+//     no error below was smaller;
+//   - the rest population's share of s p is 5 times that of direction 1: of the
+//     same number (p3, a1).  With 5/3 p and 1/3 as constants of their own, one
+//     rounded down and one up, density grew by 3e-8 s a collision.
+// Errors in float over a droplet in shear (96 x 96; M = 1, 5, 20; tau 0.79,
+// 1.5, 5) as parts of those of feq and geq formed for each pair, geometric
+// means: one collision, f 0.94 at the interface and 0.98 elsewhere, g 0.95 and
+// 0.86, sums of f 0.97 and of g 0.92; psi, rho, ux, uy after 50 to 8000
+// iterations 0.36, 0.05, 0.63, 0.53.
+// On the GPU, fields after 50 ... 100 iterations, relative to 64 bits (in
+// parentheses that form, and this one with 5/3 and 1/3 as constants): 320 x 128
+// 6e-7 (2.2e-6, 2.3e-6), 400 x 100 2.4e-7 (3.2e-6, 3.3e-6), 2048 x 1024 6.7e-7
+// (2.6e-6, 1.8e-6), 24 domains 2.7e-7 (1.1e-6, 1.2e-6); the same time within
+// 0.3 % (400 x 100: 0.8).
 template <typename T>
 FD_HD T rest(T s) {
     return T(1) - s;
@@ -208,16 +235,15 @@ FD_HD void collide(T f[9], T g[9], const Mom<T>& m, const Consts<T>& c) {
         const T jx = sr * m.ux + f3 * m.fx, jy = sr * m.uy + f3 * m.fy;
         const T kx = jx + f3 * m.fx, ky = jy + f3 * m.fy;
         // w1 A = p/3;  w0 A_0 = rho - 5/3 p
-        relax(f, om, s * (m.rho - T(5) / T(3) * m.p), s3 * m.p, m.ux * kx, m.uy * ky, m.ux * ky + m.uy * kx, jx,
-              jy);
+        relax(f, om, s * (m.rho - T(5) * m.p3), s * m.p3, m.ux * kx, m.uy * ky, m.ux * ky + m.uy * kx, jx, jy);
     }
     {
         const T om = rest(c.inv_tau_g), t = T(1) - om;
         const T t3 = t * (T(1) / T(3));
-        const T b = c.gamma * m.mu, h = t3 * m.psi;
+        const T a1 = t * (c.gamma * m.mu3), h = t3 * m.psi;
         const T hx = h * m.ux, hy = h * m.uy;
         // w1 B = gamma mu / 3;  w0 B_0 = psi - 5/3 gamma mu
-        relax(g, om, t * (m.psi - T(5) / T(3) * b), t3 * b, m.ux * hx, m.uy * hy, T(2) * (m.ux * hy), hx, hy);
+        relax(g, om, t * m.psi - T(5) * a1, a1, m.ux * hx, m.uy * hy, T(2) * (m.ux * hy), hx, hy);
     }
 }
 

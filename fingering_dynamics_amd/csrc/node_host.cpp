@@ -7,19 +7,46 @@
 #include "lbm_node.h"
 
 namespace {
-fdn::Consts<double> consts_from(const double c[9]) {
-    fdn::Consts<double> k;
-    k.inv_tau_g = c[0];
-    k.eta_n = c[1];
-    k.M = c[2];
-    k.a = c[3];
-    k.kappa = c[4];
-    k.gamma = c[5];
-    k.psi_wall = c[6];
-    k.gx = c[7];
-    k.gy = c[8];
-    k.psi_visc = 1e300;
+template <typename T = double>
+fdn::Consts<T> consts_from(const double c[9]) {
+    fdn::Consts<T> k;
+    k.inv_tau_g = (T)c[0];
+    k.eta_n = (T)c[1];
+    k.M = (T)c[2];
+    k.a = (T)c[3];
+    k.kappa = (T)c[4];
+    k.gamma = (T)c[5];
+    k.psi_wall = (T)c[6];
+    k.gx = (T)c[7];
+    k.gy = (T)c[8];
+    k.psi_visc = sizeof(T) == 4 ? (T)3e38 : (T)1e300;
     return k;
+}
+
+// Collides n nodes (f, g: [n][9]) whose psi is the sum of g; grad: [n][3],
+// the stencil's dx, dy, lap.  With per_population, in the form
+// f - (f - feq)/tau + F.
+template <typename T>
+void collide_nodes(int n, T* f, T* g, const T* grad, const double c[9], bool per_population) {
+    const fdn::Consts<T> k = consts_from<T>(c);
+    for (; n > 0; --n, f += 9, g += 9, grad += 3) {
+        T psi = g[0];
+        for (int i = 1; i < 9; ++i) psi += g[i];
+        const fdn::Mom<T> m = fdn::moments(f, psi, grad[0], grad[1], grad[2], k);
+        if (!per_population) {
+            fdn::collide(f, g, m, k);
+            continue;
+        }
+        T feq[9], geq[9];
+        fdn::equilibria(m, k, feq, geq);
+        for (int i = 0; i < 9; ++i) {
+            const T ex = T(fdn::EX[i]), ey = T(fdn::EY[i]), eu = ex * m.ux + ey * m.uy;
+            const T F = fdn::W9<T>::w(i) * (T(1) - T(0.5) * m.itau) *
+                        ((T(3) * (ex - m.ux) + T(9) * eu * ex) * m.fx + (T(3) * (ey - m.uy) + T(9) * eu * ey) * m.fy);
+            f[i] = f[i] - (f[i] - feq[i]) * m.itau + F;
+            g[i] = g[i] - (g[i] - geq[i]) * k.inv_tau_g;
+        }
+    }
 }
 }  // namespace
 
@@ -45,14 +72,24 @@ void fdn_moments_f64(const double f[9], double psi, double dpx, double dpy, doub
 
 // feq, geq for given moments (same layout as fdn_moments_f64's output).
 void fdn_equilibria_f64(const double mom[9], const double c[9], double feq[9], double geq[9]) {
-    const fdn::Mom<double> m{mom[0], mom[1], mom[2], mom[3], mom[4], mom[5], mom[6], mom[7], mom[8]};
+    const fdn::Mom<double> m{mom[0], mom[1], mom[2], mom[3], mom[4], mom[5],
+                             mom[6], mom[7], mom[8], mom[5] / 3.0, mom[2] / 3.0};
     fdn::equilibria(m, consts_from(c), feq, geq);
 }
 
 // In-place collision of f and g with the given moments.
 void fdn_collide_f64(double f[9], double g[9], const double mom[9], const double c[9]) {
-    const fdn::Mom<double> m{mom[0], mom[1], mom[2], mom[3], mom[4], mom[5], mom[6], mom[7], mom[8]};
+    const fdn::Mom<double> m{mom[0], mom[1], mom[2], mom[3], mom[4], mom[5],
+                             mom[6], mom[7], mom[8], mom[5] / 3.0, mom[2] / 3.0};
     fdn::collide(f, g, m, consts_from(c));
+}
+
+// collide_nodes in single and double precision.
+void fdn_collide_nodes_f32(int n, float* f, float* g, const float* grad, const double c[9], int per_population) {
+    collide_nodes<float>(n, f, g, grad, c, per_population != 0);
+}
+void fdn_collide_nodes_f64(int n, double* f, double* g, const double* grad, const double c[9], int per_population) {
+    collide_nodes<double>(n, f, g, grad, c, per_population != 0);
 }
 
 void fdn_inlet_f64(double f[9], double g[9], double u, double px, double py) {
