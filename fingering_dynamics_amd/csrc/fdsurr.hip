@@ -677,10 +677,13 @@ __device__ __forceinline__ void load_lds(u4v rsrc, unsigned voff, unsigned soff,
                  : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
                  : "memory", "m0");
 }
-// All but the newest N loads of this wave have arrived.
+// All but the newest N loads of this wave have arrived, and every LDS read of
+// it has returned.  The second is for buffers that later loads land in: that
+// the reads' uses come before this point is nothing the compiler has to keep
+// (it does; the wait costs nothing).
 template <int N>
 __device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0)" : : "i"(N) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "i"(N) : "memory");
 }
 // The words of make_rsrc(p, bytes), in scalar registers.
 __device__ __forceinline__ u4v rsrc_words(const void* p, int64_t bytes) {
