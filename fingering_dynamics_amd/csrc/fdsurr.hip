@@ -716,9 +716,8 @@ __global__ __launch_bounds__(512, 2) void conv_wgrad(WgradArgs a) {
     // loads of a row per wave: dy and x in 64-piece parts dealt to the
     // group's waves, the two edge columns on its first wave
     constexpr int PD = RD / 64, PX = RX / 64;
-    constexpr int ND = (PD + WG - 1) / WG, NX = (PX + WG - 1) / WG;
-    static_assert(PD % WG == 0 || WG % PD == 0, "");
-    static_assert(PX % WG == 0 || WG % PX == 0, "");
+    constexpr int ND = PD / WG, NX = PX / WG;
+    static_assert(PD % WG == 0 && PX % WG == 0, "every wave has as many parts");
     constexpr int ROW = RD + RX + (MASK ? RD : 0) + RE;         // pieces of a staged row
     constexpr int TILES = 9 * ACO * ACI;
     constexpr int NB = NS * RS;                                 // row buffers
@@ -762,13 +761,13 @@ __global__ __launch_bounds__(512, 2) void conv_wgrad(WgradArgs a) {
             r1 = min(r0 + a.rows, a.H);
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
-                const int s = ((wt + WG * i) % PD) * 64 + lane, px = s / PO, g = s % PO;
+                const int s = (wt + WG * i) * 64 + lane, px = s / PO, g = s % PO;
                 const int c = co0 + 8 * (2 * granule<GO>(g >> 1, px) + (g & 1));
                 dvo[i] = w0 + px < a.W && c < a.Cout ? (unsigned)(((w0 + px) * a.Cout + c) * 2) : kOOB;
             }
 #pragma unroll
             for (int i = 0; i < NX; ++i) {
-                const int s = ((wt + WG * i) % PX) * 64 + lane, px = s / PI, g = s % PI;
+                const int s = (wt + WG * i) * 64 + lane, px = s / PI, g = s % PI;
                 const int c = ci0 + 8 * (2 * granule<GI>(g >> 1, px) + (g & 1));
                 xvo[i] = w0 + px < a.W && c < a.Cin ? (unsigned)(((w0 + px) * a.Cin + c) * 2) : kOOB;
             }
@@ -783,8 +782,7 @@ __global__ __launch_bounds__(512, 2) void conv_wgrad(WgradArgs a) {
         const unsigned base = lds0 + (unsigned)(slot * ROW * 16);
 #pragma unroll
         for (int i = 0; i < ND; ++i) {
-            if (PD < WG && wt >= PD) break;  // waves without a part of their own
-            const unsigned part = (unsigned)((wt + WG * i) % PD) * 1024u;
+            const unsigned part = (unsigned)(wt + WG * i) * 1024u;
             load_lds(dr, dvo[i], ds, base + part);
             if (MASK)
                 load_lds(rsrc_words((const char*)a.dym + ln * db, drow ? db : 0), dvo[i], ds,
@@ -792,8 +790,7 @@ __global__ __launch_bounds__(512, 2) void conv_wgrad(WgradArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < NX; ++i) {
-            if (PX < WG && wt >= PX) break;
-            load_lds(xr, xvo[i], xs, base + (unsigned)(RD * 16) + (unsigned)((wt + WG * i) % PX) * 1024u);
+            load_lds(xr, xvo[i], xs, base + (unsigned)(RD * 16) + (unsigned)(wt + WG * i) * 1024u);
         }
         // columns w0 - 1 and w0 + 32
         if (wt == 0 && lane < RE) load_lds(xr, evo, xs, base + (unsigned)((ROW - RE) * 16));
@@ -810,11 +807,7 @@ __global__ __launch_bounds__(512, 2) void conv_wgrad(WgradArgs a) {
             wait_loads<(NS - 2) * RS * (LW + 1)>();
             __builtin_amdgcn_wave_barrier();
         } else {
-            // a wave without dy (x) parts has fewer loads in flight
-            if (PD < WG || PX < WG) {
-                constexpr int l0 = (PD >= WG ? ND * (MASK ? 2 : 1) : 0) + (PX >= WG ? NX : 0);
-                wait_loads<(NS - 2) * RS * l0>();
-            } else if (wt == 0) {
+            if (wt == 0) {
                 wait_loads<(NS - 2) * RS * (LW + 1)>();
             } else {
                 wait_loads<(NS - 2) * RS * LW>();
