@@ -3083,6 +3083,7 @@ struct fd_ensemble {
     int wx = 4, rows = 16;           // single-iteration launch shape
     int fuse = 3, fwx = 1, frows = 0;  // iterations per launch, two-iteration launch shape (0 rows: ens_rows)
     int f3wx = 1, f3rows = 0;        // three-iteration launch shape (0 rows: ens_rows)
+    int rows2 = 0, rows3 = 0;        // rows per wave of the tables as built (ens_rows)
     bool table_ok = false;
     int64_t flips = 0;               // launches since the table was built
     bool use_graph = true;
@@ -3133,7 +3134,8 @@ int ens_build(fd_ensemble* e) {
         }
     std::vector<EnsDomain> t(e->hs.size()), ft[4];
     int64_t blk = 0, fblk[4] = {0, 0, 0, 0};
-    const int depth = ens_depth(e), rows3 = ens_rows(e, e->f3rows), rows2 = ens_rows(e, e->frows);
+    const int depth = ens_depth(e), rows3 = e->rows3 = ens_rows(e, e->f3rows),
+              rows2 = e->rows2 = ens_rows(e, e->frows);
     // three iterations per launch leave remainders of two
     for (int d = 2; d <= depth; ++d) ft[d].resize(e->hs.size());
     for (size_t i = 0; i < e->hs.size(); ++i) {
@@ -3272,12 +3274,12 @@ int ens_step(fd_ensemble* e, int32_t nsteps, bool sequential) {
                     if (it == 3) {
                         const int wx3 = h->f3wx, rows3 = h->f3rows;
                         h->f3wx = e->f3wx;
-                        h->f3rows = ens_rows(e, e->f3rows);
+                        h->f3rows = e->rows3;
                         rc = launch_fused3(h, b, e->stream);
                         h->f3wx = wx3;
                         h->f3rows = rows3;
                     } else if (it == 2) {
-                        rc = launch_fused(h, b, e->stream, e->fwx, ens_rows(e, e->frows));
+                        rc = launch_fused(h, b, e->stream, e->fwx, e->rows2);
                     } else {
                         const int wx = h->wx, rows = h->rows;
                         h->wx = e->wx;
