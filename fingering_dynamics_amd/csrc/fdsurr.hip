@@ -1386,32 +1386,32 @@ __global__ __launch_bounds__(256) void net_inputs(const float* __restrict__ psi,
 // (pixels ld floats apart), d = (psi0 + o0) - psi1, x = (v0 + o) - v1:
 //   loss = sum d^2 wf / w + lambda (sum |x|^2 wf / w)
 // net_loss adds in double (a partial sum per workgroup, added in a fixed
-// order by net_loss_sum); net_loss_bwd forms the products in the order of
-// autograd's backward of that expression, so the gradients are its bits.  As
-// some forty tensor operations these were 250 us of a training step at batch
-// 64 (2.1 M pixels); both kernels take 44, bound by reading 126 MB.
+// order by net_loss_sum) and writes d, x0, x1 to res (if given), all that the
+// gradient needs: net_loss_bwd forms its products in the order of autograd's
+// backward of that expression, so the gradients are its bits.At batch 64 (2.1 M
+// pixels) net_loss takes 24 us and net_loss_bwd 10, bound by memory; forming the
+// residuals from the inputs again took 20 and 24, and kept those from changing
+// before the backward pass; as some forty tensor operations 250.
 struct LossArgs {
-    const float *out, *psi0, *psi1, *v0, *v1, *wf, *w;
+    const float *out, *psi0, *psi1, *v0, *v1, *wf;
+    float* res;
     int64_t n;
     int ld;
-    float lambda;
 };
 constexpr int kLossBlocks = 1024;
-
-__device__ __forceinline__ void loss_terms(const LossArgs& a, int64_t i, float& d, float& x0, float& x1) {
-    const float* const o = a.out + i * a.ld;
-    const float2 u = reinterpret_cast<const float2*>(a.v0)[i], v = reinterpret_cast<const float2*>(a.v1)[i];
-    d = (a.psi0[i] + o[0]) - a.psi1[i];
-    x0 = (u.x + o[1]) - v.x;
-    x1 = (u.y + o[2]) - v.y;
-}
 
 __global__ __launch_bounds__(256) void net_loss(LossArgs a, double* __restrict__ part) {
     __shared__ double sh[2][4];
     double p = 0.0, q = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * 256) {
-        float d, x0, x1;
-        loss_terms(a, i, d, x0, x1);
+        const float* const o = a.out + i * a.ld;
+        const float2 u = reinterpret_cast<const float2*>(a.v0)[i], v = reinterpret_cast<const float2*>(a.v1)[i];
+        const float d = (a.psi0[i] + o[0]) - a.psi1[i], x0 = (u.x + o[1]) - v.x, x1 = (u.y + o[2]) - v.y;
+        if (a.res) {
+            a.res[3 * i] = d;
+            a.res[3 * i + 1] = x0;
+            a.res[3 * i + 2] = x1;
+        }
         const float wf = a.wf[i];
         p += (double)(d * d * wf);
         q += (double)((x0 * x0 + x1 * x1) * wf);
@@ -1446,15 +1446,15 @@ __global__ __launch_bounds__(64) void net_loss_sum(const double* __restrict__ pa
     if (threadIdx.x == 0) *loss = (float)p / *w + lambda * ((float)q / *w);
 }
 
-__global__ __launch_bounds__(256) void net_loss_bwd(LossArgs a, const float* __restrict__ g, float* __restrict__ dout) {
+__global__ __launch_bounds__(256) void net_loss_bwd(const float* __restrict__ res, const float* __restrict__ wf,
+                                                    const float* __restrict__ w, float lambda,
+                                                    const float* __restrict__ g, float* __restrict__ dout, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= a.n) return;
-    float d, x0, x1;
-    loss_terms(a, i, d, x0, x1);
-    const float gp = *g / *a.w * a.wf[i], gu = *g * a.lambda / *a.w * a.wf[i];
-    dout[3 * i] = gp * (2.f * d);
-    dout[3 * i + 1] = gu * (2.f * x0);
-    dout[3 * i + 2] = gu * (2.f * x1);
+    if (i >= n) return;
+    const float gp = *g / *w * wf[i], gu = *g * lambda / *w * wf[i];
+    dout[3 * i] = gp * (2.f * res[3 * i]);
+    dout[3 * i + 1] = gu * (2.f * res[3 * i + 1]);
+    dout[3 * i + 2] = gu * (2.f * res[3 * i + 2]);
 }
 
 int check(int N, int H, int W, int Cin, int Cout) {
@@ -1941,23 +1941,15 @@ int fds_unet_fwd(const uint16_t* x, const float* const* w, const float* const* b
     return conv(a, nullptr, 0);
 }
 
-static int loss_args(LossArgs* a, const float* out, int32_t ld, const float* psi0, const float* psi1, const float* v0,
-                     const float* v1, const float* wf, const float* w, float lambda, int64_t n) {
-    if (!out || !psi0 || !psi1 || !v0 || !v1 || !wf || !w) return fail(FDS_E_ARG, "NULL pointer");
-    if (n < 1 || ld < 3 || n > ((int64_t)1 << 38)) return fail(FDS_E_ARG, "bad shape");
-    if (((uintptr_t)v0 | (uintptr_t)v1) & 7) return fail(FDS_E_ARG, "v0 and v1 must be 8-byte aligned");
-    *a = LossArgs{out, psi0, psi1, v0, v1, wf, w, n, ld, lambda};
-    return FDS_OK;
-}
-
 int64_t fds_net_loss_scratch(void) { return 2 * (int64_t)kLossBlocks; }
 
 int fds_net_loss(const float* out, int32_t ld, const float* psi0, const float* psi1, const float* v0, const float* v1,
-                 const float* wf, const float* w, float lambda, double* scratch, float* loss, int64_t n, void* stream) {
-    LossArgs a;
-    const int rc = loss_args(&a, out, ld, psi0, psi1, v0, v1, wf, w, lambda, n);
-    if (rc) return rc;
-    if (!scratch || !loss) return fail(FDS_E_ARG, "NULL pointer");
+                 const float* wf, const float* w, float lambda, double* scratch, float* loss, float* res, int64_t n,
+                 void* stream) {
+    if (!out || !psi0 || !psi1 || !v0 || !v1 || !wf || !w || !scratch || !loss) return fail(FDS_E_ARG, "NULL pointer");
+    if (n < 1 || ld < 3 || n > ((int64_t)1 << 38)) return fail(FDS_E_ARG, "bad shape");
+    if (((uintptr_t)v0 | (uintptr_t)v1) & 7) return fail(FDS_E_ARG, "v0 and v1 must be 8-byte aligned");
+    const LossArgs a{out, psi0, psi1, v0, v1, wf, res, n, ld};
     const int blocks = (int)std::min<int64_t>(kLossBlocks, (n + 255) / 256);
     hipLaunchKernelGGL(net_loss, dim3(blocks), dim3(256), 0, (hipStream_t)stream, a, scratch);
     FDS_HIP(hipGetLastError());
@@ -1966,14 +1958,12 @@ int fds_net_loss(const float* out, int32_t ld, const float* psi0, const float* p
     return FDS_OK;
 }
 
-int fds_net_loss_bwd(const float* out, int32_t ld, const float* psi0, const float* psi1, const float* v0,
-                     const float* v1, const float* wf, const float* w, float lambda, const float* g, float* dout,
+int fds_net_loss_bwd(const float* res, const float* wf, const float* w, float lambda, const float* g, float* dout,
                      int64_t n, void* stream) {
-    LossArgs a;
-    const int rc = loss_args(&a, out, ld, psi0, psi1, v0, v1, wf, w, lambda, n);
-    if (rc) return rc;
-    if (!g || !dout) return fail(FDS_E_ARG, "NULL pointer");
-    hipLaunchKernelGGL(net_loss_bwd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a, g, dout);
+    if (!res || !wf || !w || !g || !dout) return fail(FDS_E_ARG, "NULL pointer");
+    if (n < 1 || n > ((int64_t)1 << 38)) return fail(FDS_E_ARG, "bad shape");
+    hipLaunchKernelGGL(net_loss_bwd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, res, wf, w,
+                       lambda, g, dout, n);
     FDS_HIP(hipGetLastError());
     return FDS_OK;
 }

@@ -500,23 +500,30 @@ def _mse(out, psi0, psi1, v0, v1, wfluid, w):
 
 class _Mse(torch.autograd.Function):
     """_mse on one kernel each way: the same gradient bit for bit, the sums
-    added in double."""
+    added in double.  Like _mse it keeps the residuals, not the tensors they
+    came from, which may change before the backward pass.  They are an output
+    (the second) so that a gradient of the gradient reaches the network."""
 
     @staticmethod
     def forward(ctx, out, psi0, psi1, v0, v1, wfluid, w):
-        ctx.save_for_backward(out, psi0, psi1, v0, v1, wfluid, w)
         ctx.lam = LAMBDA_U
-        return so.net_loss(out, psi0, psi1, v0, v1, wfluid, w, ctx.lam)
+        loss, res = so.net_loss(out, psi0, psi1, v0, v1, wfluid, w, ctx.lam, residuals=ctx.needs_input_grad[0])
+        ctx.save_for_backward(res, wfluid, w)
+        ctx.set_materialize_grads(False)
+        return loss, res
 
     @staticmethod
-    def backward(ctx, g):
-        out, psi0, psi1, v0, v1, wfluid, w = ctx.saved_tensors
+    def backward(ctx, g, dres):
+        res, wfluid, w = ctx.saved_tensors
+        if g is None:
+            return (dres,) + (None,) * 6
         if torch.is_grad_enabled():
             # the gradient is to be differentiated again: tensor operations
             gp, gu = g / w * wfluid, (g * ctx.lam / w * wfluid).unsqueeze(-1)
-            return (torch.cat([(gp * (2.0 * (psi0 + out[..., 0] - psi1))).unsqueeze(-1),
-                               gu * (2.0 * (v0 + out[..., 1:3] - v1))], dim=-1),) + (None,) * 6
-        return (so.net_loss_bwd(out, psi0, psi1, v0, v1, wfluid, w, ctx.lam, g.contiguous()),) + (None,) * 6
+            dout = torch.cat([(gp * (2.0 * res[..., 0])).unsqueeze(-1), gu * (2.0 * res[..., 1:3])], dim=-1)
+        else:
+            dout = so.net_loss_bwd(res, wfluid, w, ctx.lam, g.contiguous())
+        return (dout if dres is None else dout + dres,) + (None,) * 6
 
 
 def _mse_native(out, psi0, psi1, v0, v1, wfluid):
@@ -546,8 +553,8 @@ def loss_fn(model, x, psi0, psi1, v0, v1, wfluid):
     if LOSS_BAND > 0:
         wfluid = wfluid * near_interface(psi0, LOSS_BAND)
     w = wfluid.sum().clamp(min=1.0)
-    mse = _Mse.apply if _mse_native(out, psi0, psi1, v0, v1, wfluid) else _mse
-    loss = mse(out, psi0, psi1, v0, v1, wfluid, w)
+    args = (out, psi0, psi1, v0, v1, wfluid)
+    loss = _Mse.apply(*args, w)[0] if _mse_native(*args) else _mse(*args, w)
     if LAMBDA_V > 0.0:
         # networks whose jumps add too little volume lag in the coupled run
         # (the mass correction scales their smeared increments up instead)

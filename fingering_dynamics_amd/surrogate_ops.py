@@ -32,8 +32,8 @@ EXPORTS = {
     "fds_unet_scratch": (ctypes.c_int64, [_I32] * 3 + [_VP]),
     "fds_unet_fwd": (ctypes.c_int, [_VP] * 5 + [_I32] * 3 + [_VP, _VP]),
     "fds_net_loss_scratch": (ctypes.c_int64, []),
-    "fds_net_loss": (ctypes.c_int, [_VP, _I32] + [_VP] * 6 + [ctypes.c_float, _VP, _VP, ctypes.c_int64, _VP]),
-    "fds_net_loss_bwd": (ctypes.c_int, [_VP, _I32] + [_VP] * 6 + [ctypes.c_float, _VP, _VP, ctypes.c_int64, _VP]),
+    "fds_net_loss": (ctypes.c_int, [_VP, _I32] + [_VP] * 6 + [ctypes.c_float] + [_VP] * 3 + [ctypes.c_int64, _VP]),
+    "fds_net_loss_bwd": (ctypes.c_int, [_VP] * 3 + [ctypes.c_float, _VP, _VP, ctypes.c_int64, _VP]),
     "fds_last_error": (ctypes.c_char_p, []),
 }
 
@@ -344,7 +344,10 @@ def pixel_ld(out):
     return ld if out.stride() == (H * W * ld, W * ld, ld, 1) and ld >= 3 else None
 
 
-def _loss_ptrs(out, psi0, psi1, v0, v1, wf, w):
+def net_loss(out, psi0, psi1, v0, v1, wf, w, lam, residuals=False):
+    """(loss, res): sum(d^2 wf) / w + lam sum(|x|^2 wf) / w with d = psi0 +
+    out[..., 0] - psi1 and x = v0 + out[..., 1:3] - v1, a 0-d float32 tensor,
+    and, if asked for, d and x as [N, H, W, 3] float32 (else None)."""
     ld = pixel_ld(out)
     shape = tuple(out.shape[:3])
     if (ld is None or any(t.dtype != torch.float32 or not t.is_contiguous() for t in (psi0, psi1, v0, v1, wf, w))
@@ -352,25 +355,20 @@ def _loss_ptrs(out, psi0, psi1, v0, v1, wf, w):
             or any(tuple(t.shape) != shape + (2,) for t in (v0, v1))):
         raise ValueError("expected contiguous float32 tensors shaped like the network's output")
     _same_device(out, psi0, psi1, v0, v1, wf, w)
-    return [_p(out), ld] + [_p(t) for t in (psi0, psi1, v0, v1, wf, w)]
-
-
-def net_loss(out, psi0, psi1, v0, v1, wf, w, lam):
-    """sum(d^2 wf) / w + lam sum(|x|^2 wf) / w with d = psi0 + out[..., 0] -
-    psi1 and x = v0 + out[..., 1:3] - v1: a 0-d float32 tensor."""
-    ptrs = _loss_ptrs(out, psi0, psi1, v0, v1, wf, w)
     scratch = torch.empty(load().fds_net_loss_scratch(), dtype=torch.float64, device=out.device)
     loss = torch.empty((), dtype=torch.float32, device=out.device)
-    _check(load().fds_net_loss(*ptrs, lam, _p(scratch), _p(loss), wf.numel(), _stream()))
-    return loss
+    res = torch.empty(tuple(out.shape), dtype=torch.float32, device=out.device) if residuals else None
+    _check(load().fds_net_loss(_p(out), ld, *[_p(t) for t in (psi0, psi1, v0, v1, wf, w)], lam, _p(scratch), _p(loss),
+                               _p(res), wf.numel(), _stream()))
+    return loss, res
 
 
-def net_loss_bwd(out, psi0, psi1, v0, v1, wf, w, lam, g):
+def net_loss_bwd(res, wf, w, lam, g):
     """g times the gradient of net_loss in out, [N, H, W, 3] float32."""
-    ptrs = _loss_ptrs(out, psi0, psi1, v0, v1, wf, w)
-    if g.dtype != torch.float32 or g.numel() != 1:
-        raise ValueError("g must be one float32 value")
-    _same_device(out, g)
-    dout = torch.empty(tuple(out.shape), dtype=torch.float32, device=out.device)
-    _check(load().fds_net_loss_bwd(*ptrs, lam, _p(g), _p(dout), wf.numel(), _stream()))
+    if (any(t.dtype != torch.float32 or not t.is_contiguous() for t in (res, wf, w, g)) or w.numel() != 1
+            or g.numel() != 1 or tuple(res.shape) != (*wf.shape, 3)):
+        raise ValueError("expected contiguous float32 tensors, w and g of one value")
+    _same_device(res, wf, w, g)
+    dout = torch.empty_like(res)
+    _check(load().fds_net_loss_bwd(_p(res), _p(wf), _p(w), lam, _p(g), _p(dout), wf.numel(), _stream()))
     return dout

@@ -129,14 +129,15 @@ int fds_unet_fwd(const uint16_t* x, const float* const* w, const float* const* b
  * floats apart), d = psi0 + o[0] - psi1 and x = v0 + o[1..2] - v1 (v0, v1: two
  * floats a pixel, 8-byte aligned), loss = sum(d^2 wf) / w + lambda sum(|x|^2
  * wf) / w; w: one float.  scratch: fds_net_loss_scratch doubles.
- * Deterministic.  fds_net_loss_bwd: dout (3 floats a pixel) = g (one float)
- * times the gradient of the loss in o, in the order of products of
- * PyTorch's autograd for that expression. */
+ * Deterministic.  res (3 floats a pixel, or NULL): d and x, from which
+ * fds_net_loss_bwd forms dout (3 floats a pixel) = g (one float) times the
+ * gradient of the loss in o, in the order of products of PyTorch's autograd
+ * for that expression. */
 int64_t fds_net_loss_scratch(void);
 int fds_net_loss(const float* out, int32_t ld, const float* psi0, const float* psi1, const float* v0, const float* v1,
-                 const float* wf, const float* w, float lambda, double* scratch, float* loss, int64_t n, void* stream);
-int fds_net_loss_bwd(const float* out, int32_t ld, const float* psi0, const float* psi1, const float* v0,
-                     const float* v1, const float* wf, const float* w, float lambda, const float* g, float* dout,
+                 const float* wf, const float* w, float lambda, double* scratch, float* loss, float* res, int64_t n,
+                 void* stream);
+int fds_net_loss_bwd(const float* res, const float* wf, const float* w, float lambda, const float* g, float* dout,
                      int64_t n, void* stream);
 
 /* Message of the last failed call on this thread. */

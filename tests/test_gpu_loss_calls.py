@@ -1,0 +1,49 @@
+"""Calls that the training loss takes on its kernels as it does as tensor
+operations: with inputs that change between the forward and the backward
+pass."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(seed=0, N=3, H=17, W=5):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    head = rnd(N, H, W, 8).requires_grad_(True)
+    return head, (rnd(N, H, W), rnd(N, H, W), rnd(N, H, W, 2), rnd(N, H, W, 2), rnd(N, H, W).abs())
+
+
+def _both(head, args):
+    """loss_fn on the kernels and as tensor operations, [(loss, output)]"""
+    from fingering_dynamics_amd import surrogate as sg
+    w = args[-1].sum().clamp(min=1.0)
+    out = []
+    for native in (True, False):
+        o = head[..., :3] * 1.0
+        loss = sg.loss_fn(lambda x: o, None, *args) if native else sg._mse(o, *args, w)
+        assert (type(loss.grad_fn).__name__ == "_MseBackward") == native
+        out.append((loss, o))
+    return out
+
+
+@pytest.mark.parametrize("changed", ["psi0", "psi1", "v0", "v1", "output"])
+def test_inputs_change_before_the_backward_pass(changed):
+    grads = []
+    for native in (0, 1):
+        head, args = _case(1)
+        loss, out = _both(head, args)[native]
+        t = out if changed == "output" else args[("psi0", "psi1", "v0", "v1").index(changed)]
+        with torch.no_grad():
+            t.mul_(3.0).add_(1.0)
+        grads.append(torch.autograd.grad(loss, head)[0])
+    assert torch.equal(*grads)
+
+
+def test_a_changed_weight_is_an_error():
+    for native in (0, 1):
+        head, args = _case(2)
+        loss, _ = _both(head, args)[native]
+        args[-1].mul_(2.0)
+        with pytest.raises(RuntimeError, match="inplace"):
+            torch.autograd.grad(loss, head)
