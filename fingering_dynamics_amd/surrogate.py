@@ -517,8 +517,9 @@ class _Mse(torch.autograd.Function):
         res, wfluid, w = ctx.saved_tensors
         if g is None:
             return (dres,) + (None,) * 6
-        if torch.is_grad_enabled():
-            # the gradient is to be differentiated again: tensor operations
+        if torch.is_grad_enabled() or not so.plain(g, grad=True):
+            # a gradient that is to be differentiated again, or a batch of
+            # them: tensor operations
             gp, gu = g / w * wfluid, (g * ctx.lam / w * wfluid).unsqueeze(-1)
             dout = torch.cat([(gp * (2.0 * res[..., 0])).unsqueeze(-1), gu * (2.0 * res[..., 1:3])], dim=-1)
         else:

@@ -1,6 +1,6 @@
 """Calls that the training loss takes on its kernels as it does as tensor
-operations: with inputs that change between the forward and the backward
-pass."""
+operations: a batch of gradients, and inputs that change between the forward
+and the backward pass."""
 import pytest
 import torch
 
@@ -25,6 +25,19 @@ def _both(head, args):
         assert (type(loss.grad_fn).__name__ == "_MseBackward") == native
         out.append((loss, o))
     return out
+
+
+def test_a_batch_of_gradients():
+    head, args = _case()
+    scales = torch.tensor([1.0, -0.37, 2.5], device="cuda")
+    got, want = [torch.autograd.grad(loss, head, scales, is_grads_batched=True, retain_graph=True)[0]
+                 for loss, _ in _both(head, args)]
+    assert got.shape == (3, *head.shape) and torch.equal(got, want)
+    (loss, _), _ = _both(head, args)
+    for k in range(3):
+        assert torch.equal(torch.autograd.grad(loss, head, scales[k], retain_graph=True)[0], got[k])
+    vm = torch.func.vmap(lambda v: torch.autograd.grad(loss, head, v, retain_graph=True)[0])(scales)
+    assert torch.equal(vm, got)
 
 
 @pytest.mark.parametrize("changed", ["psi0", "psi1", "v0", "v1", "output"])
