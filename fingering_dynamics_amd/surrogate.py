@@ -164,16 +164,19 @@ def pool_skip(s):
     return _PoolSkip.apply(s)
 
 
+def _layers(c0, c1, c2, c3):
+    """(name, Cin, Cout) of the network's convolutions for its level widths."""
+    return [("e0a", IN_CH, c0), ("e0b", c0, c0), ("e1a", c0, c1), ("e1b", c1, c1), ("e2a", c1, c2),
+            ("e2b", c2, c2), ("e3a", c2, c3), ("e3b", c3, c3), ("d2a", c3 + c2, c2), ("d2b", c2, c2),
+            ("d1a", c2 + c1, c1), ("d1b", c1, c1), ("d0a", c1 + c0, c0), ("d0b", c0, c0), ("head", c0, 8)]
+
+
 class UNet(torch.nn.Module):
     def __init__(self, channels=CHANNELS, seed=0):
         super().__init__()
         g = torch.Generator().manual_seed(seed)
-        c0, c1, c2, c3 = channels
-        plan = [("e0a", IN_CH, c0), ("e0b", c0, c0), ("e1a", c0, c1), ("e1b", c1, c1), ("e2a", c1, c2),
-                ("e2b", c2, c2), ("e3a", c2, c3), ("e3b", c3, c3), ("d2a", c3 + c2, c2), ("d2b", c2, c2),
-                ("d1a", c2 + c1, c1), ("d1b", c1, c1), ("d0a", c1 + c0, c0), ("d0b", c0, c0), ("head", c0, 8)]
+        plan = _layers(*channels)
         self.names = [p[0] for p in plan]
-        self._plan, self._widths = plan, tuple(channels)
         for name, cin, cout in plan:
             std = math.sqrt(2.0 / (9 * cin)) * (0.1 if name == "head" else 1.0)
             self.register_parameter("w_" + name, torch.nn.Parameter(torch.randn(cout, 3, 3, cin, generator=g) * std))
@@ -184,10 +187,11 @@ class UNet(torch.nn.Module):
         return conv(x, getattr(self, "w_" + name), getattr(self, "b_" + name), relu, out_f32, dy_masked, w16, wt)
 
     def _native(self, x):
-        """The layers' weights and biases if forward(x) can be one native
-        call - no gradient or transformation is asked for (surrogate_ops.plain)
-        and the input and the parameters are laid out as the constructor's -
-        else None."""
+        """The layers' weights and biases and the level widths if forward(x)
+        can be one native call - no gradient or transformation is asked for
+        (surrogate_ops.plain) and the input and the parameters are laid out as
+        the constructor's - else None.  The widths are the parameters', not
+        the constructor's arguments, which a pickled network need not hold."""
         if (x.dim() != 4 or x.dtype != torch.bfloat16 or x.shape[3] != IN_CH or x.shape[1] % 8 or x.shape[2] % 8
                 or not x.numel() or not x.is_contiguous()):
             return None
@@ -198,11 +202,12 @@ class UNet(torch.nn.Module):
         if not so.plain(x, *ws, *bs):
             return None
         f32 = torch.float32
-        for w, b, (_, cin, cout) in zip(ws, bs, self._plan):
+        widths = tuple(w.shape[0] if w.dim() else 0 for w in ws[:8:2])
+        for w, b, (_, cin, cout) in zip(ws, bs, _layers(*widths)):
             if (w.shape != (cout, 3, 3, cin) or w.dtype != f32 or not w.is_contiguous() or b.shape != (cout,)
                     or b.dtype != f32 or not b.is_contiguous() or cout % 8):
                 return None
-        return ws, bs
+        return ws, bs, widths
 
     def forward(self, x):
         """x [N, H, W, 8] bf16 (H, W multiples of 8) -> [N, H, W, 3] fp32:
@@ -212,7 +217,7 @@ class UNet(torch.nn.Module):
             # a prediction: every launch from one native call.  Through the
             # functions below a 128 x 256 sample takes 550 us, of which the
             # GPU works 110
-            return so.unet_fwd(x, *layers, self._widths)[..., :3]
+            return so.unet_fwd(x, *layers)[..., :3]
         # every layer's bf16 weights and flipped weights in one launch
         w16, wt = so.cast_flip([getattr(self, "w_" + n).detach() for n in self.names])
         self._w = dict(zip(self.names, zip(w16, wt)))

@@ -284,3 +284,23 @@ def test_channel_slice_layout_of_the_pooled_skip_gradient():
     assert so.channel_slice_ld(wide.permute(0, 2, 1, 3)) is None
     assert so.channel_slice_ld(wide.float()) is None
     assert so.channel_slice_ld(torch.zeros(2, 4, 6, 12, dtype=torch.bfloat16)) is None   # pixels 12 apart
+
+
+def test_a_network_pickled_without_the_plan_predicts(monkeypatch):
+    """A prediction takes the level widths from the parameters: a network
+    that was pickled whole before it kept them otherwise is still one."""
+    from fingering_dynamics_amd import surrogate_ops as so
+    seen = []
+    monkeypatch.setattr(so, "plain", lambda *ts, **kw: True)
+    monkeypatch.setattr(so, "unet_fwd", lambda x, ws, bs, widths: seen.append((len(ws), len(bs), widths)) or
+                        torch.zeros(*x.shape[:3], 8))
+    model = sg.UNet(channels=(8, 16, 24, 40))
+    kept = ("training", "_parameters", "_buffers", "_modules", "names")
+    for k in [k for k in model.__dict__ if k not in kept and not k.endswith("hooks") and "hooks_" not in k
+              and k != "_non_persistent_buffers_set"]:
+        del model.__dict__[k]
+    with torch.no_grad():
+        y = model(torch.zeros(2, 8, 16, 8, dtype=torch.bfloat16))
+    assert y.shape == (2, 8, 16, 3) and seen == [(15, 15, (8, 16, 24, 40))]
+    model.register_parameter("w_e1a", torch.nn.Parameter(torch.zeros(16, 3, 3, 16)))   # not the chain's shape
+    assert model._native(torch.zeros(2, 8, 16, 8, dtype=torch.bfloat16)) is None
