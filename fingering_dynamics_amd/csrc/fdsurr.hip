@@ -1388,7 +1388,7 @@ __global__ __launch_bounds__(256) void net_inputs(const float* __restrict__ psi,
 // net_loss adds in double (a partial sum per workgroup, added in a fixed
 // order by net_loss_sum) and writes d, x0, x1 to res (if given), all that the
 // gradient needs: net_loss_bwd forms its products in the order of autograd's
-// backward of that expression, so the gradients are its bits.At batch 64 (2.1 M
+// backward of that expression, so the gradients are its bits.  At batch 64 (2.1 M
 // pixels) net_loss takes 24 us and net_loss_bwd 10, bound by memory; forming the
 // residuals from the inputs again took 20 and 24, and kept those from changing
 // before the backward pass; as some forty tensor operations 250.

@@ -298,12 +298,18 @@ class Compute:
     def fields_device(self, out=None):
         """(psi, rho, ux, uy) of the last completed iteration as a float32
         [4][H][W] device tensor, enqueued on the handle's stream
-        (fd_fields_device).  `out` is reused when given."""
+        (fd_fields_device).  `out` is reused when given (a tensor, or four
+        tensors with room for a field each)."""
         import torch
         if out is None:
             with torch.cuda.stream(self.torch_stream()):
                 out = torch.empty((4, self.H, self.W), dtype=torch.float32, device="cuda")
         self._check_dev(out[0])
+        if not isinstance(out, torch.Tensor):
+            # the kernel writes them itself: no copy checks their extent
+            for a in (out[1], out[2], out[3]):
+                if a.untyped_storage().nbytes() - a.storage_offset() * a.element_size() < 4 * self.H * self.W:
+                    raise ValueError("expected room for float32 [H][W] in every output")
         _native.check(self._lib.fd_fields_device(self._h, *[out[i].data_ptr() for i in range(4)]))
         return out
 

@@ -134,3 +134,19 @@ def test_plumbing_wrappers_check_arguments_before_any_launch():
         so.pool_skip_bwd(_bf(2, 4, 4, 16), _bf(2, 8, 8, 20)[..., 2:18], s)
     with pytest.raises(ValueError, match="same GPU device"):
         so.pool_skip_bwd(_bf(2, 4, 4, 16), _bf(2, 8, 8, 32)[..., 8:24], s)
+
+
+def test_field_outputs_need_room_before_the_kernel_writes_them():
+    c = _bare_compute(8, 16)
+    c._check_dev = lambda a: None          # host tensors stand in for device ones
+    f = lambda *s: torch.zeros(s)
+    for k in (1, 2, 3):
+        outs = [f(8, 16) for _ in range(4)]
+        for short in (f(8, 15), f(2, 8, 16).view(-1)[129:], torch.zeros(8, 16, dtype=torch.float16)):
+            outs[k] = short
+            with pytest.raises(ValueError, match="room"):
+                c.fields_device(outs)
+    assert c._lib.calls == []
+    c.fields_device([f(8, 16), f(128), f(2, 8, 16)[1], f(8, 17)])
+    c.fields_device(f(4, 8, 16))
+    assert c._lib.calls == ["fd_fields_device"] * 2
