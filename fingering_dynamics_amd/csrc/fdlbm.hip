@@ -1024,10 +1024,11 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
 #pragma unroll
         for (int q = 0; q < 2; ++q) piece[q] = *reinterpret_cast<const float4*>(out_at + 256 * q);
         asm volatile("" ::: "memory");
-        // A store of more than eight bytes reads its registers after it was issued, and the link masks that
-        // the next phase makes by inline asm are no writes that the compiler's hazard table sees: without
-        // these wait states, with the registers as operands to keep them whole, the last store of a phase
-        // put masks into memory wherever the allocator had reused its registers at once.
+        // A buffer store of more than eight bytes reads its registers after it was issued.  With a constant
+        // scalar offset the compiler puts wait states before the next write to them; with the offset in a
+        // scalar register, as here, it puts none, whatever writes next, and the masks that the next phase
+        // makes reached memory wherever the allocator had reused the registers at once.  Every such store
+        // needs wait states of its own, with the registers as operands to keep them whole.
         const u4v piece0 = __builtin_bit_cast(u4v, piece[0]), piece1 = __builtin_bit_cast(u4v, piece[1]);
         __builtin_amdgcn_raw_buffer_store_b128(piece0, dst, ov[0], row * 4, 0);
         __builtin_amdgcn_raw_buffer_store_b128(piece1, dst, ov[1], row * 4, 0);
@@ -1041,7 +1042,7 @@ __device__ __forceinline__ void fused3_march(const KParams& k, const KBufs& b, i
     const unsigned side = (zh.lane_in ? 0u : 2u) * (unsigned)k.H * 4u;   // of side_in and side_out
     const rsrc_t sin = make_rsrc(b.side_in, 16u * (unsigned)k.H), sout = make_rsrc(b.side_out, 16u * (unsigned)k.H);
     const rsrc_t uprof = make_rsrc(b.uprof, 4u * (unsigned)k.H);
-    // a value of column 0 (lane 6 of strip 0), kept in a scalar register
+    // a value of column 0 (lane kHalo3 of strip 0), kept in a scalar register
     auto of_inlet = [](float v) {
         return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), kHalo3));
     };
@@ -2060,11 +2061,10 @@ bool fusable(const fd_handle* h) { return h->fuse >= 2 && geom_fusable(h->p); }
 
 // Waves of the three-iteration kernel the device holds at once (one-wave
 // workgroups): the quantum of its launch rounds.
-int fused3_slots(int dev, const hipDeviceProp_t& prop, int* slots) {
+int fused3_slots(const hipDeviceProp_t& prop, int* slots) {
     int per_cu = 0;
     FD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&fused3_kernel<1>), 64,
                                                         0));
-    (void)dev;
     *slots = std::max(1, per_cu) * std::max(1, prop.multiProcessorCount);
     return FD_OK;
 }
@@ -2081,7 +2081,7 @@ int fuse3_edge_rows(int rows) { return std::max(4, rows * 5 / 8 - 1); }
 int fuse3_grid(KParams& k, int rows, int wx, int pad) {
     k.rows = rows;
     k.rows_e = fuse3_edge_rows(rows);
-const int last = 64 - kHalo3 + 1;   // an inner strip's lanes end at column W - 2
+    const int last = 64 - kHalo3 + 1;   // an inner strip's lanes end at column W - 2
     k.nin = k.W >= kFuse3Cols + last ? (k.W - last) / kFuse3Cols : 0;
     k.nes = (k.W + kFuse3Cols - 1) / kFuse3Cols - k.nin;
     const int e = (k.nes + wx - 1) / wx * ((k.H + k.rows_e - 1) / k.rows_e);
@@ -2417,7 +2417,7 @@ int fd_create(const fd_params* p, const uint8_t* solid, const uint8_t* links, fd
         h->rows = (int)std::min<int64_t>(16, std::max<int64_t>(1, (strips64 * p->H + 4096) / 8192));
         h->fwx = 1;
         int slots = 0;
-        if ((rc = fused3_slots(dev, prop, &slots))) {
+        if ((rc = fused3_slots(prop, &slots))) {
             delete h;
             return rc;
         }

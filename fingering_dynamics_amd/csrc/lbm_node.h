@@ -179,8 +179,8 @@ FD_HD void equilibria(const Mom<T>& m, const Consts<T>& c, T feq[9], T geq[9]) {
 // py = uy Ky and the cross term ux Ky + uy Kx serve all nine directions; the
 // same for g with H = 3 w1 t psi u in place of both.  The kernels spend most
 // of their time issuing vector instructions; this form and the moments'
-// shared differences and reciprocals take 75 fewer of them per node than
-// equilibria formed for each pair (350 -> 275): 100 x 400 on tiles 8.0 ->
+// shared differences and reciprocals take 74 fewer of them per node than
+// equilibria formed for each pair (350 -> 276): 100 x 400 on tiles 8.0 ->
 // 7.7 us per iteration, 2048 x 1024 45.7 -> 43.9, 24 domains of an ensemble
 // 343 -> 325 per launch of three.
 // Conservation.  A collision keeps the sums of f and of g if every rounded
