@@ -995,7 +995,8 @@ __global__ __launch_bounds__(512, 2) void conv_wgrad(WgradArgs a) {
 }
 
 // The general weight gradient, for operands that conv_wgrad does not
-// take (unaligned, or an image beyond its 31-bit offsets).  Each
+// take (unaligned, or an image beyond its 31-bit offsets) and where it is the
+// faster one (bwd_w_general).  Each
 // 64-pixel step loads dy (64 px x 64 co) and the shifted x (64 px x 64 ci)
 // with 16-byte loads (8 channels of one pixel) and stores them TRANSPOSED
 // in LDS, [channel][pixel] with rows padded to 72 elements, so that every
@@ -1477,7 +1478,11 @@ struct BwdWPlan {
     int bco, bci, wk;
     int ncb, nib;
     int strips, chunks, rows, items, slices;
+    float us;       // what it takes with reduce_slices (below)
 };
+
+// The partial sums of S slices, MB.
+float partial_mb(int64_t S, int Cin, int Cout) { return (float)(S * Cout * (9 * (int64_t)Cin + 1)) * 4e-6f; }
 
 BwdWPlan bwd_w_plan(int N, int H, int W, int Cin, int Cout) {
     BwdWPlan pl{};
@@ -1493,7 +1498,7 @@ BwdWPlan bwd_w_plan(int N, int H, int W, int Cin, int Cout) {
     const int64_t nblk = (int64_t)pl.ncb * pl.nib;
     const int64_t cap = std::max<int64_t>(1, 256 / nblk);
     const int64_t sum = nblk * pl.bco * pl.bci * 5 / 8;  // 65536ths of a step per slice
-    int64_t best = -1;
+    int64_t best = -1, steps = 0;
     for (int c = 1; c <= H && c <= 256; c = c < 4 ? c + 1 : c + c / 2) {
         const int rows = (H + c - 1) / c, chunks = (H + rows - 1) / rows;
         const int64_t items = (int64_t)N * pl.strips * chunks;
@@ -1507,27 +1512,53 @@ BwdWPlan bwd_w_plan(int N, int H, int W, int Cin, int Cout) {
                 pl.rows = rows;
                 pl.items = (int)items;
                 pl.slices = (int)slices;
+                steps = per * (rows + 2);
             }
             if (slices == 1) break;
         }
     }
+    const bool thin = pl.kind >= 4;
+    pl.us = (thin ? 10.f : 14.5f) + (thin ? 0.75f : 1.05f) * (float)steps + 3.6f / 256 * (float)(pl.slices * nblk) +
+            0.26f * partial_mb(pl.slices, Cin, Cout);
     return pl;
 }
 
 // The general kernel's split: pixel slices of whole 64-pixel steps, about
-// 2048 workgroups (1..256 slices), at least 512 pixels each.
+// 2048 workgroups (1..256 slices), at least 64 to 512 pixels each: what takes
+// the least time.
+//
+// Which of the two kernels a layer takes is the smaller of their times, `us`.
+// conv_wgrad reads strips of 32 columns and needs some 14 us before its first
+// step counts, so narrow images and small problems are the general kernel's:
+// 96 -> 96 channels on 67 x 201 x 2 take 79 us there and 159 in conv_wgrad,
+// 64 -> 64 on 64 x 16 x 8 16 and 28, 32 -> 32 on 1 x 64 x 64 10 and 18; on
+// 64 x 64 x 64 64 -> 64 takes 88 and 40.  Both times
+// are fits of 513 measured layers of 256 to 120,000 pixels (19 pairs of
+// channels, 27 sizes; the general kernel at four slice heights each) and
+// within 6 % of them (rms): steps of a workgroup, rounds of workgroups over
+// the CUs, and the bytes of the partial sums.  A narrow image's pixel
+// coordinates advance in a loop, hence the terms with 1 / W.
 struct BwdWGeneral {
     int64_t chunk;
     int S;
+    float us;
 };
 
 BwdWGeneral bwd_w_general(int N, int H, int W, int Cin, int Cout) {
     const int64_t P = (int64_t)N * H * W;
     const int64_t per_slice = (int64_t)((Cout + 63) / 64) * 9 * ((Cin + 63) / 64);
     const int64_t want = std::min<int64_t>(256, std::max<int64_t>(1, (2048 + per_slice - 1) / per_slice));
-    int64_t c = (P + want - 1) / want;
-    c = std::max<int64_t>((c + kStep - 1) / kStep * kStep, 512);
-    return BwdWGeneral{c, (int)((P + c - 1) / c)};
+    const int64_t c0 = ((P + want - 1) / want + kStep - 1) / kStep * kStep;
+    BwdWGeneral best{0, 0, 0.f};
+    for (int64_t least = 64; least <= 512; least *= 2) {
+        const int64_t c = std::max(c0, least), S = (P + c - 1) / c;
+        const float steps = (float)((std::min(c, P) + kStep - 1) / kStep);
+        const float more = std::max(0.f, (float)(S * per_slice) / 256.f - 1.f);   // rounds beyond one
+        const float us = 7.3f + steps * (1.07f + 0.29f * more + (3.4f + 0.84f * more) / (float)W) + 0.97f * more +
+                         0.4f * partial_mb(S, Cin, Cout);
+        if (!best.S || us < best.us) best = BwdWGeneral{c, (int)S, us};
+    }
+    return best;
 }
 
 }  // namespace
@@ -1781,6 +1812,8 @@ int fds_conv3x3_bwd_data(const uint16_t* dy, const uint16_t* wt, const uint16_t*
     return conv_fwd_checked(dy, relu_y, wt, nullptr, dx32, dx16, N, H, W, Cout, Cin, 0, stream);
 }
 
+// The floats of scratch of either kernel: unaligned operands take the general
+// one whatever its time.
 int64_t fds_bwd_weight_scratch(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
     int64_t S = bwd_w_general(N, H, W, Cin, Cout).S;
     if (wgrad_fits(N, H, W, Cin, Cout)) S = std::max<int64_t>(S, bwd_w_plan(N, H, W, Cin, Cout).slices);
@@ -1795,20 +1828,21 @@ int fds_conv3x3_bwd_weight(const uint16_t* x, const uint16_t* dy, const uint16_t
     if (!x || !dy || !dw || !scratch) return fail(FDS_E_ARG, "NULL pointer");
     hipStream_t st = (hipStream_t)stream;
     const int64_t nw = (int64_t)Cout * 9 * Cin;
-    if (wgrad_fits(N, H, W, Cin, Cout) && aligned16(x) && aligned16(dy) && aligned16(relu_y)) {
-        const BwdWPlan pl = bwd_w_plan(N, H, W, Cin, Cout);
-        const WgradArgs a{x, dy, relu_y, scratch, dbias != nullptr, N, H, W, Cin, Cout, pl.strips, pl.chunks, pl.rows,
-                          pl.items, pl.slices, pl.ncb, pl.nib};
-        if (relu_y) launch_wgrad<true>(a, pl, st);
-        else launch_wgrad<false>(a, pl, st);
+    const BwdWGeneral pl = bwd_w_general(N, H, W, Cin, Cout);
+    const bool fits = wgrad_fits(N, H, W, Cin, Cout) && aligned16(x) && aligned16(dy) && aligned16(relu_y);
+    const BwdWPlan pw = fits ? bwd_w_plan(N, H, W, Cin, Cout) : BwdWPlan{};
+    if (fits && pl.us >= 0.98f * pw.us) {
+        const WgradArgs a{x, dy, relu_y, scratch, dbias != nullptr, N, H, W, Cin, Cout, pw.strips, pw.chunks, pw.rows,
+                          pw.items, pw.slices, pw.ncb, pw.nib};
+        if (relu_y) launch_wgrad<true>(a, pw, st);
+        else launch_wgrad<false>(a, pw, st);
         FDS_HIP(hipGetLastError());
         const int64_t n = dbias ? nw + Cout : nw;
         hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, st, scratch, nw + Cout,
-                           pl.slices, n, dw, nw, dbias);
+                           pw.slices, n, dw, nw, dbias);
         FDS_HIP(hipGetLastError());
         return FDS_OK;
     }
-    const BwdWGeneral pl = bwd_w_general(N, H, W, Cin, Cout);
     const int S = pl.S;
     float* bp = dbias ? scratch + (int64_t)S * nw : nullptr;
     const dim3 grid((unsigned)S * (unsigned)(((Cout + 63) / 64) * 9 * ((Cin + 63) / 64)));
