@@ -1611,6 +1611,21 @@ int64_t blocks_of(const ConvArgs& a) {
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
+// Whether images of up to eight columns are conv_fwd's: the staged kernels
+// compute 32 columns of them, conv_fwd only the pixels there are.  Estimates
+// of both, us (Cout outputs of Cin channels; fits of 336 measured layers of 1
+// to 8 columns and 1,000 to 65,536 rows):
+//   48 -> 96   on 67 x 201 x 2   25 here, 51 staged    on 64 x 64 x 2    23, 13
+//   64 -> 64   on 256 x 256 x 1  28, 135               on 64 x 64 x 4    20, 13
+//   128 -> 128 on 256 x 256 x 4  253, 471              on 64 x 256 x 8   140, 126
+bool narrow(int N, int H, int W, int Cin, int Cout, bool mask) {
+    if (W > 8) return false;
+    const double rows = (double)N * ((H + 7) / 8 * 8), cc = (double)Cin * Cout;
+    const double staged = 4. + rows * std::max(cc / (Cin % 32 ? 1.5e6 : 2.3e6), 1. / 3300);
+    const double rate = (Cout >= 64 ? 1.2e7 : (Cout >= 32 ? 1e7 : 2.5e6)) * (mask ? 0.5 : 1.);
+    return std::max(15. + 0.19 * Cin, (double)N * H * W * cc / rate) < 0.9 * staged;
+}
+
 template <bool MASK>
 void launch_fwd(const uint16_t* x, const uint16_t* xm, const uint16_t* w, const float* bias, float* y32, uint16_t* y16,
                 int N, int H, int W, int Cin, int Cout, int relu, hipStream_t st) {
@@ -1621,7 +1636,7 @@ void launch_fwd(const uint16_t* x, const uint16_t* xm, const uint16_t* w, const 
     const bool staged = !(y32 && y16) && (int64_t)H * W * Cin * 2 < kMaxBytes &&
                         (int64_t)H * W * Cout * (y32 ? 4 : 2) < kMaxBytes && (int64_t)Cout * 9 * Cin * 2 < kMaxBytes &&
                         P < ((int64_t)1 << 28) && P * ((Cout + 15) / 16) < ((int64_t)1 << 31) && aligned16(x) && aligned16(xm) && aligned16(w) && aligned16(y32) &&
-                        aligned16(y16);
+                        aligned16(y16) && !narrow(N, H, W, Cin, Cout, MASK);
     if (staged && Cin % 32 == 0) {
         // The block shape, by what was measured at batch 64 on 128 x 256
         // (thin layers) to 32 x 64 (wide ones), us a layer for the shape
