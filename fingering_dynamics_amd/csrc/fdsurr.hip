@@ -1616,14 +1616,16 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // of both, us (Cout outputs of Cin channels; fits of 336 measured layers of 1
 // to 8 columns and 1,000 to 65,536 rows):
 //   48 -> 96   on 67 x 201 x 2   25 here, 51 staged    on 64 x 64 x 2    23, 13
-//   64 -> 64   on 256 x 256 x 1  28, 135               on 64 x 64 x 4    20, 13
+//   64 -> 64   on 256 x 256 x 1  28, 135               on 64 x 64 x 4    28, 12
+//   16 -> 96   on 67 x 201 x 2   18, 24                on 64 x 256 x 8   38, 25
 //   128 -> 128 on 256 x 256 x 4  253, 471              on 64 x 256 x 8   140, 126
 bool narrow(int N, int H, int W, int Cin, int Cout, bool mask) {
     if (W > 8) return false;
     const double rows = (double)N * ((H + 7) / 8 * 8), cc = (double)Cin * Cout;
     const double staged = 4. + rows * std::max(cc / (Cin % 32 ? 1.5e6 : 2.3e6), 1. / 3300);
     const double rate = (Cout >= 64 ? 1.2e7 : (Cout >= 32 ? 1e7 : 2.5e6)) * (mask ? 0.5 : 1.);
-    return std::max(15. + 0.19 * Cin, (double)N * H * W * cc / rate) < 0.9 * staged;
+    const double outputs = (double)N * H * W * Cout;   // few input channels: bound by the stores
+    return std::max(15. + 0.19 * Cin, std::max(outputs * Cin / rate, outputs / 3.3e5)) < 0.9 * staged;
 }
 
 template <bool MASK>
