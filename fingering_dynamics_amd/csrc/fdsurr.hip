@@ -1022,8 +1022,7 @@ constexpr int kLds = kStep + 8;
 
 __global__ __launch_bounds__(256) void conv_bwd_w(const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy,
                                                   const uint16_t* __restrict__ dym, float* __restrict__ part,
-                                                  float* __restrict__ bpart, int N, int H, int W, int Cin, int Cout,
-                                                  int64_t chunk) {
+                                                  int bias, int N, int H, int W, int Cin, int Cout, int64_t chunk) {
     __shared__ __align__(16) uint16_t sdy[2][64][kLds];
     __shared__ __align__(16) uint16_t sx[2][64][kLds];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1049,7 +1048,7 @@ __global__ __launch_bounds__(256) void conv_bwd_w(const uint16_t* __restrict__ x
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
     v4f accb[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
-    const bool with_bias = bpart != nullptr && tap == 0 && ib == 0 && wcol == 0;
+    const bool with_bias = bias && tap == 0 && ib == 0 && wcol == 0;
     const u4v ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};  // eight bf16 1.0
     // Thread t loads channels g8 .. g8 + 7 (g8 = 8 (t & 7)) of pixels
     // pl = t >> 3 and pl + 32 of the step: eight consecutive lanes read one
@@ -1170,6 +1169,7 @@ __global__ __launch_bounds__(256) void conv_bwd_w(const uint16_t* __restrict__ x
         buf ^= 1;
     }
     const int64_t K = 9 * (int64_t)Cin;
+    float* out = part + slice * (Cout * K + Cout);   // a slice: the weights' sums, then the bias's
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1178,7 +1178,7 @@ __global__ __launch_bounds__(256) void conv_bwd_w(const uint16_t* __restrict__ x
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int co = co0 + 32 * wrow + 16 * i + 4 * (lane >> 4) + r;
-                if (co < Cout && ci < Cin) part[((int64_t)slice * Cout + co) * K + tap * Cin + ci] = acc[i][j][r];
+                if (co < Cout && ci < Cin) out[co * K + tap * Cin + ci] = acc[i][j][r];
             }
         }
     if (with_bias && (lane & 15) == 0) {
@@ -1187,7 +1187,7 @@ __global__ __launch_bounds__(256) void conv_bwd_w(const uint16_t* __restrict__ x
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int co = co0 + 32 * wrow + 16 * i + 4 * (lane >> 4) + r;
-                if (co < Cout) bpart[(int64_t)slice * Cout + co] = accb[i][r];
+                if (co < Cout) out[Cout * K + co] = accb[i][r];
             }
     }
 }
@@ -1844,7 +1844,8 @@ int fds_conv3x3_bwd_weight(const uint16_t* x, const uint16_t* dy, const uint16_t
     if (Cout % 8) return fail(FDS_E_ARG, "Cout must be a multiple of 8");
     if (!x || !dy || !dw || !scratch) return fail(FDS_E_ARG, "NULL pointer");
     hipStream_t st = (hipStream_t)stream;
-    const int64_t nw = (int64_t)Cout * 9 * Cin;
+    const int64_t nw = (int64_t)Cout * 9 * Cin, n = dbias ? nw + Cout : nw;
+    int S;
     const BwdWGeneral pl = bwd_w_general(N, H, W, Cin, Cout);
     const bool fits = wgrad_fits(N, H, W, Cin, Cout) && aligned16(x) && aligned16(dy) && aligned16(relu_y);
     const BwdWPlan pw = fits ? bwd_w_plan(N, H, W, Cin, Cout) : BwdWPlan{};
@@ -1853,26 +1854,17 @@ int fds_conv3x3_bwd_weight(const uint16_t* x, const uint16_t* dy, const uint16_t
                           pw.items, pw.slices, pw.ncb, pw.nib};
         if (relu_y) launch_wgrad<true>(a, pw, st);
         else launch_wgrad<false>(a, pw, st);
-        FDS_HIP(hipGetLastError());
-        const int64_t n = dbias ? nw + Cout : nw;
-        hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, st, scratch, nw + Cout,
-                           pw.slices, n, dw, nw, dbias);
-        FDS_HIP(hipGetLastError());
-        return FDS_OK;
+        S = pw.slices;
+    } else {
+        S = pl.S;
+        const dim3 grid((unsigned)S * (unsigned)(((Cout + 63) / 64) * 9 * ((Cin + 63) / 64)));
+        hipLaunchKernelGGL(conv_bwd_w, grid, dim3(256), 0, st, x, dy, relu_y, scratch, dbias != nullptr, N, H, W, Cin,
+                           Cout, pl.chunk);
     }
-    const int S = pl.S;
-    float* bp = dbias ? scratch + (int64_t)S * nw : nullptr;
-    const dim3 grid((unsigned)S * (unsigned)(((Cout + 63) / 64) * 9 * ((Cin + 63) / 64)));
-    hipLaunchKernelGGL(conv_bwd_w, grid, dim3(256), 0, st, x, dy, relu_y, scratch, bp, N, H, W, Cin, Cout, pl.chunk);
     FDS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((nw + 31) / 32)), dim3(256), 0, st, scratch, nw, S, nw, dw, nw,
-                       dbias);
+    hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, st, scratch, nw + Cout, S, n, dw,
+                       nw, dbias);
     FDS_HIP(hipGetLastError());
-    if (dbias) {
-        hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((Cout + 31) / 32)), dim3(256), 0, st, bp, (int64_t)Cout, S,
-                           (int64_t)Cout, dbias, (int64_t)Cout, dbias);
-        FDS_HIP(hipGetLastError());
-    }
     return FDS_OK;
 }
 
