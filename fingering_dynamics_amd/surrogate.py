@@ -39,6 +39,7 @@ the plain LBM runs K + R iterations instead.  Breakthrough is checked after
 every cycle at the probe column.  Every array stays on the device and
 every launch goes to the solver's stream.
 """
+import functools
 import math
 import time
 
@@ -164,11 +165,12 @@ def pool_skip(s):
     return _PoolSkip.apply(s)
 
 
+@functools.lru_cache(maxsize=16)
 def _layers(c0, c1, c2, c3):
     """(name, Cin, Cout) of the network's convolutions for its level widths."""
-    return [("e0a", IN_CH, c0), ("e0b", c0, c0), ("e1a", c0, c1), ("e1b", c1, c1), ("e2a", c1, c2),
+    return (("e0a", IN_CH, c0), ("e0b", c0, c0), ("e1a", c0, c1), ("e1b", c1, c1), ("e2a", c1, c2),
             ("e2b", c2, c2), ("e3a", c2, c3), ("e3b", c3, c3), ("d2a", c3 + c2, c2), ("d2b", c2, c2),
-            ("d1a", c2 + c1, c1), ("d1b", c1, c1), ("d0a", c1 + c0, c0), ("d0b", c0, c0), ("head", c0, 8)]
+            ("d1a", c2 + c1, c1), ("d1b", c1, c1), ("d0a", c1 + c0, c0), ("d0b", c0, c0), ("head", c0, 8))
 
 
 class UNet(torch.nn.Module):
@@ -522,9 +524,10 @@ class _Mse(torch.autograd.Function):
         res, wfluid, w = ctx.saved_tensors
         if g is None:
             return (dres,) + (None,) * 6
-        if torch.is_grad_enabled() or not so.plain(g, grad=True):
+        if (torch.is_grad_enabled() or not so.plain(g, grad=True)
+                or torch._C._functorch.is_legacy_batchedtensor(g)):
             # a gradient that is to be differentiated again, or a batch of
-            # them: tensor operations
+            # them (vmap, is_grads_batched): tensor operations
             gp, gu = g / w * wfluid, (g * ctx.lam / w * wfluid).unsqueeze(-1)
             dout = torch.cat([(gp * (2.0 * res[..., 0])).unsqueeze(-1), gu * (2.0 * res[..., 1:3])], dim=-1)
         else:

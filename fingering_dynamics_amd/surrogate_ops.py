@@ -293,8 +293,7 @@ def plain(*ts, grad=False):
     if not ts[0].is_cuda:
         return False
     dev, kinds, strided = torch.cuda.current_device(), (torch.Tensor, torch.nn.Parameter), torch.strided
-    batched = torch._C._functorch.is_legacy_batchedtensor      # autograd.grad(is_grads_batched=True)
-    return all(type(t) in kinds and t.layout is strided and t.get_device() == dev and not batched(t) for t in ts)
+    return all(type(t) in kinds and t.layout is strided and t.get_device() == dev for t in ts)
 
 
 def net_inputs(psi, ux, uy, solid, lm, th, scale):
