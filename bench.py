@@ -139,8 +139,9 @@ def ensemble_bench(n, steps, warmup):
     """Aggregate MLUPS of n independent domains (the seeded many-domain
     workload of fingering_dynamics_amd.ensemble.domain_spec) advanced by
     graph-replayed batched launches of three iterations each, against one
-    launch per domain per launch step on the same stream, and against
-    batched launches of one iteration.  Prints one JSON line."""
+    launch per domain per launch step on the same stream (at the height
+    fastest for that: a launch of one domain fills a part of the device), and
+    against batched launches of one iteration.  Prints one JSON line."""
     from fingering_dynamics_amd.ensemble import Ensemble, domain_spec, build_domain
     from fingering_dynamics_amd.lbm import Compute
     t0 = time.perf_counter()
@@ -152,11 +153,20 @@ def ensemble_bench(n, steps, warmup):
     ens.synchronize()
     nodes = ens.nodes
     res = {}
-    fusion, depth = ens.fusion, ens.depth
+    fusion, depth, seq_rows = ens.fusion, ens.depth, 0
     for mode in ("graph", "eager", "sequential", "one_iteration_per_launch"):
         k = steps if mode != "sequential" else max(steps // 8, 10)
         k += k & 1
         ens.use_graph(mode != "eager")
+        if mode == "sequential" and depth >= 2:
+            alone = {}
+            for rows in (4, 6, 8, 12, 16, fusion[2]):
+                ens.set_fusion(depth, 1, rows)
+                ens.step_sequential(6)
+                ens.step_sequential(6)
+                alone[rows] = ens.last_step_ms()
+            seq_rows = min(alone, key=alone.get)
+            ens.set_fusion(depth, 1, seq_rows)
         if mode == "one_iteration_per_launch":
             ens.set_fusion(1)
             ens.step(4)
@@ -178,7 +188,7 @@ def ensemble_bench(n, steps, warmup):
         "speedup_vs_sequential": round(res["graph"]["mlups"] / res["sequential"]["mlups"], 2),
         "iterations_per_launch": depth,
         "autotune_ms_per_step": {"%dx%d" % t: round(v, 4) for t, v in tune.items()},
-        "shape": "%dx%d" % fusion[1:], "tile_one_iteration": "%dx%d" % ens.tile, "setup_s": round(setup_s, 1),
+        "shape": "%dx%d" % fusion[1:], "rows_sequential": seq_rows, "tile_one_iteration": "%dx%d" % ens.tile, "setup_s": round(setup_s, 1),
         "domains_non_finite": int(sum(1 for v in bad if v)), "iterations_run": int(cs[0].t),
     }
     ens.close()
