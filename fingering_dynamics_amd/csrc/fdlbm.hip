@@ -809,7 +809,8 @@ __device__ __forceinline__ float collide_node(const KParams& k, float f[9], floa
 //
 // What bounds a launch, 2048 x 1024: its vector instructions, 86 % of the
 // cycles of two waves per SIMD while they are there, and that waves differ by
-// 20 %; 4096 x 2048: its stores.  With all of them to one row it takes 87 us
+// 20 %; 4096 x 2048: its stores and, at the 1.7 to 1.9 GHz the clock falls to,
+// its vector instructions.  With all stores to one row it takes 87 us
 // per iteration instead of 123, and 52 output columns (208 bytes, sectors
 // shared by neighbouring strips), which leave less margin, take 118 instead
 // of 107; 3000 x 1500 68.4 and 59.8, 2048 x 1024 29.4 and 29.5, 1024 x 1024
@@ -2095,7 +2096,7 @@ int fuse3_grid(KParams& k, int rows, int wx, int pad) {
 // save work, and a launch that just exceeds a round pays a whole one more:
 // 2048 x 1024 takes 29.5 us per iteration at 23 rows (one round), 39.3 at 22;
 // 1024 x 1024 17.0 at 13, 23 at 12; 3000 x 1500 59.8 at 51 (one round), 64.9
-// at 26 (two); 4096 x 2048 107 at 94, 110 at 46, 114 at 31.
+// at 26 (two); 4096 x 2048 107 at 94 (105 over long runs), 110 at 46, 114 at 31.
 constexpr int kFuse3Tall = 96;
 
 int fuse3_rows(const KParams& k0, int H, int64_t slots) {
